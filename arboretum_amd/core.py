@@ -356,11 +356,12 @@ class Garden(object):
         _check(_LIB.AGardenGetTreeDepth(self.handle, t, ctypes.byref(d)))
         depth = d.value
         ni, nl = (1 << (depth - 1)) - 1, 1 << (depth - 1)
-        fid, q = np.empty(ni, np.int32), np.empty(ni, np.int32)
-        thr, gain, w = np.empty(ni, np.float32), np.empty(ni, np.float32), np.empty(nl, np.float32)
-        vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)
-        _check(_LIB.AGardenGetTree(self.handle, t, vp(fid), vp(q), vp(thr), vp(gain), vp(w)))
-        return {"fid": fid, "quantized": q, "threshold": thr, "gain": gain, "weights": w}
+        words = np.empty(4 * ni + nl, np.int32)  # the five arrays one after the other
+        at = words.ctypes.data
+        _check(_LIB.AGardenGetTree(self.handle, t, at, at + 4 * ni, at + 8 * ni, at + 12 * ni, at + 16 * ni))
+        floats = words.view(np.float32)
+        return {"fid": words[:ni], "quantized": words[ni:2 * ni], "threshold": floats[2 * ni:3 * ni],
+                "gain": floats[3 * ni:4 * ni], "weights": floats[4 * ni:]}
 
     def leaves(self):
         out = np.empty(self.data.rows, dtype=np.uint32)

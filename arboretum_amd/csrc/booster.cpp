@@ -1,61 +1,16 @@
 #include "booster.h"
 
+#include "parallel.h"
+
 #include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
-#include <exception>
 #include <limits>
 #include <mutex>
 #include <stdexcept>
-#include <thread>
 
 namespace arb {
-
-namespace {
-// Runs the workers on threads of their own (the caller's included) and hands the first
-// exception of any of them back to the caller instead of ending the process.
-void RunWorkers(size_t workers, const std::function<void(size_t)> &work) {
-  std::exception_ptr failed;
-  std::mutex guard;
-  auto run = [&](size_t t) {
-    try {
-      work(t);
-    } catch (...) {
-      std::lock_guard<std::mutex> lock(guard);
-      if (!failed) failed = std::current_exception();
-    }
-  };
-  std::vector<std::thread> th;
-  for (size_t t = 1; t < workers; ++t) th.emplace_back(run, t);
-  run(0);
-  for (auto &t : th) t.join();
-  if (failed) std::rethrow_exception(failed);
-}
-}  // namespace
-
-void ParallelFor(size_t n, const std::function<void(size_t, size_t)> &fn) {
-  unsigned hw = std::thread::hardware_concurrency();
-  size_t nt = std::max<size_t>(1, std::min<size_t>(hw ? hw : 1, 16));
-  if (n < 65536 || nt == 1) {
-    fn(0, n);
-    return;
-  }
-  const size_t chunk = (n + nt - 1) / nt;
-  RunWorkers(nt, [&](size_t t) {
-    const size_t b = t * chunk, e = std::min(n, b + chunk);
-    if (b < e) fn(b, e);
-  });
-}
-
-void ParallelTasks(size_t n, const std::function<void(size_t)> &fn) {
-  const unsigned hw = std::thread::hardware_concurrency();
-  const size_t nt = std::max<size_t>(1, std::min<size_t>({(size_t)(hw ? hw : 1), (size_t)16, n}));
-  std::atomic<size_t> next{0};
-  RunWorkers(nt, [&](size_t) {
-    for (size_t i = next++; i < n; i = next++) fn(i);
-  });
-}
 
 namespace {
 std::atomic<uint64_t> g_next_matrix_uid{1};
@@ -67,6 +22,48 @@ DataMatrix::DataMatrix(size_t rows, size_t columns, size_t columns_category)
 DataMatrix::~DataMatrix() {
   if (device) FreeDeviceMatrix(device);
   if (exact_sort) FreeExactSortData(exact_sort);
+}
+
+void DataMatrix::SetY(const float *v) {
+  y.resize(rows);
+  std::mutex guard;
+  TargetFacts all;
+  ParallelFor(rows, [&](size_t b, size_t e) {
+    TargetFacts f;
+    for (size_t i = b; i < e; ++i) {
+      const float x = v[i];
+      y[i] = x;
+      f.finite = f.finite && std::isfinite(x);
+      f.zero_one = f.zero_one && (x == 0.0f || x == 1.0f);
+      f.least = std::min(f.least, x);
+      f.most = std::max(f.most, x);
+    }
+    std::lock_guard<std::mutex> lock(guard);
+    all.finite = all.finite && f.finite;
+    all.zero_one = all.zero_one && f.zero_one;
+    all.least = std::min(all.least, f.least);
+    all.most = std::max(all.most, f.most);
+  });
+  y_facts = all;
+  std::lock_guard<std::mutex> lock(target_mutex_);
+  device_y_.reset();
+}
+
+void DataMatrix::SetLabels(const unsigned char *v) {
+  labels.assign(v, v + rows);
+  std::lock_guard<std::mutex> lock(target_mutex_);
+  device_labels_.reset();
+}
+
+void DataMatrix::ResetYHat(size_t count, float value) {
+  y_hat_.clear();
+  y_hat_count_ = count;
+  y_hat_start_ = value;
+}
+
+std::vector<float> &DataMatrix::YHat() {
+  if (y_hat_.size() != y_hat_count_) y_hat_.assign(y_hat_count_, y_hat_start_);
+  return y_hat_;
 }
 
 RegTree::RegTree(unsigned depth, unsigned label) : depth(depth), label(label) {
@@ -183,18 +180,11 @@ void Garden::GrowTree(DataMatrix *data, const float *grad) {
     throw std::runtime_error("colsample_bytree is too small");
   if ((int)(cfg.tree.colsample_bytree * cfg.tree.colsample_bylevel * columns) == 0)
     throw std::runtime_error("colsample_bytree and colsample_bylevel are too small");
-  if (!builder_ && cfg.objective < kSoftMaxOneVsAll) {
-    // Gradients are accumulated in fixed point scaled by the largest one; a
-    // target that is NaN or infinite has no scale (the reference would carry
-    // the NaN into every sum it touches).
-    std::atomic<bool> bad{false};
-    ParallelFor(data->rows, [&](size_t b, size_t e) {
-      bool any = false;
-      for (size_t i = b; i < e; ++i) any = any || !std::isfinite(data->y[i]);
-      if (any) bad = true;
-    });
-    if (bad) throw std::runtime_error("y must be finite");
-  }
+  // Gradients are accumulated in fixed point scaled by the largest one; a
+  // target that is NaN or infinite has no scale (the reference would carry
+  // the NaN into every sum it touches).
+  if (!builder_ && cfg.objective < kSoftMaxOneVsAll && !data->y_facts.finite)
+    throw std::runtime_error("y must be finite");
   if (DeviceCount() <= 0) throw std::runtime_error("no HIP device available: training needs an MI355X");
   if (!builder_) {
     // upload_features = false keeps the bins in pinned host memory and streams
@@ -239,14 +229,14 @@ void Garden::Predict(const DataMatrix *data, float *out, int n_rounds) const {
 
 void Garden::UpdateByLastTree(DataMatrix *data) {
   const size_t K = cfg.tree.labels_count;
-  if (data->y_hat.empty()) data->y_hat.assign(data->rows * K, IntoInternal(cfg.tree.initial_y));
+  if (!data->HasYHat()) data->ResetYHat(data->rows * K, IntoInternal(cfg.tree.initial_y));
   if (trees_.size() < K) return;
   SyncTrees();
-  for (size_t t = trees_.size() - K; t < trees_.size(); ++t) trees_[t].Predict(*data, data->y_hat.data());
+  for (size_t t = trees_.size() - K; t < trees_.size(); ++t) trees_[t].Predict(*data, data->YHat().data());
 }
 
-void Garden::GetY(const DataMatrix *data, std::vector<float> *out) const {
-  FromInternal(data->y_hat, out);
+void Garden::GetY(DataMatrix *data, std::vector<float> *out) const {
+  FromInternal(data->YHat(), out);
 }
 
 // src/core/model_helper.cpp:16-23, json_conversion.h:13-40

@@ -8,17 +8,13 @@
 #include <cstdint>
 #include <functional>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "config.h"
 
 namespace arb {
-
-// Runs fn(begin, end) over [0, n) on a few host threads.
-void ParallelFor(size_t n, const std::function<void(size_t, size_t)> &fn);
-// fn(i) for every i in [0, n), a few long tasks (columns) handed out one at a time to up to 16 threads.
-void ParallelTasks(size_t n, const std::function<void(size_t)> &fn);
 
 struct DeviceMatrix;  // quantised bins resident in HBM (device_builder.hip)
 struct ExactSortData;  // ranks and sorted row lists of every feature (exact_builder.hip)
@@ -44,9 +40,26 @@ class DataMatrix {
   std::vector<std::vector<unsigned>> data_categories;
 
   std::vector<float> y;
-  std::vector<float> y_hat;
   std::vector<unsigned char> labels;
   std::vector<float> weights;
+  // What a booster asks of its target, found while the target is copied in.
+  struct TargetFacts {
+    bool finite = true, zero_one = true;
+    float least = 0.0f, most = 1.0f;  // of the targets, 0 and 1
+  } y_facts;
+  void SetY(const float *v);
+  void SetLabels(const unsigned char *v);
+  // Predictions of this matrix that AAppendLastTree advances and AGetY reads (internal scale,
+  // class-major).  ResetYHat only notes the starting value: a training matrix' own is rarely read.
+  void ResetYHat(size_t count, float value);
+  std::vector<float> &YHat();
+  bool HasYHat() const { return y_hat_count_ != 0; }
+
+  // The target in device memory, copied there when the first booster asks and kept with the matrix
+  // like its bins (device_builder.hip); null when it is not set.  The copy is complete when the call
+  // returns, and stays whole for as long as a booster holds it, whatever is set here afterwards.
+  std::shared_ptr<const float> DeviceY();
+  std::shared_ptr<const unsigned char> DeviceLabels();
 
   // Quantiser output (io.h:24, 32): thresholds[f] has hist_size entries,
   // reduced_size[f] real bins.
@@ -74,6 +87,14 @@ class DataMatrix {
     const uint32_t q = stream_blocks[i / stream_block_rows][(f >> 2) * stream_block_rows + i % stream_block_rows];
     return (float)((q >> (8 * (f & 3))) & 255u);
   }
+
+ private:
+  std::vector<float> y_hat_;
+  size_t y_hat_count_ = 0;
+  float y_hat_start_ = 0.0f;
+  std::mutex target_mutex_;  // boosters of several threads may ask at once
+  std::shared_ptr<const float> device_y_;
+  std::shared_ptr<const unsigned char> device_labels_;
 };
 
 // Heap-ordered tree (src/core/reg_tree.h:16-45, garden.h:32-67).
@@ -180,7 +201,7 @@ class Garden {
   // out: rows * labels_count floats
   void Predict(const DataMatrix *data, float *out, int n_rounds) const;  // :643-657
   void UpdateByLastTree(DataMatrix *data);                   // :627-635
-  void GetY(const DataMatrix *data, std::vector<float> *out) const;  // :637-641
+  void GetY(DataMatrix *data, std::vector<float> *out) const;  // :637-641
   const char *GetModel();                                    // :659-665
   void Restore(const char *json_model);                      // :667-677
 

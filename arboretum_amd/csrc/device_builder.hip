@@ -68,6 +68,9 @@
 #include "kernels_quantise.h"
 #include "kernels_split.h"
 #include "kernels_stream.h"
+#include "memory_pool.h"
+#include "parallel.h"
+#include "staging.h"
 
 namespace arb {
 
@@ -120,6 +123,25 @@ void CopyProbe(size_t bytes) {
   HIP_OK(hipFree(dst));
 }
 
+// ---- the target of a matrix in device memory
+template <typename T>
+static std::shared_ptr<const T> OnDevice(const std::vector<T> &v) {
+  // (whoever lets go of it last, a booster or the matrix, has waited for the kernels that read it)
+  std::shared_ptr<T> p(DevAlloc<T>(v.size()), [](T *q) { DevicePoolGive(q); });
+  CopyToDevice(p.get(), v.data(), v.size() * sizeof(T), nullptr);
+  return p;
+}
+std::shared_ptr<const float> DataMatrix::DeviceY() {
+  std::lock_guard<std::mutex> lock(target_mutex_);
+  if (!device_y_ && !y.empty()) device_y_ = OnDevice(y);
+  return device_y_;
+}
+std::shared_ptr<const unsigned char> DataMatrix::DeviceLabels() {
+  std::lock_guard<std::mutex> lock(target_mutex_);
+  if (!device_labels_ && !labels.empty()) device_labels_ = OnDevice(labels);
+  return device_labels_;
+}
+
 int DeviceCount() {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess) return 0;
@@ -128,10 +150,12 @@ int DeviceCount() {
 
 void FreeDeviceMatrix(DeviceMatrix *m) {
   if (!m) return;
-  if (m->bins) (void)hipFree(m->bins);
-  if (m->rec) (void)hipFree(m->rec);
-  if (m->bytes) (void)hipFree(m->bytes);
-  if (m->hibits) (void)hipFree(m->hibits);
+  // what goes back to the pool has no work pending on it
+  if (m->bins || m->rec || m->bytes || m->hibits) (void)hipDeviceSynchronize();
+  DevicePoolGive(m->bins);
+  DevicePoolGive(m->rec);
+  DevicePoolGive(m->bytes);
+  DevicePoolGive(m->hibits);
   if (m->owns_blocks)
     for (uint32_t *b : m->host_blocks)
       if (b) (void)hipHostFree(b);
@@ -297,14 +321,14 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
       dm->bits = 16;
       dm->slots = slots;
       dm->Q = dm->cols = (F + 1) / 2;
-      HIP_OK(hipFree(dm->bins));
+      DevicePoolGive(dm->bins);
       dm->bins = DevAlloc<uint32_t>((size_t)dm->Q * dm->stride);
       uint16_t *d_in = DevAlloc<uint16_t>(n * F);
       HIP_OK(hipMemcpy(d_in, ranks.data(), n * F * sizeof(uint16_t), hipMemcpyHostToDevice));
       hipLaunchKernelGGL(k_pack_prebinned16, dim3(GridFor(n, 256)), dim3(256), 0, 0, d_in, F, dm->Q, dm->bins,
                          dm->stride, n);
       HIP_OK(hipDeviceSynchronize());
-      HIP_OK(hipFree(d_in));
+      DevicePoolGive(d_in);
     }
   }
   if (exact && dm->bits == 16) {
@@ -321,7 +345,7 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
       hipLaunchKernelGGL(k_pack_prebinned, dim3(GridFor(n, 256)), dim3(256), 0, 0, d_in, F, dm->Q,
                          dm->bins, dm->stride, n);
       HIP_OK(hipDeviceSynchronize());
-      HIP_OK(hipFree(d_in));
+      DevicePoolGive(d_in);
     } else {
       // pack block by block: row-major bytes up, quads down into the pinned block
       uint8_t *d_in = DevAlloc<uint8_t>(block_rows * F);
@@ -333,8 +357,8 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
                            block_rows, rows);
         HIP_OK(hipMemcpy(dm->host_blocks[b], d_out, (size_t)dm->Q * block_rows * sizeof(uint32_t), hipMemcpyDeviceToHost));
       }
-      HIP_OK(hipFree(d_in));
-      HIP_OK(hipFree(d_out));
+      DevicePoolGive(d_in);
+      DevicePoolGive(d_out);
       std::vector<uint8_t>().swap(data->prebinned);  // the pinned blocks are the only copy from here on
     }
   } else {
@@ -407,7 +431,7 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
       int slots = kSlots;
       while (slots < hist_size + 1) slots *= 2;
       if (slots > kMaxWideSlots) throw std::runtime_error("hist_size above 4095 is not supported");
-      HIP_OK(hipFree(dm->bins));
+      DevicePoolGive(dm->bins);
       dm->bins = nullptr;
       dm->bits = 16;
       dm->slots = slots;
@@ -418,13 +442,13 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
       dm->bins = DevAlloc<uint32_t>((size_t)dm->Q * dm->stride);
       if (!quantise_columns(16)) throw std::runtime_error("internal: 16-bit quantisation failed");
     }
-    HIP_OK(hipFree(d_x));
-    HIP_OK(hipFree(d_thr));
-    HIP_OK(hipFree(d_size));
+    DevicePoolGive(d_x);
+    DevicePoolGive(d_thr);
+    DevicePoolGive(d_size);
     for (int k = 0; k < 2; ++k) HIP_OK(hipHostFree(stage[k]));
   }
-  if (d_col) HIP_OK(hipFree(d_col));
-  if (streamed && d_hi) HIP_OK(hipFree(d_hi));
+  if (d_col) DevicePoolGive(d_col);
+  if (streamed && d_hi) DevicePoolGive(d_hi);
   if (dm->hi) dm->slots = kSlots + 1;
   if (streamed) {
     data->stream_blocks = dm->host_blocks;
@@ -621,7 +645,7 @@ class HipTreeBuilder : public TreeBuilder {
     if (cfg.objective < kSoftMaxOneVsAll && K_ != 1) throw std::runtime_error("labels_count must be 1 for this objective");
     const int last_nodes = 1 << (D_ - 2);
     if (last_nodes > kMaxPlanNodes) throw std::runtime_error("unsupported depth: at most 4096 nodes per level");
-    HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    stream_ = StreamPoolTake();
 
     // quads per histogram launch, limited by LDS
     // whole 16-feature blocks per launch
@@ -670,29 +694,28 @@ class HipTreeBuilder : public TreeBuilder {
     }
 
     // per-row state in original order
-    d_y_ = DevAlloc<float>(n_);
-    d_labels_ = DevAlloc<uint8_t>(n_);
+    y_held_ = data->DeviceY();
+    labels_held_ = data->DeviceLabels();
+    d_y_ = y_held_.get();
+    d_labels_ = labels_held_.get();
     d_yhat_ = DevAlloc<float>(n_ * K_);
     streamed_ = dm_->streamed;
     // Logistic gradients of 0/1 labels travel as one float per row (PackGrad):
     // there is no h array then, and kernels given h == nullptr unpack g.
     // (never together with rows kept in place: those kernels take g and h as two arrays)
     pack_ = cfg.objective == kLogisticRegression && !streamed_ && !wide_ && !indexed_ && Q_ <= kMaxGroupQuads &&
-            data->y.size() == n_ &&
-            std::all_of(data->y.begin(), data->y.end(), [](float v) { return v == 0.0f || v == 1.0f; });
+            data->y.size() == n_ && data->y_facts.zero_one;
     d_g_ = DevAlloc<float>(n_ * K_);
     d_h_ = pack_ ? nullptr : DevAlloc<float>(n_ * K_);
     d_leaf_ = DevAlloc<unsigned>(n_);
-    if (!data->y.empty()) HIP_OK(hipMemcpy(d_y_, data->y.data(), n_ * sizeof(float), hipMemcpyHostToDevice));
-    if (!data->labels.empty()) HIP_OK(hipMemcpy(d_labels_, data->labels.data(), n_, hipMemcpyHostToDevice));
     float init = cfg.tree.initial_y;
     if (cfg.objective == kLogisticRegression) init = std::log(init / (1 - init));  // objective.h:55-57
     hipLaunchKernelGGL(k_fill_f32, dim3(GridFor(n_ * K_, 256)), dim3(256), 0, stream_, d_yhat_, init, n_ * K_);
-    data->y_hat.assign(n_ * K_, init);  // garden.cu:104
+    data->ResetYHat(n_ * K_, init);  // garden.cu:104
 
     if (streamed_) {
       const size_t br = dm_->block_rows;
-      HIP_OK(hipStreamCreateWithFlags(&copy_stream_, hipStreamNonBlocking));
+      copy_stream_ = StreamPoolTake();
       for (int b = 0; b < 2; ++b) {
         blk_[b] = DevAlloc<uint32_t>((size_t)W_ * br);
         HIP_OK(hipEventCreateWithFlags(&ev_ready_[b], hipEventDisableTiming));
@@ -730,7 +753,7 @@ class HipTreeBuilder : public TreeBuilder {
         HIP_OK(hipGetLastError());
         HIP_OK(hipMemcpyAsync(&dm_->rec_largest_id, d_largest, sizeof(unsigned), hipMemcpyDeviceToHost, stream_));
         HIP_OK(hipStreamSynchronize(stream_));
-        HIP_OK(hipFree(d_largest));
+        DevicePoolGive(d_largest);
       }
       // the histogram over the records is sized by max_bin and does not look at the ids again
       if ((int)dm_->rec_largest_id > data->max_bin)
@@ -758,13 +781,15 @@ class HipTreeBuilder : public TreeBuilder {
       d_tot_[b] = DevAlloc<NodeSum>(max_nodes);
       d_seg_[b] = DevAlloc<unsigned>(max_nodes);
       d_hg_[b] = DevAlloc<long long>((size_t)last_nodes * nbin_total_);
-      d_hh_[b] = DevAlloc<long long>((size_t)last_nodes * nbin_total_);
+      if (pair_) d_hh_[b] = DevAlloc<long long>((size_t)last_nodes * nbin_total_);  // (null without hessians: the kernels leave it out)
       d_hc_[b] = DevAlloc<unsigned long long>((size_t)last_nodes * nbin_total_);
       // cells of bins that no row can have are never written (rows in place with fewer than 256
       // bins in use) and must read as zero
-      HIP_OK(hipMemsetAsync(d_hg_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(long long), stream_));
-      HIP_OK(hipMemsetAsync(d_hh_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(long long), stream_));
-      HIP_OK(hipMemsetAsync(d_hc_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(unsigned long long), stream_));
+      if (indexed_ && rec_one_launch_ && rec_slots_ < kSlots) {
+        HIP_OK(hipMemsetAsync(d_hg_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(long long), stream_));
+        if (pair_) HIP_OK(hipMemsetAsync(d_hh_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(long long), stream_));
+        HIP_OK(hipMemsetAsync(d_hc_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(unsigned long long), stream_));
+      }
     }
     d_split_ = DevAlloc<SplitRec>(last_nodes);
     d_cand_ = DevAlloc<Cand>((size_t)last_nodes * F_);
@@ -821,12 +846,7 @@ class HipTreeBuilder : public TreeBuilder {
     if (cfg.objective == kLogisticRegression) {
       shifts[1] = 32;  // 0 <= h <= 1/4
       // labels outside [0, 1] widen the gradient range
-      float ymin = 0.0f, ymax = 1.0f;
-      for (float v : data->y) {
-        ymin = std::min(ymin, v);
-        ymax = std::max(ymax, v);
-      }
-      shifts[0] = LogisticGradShift(ymin, ymax);
+      shifts[0] = LogisticGradShift(data->y_facts.least, data->y_facts.most);
     }
     if (cfg.objective >= kSoftMaxOneVsAll) shifts[1] = 31;     // 0 <= h <= 1/2
     HIP_OK(hipMemcpyAsync(d_shifts_, shifts, sizeof(shifts), hipMemcpyHostToDevice, stream_));
@@ -836,32 +856,32 @@ class HipTreeBuilder : public TreeBuilder {
 
   void Release() noexcept {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    void *ptrs[] = {d_y_, d_labels_, d_yhat_, d_g_, d_h_, d_leaf_, d_split_, d_cand_, d_node_first2_,
+    void *ptrs[] = {d_yhat_, d_g_, d_h_, d_leaf_, d_split_, d_cand_, d_node_first2_,
                     d_node_items2_, d_hwork_, d_pwork_, d_nwork_, d_wave_left_, d_item_left_, d_slab_,
                     d_shifts_, d_gmax_, d_rows_scanned_, d_tfid_, d_tbin_, d_tgain_, d_weights_, d_active_, d_overflow_, d_records_, d_cursor2_};
     for (void *p : ptrs)
-      if (p) (void)hipFree(p);
+      DevicePoolGive(p);
     for (int b = 0; b < 2; ++b) {
       void *q[] = {buf_[b].bins, buf_[b].g, buf_[b].h, buf_[b].ids, d_tot_[b], d_seg_[b], d_hg_[b], d_hh_[b], d_hc_[b]};
       for (void *p : q)
-        if (p) (void)hipFree(p);
+        DevicePoolGive(p);
     }
     for (hipEvent_t e : event_pool_) (void)hipEventDestroy(e);
     for (uint32_t *p : resident_)
-      if (p) (void)hipFree(p);
+      DevicePoolGive(p);
     if (streamed_) {
       if (copy_stream_) (void)hipStreamSynchronize(copy_stream_);
       void *sp[] = {blk_[0], blk_[1], stage_.bins, stage_.g, stage_.h, d_node_of_, d_blk_cnt_, d_blk_seg_,
                     d_cursor_, d_blk_tot_};
       for (void *p : sp)
-        if (p) (void)hipFree(p);
+        DevicePoolGive(p);
       for (int b = 0; b < 2; ++b) {
         if (ev_ready_[b]) (void)hipEventDestroy(ev_ready_[b]);
         if (ev_free_[b]) (void)hipEventDestroy(ev_free_[b]);
       }
-      if (copy_stream_) (void)hipStreamDestroy(copy_stream_);
+      StreamPoolGive(copy_stream_);
     }
-    if (stream_) (void)hipStreamDestroy(stream_);
+    StreamPoolGive(stream_);
   }
 
  public:
@@ -903,8 +923,7 @@ class HipTreeBuilder : public TreeBuilder {
     const int internal = (1 << (D_ - 1)) - 1, leaves = 1 << (D_ - 1);
     const size_t words = RecordWords();
     std::vector<uint32_t> rec(words * pending_.size());
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(rec.data(), d_records_, rec.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    CopyToHost(rec.data(), d_records_, rec.size() * sizeof(uint32_t), stream_);
     bool overflow = false;
     for (size_t k = 0; k < pending_.size(); ++k) {
       RegTree &tree = (*owner_)[pending_[k]];
@@ -933,12 +952,10 @@ class HipTreeBuilder : public TreeBuilder {
       HIP_OK(hipGetLastError());
       leaf_valid_ = true;
     }
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(out, d_leaf_, n_ * sizeof(unsigned), hipMemcpyDeviceToHost));
+    CopyToHost(out, d_leaf_, n_ * sizeof(unsigned), stream_);
   }
   void GetYHat(float *out) override {
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(out, d_yhat_, n_ * K_ * sizeof(float), hipMemcpyDeviceToHost));
+    CopyToHost(out, d_yhat_, n_ * K_ * sizeof(float), stream_);
   }
   void GetGrad(float *g, float *h) override {
     if (!inspect_) throw std::runtime_error("gradients of the last round are only kept with inspection on");
@@ -1422,6 +1439,7 @@ class HipTreeBuilder : public TreeBuilder {
     const size_t nblocks = dm_->host_blocks.size();
     const size_t block_bytes = (size_t)W_ * dm_->block_rows * sizeof(uint32_t);
     size_t free_b = 0, total_b = 0;
+    DevicePoolTrim();  // (idle blocks are free memory)
     HIP_OK(hipMemGetInfo(&free_b, &total_b));
     size_t allowed = (size_t)(0.9 * (double)free_b);
     if (budget >= 0) allowed = std::min(allowed, (size_t)budget);
@@ -1734,7 +1752,7 @@ class HipTreeBuilder : public TreeBuilder {
     std::vector<unsigned long long> c(cells);
     HIP_OK(hipStreamSynchronize(stream_));
     HIP_OK(hipMemcpy(g.data(), d_hg_[hb], cells * sizeof(long long), hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(h.data(), d_hh_[hb], cells * sizeof(long long), hipMemcpyDeviceToHost));
+    if (pair_) HIP_OK(hipMemcpy(h.data(), d_hh_[hb], cells * sizeof(long long), hipMemcpyDeviceToHost));
     HIP_OK(hipMemcpy(c.data(), d_hc_[hb], cells * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     // keep [node][F][slots][3] (padding features of the last quad dropped)
     std::vector<NodeSum> tot;
@@ -1809,8 +1827,11 @@ class HipTreeBuilder : public TreeBuilder {
   bool grad_ready_ = false;
   int quads_per_group_ = 1;
   hipStream_t stream_ = nullptr;
-  float *d_y_ = nullptr, *d_yhat_ = nullptr, *d_g_ = nullptr, *d_h_ = nullptr, *d_weights_ = nullptr, *d_tgain_ = nullptr;
-  uint8_t *d_labels_ = nullptr;
+  const float *d_y_ = nullptr;
+  float *d_yhat_ = nullptr, *d_g_ = nullptr, *d_h_ = nullptr, *d_weights_ = nullptr, *d_tgain_ = nullptr;
+  const uint8_t *d_labels_ = nullptr;
+  std::shared_ptr<const float> y_held_;  // the matrix' target (d_y_, d_labels_)
+  std::shared_ptr<const unsigned char> labels_held_;
   unsigned *d_overflow_ = nullptr;     // set by the planner when a launch bound was too small
   unsigned char *d_active_ = nullptr;  // [level][feature] 1 = sampled at that level
   std::vector<unsigned char> active_host_;

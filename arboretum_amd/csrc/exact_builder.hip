@@ -31,6 +31,9 @@
 #include "kernels_objective.h"
 #include "kernels_plan.h"
 #include "kernels_split.h"
+#include "memory_pool.h"
+#include "parallel.h"
+#include "staging.h"
 
 namespace arb {
 
@@ -44,9 +47,10 @@ struct ExactSortData {
 
 void FreeExactSortData(ExactSortData *d) {
   if (!d) return;
-  if (d->ranks) (void)hipFree(d->ranks);
-  if (d->lists) (void)hipFree(d->lists);
-  if (d->list_ranks) (void)hipFree(d->list_ranks);
+  (void)hipDeviceSynchronize();  // what goes back to the pool has no work pending on it
+  DevicePoolGive(d->ranks);
+  DevicePoolGive(d->lists);
+  DevicePoolGive(d->list_ranks);
   delete d;
 }
 
@@ -145,28 +149,27 @@ class ExactSortBuilder : public TreeBuilder {
     if (F_ > 65535) throw std::runtime_error("the exact method over sorted lists takes at most 65535 features");
     const int last_nodes = 1 << (D_ - 2);
     if (last_nodes > kMaxPlanNodes) throw std::runtime_error("unsupported depth: at most 4096 nodes per level");
-    HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    stream_ = StreamPoolTake();
     max_items_ = (unsigned)(n_ / kExItem) + 2u * (unsigned)last_nodes + 2u;
 
-    d_y_ = DevAlloc<float>(n_);
-    d_labels_ = DevAlloc<uint8_t>(n_);
+    y_held_ = data->DeviceY();
+    labels_held_ = data->DeviceLabels();
+    d_y_ = y_held_.get();
+    d_labels_ = labels_held_.get();
     d_yhat_ = DevAlloc<float>(n_ * K_);
     // Logistic gradients of 0/1 labels travel as one float per row (PackGrad): no h array, and
     // 12 instead of 16 bytes per place of the lists.
-    pack_ = cfg.objective == kLogisticRegression && data->y.size() == n_ &&
-            std::all_of(data->y.begin(), data->y.end(), [](float v) { return v == 0.0f || v == 1.0f; });
+    pack_ = cfg.objective == kLogisticRegression && data->y.size() == n_ && data->y_facts.zero_one;
     harr_ = pair_ && !pack_;
     d_g_ = DevAlloc<float>(n_ * K_);
     d_h_ = harr_ ? DevAlloc<float>(n_ * K_) : nullptr;
     d_leaf_ = DevAlloc<unsigned>(n_);
     HIP_OK(hipMemsetAsync(d_leaf_, 0, n_ * sizeof(unsigned), stream_));  // (asked for before the first tree: the root)
     d_node_of_ = DevAlloc<unsigned>(n_);
-    if (!data->y.empty()) HIP_OK(hipMemcpy(d_y_, data->y.data(), n_ * sizeof(float), hipMemcpyHostToDevice));
-    if (!data->labels.empty()) HIP_OK(hipMemcpy(d_labels_, data->labels.data(), n_, hipMemcpyHostToDevice));
     float init = cfg.tree.initial_y;
     if (cfg.objective == kLogisticRegression) init = std::log(init / (1 - init));  // objective.h:55-57
     hipLaunchKernelGGL(k_fill_f32, dim3(GridFor(n_ * K_, 256)), dim3(256), 0, stream_, d_yhat_, init, n_ * K_);
-    data->y_hat.assign(n_ * K_, init);  // garden.cu:104
+    data->ResetYHat(n_ * K_, init);  // garden.cu:104
 
     d_went_right_ = DevAlloc<unsigned long long>(stride_ / 64);
     d_gh_ = harr_ ? DevAlloc<float2>(n_) : nullptr;
@@ -215,12 +218,8 @@ class ExactSortBuilder : public TreeBuilder {
     int shifts[2] = {30, 0};
     if (cfg.objective == kLogisticRegression) {
       shifts[1] = 32;  // 0 <= h <= 1/4
-      float ymin = 0.0f, ymax = 1.0f;  // labels outside [0, 1] widen the gradient range
-      for (float v : data->y) {
-        ymin = std::min(ymin, v);
-        ymax = std::max(ymax, v);
-      }
-      shifts[0] = LogisticGradShift(ymin, ymax);
+      // labels outside [0, 1] widen the gradient range
+      shifts[0] = LogisticGradShift(data->y_facts.least, data->y_facts.most);
     }
     if (cfg.objective >= kSoftMaxOneVsAll) shifts[1] = 31;  // 0 <= h <= 1/2
     HIP_OK(hipMemcpyAsync(d_shifts_, shifts, sizeof(shifts), hipMemcpyHostToDevice, stream_));
@@ -229,14 +228,14 @@ class ExactSortBuilder : public TreeBuilder {
 
   void Release() noexcept {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    void *all[] = {d_y_, d_labels_, d_yhat_, d_g_, d_h_, d_leaf_, d_node_of_, d_went_right_, d_gh_, d_ids_[0], d_ids_[1], d_ranks_[0],
+    void *all[] = {d_yhat_, d_g_, d_h_, d_leaf_, d_node_of_, d_went_right_, d_gh_, d_ids_[0], d_ids_[1], d_ranks_[0],
                    d_ranks_[1], d_lg_[0], d_lg_[1], d_lh_[0], d_lh_[1], d_tot_[0],
                    d_tot_[1], d_seg_[0], d_seg_[1], d_split_, d_cand_, d_work_, d_n_work_, d_node_first_,
                    d_node_items_, d_part_, d_off_, d_best_, d_lefts_, d_left_off_, d_left_bits_, d_shifts_, d_records_, d_gmax_,
                    d_overflow_, d_tfid_, d_tbin_, d_tgain_, d_weights_, d_active_};
     for (void *p : all)
-      if (p) (void)hipFree(p);
-    if (stream_) (void)hipStreamDestroy(stream_);
+      DevicePoolGive(p);
+    StreamPoolGive(stream_);
   }
 
  public:
@@ -265,8 +264,7 @@ class ExactSortBuilder : public TreeBuilder {
     const int internal = (1 << (D_ - 1)) - 1, leaves = 1 << (D_ - 1);
     const size_t words = RecordWords();
     std::vector<uint32_t> rec(words * pending_.size());
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(rec.data(), d_records_, rec.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    CopyToHost(rec.data(), d_records_, rec.size() * sizeof(uint32_t), stream_);
     bool overflow = false;
     for (size_t k = 0; k < pending_.size(); ++k) {
       RegTree &tree = (*owner_)[pending_[k]];
@@ -289,12 +287,10 @@ class ExactSortBuilder : public TreeBuilder {
 
   void SetInspect(bool on) override { inspect_ = on; }
   void GetLeaves(uint32_t *out) override {
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(out, d_leaf_, n_ * sizeof(unsigned), hipMemcpyDeviceToHost));
+    CopyToHost(out, d_leaf_, n_ * sizeof(unsigned), stream_);
   }
   void GetYHat(float *out) override {
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(out, d_yhat_, n_ * K_ * sizeof(float), hipMemcpyDeviceToHost));
+    CopyToHost(out, d_yhat_, n_ * K_ * sizeof(float), stream_);
   }
   void GetGrad(float *g, float *h) override {
     if (!inspect_) throw std::runtime_error("gradients of the last round are only kept with inspection on");
@@ -467,8 +463,11 @@ class ExactSortBuilder : public TreeBuilder {
   std::vector<RegTree> *owner_ = nullptr;
   std::vector<size_t> pending_;
 
-  float *d_y_ = nullptr, *d_yhat_ = nullptr, *d_g_ = nullptr, *d_h_ = nullptr, *d_tgain_ = nullptr, *d_weights_ = nullptr;
-  uint8_t *d_labels_ = nullptr;
+  const float *d_y_ = nullptr;
+  float *d_yhat_ = nullptr, *d_g_ = nullptr, *d_h_ = nullptr, *d_tgain_ = nullptr, *d_weights_ = nullptr;
+  const uint8_t *d_labels_ = nullptr;
+  std::shared_ptr<const float> y_held_;  // the matrix' target (d_y_, d_labels_)
+  std::shared_ptr<const unsigned char> labels_held_;
   unsigned *d_leaf_ = nullptr, *d_node_of_ = nullptr, *d_seg_[2] = {nullptr, nullptr}, *d_n_work_ = nullptr,
            *d_node_first_ = nullptr, *d_node_items_ = nullptr, *d_lefts_ = nullptr, *d_left_off_ = nullptr,
            *d_gmax_ = nullptr, *d_overflow_ = nullptr;

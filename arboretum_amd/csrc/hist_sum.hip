@@ -21,6 +21,7 @@
 #include "kernels_launch.h"
 #include "kernels_partition.h"
 #include "kernels_plan.h"
+#include "memory_pool.h"
 
 namespace arb {
 namespace {
@@ -70,14 +71,23 @@ HistSumScratch Carve(unsigned char *base, int max_nodes, unsigned max_items) {
 
 // Node sizes and segment starts from the offsets the caller passes (the
 // reference's node_size array: nodes + 1 non-decreasing row offsets), the
-// fixed-point shifts, cleared counters.  status (optional): 0, or 1 when the
-// offsets are not non-decreasing within [0, nrow].  One workgroup.
+// fixed-point shifts, and the work plan over those segments.  One workgroup:
+// three kernels of a few microseconds each (set-up, plan, status) made one.
+// status: 0, 1 when the offsets are not non-decreasing within [0, nrow] (such
+// a segment is skipped), 2 when the plan does not fit its launch bound.  It may
+// lie in host memory.
 __global__ void __launch_bounds__(1024)
-k_hist_sum_setup(const unsigned *__restrict__ node_size, int nodes, unsigned nrow, int shift_g, int shift_h,
-                 NodeSum *__restrict__ tot, unsigned *__restrict__ seg, unsigned *__restrict__ n_work,
-                 unsigned *__restrict__ overflow, int *__restrict__ shifts, unsigned *__restrict__ status) {
+k_hist_sum_plan(const unsigned *__restrict__ node_size, int nodes, unsigned nrow, int shift_g, int shift_h, NodeSum *tot,
+                unsigned *seg, int select, unsigned rows_per_item, WorkItem *work, unsigned *n_work,
+                unsigned *node_first, unsigned *node_items, unsigned max_items, unsigned *overflow, int *shifts,
+                unsigned *__restrict__ status) {
   __shared__ unsigned s_bad;
-  if (threadIdx.x == 0) s_bad = 0;
+  if (threadIdx.x == 0) {
+    s_bad = 0;
+    *overflow = 0;
+    shifts[0] = shift_g;
+    shifts[1] = shift_h;
+  }
   __syncthreads();
   for (int nd = threadIdx.x; nd < nodes; nd += blockDim.x) {
     const unsigned b = node_size[nd], e = node_size[nd + 1];
@@ -90,19 +100,10 @@ k_hist_sum_setup(const unsigned *__restrict__ node_size, int nodes, unsigned nro
     tot[nd] = t;
     seg[nd] = ok ? b : 0;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    *n_work = 0;
-    *overflow = 0;
-    shifts[0] = shift_g;
-    shifts[1] = shift_h;
-    if (status) *status = s_bad;
-  }
-}
-
-// A work plan that did not fit its launch bound is reported as status 2.
-__global__ void k_hist_sum_status(const unsigned *__restrict__ overflow, unsigned *__restrict__ status) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && *overflow != 0 && *status == 0) *status = 2;
+  __syncthreads();  // the plan reads what this workgroup has just written
+  PlanBody(tot, seg, nodes, select, rows_per_item, work, n_work, node_first, node_items, nullptr, nullptr, max_items,
+           overflow);
+  if (threadIdx.x == 0) *status = s_bad != 0 ? 1u : *overflow != 0 ? 2u : 0u;  // (thread 0 wrote *overflow)
 }
 
 struct Shape {
@@ -152,11 +153,9 @@ void Enqueue(const HistSumArgs &a, const Shape &sh, unsigned char *mem, unsigned
   const bool pair = a.hess != nullptr;
   HistSumScratch s = Carve(mem, a.nodes, max_items);
   if (slab_base) s.slab = reinterpret_cast<unsigned long long *>(slab_base);
-  hipLaunchKernelGGL(k_hist_sum_setup, dim3(1), dim3(1024), 0, st, a.node_size, a.nodes, (unsigned)a.nrow, a.shift_g,
-                     a.shift_h, s.tot, s.seg, s.n_work, s.overflow, s.shifts, status);
-  hipLaunchKernelGGL(k_plan, dim3(1), dim3(1024), 0, st, s.tot, s.seg, a.nodes, a.use_trick ? 1 : 0, per_item, s.work,
-                     s.n_work, s.node_first, s.node_items, (unsigned long long *)nullptr, (const SplitRec *)nullptr,
-                     max_items, s.overflow, 0u);
+  hipLaunchKernelGGL(k_hist_sum_plan, dim3(1), dim3(1024), 0, st, a.node_size, a.nodes, (unsigned)a.nrow, a.shift_g,
+                     a.shift_h, s.tot, s.seg, a.use_trick ? 1 : 0, per_item, s.work, s.n_work, s.node_first,
+                     s.node_items, max_items, s.overflow, s.shifts, status);
   const unsigned grid = (unsigned)std::min<size_t>((size_t)a.nrow / per_item + 2 * (size_t)a.nodes + 1, max_items);
   for (int q0 = 0; q0 < sh.Q; q0 += sh.quads_per_group) {
     const int nq = std::min(sh.quads_per_group, sh.Q - q0);
@@ -178,7 +177,6 @@ void Enqueue(const HistSumArgs &a, const Shape &sh, unsigned char *mem, unsigned
                        s.node_first, s.node_items, 0, (const SplitRec *)nullptr, (const NodeSum *)nullptr, a.sum_g,
                        a.sum_h, a.bin_count, a.parent_g, a.parent_h, a.parent_c, a.use_trick ? 1 : 0, 0, 0,
                        HistBlocks(sh.quads_per_group));
-  if (status) hipLaunchKernelGGL(k_hist_sum_status, dim3(1), dim3(64), 0, st, s.overflow, status);
   HIP_OK(hipGetLastError());
 }
 
@@ -251,21 +249,28 @@ void HistSum(const HistSumArgs &a) {
   // one work item per CU and round where the rows allow it, as the tree builder plans a level
   const unsigned per_item = HistSumRowsPerItem((size_t)a.nrow, a.nodes);
   const unsigned max_items = (unsigned)((size_t)a.nrow / per_item + 2 * (size_t)a.nodes + 2);
-  const size_t bytes = HistSumHeadBytes(a.nodes, max_items) + (size_t)max_items * sh.slab_words * 8 + 256;
-  unsigned char *mem = nullptr;
-  HIP_OK(hipMalloc((void **)&mem, bytes));
-  unsigned *status = reinterpret_cast<unsigned *>(mem + bytes - 256);
-  unsigned host_status = 0;
+  // The work memory (tens of MB) comes out of the pool: taken from the driver and given back on every
+  // call it cost 0.5 to 2 ms beside the 57 us of kernels (4 M rows x 28, 16 nodes).  The status is
+  // a word of pinned memory that the plan writes: no copy back.
+  struct Work {
+    unsigned char *mem = nullptr;
+    unsigned *status = nullptr;
+    ~Work() {
+      DevicePoolGive(mem);
+      PinnedPoolGive(status);
+    }
+  } work;
+  work.mem = static_cast<unsigned char *>(DevicePoolTake(HistSumHeadBytes(a.nodes, max_items) + (size_t)max_items * sh.slab_words * 8));
+  work.status = static_cast<unsigned *>(PinnedPoolTake(sizeof(unsigned)));
   hipStream_t st = static_cast<hipStream_t>(a.stream);
   try {
-    Enqueue(a, sh, mem, max_items, per_item, status, st);
+    Enqueue(a, sh, work.mem, max_items, per_item, work.status, st);
     HIP_OK(hipStreamSynchronize(st));
-    HIP_OK(hipMemcpy(&host_status, status, sizeof(unsigned), hipMemcpyDeviceToHost));
   } catch (...) {
-    (void)hipFree(mem);
+    (void)hipStreamSynchronize(st);  // nothing pending on what goes back to the pool
     throw;
   }
-  HIP_OK(hipFree(mem));
+  const unsigned host_status = *work.status;
   if (host_status == 1) throw std::runtime_error("node_size must hold non-decreasing row offsets within the matrix");
   if (host_status != 0) throw std::runtime_error("internal: work plan exceeded its launch bound");
 }

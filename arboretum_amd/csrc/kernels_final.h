@@ -3,6 +3,7 @@
 #define ARBORETUM_AMD_KERNELS_FINAL_H_
 #include "device_common.h"
 #include "kernels_hist.h"
+#include "memory_pool.h"
 
 namespace arb {
 namespace {
@@ -378,11 +379,10 @@ __global__ void k_fill_f32(float *p, float v, size_t n) {
     p[i] = v;
 }
 
+// Device memory out of the pool (DevicePoolGive it back, with no work pending on it).
 template <typename T>
 T *DevAlloc(size_t n) {
-  void *p = nullptr;
-  HIP_OK(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)));
-  return static_cast<T *>(p);
+  return static_cast<T *>(DevicePoolTake(std::max<size_t>(n, 1) * sizeof(T)));
 }
 
 inline int GridFor(size_t n, int block, int cap = 4096) {

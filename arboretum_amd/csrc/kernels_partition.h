@@ -820,17 +820,18 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
 // row, NaN included, sits in exactly one slot).  Replaces the reduction over
 // the gradient array of garden.cu:432-435.  One wave.
 // hi_cell > 0: the cell of feature 0's bin 256 (matrices with a ninth-bit word).
+// hh may be null (no hessians).
 __global__ void __launch_bounds__(64)
 k_root_from_hist(const long long *__restrict__ hg, const long long *__restrict__ hh,
                  NodeSum *__restrict__ tot, int slots, int hi_cell = 0) {
   long long a = 0, b = 0;
   for (int i = threadIdx.x; i < slots; i += 64) {
     a += hg[i];
-    b += hh[i];
+    if (hh != nullptr) b += hh[i];
   }
   if (hi_cell > 0 && threadIdx.x == 0) {
     a += hg[hi_cell];
-    b += hh[hi_cell];
+    if (hh != nullptr) b += hh[hi_cell];
   }
   a = WaveSumLL(a);
   b = WaveSumLL(b);

@@ -221,7 +221,7 @@ __global__ void k_sibling(long long *__restrict__ hg, long long *__restrict__ hh
   const size_t o = (size_t)nd * nbin_total + e, so = (size_t)(nd ^ 1u) * nbin_total + e,
                po = (size_t)(nd >> 1) * nbin_total + e;
   hg[o] = pg[po] - hg[so];
-  hh[o] = ph[po] - hh[so];
+  if (hh != nullptr) hh[o] = ph[po] - hh[so];  // (null without hessians)
   hc[o] = pc[po] - hc[so];
 }
 

@@ -16,6 +16,8 @@
 #include <vector>
 
 #include "booster.h"
+#include "memory_pool.h"
+#include "parallel.h"
 
 namespace arb {
 namespace {
@@ -126,13 +128,13 @@ template <typename T>
 struct DevBuf {
   T *p = nullptr;
   size_t n = 0;
-  ~DevBuf() { if (p) (void)hipFree(p); }
+  ~DevBuf() { DevicePoolGive(p); }
   void Reserve(size_t want) {
     if (want <= n) return;
-    if (p) HIP_OK(hipFree(p));
+    if (p) DevicePoolGive(p);
     p = nullptr;
     n = 0;
-    HIP_OK(hipMalloc((void **)&p, want * sizeof(T)));
+    p = static_cast<decltype(p)>(DevicePoolTake(want * sizeof(T)));
     n = want;
   }
   // blocking: the vector may be gone when the call returns

@@ -17,6 +17,8 @@
 #include <vector>
 
 #include "booster.h"
+#include "memory_pool.h"
+#include "parallel.h"
 
 namespace arb {
 namespace {
@@ -299,13 +301,13 @@ SortWorkspace *CreateSortWorkspace(size_t n, int hist_size) {
   ws->n = n;
   ws->hist_size = hist_size;
   ws->nblk = (unsigned)((n + kSortTile - 1) / kSortTile);
-  HIP_OK(hipMalloc((void **)&ws->keys[0], n * sizeof(unsigned)));
-  HIP_OK(hipMalloc((void **)&ws->keys[1], n * sizeof(unsigned)));
-  HIP_OK(hipMalloc((void **)&ws->counts, (size_t)256 * ws->nblk * sizeof(unsigned)));
-  HIP_OK(hipMalloc((void **)&ws->digit_total, 256 * sizeof(unsigned)));
-  HIP_OK(hipMalloc((void **)&ws->thr, (size_t)hist_size * sizeof(unsigned)));
-  HIP_OK(hipMalloc((void **)&ws->thr_f, (size_t)hist_size * sizeof(float)));
-  HIP_OK(hipMalloc((void **)&ws->has_nan, sizeof(unsigned)));
+  ws->keys[0] = static_cast<unsigned *>(DevicePoolTake(n * sizeof(unsigned)));
+  ws->keys[1] = static_cast<unsigned *>(DevicePoolTake(n * sizeof(unsigned)));
+  ws->counts = static_cast<unsigned *>(DevicePoolTake((size_t)256 * ws->nblk * sizeof(unsigned)));
+  ws->digit_total = static_cast<unsigned *>(DevicePoolTake(256 * sizeof(unsigned)));
+  ws->thr = static_cast<unsigned *>(DevicePoolTake((size_t)hist_size * sizeof(unsigned)));
+  ws->thr_f = static_cast<float *>(DevicePoolTake((size_t)hist_size * sizeof(float)));
+  ws->has_nan = static_cast<unsigned *>(DevicePoolTake(sizeof(unsigned)));
   return ws;
 }
 
@@ -313,7 +315,7 @@ void FreeSortWorkspace(SortWorkspace *ws) {
   if (!ws) return;
   void *p[] = {ws->keys[0], ws->keys[1], ws->counts, ws->digit_total, ws->thr, ws->thr_f, ws->has_nan};
   for (void *q : p)
-    if (q) (void)hipFree(q);
+    DevicePoolGive(q);
   delete ws;
 }
 

@@ -1,0 +1,101 @@
+#include "staging.h"
+
+#include <algorithm>
+#include <cstring>
+#include <stdexcept>
+#include <string>
+
+#include "memory_pool.h"
+#include "parallel.h"
+
+namespace arb {
+namespace {
+
+#define HIP_OK(expr)                                                                        \
+  do {                                                                                      \
+    hipError_t e_ = (expr);                                                                 \
+    if (e_ != hipSuccess)                                                                   \
+      throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_) + " in " #expr); \
+  } while (0)
+
+constexpr size_t kCopyGrain = (size_t)256 << 10;  // bytes a host thread takes at a time
+
+void ParallelCopy(void *dst, const void *src, size_t bytes) {
+  ParallelFor(bytes, [&](size_t b, size_t e) { std::memcpy((char *)dst + b, (const char *)src + b, e - b); }, kCopyGrain);
+}
+
+// Up to kStageSlots pinned blocks and the event of the last copy that touched each.
+struct Slots {
+  explicit Slots(int count, size_t bytes, hipStream_t stream) : count(count), stream(stream) {
+    try {
+      for (int k = 0; k < count; ++k) {
+        block[k] = PinnedPoolTake(bytes);
+        HIP_OK(hipEventCreateWithFlags(&copied[k], hipEventDisableTiming));
+      }
+    } catch (...) {
+      Release();
+      throw;
+    }
+  }
+  ~Slots() {
+    (void)hipStreamSynchronize(stream);  // (a failed call may leave a copy pending; else this was waited for)
+    Release();
+  }
+  void Release() {
+    for (int k = 0; k < kStageSlots; ++k) {
+      PinnedPoolGive(block[k]);
+      if (copied[k]) (void)hipEventDestroy(copied[k]);
+    }
+  }
+  const int count;
+  hipStream_t stream;
+  void *block[kStageSlots] = {};
+  hipEvent_t copied[kStageSlots] = {};
+};
+
+}  // namespace
+
+void CopyToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+  if (bytes == 0) return;
+  const size_t pieces = (bytes + kStageBytes - 1) / kStageBytes;
+  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::min(bytes, kStageBytes), stream);
+  auto start = [&](size_t k) {
+    const size_t at = k * kStageBytes, len = std::min(kStageBytes, bytes - at);
+    HIP_OK(hipMemcpyAsync(s.block[k % s.count], (const char *)src + at, len, hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipEventRecord(s.copied[k % s.count], stream));
+  };
+  for (size_t k = 0; k < pieces && k < (size_t)s.count; ++k) start(k);
+  for (size_t k = 0; k < pieces; ++k) {
+    const size_t at = k * kStageBytes, len = std::min(kStageBytes, bytes - at);
+    HIP_OK(hipEventSynchronize(s.copied[k % s.count]));
+    ParallelCopy((char *)dst + at, s.block[k % s.count], len);
+    if (k + s.count < pieces) start(k + s.count);
+  }
+}
+
+void StageToDevice(size_t pieces, const std::function<size_t(size_t)> &bytes_of,
+                   const std::function<void(size_t, void *)> &fill, const std::function<void *(size_t)> &dst_of,
+                   const std::function<void(size_t)> &then, hipStream_t stream) {
+  if (pieces == 0) return;
+  size_t most = 0;
+  for (size_t k = 0; k < pieces; ++k) most = std::max(most, bytes_of(k));
+  if (most > kStageBytes) throw std::runtime_error("internal: staging piece too large");
+  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::max<size_t>(most, 1), stream);
+  for (size_t k = 0; k < pieces; ++k) {
+    const int slot = (int)(k % s.count);
+    if (k >= (size_t)s.count) HIP_OK(hipEventSynchronize(s.copied[slot]));
+    fill(k, s.block[slot]);
+    HIP_OK(hipMemcpyAsync(dst_of(k), s.block[slot], bytes_of(k), hipMemcpyHostToDevice, stream));
+    HIP_OK(hipEventRecord(s.copied[slot], stream));
+    if (then) then(k);
+  }
+}
+
+void CopyToDevice(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+  auto bytes_of = [&](size_t k) { return std::min(kStageBytes, bytes - k * kStageBytes); };
+  StageToDevice((bytes + kStageBytes - 1) / kStageBytes, bytes_of,
+                [&](size_t k, void *p) { ParallelCopy(p, (const char *)src + k * kStageBytes, bytes_of(k)); },
+                [&](size_t k) { return (void *)((char *)dst + k * kStageBytes); }, nullptr, stream);
+}
+
+}  // namespace arb

@@ -12,6 +12,7 @@
 #include "../../include/arboretum_ext.h"
 #include "booster.h"
 #include "hist_sum.h"
+#include "parallel.h"
 
 using namespace arb;
 
@@ -77,15 +78,7 @@ const char *ACreateFromDenseMatrix(const float *data, const unsigned int *catego
     const size_t rows = (size_t)nrow, cols = (size_t)ncol;
     // the columns are allocated (and their pages first touched) by several threads
     mat->data.resize(cols);
-    {
-      const size_t nt = std::min<size_t>(cols, 16);
-      std::vector<std::thread> th;
-      for (size_t t = 0; t < nt; ++t)
-        th.emplace_back([&, t] {
-          for (size_t f = t; f < cols; f += nt) mat->data[f].resize(rows);
-        });
-      for (auto &x : th) x.join();
-    }
+    ParallelTasks(cols, [&](size_t f) { mat->data[f].resize(rows); });
     // row-major -> column-major in tiles of 256 rows, so that a tile's lines of every
     // column stay in cache while its rows are read once
     ParallelFor(rows, [&](size_t b, size_t e) {
@@ -110,7 +103,7 @@ const char *ASetY(VoidPointer data, const float *y) {
   return Guard([&] {
     DataMatrix *d = AsData(data);
     if (!y) throw std::runtime_error("null y");
-    d->y.assign(y, y + d->rows);
+    d->SetY(y);
   });
 }
 
@@ -118,7 +111,7 @@ const char *ASetLabel(VoidPointer data, const unsigned char *labels) {
   return Guard([&] {
     DataMatrix *d = AsData(data);
     if (!labels) throw std::runtime_error("null labels");
-    d->labels.assign(labels, labels + d->rows);
+    d->SetLabels(labels);
   });
 }
 
