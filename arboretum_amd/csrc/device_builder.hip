@@ -819,22 +819,25 @@ class HipTreeBuilder : public TreeBuilder {
         max_hist_items_ = std::max(max_hist_items_, BalancedPlanItems(plan_rows, 1u << level, kMaxHistRows, hist_cus_));
       max_hist_items_ = std::max(max_hist_items_, BalancedPlanItems(plan_rows, 1u, kMaxHistRows, cus_));
     }
-    max_part_items_ = std::max<unsigned>((unsigned)(plan_rows / kPartRows + 1) + 2 * last_nodes, max_hist_items_);
+    // Rows per work item of a partition that builds no histogram: two workgroups per CU as long as
+    // an item of kPartRows rows, the most a workgroup takes, would leave CUs without one.  (At 16384 rows
+    // whatever the matrix, 500,000 rows were 31 workgroups on 256 CUs: 33 us for a pass that moves 40 MB.)
+    part_rows_ = (unsigned)std::min<size_t>(std::max<size_t>((plan_rows / (2 * cus_) + 1023) / 1024 * 1024, 1024), kPartRows);
+    max_part_items_ = std::max<unsigned>((unsigned)(plan_rows / part_rows_ + 1) + 2 * last_nodes, max_hist_items_);
     d_hwork_ = DevAlloc<WorkItem>(max_hist_items_);
     d_pwork_ = DevAlloc<WorkItem>(max_part_items_);
     d_nwork_ = DevAlloc<unsigned>(2);
     d_wave_left_ = DevAlloc<unsigned>((size_t)max_part_items_ * kItemWaves);
     d_item_left_ = DevAlloc<unsigned>((size_t)2 * max_part_items_);  // also the claimed bases of the fused pass
     d_cursor2_ = DevAlloc<unsigned>((size_t)2 * last_nodes);
-    d_slab_ = DevAlloc<unsigned long long>((size_t)std::max(max_hist_items_, max_part_items_) * slab_stride_ * (pair_ ? 2 : 1));
+    d_slab_ = DevAlloc<unsigned long long>((size_t)max_hist_items_ * slab_stride_ * (pair_ ? 2 : 1));
     d_shifts_ = DevAlloc<int>(2);
     d_records_ = DevAlloc<uint32_t>(kRecordRing * RecordWords());
-    d_gmax_ = DevAlloc<unsigned>(1);
+    d_gmax_ = DevAlloc<float>(std::max<size_t>(kGmaxParts, streamed_ ? dm_->host_blocks.size() * kStreamFinalGrid : 0));
     d_rows_scanned_ = DevAlloc<unsigned long long>(kScanLevels);  // one counter per tree level
     d_overflow_ = DevAlloc<unsigned>(1);
     HIP_OK(hipMemsetAsync(d_overflow_, 0, sizeof(unsigned), stream_));
     HIP_OK(hipMemsetAsync(d_rows_scanned_, 0, kScanLevels * sizeof(unsigned long long), stream_));
-    HIP_OK(hipMemsetAsync(d_gmax_, 0, sizeof(unsigned), stream_));
     const int internal = (1 << (D_ - 1)) - 1;
     d_tfid_ = DevAlloc<int>(internal);
     d_tbin_ = DevAlloc<int>(internal);
@@ -891,7 +894,8 @@ class HipTreeBuilder : public TreeBuilder {
     if (!grad_ready_) {
       Mark(kGrad);
       if (cfg_.objective == kLinearRegression) {
-        hipLaunchKernelGGL(k_grad_squared, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
+        gmax_parts_ = (unsigned)GridFor(n_, 256, kGmaxParts);
+        hipLaunchKernelGGL(k_grad_squared, dim3(gmax_parts_), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
       } else if (cfg_.objective == kLogisticRegression) {
         hipLaunchKernelGGL(k_grad_logistic, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, d_h_, n_);
       } else {
@@ -899,7 +903,7 @@ class HipTreeBuilder : public TreeBuilder {
       }
     }
     if (cfg_.objective == kLinearRegression)
-      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(64), 0, stream_, d_gmax_, d_shifts_);
+      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(1024), 0, stream_, d_gmax_, gmax_parts_, d_shifts_);
     grad_ready_ = false;
     Mark(kNone);
     owner_ = trees;
@@ -1180,8 +1184,8 @@ class HipTreeBuilder : public TreeBuilder {
   // zero: k_init_root).
   void RootTotals(int hb, int state, const RowBuffers &orig) {
     if (hi_skip_)
-      hipLaunchKernelGGL(k_sum_grad, dim3(GridFor(n_, 256, 2048)), dim3(256), 0, stream_, orig.g, pair_ ? orig.h : nullptr,
-                         n_, d_shifts_, d_tot_[state]);
+      hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, orig.g,
+                         pair_ ? orig.h : nullptr, 0, n_, d_shifts_, d_tot_[state]);
     else
       hipLaunchKernelGGL(k_root_from_hist, dim3(1), dim3(64), 0, stream_, d_hg_[hb], d_hh_[hb], d_tot_[state], slots_,
                          hi_base_);
@@ -1274,7 +1278,7 @@ class HipTreeBuilder : public TreeBuilder {
     // (the last pass of the previous tree has done this when it built the root histogram)
     if (!root_hist_ready_)
       hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0],
-                         (unsigned long long)n_, (unsigned *)nullptr);
+                         (unsigned long long)n_);
     // The last pass of the tree can also build the root histogram of the next
     // one: logistic objective, gradients of the next round wanted, all quads in
     // one LDS histogram next to the node arrays.
@@ -1350,9 +1354,9 @@ class HipTreeBuilder : public TreeBuilder {
           }
           Reduce(L, hb, true, ps, true, false, own_scan_ && !last ? state : -1);
         } else {
-          const unsigned grid = (unsigned)std::min<size_t>(n_ / kPartRows + 2 * PL + 1, max_part_items_);
+          const unsigned grid = (unsigned)std::min<size_t>(n_ / part_rows_ + 2 * PL + 1, max_part_items_);
           Mark(kPlan);
-          Plan(ps, PL, 0, kPartRows, d_pwork_, d_nwork_ + 1, -1, nullptr, grid, 0, indexed_ ? d_cursor2_ : nullptr);
+          Plan(ps, PL, 0, part_rows_, d_pwork_, d_nwork_ + 1, -1, nullptr, grid, 0, indexed_ ? d_cursor2_ : nullptr);
           Mark(kPartition);
           if (indexed_) {
             // decisions, claims of the children's ranges and the move of (row id, g, h) in one launch
@@ -1383,7 +1387,6 @@ class HipTreeBuilder : public TreeBuilder {
     Mark(kLeaf);
     bool record_written = false;
     {
-      if (cfg_.objective == kLinearRegression) HIP_OK(hipMemsetAsync(d_gmax_, 0, sizeof(unsigned), stream_));
       if (final_hist) {
         // leaf weights, tree record, state and plan of the next tree's root in
         // one launch, then one pass: leaves, predictions, gradients and the
@@ -1556,7 +1559,7 @@ class HipTreeBuilder : public TreeBuilder {
 
   // launch bound of the fused pass over PL parent nodes
   unsigned FusedGrid(int PL) const {
-    return (unsigned)std::min<size_t>(n_ / FusedRowsPerItem(PL) + 2 * PL + 1, max_part_items_);
+    return (unsigned)std::min<size_t>(n_ / FusedRowsPerItem(PL) + 2 * PL + 1, max_hist_items_);  // (a slab each)
   }
   // Rows per work item of the fused pass over PL parents.  A CU runs one
   // workgroup at a time, so the pass takes as many rounds as items / CUs rounded
@@ -1588,7 +1591,11 @@ class HipTreeBuilder : public TreeBuilder {
     const int internal = (1 << (D_ - 1)) - 1;
     const size_t lds = (size_t)internal * 2 * sizeof(int);
     float *yh = d_yhat_ + (size_t)label * n_ + row0;
-    const int grid = GridFor(rows, 256, 8192);
+    // few enough workgroups that their shares of the maximum and the tree's nodes, which each of them
+    // reads, do not weigh; enough for every wave slot of the chip
+    const int grid = streamed_ ? (int)kStreamFinalGrid : GridFor(rows, 256, (int)kGmaxParts);
+    const size_t first_part = streamed_ ? row0 / dm_->block_rows * kStreamFinalGrid : 0;
+    gmax_parts_ = (unsigned)(first_part + grid);
     // the byte columns of a matrix whose rows stay in place (whole matrix only)
     const uint8_t *walk_bytes = indexed_ && bins == dm_->bins && row0 == 0 ? dm_->bytes : nullptr;
     int mode = 0;
@@ -1596,7 +1603,7 @@ class HipTreeBuilder : public TreeBuilder {
     if (next_grad && cfg_.objective == kLogisticRegression) mode = 2;
 #define ARB_FINAL(M, N) \
   hipLaunchKernelGGL((k_final<M, N>), dim3(grid), dim3(256), lds, stream_, bins, stride, d_tfid_, d_tbin_, D_, \
-                     d_weights_, yh, d_y_ + row0, d_leaf_ + row0, d_g_ + row0, d_h_ ? d_h_ + row0 : nullptr, d_gmax_, rows, code_, \
+                     d_weights_, yh, d_y_ + row0, d_leaf_ + row0, d_g_ + row0, d_h_ ? d_h_ + row0 : nullptr, d_gmax_ + first_part, rows, code_, \
                      walk_bytes, dm_->stride8, hi_word_)
 #define ARB_FINAL_Q(N) \
   do { if (mode == 1) ARB_FINAL(1, N); else if (mode == 2) ARB_FINAL(2, N); else ARB_FINAL(0, N); } while (0)
@@ -1644,8 +1651,7 @@ class HipTreeBuilder : public TreeBuilder {
   void GrowOneStreamed(int label, const RowBuffers &orig, const GainParams &gp) {
     const size_t br = dm_->block_rows;
     const size_t nblocks = dm_->host_blocks.size();
-    hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0],
-                       (unsigned long long)n_, (unsigned *)nullptr);
+    hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0], (unsigned long long)n_);
     int state = 0;
     for (int level = 0; level + 1 < D_; ++level) {
       const int L = 1 << level;
@@ -1709,7 +1715,6 @@ class HipTreeBuilder : public TreeBuilder {
     // leaves, y_hat, next gradients: one more pass over the blocks
     Mark(kLeaf);
     const bool next_grad = !inspect_ && K_ == 1;
-    if (cfg_.objective == kLinearRegression) HIP_OK(hipMemsetAsync(d_gmax_, 0, sizeof(unsigned), stream_));
     for (size_t b = 0; b < nblocks; ++b) {
       const size_t row0 = b * br;
       const size_t rows = std::min(br, n_ - row0);
@@ -1825,6 +1830,8 @@ class HipTreeBuilder : public TreeBuilder {
   unsigned sample_every_ = 1;
   unsigned long long trees_grown_ = 0;
   bool grad_ready_ = false;
+  float *d_gmax_ = nullptr;    // partial maxima of |g| of the pass that wrote the gradients
+  unsigned gmax_parts_ = 0;    // ... how many
   int quads_per_group_ = 1;
   hipStream_t stream_ = nullptr;
   const float *d_y_ = nullptr;
@@ -1840,7 +1847,7 @@ class HipTreeBuilder : public TreeBuilder {
   unsigned *d_node_first2_ = nullptr, *d_node_items2_ = nullptr;  // both sets; d_node_first_ / d_node_items_: the one in use
   bool own_scan_ = false;  // the fused passes find the splits of their parents themselves (LevelScan)
   unsigned *d_leaf_ = nullptr, *d_node_first_ = nullptr, *d_node_items_ = nullptr, *d_nwork_ = nullptr,
-           *d_wave_left_ = nullptr, *d_item_left_ = nullptr, *d_gmax_ = nullptr, *d_cursor2_ = nullptr;
+           *d_wave_left_ = nullptr, *d_item_left_ = nullptr, *d_cursor2_ = nullptr;
   RowBuffers buf_[2];
   // streamed matrices: two block buffers filled by the copy stream, a staging
   // buffer with the rows of the built nodes, a resident node id per row
@@ -1866,6 +1873,7 @@ class HipTreeBuilder : public TreeBuilder {
   Cand *d_cand_ = nullptr;
   WorkItem *d_hwork_ = nullptr, *d_pwork_ = nullptr;
   unsigned max_hist_items_ = 0, max_part_items_ = 0;
+  unsigned part_rows_ = kPartRows;  // rows per work item of a stand-alone partition
   unsigned long long *d_slab_ = nullptr, *d_rows_scanned_ = nullptr;
   int *d_shifts_ = nullptr, *d_tfid_ = nullptr, *d_tbin_ = nullptr;
   std::vector<std::vector<int64_t>> kept_hist_;

@@ -28,6 +28,8 @@ constexpr int kMaxGroupQuads = 8;         // quads per histogram launch (compile
 constexpr unsigned kMaxHistRows = 64512;  // rows per histogram work item (< 2^16)
 constexpr int kCountShift = 47;           // word0 = count << 47 | g
 constexpr int kMaxPlanNodes = 4096;       // nodes per level the planner handles
+constexpr unsigned kGmaxParts = 2048;       // most workgroups of a pass that leaves partial maxima of |g|
+constexpr unsigned kStreamFinalGrid = 1024;  // ... of such a pass over one block of a streamed matrix
 constexpr size_t kLdsBudget = 160 * 1024;
 // LDS histograms are laid out bin-major with the features of a bin in blocks
 // of 16 (4 quads): in 64-bit words, one word per entry,
@@ -136,19 +138,26 @@ __device__ __forceinline__ float WaveMaxF(float v) {
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_down(v, off));
   return v;
 }
+// The largest v >= 0 of a workgroup of up to 1024 threads, valid in thread 0.  Called by all threads.
+__device__ __forceinline__ float BlockMaxF(float v) {
+  __shared__ float s_max[16];
+  v = WaveMaxF(v);
+  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x < 64) v = WaveMaxF(threadIdx.x < blockDim.x / 64 ? s_max[threadIdx.x] : 0.0f);
+  return v;
+}
 __device__ __forceinline__ long long WaveSumLL(long long v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
   return v;
 }
 
-__global__ void k_init_root(NodeSum *tot, unsigned *seg_start, unsigned long long n,
-                            unsigned *gmax_bits) {  // gmax_bits may be NULL
+__global__ void k_init_root(NodeSum *tot, unsigned *seg_start, unsigned long long n) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     tot[0].g = 0;
     tot[0].h = 0;
     tot[0].c = n;
     seg_start[0] = 0;
-    if (gmax_bits) *gmax_bits = 0;
   }
 }
 

@@ -205,7 +205,7 @@ class ExactSortBuilder : public TreeBuilder {
     d_left_bits_ = DevAlloc<uint8_t>((size_t)F_ * max_items_ * kExThreads);
     d_shifts_ = DevAlloc<int>(2);
     d_records_ = DevAlloc<uint32_t>(kRecordRing * RecordWords());
-    d_gmax_ = DevAlloc<unsigned>(1);
+    d_gmax_ = DevAlloc<float>(kGmaxParts);
     d_overflow_ = DevAlloc<unsigned>(1);
     HIP_OK(hipMemsetAsync(d_overflow_, 0, sizeof(unsigned), stream_));
     const int internal = (1 << (D_ - 1)) - 1;
@@ -241,9 +241,9 @@ class ExactSortBuilder : public TreeBuilder {
  public:
   void GrowRound(std::vector<RegTree> *trees) override {
     if (cfg_.objective == kLinearRegression) {
-      HIP_OK(hipMemsetAsync(d_gmax_, 0, sizeof(unsigned), stream_));
-      hipLaunchKernelGGL(k_grad_squared, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
-      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(64), 0, stream_, d_gmax_, d_shifts_);
+      const unsigned parts = (unsigned)GridFor(n_, 256, kGmaxParts);
+      hipLaunchKernelGGL(k_grad_squared, dim3(parts), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
+      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(1024), 0, stream_, d_gmax_, parts, d_shifts_);
     } else if (cfg_.objective == kLogisticRegression) {
       hipLaunchKernelGGL(k_grad_logistic, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, d_h_, n_);  // (no d_h_: packed)
     } else {
@@ -362,12 +362,9 @@ class ExactSortBuilder : public TreeBuilder {
     const float *g = d_g_ + (size_t)label * n_;
     const float *h = d_h_ ? d_h_ + (size_t)label * n_ : nullptr;
     SampleColumns();
-    hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0], (unsigned long long)n_,
-                       (unsigned *)nullptr);
-    if (pack_)
-      hipLaunchKernelGGL(k_ex_sum_packed, dim3(GridFor(n_, 256, 1024)), dim3(256), 0, stream_, g, n_, d_shifts_, d_tot_[0]);
-    else
-      hipLaunchKernelGGL(k_sum_grad, dim3(GridFor(n_, 256, 1024)), dim3(256), 0, stream_, g, h, n_, d_shifts_, d_tot_[0]);
+    hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0], (unsigned long long)n_);
+    hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, g, h, pack_ ? 1 : 0, n_, d_shifts_,
+                       d_tot_[0]);
     HIP_OK(hipMemsetAsync(d_node_of_, 0, n_ * sizeof(unsigned), stream_));
     int state = 0;
     // the root's lists: every row, sorted once; this tree's gradients in that order
@@ -388,7 +385,7 @@ class ExactSortBuilder : public TreeBuilder {
       const dim3 per_item(grid_items, (unsigned)F_), per_node((unsigned)L, (unsigned)F_);
       hipLaunchKernelGGL(k_plan, dim3(1), dim3(1024), 0, stream_, d_tot_[state], d_seg_[state], L, 0, kExItem, d_work_,
                          d_n_work_, d_node_first_, d_node_items_, (unsigned long long *)nullptr,
-                         (const SplitRec *)nullptr, grid_items, d_overflow_, 0u, (unsigned *)nullptr);
+                         (const SplitRec *)nullptr, grid_items, d_overflow_, 0u);
 #define ARB_EX(P, D, K)                                                                                               \
   do {                                                                                                                \
     hipLaunchKernelGGL((k_ex_partial<P, K>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_,      \
@@ -470,7 +467,8 @@ class ExactSortBuilder : public TreeBuilder {
   std::shared_ptr<const unsigned char> labels_held_;
   unsigned *d_leaf_ = nullptr, *d_node_of_ = nullptr, *d_seg_[2] = {nullptr, nullptr}, *d_n_work_ = nullptr,
            *d_node_first_ = nullptr, *d_node_items_ = nullptr, *d_lefts_ = nullptr, *d_left_off_ = nullptr,
-           *d_gmax_ = nullptr, *d_overflow_ = nullptr;
+           *d_overflow_ = nullptr;
+  float *d_gmax_ = nullptr;  // partial maxima of |g|
   uint32_t *d_ids_[2] = {nullptr, nullptr}, *d_ranks_[2] = {nullptr, nullptr}, *d_records_ = nullptr;
   float *d_lg_[2] = {nullptr, nullptr}, *d_lh_[2] = {nullptr, nullptr};
   unsigned long long *d_went_right_ = nullptr;

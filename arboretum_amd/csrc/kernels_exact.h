@@ -101,26 +101,6 @@ __device__ __forceinline__ void ExLoadSums(const ExLists &ls, size_t fbase, unsi
   }
 }
 
-// Sum of the fixed-point gradients of all rows from packed logistic gradients: the totals of
-// the root.  tot[0].g / .h must be zero at launch; integer sums, any order.
-__global__ void __launch_bounds__(256)
-k_ex_sum_packed(const float *__restrict__ packed, size_t n, const int *__restrict__ shifts, NodeSum *__restrict__ tot) {
-  const int sg = shifts[0], sh = shifts[1];
-  long long a = 0, b = 0;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    float g1, h1;
-    UnpackGrad(packed[i], &g1, &h1);
-    a += ToFixed(g1, sg);
-    b += ToFixed(h1, sh);
-  }
-  a = WaveSumLL(a);
-  b = WaveSumLL(b);
-  if ((threadIdx.x & 63) == 0) {
-    atomicAdd(reinterpret_cast<unsigned long long *>(&tot[0].g), (unsigned long long)a);
-    atomicAdd(reinterpret_cast<unsigned long long *>(&tot[0].h), (unsigned long long)b);
-  }
-}
-
 // grid (items, F): the sum of the gradients over every work item's piece of every feature's list.
 template <bool PAIR, bool PACK>
 __global__ void __launch_bounds__(kExThreads)

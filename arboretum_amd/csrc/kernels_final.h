@@ -109,7 +109,7 @@ k_tree_end(const SplitRec *__restrict__ split, const NodeSum *__restrict__ tot, 
 // (bin >= q+1 goes right, builder.h:107-123), record the leaf, add its weight
 // to y_hat (update_by_last_tree, garden.cu:45-76) and, when NEXT_GRAD is not
 // 0, write the gradients of the next round (objective.cu:28-56):
-// 1 = squared (also max |g|), 2 = logistic (h == nullptr: packed into g, PackGrad).
+// 1 = squared (also max |g| of every workgroup, gmax_parts), 2 = logistic (h == nullptr: packed into g, PackGrad).
 // NQ > 0: the matrix has NQ quads, all loaded up front (coalesced, independent
 // loads) and selected in registers; NQ == 0: any width, one dependent load per
 // level, from the byte columns when the matrix has them (bytes != null).
@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(256)
 k_final(const uint32_t *__restrict__ bins, size_t stride, const int *__restrict__ t_fid,
         const int *__restrict__ t_bin, int depth, const float *__restrict__ weights,
         float *__restrict__ yhat, const float *__restrict__ y, unsigned *__restrict__ leaf_of,
-        float *__restrict__ g, float *__restrict__ h, unsigned *__restrict__ gmax_bits, size_t n,
+        float *__restrict__ g, float *__restrict__ h, float *__restrict__ gmax_parts, size_t n,
         BinCode code, const uint8_t *__restrict__ bytes, size_t stride8, int hi_word) {
   extern __shared__ int s_nodes[];  // fid[internal], bin[internal]
   const int internal = (1 << (depth - 1)) - 1;
@@ -178,8 +178,8 @@ k_final(const uint32_t *__restrict__ bins, size_t stride, const int *__restrict_
     }
   }
   if (NEXT_GRAD == 1) {
-    m = WaveMaxF(m);
-    if ((threadIdx.x & 63) == 0) atomicMax(gmax_bits, __float_as_uint(m));
+    m = BlockMaxF(m);
+    if (threadIdx.x == 0) gmax_parts[blockIdx.x] = m;
   }
 }
 
