@@ -58,6 +58,7 @@
 #include "booster.h"
 #include "device_common.h"
 #include "gain.h"
+#include "fused_pass.h"
 #include "kernels_final.h"
 #include "kernels_hist.h"
 #include "kernels_indexed.h"
@@ -547,52 +548,6 @@ struct RowBuffers {
   float *g = nullptr, *h = nullptr;
   unsigned *ids = nullptr;  // indexed mode: the row at each position (null: position = row)
 };
-
-struct FusedArgs {
-  const uint32_t *bins;
-  uint32_t *bins_out;
-  size_t stride;
-  int F;
-  const float *g;
-  float *g_out;
-  const float *h;
-  float *h_out;
-  const int *shifts;
-  const SplitRec *split;
-  const NodeSum *tot;
-  const unsigned *seg_start;
-  const WorkItem *work;
-  const unsigned *n_work;
-  unsigned *cursor;     // claims destinations (null: read item_base)
-  unsigned *item_base;  // claimed destination bases, two per work item
-  unsigned long long *slab;
-  int slab_entries;
-  const uint32_t *split_bins;  // start of the whole matrix
-  int q0;                      // first quad of this launch
-  LevelScan scan;              // hg set: the pass finds the splits of its parents itself
-};
-
-template <bool PAIR, int NQ, bool WRITE, bool GROUP, bool PACK, int HI>
-void LaunchFusedNQ(hipStream_t st, unsigned grid, const FusedArgs &a) {
-  const size_t lds = HistLdsBytes(NQ, PAIR, HI != 0);
-  static std::once_flag configured;
-  AllowLdsOnce(configured, k_part_hist<PAIR, NQ, WRITE, GROUP, PACK, HI>, lds);
-  hipLaunchKernelGGL((k_part_hist<PAIR, NQ, WRITE, GROUP, PACK, HI>), dim3(grid), dim3(kHistThreads), lds, st,
-                     a.bins + (size_t)a.q0 * a.stride, a.bins_out ? a.bins_out + (size_t)a.q0 * a.stride : nullptr,
-                     a.stride, a.F, a.g, a.g_out, a.h, a.h_out, a.shifts, a.split, a.tot, a.seg_start, a.work,
-                     a.n_work, a.cursor, a.item_base, a.slab, a.slab_entries, a.split_bins, a.q0, a.scan);
-}
-
-template <bool PAIR, bool WRITE, bool GROUP, bool PACK, int HI = 0>
-void LaunchFused(int nq, hipStream_t st, unsigned grid, const FusedArgs &a) {
-#define ARB_CASE(N) \
-  case N: LaunchFusedNQ<PAIR, N, WRITE, GROUP, PACK, HI>(st, grid, a); break;
-  switch (nq) {
-    ARB_CASE(1) ARB_CASE(2) ARB_CASE(3) ARB_CASE(4) ARB_CASE(5) ARB_CASE(6) ARB_CASE(7) ARB_CASE(8)
-    default: throw std::runtime_error("internal: bad quad count");
-  }
-#undef ARB_CASE
-}
 
 class HipTreeBuilder : public TreeBuilder {
  public:
@@ -1332,23 +1287,9 @@ class HipTreeBuilder : public TreeBuilder {
                         q0 == 0 ? dst.h : nullptr, d_shifts_, d_split_, d_tot_[ps], d_seg_[ps], d_pwork_,
                         d_nwork_ + 1, q0 == 0 ? d_cursor2_ : nullptr, d_item_left_, d_slab_, slab_stride_, src.bins,
                         q0, scan};
-#define ARB_FUSED(P, W)                                                       \
-  do {                                                                        \
-    if (hi_rows_ && P && pack_) LaunchFused<P, W, false, P, 1>(nq, stream_, grid, a); \
-    else if (hi_rows_) LaunchFused<P, W, false, false, 1>(nq, stream_, grid, a);   \
-    else if (P && pack_ && single_group_) LaunchFused<P, W, false, P>(nq, stream_, grid, a); \
-    else if (P && pack_) LaunchFused<P, W, true, P>(nq, stream_, grid, a);    \
-    else if (single_group_) LaunchFused<P, W, false, false>(nq, stream_, grid, a); \
-    else LaunchFused<P, W, true, false>(nq, stream_, grid, a);                \
-  } while (0)
-            if (pair_) {
-              if (last) ARB_FUSED(true, false);
-              else ARB_FUSED(true, true);
-            } else {
-              if (last) ARB_FUSED(false, false);
-              else ARB_FUSED(false, true);
-            }
-#undef ARB_FUSED
+            const bool group = !single_group_ && !hi_rows_;
+            if (pair_) LaunchFusedPair(!last, group, pack_, hi_rows_, nq, stream_, grid, a);
+            else LaunchFusedSingle(!last, group, hi_rows_, nq, stream_, grid, a);
             if (timing_ && (last || !dominant_only_ || trees_grown_ % sample_every_ == 0))
             ++(last ? timings_.fused_last_launches : timings_.hist_deep_launches);
           }

@@ -10,6 +10,28 @@
 #include "gain.h"
 
 namespace arb {
+
+struct NodeSum {
+  long long g;
+  long long h;
+  unsigned long long c;
+};
+
+struct SplitRec {
+  float gain;
+  int fid;   // -1: not split (every row stays left)
+  int bin;
+  unsigned pad;
+  NodeSum left;
+};
+
+struct WorkItem {
+  unsigned node;
+  unsigned begin;  // row range in the current order
+  unsigned end;
+  unsigned first;  // index of the first work item of this node
+};
+
 namespace {
 
 #define HIP_OK(expr)                                                                        \
@@ -73,27 +95,6 @@ __host__ __device__ __forceinline__ void UnpackGrad(float u, float *g, float *h)
   *g = y - s;
   *h = s * (1.0f - s);
 }
-
-struct NodeSum {
-  long long g;
-  long long h;
-  unsigned long long c;
-};
-
-struct SplitRec {
-  float gain;
-  int fid;   // -1: not split (every row stays left)
-  int bin;
-  unsigned pad;
-  NodeSum left;
-};
-
-struct WorkItem {
-  unsigned node;
-  unsigned begin;  // row range in the current order
-  unsigned end;
-  unsigned first;  // index of the first work item of this node
-};
 
 // How bin ids are packed in the 32-bit words of a row: 8 bits (four features
 // per word) or 16 bits (two features per word).

@@ -1,6 +1,8 @@
 // Row partition, the fused partition + histogram pass, slab reduction.
 #ifndef ARBORETUM_AMD_KERNELS_PARTITION_H_
 #define ARBORETUM_AMD_KERNELS_PARTITION_H_
+#include <type_traits>
+
 #include "device_common.h"
 #include "kernels_hist.h"
 #include "kernels_plan.h"
@@ -141,24 +143,31 @@ __device__ __forceinline__ unsigned CountWaveLefts(const WorkItem &it, const Spl
       if constexpr (HI != 0) return test.Right(v);
       else return (int)((v >> fs) & 255u) > s.bin;
     };
-    constexpr int kBatch = 24;  // loads in flight per wave: all of a typical item at once
-    for (int k0 = nk - 1; k0 >= 0; k0 -= kBatch) {
-      uint32_t v0[kBatch], v1[kBatch];
+    // Loads in flight per wave: as many as the item has chunks, up to 24 at a time (all of a typical
+    // item of a large matrix at once; the ones past the last chunk read its first rows again).
+    auto batches = [&](auto size) {
+      constexpr int kBatch = decltype(size)::value;
+      for (int k0 = nk - 1; k0 >= 0; k0 -= kBatch) {
+        uint32_t v0[kBatch], v1[kBatch];
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const int k = max(k0 - j, 0);
-        const unsigned r0 = wb + (unsigned)k * kChunkStep + lane, r1 = r0 + 64;
-        v0[j] = col[min(r0, we - 1)];
-        v1[j] = col[min(r1, we - 1)];
-      }
+        for (int j = 0; j < kBatch; ++j) {
+          const int k = max(k0 - j, 0);
+          const unsigned r0 = wb + (unsigned)k * kChunkStep + lane, r1 = r0 + 64;
+          v0[j] = col[min(r0, we - 1)];
+          v1[j] = col[min(r1, we - 1)];
+        }
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const int k = k0 - j;
-        const unsigned r0 = wb + (unsigned)max(k, 0) * kChunkStep + lane, r1 = r0 + 64;
-        if (k >= 0 && r0 >= it.begin && r0 < we) cnt += right(v0[j]) ? 0u : 1u;
-        if (k >= 0 && r1 < we) cnt += right(v1[j]) ? 0u : 1u;
+        for (int j = 0; j < kBatch; ++j) {
+          const int k = k0 - j;
+          const unsigned r0 = wb + (unsigned)max(k, 0) * kChunkStep + lane, r1 = r0 + 64;
+          if (k >= 0 && r0 >= it.begin && r0 < we) cnt += right(v0[j]) ? 0u : 1u;
+          if (k >= 0 && r1 < we) cnt += right(v1[j]) ? 0u : 1u;
+        }
       }
-    }
+    };
+    // (an item of 2048 rows, one chunk per wave, spent 5 us on 23 loads it did not need)
+    if (nk <= 8) batches(std::integral_constant<int, 8>());
+    else batches(std::integral_constant<int, 24>());
   }
   for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
   return cnt;
@@ -166,7 +175,7 @@ __device__ __forceinline__ unsigned CountWaveLefts(const WorkItem &it, const Spl
 
 // Destination offsets of a wave of the fused pass without a counting launch:
 // the waves count their rows going left (CountWaveLefts), the workgroup claims
-// its share of the two children's row ranges with one atomic add per child on
+// its share of the two children's row ranges with one atomic add on
 // the node's pair of cursors (zero at launch), and the waves take their parts
 // in wave order.  The order of the work items inside a child's range depends
 // on the order of the claims; no result depends on it (all sums are integers).
@@ -187,8 +196,11 @@ __device__ __forceinline__ void ClaimWithCount(const WorkItem &it, unsigned w, c
       unsigned lefts = 0;
       for (int k = 0; k < kItemWaves; ++k) lefts += s_tmp[k];
       const unsigned rows = it.end - it.begin;
-      item_base[2 * w] = s_tmp[kItemWaves] = atomicAdd(&cursor[2 * it.node], lefts);
-      item_base[2 * w + 1] = s_tmp[kItemWaves + 1] = atomicAdd(&cursor[2 * it.node + 1], rows - lefts);
+      // both cursors of the node in one atomic (neither passes the rows of its child, so nothing carries over)
+      const unsigned long long claim = atomicAdd(reinterpret_cast<unsigned long long *>(cursor) + it.node,
+                                                 (unsigned long long)lefts | ((unsigned long long)(rows - lefts) << 32));
+      item_base[2 * w] = s_tmp[kItemWaves] = (unsigned)claim;
+      item_base[2 * w + 1] = s_tmp[kItemWaves + 1] = (unsigned)(claim >> 32);
     } else {
       s_tmp[kItemWaves] = item_base[2 * w];
       s_tmp[kItemWaves + 1] = item_base[2 * w + 1];
@@ -417,18 +429,30 @@ k_part_hist(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
   if (own_scan && w == 0) WriteEmptyNodes(scan, tot, seg_start);
   if (w >= *n_work) return;
   const WorkItem it = work[w];
+  static_assert(!(HI && GROUP), "ninth bits: one group of quads only");
+  constexpr int NW = NQ + HI;  // words of a row
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
+  auto load_rows = [&](RowSet<NW> &R, unsigned base) {
+    const unsigned a0 = min(base + lane, we - 1), a1 = min(base + 64 + lane, we - 1);
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      R.b0[q] = __builtin_nontemporal_load(&bins[(size_t)q * stride + a0]);
+      R.b1[q] = __builtin_nontemporal_load(&bins[(size_t)q * stride + a1]);
+    }
+    R.g0 = __builtin_nontemporal_load(&g[a0]);
+    R.g1 = __builtin_nontemporal_load(&g[a1]);
+    R.h0 = PAIR && !PACK ? __builtin_nontemporal_load(&h[a0]) : 0.0f;
+    R.h1 = PAIR && !PACK ? __builtin_nontemporal_load(&h[a1]) : 0.0f;
+  };
   const SplitRec s = own_scan ? SelectInPass(scan, (int)it.node, tot[it.node], seg_start,
                                              w == scan.node_first[it.node], &s_rec)
                               : split[it.node];
   const unsigned long long cl = s.left.c, cr = tot[it.node].c - cl;
   const bool build_right = cl > cr;  // ties -> left (hist_grad_sum.cu:288-290)
-  static_assert(!(HI && GROUP), "ninth bits: one group of quads only");
-  constexpr int NW = NQ + HI;  // words of a row
   constexpr int words = (int)(HistLdsBytes(NQ, PAIR, HI != 0) / 8);
   for (int i = threadIdx.x; i < words; i += kHistThreads) lds[i] = 0ull;
   const int sg = shifts[0], sh = shifts[1];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
   // which word of a row decides, and how (HI: the ninth-bit word for a split at bin 255; without
   // ninth bits the byte test is spelled out, the pass has no register to spare)
   const SplitTest test = MakeSplitTest(s, BinCode{2, 8}, HI ? NQ : -1);
@@ -452,21 +476,15 @@ k_part_hist(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
     // row of the item) and the sets are never copied, so every wait in the loop
     // is for exactly the set that is needed next.
     const uint32_t *split_col = split_bins + (size_t)fq * stride;
-    auto load = [&](RowSet<NW> &R, unsigned base) {
-      const unsigned a0 = min(base + lane, we - 1), a1 = min(base + 64 + lane, we - 1);
-#pragma unroll
-      for (int q = 0; q < NW; ++q) {
-        R.b0[q] = __builtin_nontemporal_load(&bins[(size_t)q * stride + a0]);
-        R.b1[q] = __builtin_nontemporal_load(&bins[(size_t)q * stride + a1]);
-      }
+    auto load_split = [&](RowSet<NW> &R, unsigned base) {
       if (GROUP) {  // the quad of the split feature, wherever it lives
-        R.s0 = split_col[a0];
-        R.s1 = split_col[a1];
+        R.s0 = split_col[min(base + lane, we - 1)];
+        R.s1 = split_col[min(base + 64 + lane, we - 1)];
       }
-      R.g0 = __builtin_nontemporal_load(&g[a0]);
-      R.g1 = __builtin_nontemporal_load(&g[a1]);
-      R.h0 = PAIR && !PACK ? __builtin_nontemporal_load(&h[a0]) : 0.0f;
-      R.h1 = PAIR && !PACK ? __builtin_nontemporal_load(&h[a1]) : 0.0f;
+    };
+    auto load = [&](RowSet<NW> &R, unsigned base) {
+      load_rows(R, base);
+      load_split(R, base);
     };
     auto process = [&](const RowSet<NW> &R, unsigned base) {
       const unsigned r0 = base + lane, r1 = r0 + 64;

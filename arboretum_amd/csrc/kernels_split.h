@@ -5,14 +5,36 @@
 #include "kernels_plan.h"
 
 namespace arb {
-namespace {
 
-// --------------------------------------------------------------- split scan
+// The best candidate of one feature of a node (bin -1: none).
 struct Cand {
   float gain;
   int bin;
   NodeSum left;
 };
+
+// What a fused pass over the rows of a level's nodes needs to select the splits of those nodes
+// itself, in its prologue, from the per-feature candidates of the split scan (k_split_scan)
+// instead of reading them from a selection kernel launched before it: one launch less per level
+// on the critical path.  Every workgroup of the pass selects for ITS node; the node's first work
+// item also writes the node's record.  cand == null: the splits are read from `split` as before.
+struct LevelScan {
+  const Cand *cand;
+  int F, L;
+  NodeSum *tot_next;
+  unsigned *seg_next;
+  SplitRec *split;
+  int *t_fid, *t_bin;
+  float *t_gain;
+  int heap_off;
+  const unsigned char *active;
+  const unsigned *node_first;         // first work item of every node: that item writes the node's record
+  unsigned long long *rows_scanned;   // advanced by the rows of the smaller side of every split
+};
+
+namespace {
+
+// --------------------------------------------------------------- split scan
 
 // One wave scans one (feature, node): inclusive prefix over the slots, gain
 // per bin < hist_size, arg-max with ties to the HIGHEST bin (builder.h:39-49),
@@ -160,24 +182,31 @@ __device__ __forceinline__ SplitRec WriteNode(int nd, const NodeSum &t, float ga
   return rec;
 }
 
-// What a fused pass over the rows of a level's nodes needs to select the splits of those nodes
-// itself, in its prologue, from the per-feature candidates of the split scan (k_split_scan)
-// instead of reading them from a selection kernel launched before it: one launch less per level
-// on the critical path.  Every workgroup of the pass selects for ITS node; the node's first work
-// item also writes the node's record.  cand == null: the splits are read from `split` as before.
-struct LevelScan {
-  const Cand *cand;
-  int F, L;
-  NodeSum *tot_next;
-  unsigned *seg_next;
-  SplitRec *split;
-  int *t_fid, *t_bin;
-  float *t_gain;
-  int heap_off;
-  const unsigned char *active;
-  const unsigned *node_first;         // first work item of every node: that item writes the node's record
-  unsigned long long *rows_scanned;   // advanced by the rows of the smaller side of every split
-};
+
+// The best of a node's per-feature candidates over the features active at its level: the highest
+// gain, ties to the lowest feature id (hist_tree_grower.cu:59-60).  One wave; every lane gets the
+// feature (-1: no candidate) and the candidate.  Gains of candidates are positive, so their bits order
+// like the gains, and one 64-bit maximum of (gain, ~feature) decides: two shuffles per step instead of
+// one for every word of a candidate (2.4 -> 1.6 us of the prologue of a pass).
+__device__ __forceinline__ int BestOfNode(const Cand *__restrict__ cand, int F, const unsigned char *__restrict__ active,
+                                          int lane, Cand *best) {
+  unsigned long long key = 0;  // larger than that of no candidate: the gain of a candidate is positive
+  for (int f = lane; f < F; f += 64) {
+    if (active && !active[f]) continue;  // feature not sampled at this level
+    if (cand[f].bin < 0) continue;
+    const unsigned long long k = ((unsigned long long)__float_as_uint(cand[f].gain) << 32) | (0xffffffffu - (unsigned)f);
+    key = max(key, k);
+  }
+  for (int off = 32; off > 0; off >>= 1) key = max(key, (unsigned long long)__shfl_xor(key, off));
+  best->gain = 0.0f;
+  best->bin = -1;
+  best->left.g = best->left.h = 0;
+  best->left.c = 0;
+  if (key == 0) return -1;  // uniform
+  const int fid = (int)__builtin_amdgcn_readfirstlane(0xffffffffu - (unsigned)key);
+  *best = cand[fid];
+  return fid;
+}
 
 // Split of node nd (totals t) from its candidates: wave 0 of the workgroup keeps the candidate
 // with the highest gain, ties to the lowest feature id (hist_tree_grower.cu:59-60), over the
@@ -189,40 +218,15 @@ __device__ __forceinline__ SplitRec SelectInPass(const LevelScan &a, int nd, con
                                                  SplitRec *s_rec) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (wave == 0) {
-    float gain = 0.0f;
-    int fid = -1, bin = -1;
-    long long lg = 0, lh = 0;
-    unsigned long long lc = 0;
-    if (t.c != 0) {
-      for (int f = lane; f < a.F; f += 64) {
-        if (a.active && !a.active[f]) continue;  // feature not sampled at this level
-        const Cand c = a.cand[(size_t)nd * a.F + f];
-        if (c.bin >= 0 && (fid < 0 || gain < c.gain)) {
-          gain = c.gain;
-          fid = f;
-          bin = c.bin;
-          lg = c.left.g;
-          lh = c.left.h;
-          lc = c.left.c;
-        }
-      }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      const float og = __shfl_down(gain, off);
-      const int of = __shfl_down(fid, off);
-      const int ob = __shfl_down(bin, off);
-      const long long olg = __shfl_down(lg, off);
-      const long long olh = __shfl_down(lh, off);
-      const unsigned long long olc = __shfl_down(lc, off);
-      if (of >= 0 && (fid < 0 || og > gain || (og == gain && of < fid))) {
-        gain = og;
-        fid = of;
-        bin = ob;
-        lg = olg;
-        lh = olh;
-        lc = olc;
-      }
-    }
+    Cand c;
+    c.gain = 0.0f;
+    c.bin = -1;
+    c.left = NodeSum{0, 0, 0};
+    const int fid = t.c == 0 ? -1 : BestOfNode(a.cand + (size_t)nd * a.F, a.F, a.active, lane, &c);
+    const float gain = c.gain;
+    const int bin = c.bin;
+    const long long lg = c.left.g, lh = c.left.h;
+    const unsigned long long lc = c.left.c;
     if (lane == 0) {
       SplitRec rec;
       if (write) {
@@ -295,42 +299,14 @@ __device__ __forceinline__ void SelectNode(int nd, int lane, const Cand *__restr
                                            int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
                                            const unsigned char *__restrict__ active) {
   const NodeSum t = tot[nd];
-  float gain = 0.0f;
-  int fid = -1, bin = -1;
-  long long lg = 0, lh = 0;
-  unsigned long long lc = 0;
-  if (t.c != 0) {
-    for (int f = lane; f < F; f += 64) {
-      if (active && !active[f]) continue;  // feature not sampled at this level
-      const Cand c = cand[(size_t)nd * F + f];
-      if (c.bin >= 0 && (fid < 0 || gain < c.gain)) {
-        gain = c.gain;
-        fid = f;
-        bin = c.bin;
-        lg = c.left.g;
-        lh = c.left.h;
-        lc = c.left.c;
-      }
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    const float og = __shfl_down(gain, off);
-    const int of = __shfl_down(fid, off);
-    const int ob = __shfl_down(bin, off);
-    const long long olg = __shfl_down(lg, off);
-    const long long olh = __shfl_down(lh, off);
-    const unsigned long long olc = __shfl_down(lc, off);
-    if (of >= 0 && (fid < 0 || og > gain || (og == gain && of < fid))) {
-      gain = og;
-      fid = of;
-      bin = ob;
-      lg = olg;
-      lh = olh;
-      lc = olc;
-    }
-  }
+  Cand c;
+  c.gain = 0.0f;
+  c.bin = -1;
+  c.left = NodeSum{0, 0, 0};
+  const int fid = t.c == 0 ? -1 : BestOfNode(cand + (size_t)nd * F, F, active, lane, &c);
   if (lane != 0) return;
-  WriteNode(nd, t, gain, fid, bin, lg, lh, lc, seg_start, tot_next, seg_next, split, t_fid, t_bin, t_gain, heap_off);
+  WriteNode(nd, t, c.gain, fid, c.bin, c.left.g, c.left.h, c.left.c, seg_start, tot_next, seg_next, split, t_fid, t_bin,
+            t_gain, heap_off);
 }
 
 // grid ceil(L / 16), 1024 threads: one wave per node

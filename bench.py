@@ -37,7 +37,7 @@ TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "hbm_traffic_headline_10.5Mx28_
 # every source that shapes the dominant launch: the kernel, the LDS update order, the work plan
 # (item sizes, claims) and the host code that sizes and launches it
 KERNEL_SOURCES = ["kernels_partition.h", "kernels_hist.h", "device_common.h", "kernels_plan.h", "kernels_launch.h",
-                  "kernels_split.h", "device_builder.hip"]
+                  "kernels_split.h", "fused_pass_launch.h", "device_builder.hip"]
 # The LDS co-limit of the kernels that accumulate histograms: an update of one wave (64 rows, one
 # feature each) is two ds_add_u64 wave instructions (sum of g with the count, sum of h); the LDS
 # atomic unit of a compute unit sustains one such instruction per 7.3 cycles at 2.4 GHz when no
