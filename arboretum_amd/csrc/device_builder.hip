@@ -969,6 +969,7 @@ class HipTreeBuilder : public TreeBuilder {
   void RowsScannedByLevel(unsigned long long *out) override {  // kScanLevels entries
     HIP_OK(hipStreamSynchronize(stream_));
     HIP_OK(hipMemcpy(out, d_rows_scanned_, kScanLevels * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    out[0] += root_rows_scanned_;  // (root histograms of resident matrices are counted on the host)
   }
   void StreamResidency(unsigned long long *resident, unsigned long long *blocks) override {
     *resident = resident_blocks_;
@@ -1035,13 +1036,6 @@ class HipTreeBuilder : public TreeBuilder {
   // the counter of rows accumulated into histograms at `level` (levels past the last counter share it)
   unsigned long long *ScanCounter(int level) { return d_rows_scanned_ + std::min(level, kScanLevels - 1); }
   // count_level >= 0: the planned rows are histogram work of that tree level
-  // cursor: two claim cursors per node, cleared by the plan (passes that claim their output ranges)
-  void Plan(int state, int L, int select, unsigned rows_per_item, WorkItem *work, unsigned *n_work,
-            int count_level, const SplitRec *split, unsigned max_items, unsigned balance_cus = 0,
-            unsigned *cursor = nullptr) {
-    PlanOn(d_tot_[state], d_seg_[state], L, select, rows_per_item, work, n_work, count_level, split, max_items,
-           balance_cus, cursor);
-  }
   void PlanOn(const NodeSum *tot, const unsigned *seg, int L, int select, unsigned rows_per_item, WorkItem *work,
               unsigned *n_work, int count_level, const SplitRec *split, unsigned max_items,
               unsigned balance_cus = 0, unsigned *cursor = nullptr) {
@@ -1051,37 +1045,48 @@ class HipTreeBuilder : public TreeBuilder {
                        d_overflow_, balance_cus, cursor);
   }
 
-  // Histograms of contiguous node ranges in `cur` (level order), feature group by group.
-  void HistOfNodes(const RowBuffers &cur, int state, int L, bool select_smaller, size_t rows_max, bool root, int level) {
-    // A CU holds one work item at a time, so the launch runs in rounds of cus_ items: the planner
-    // sizes the items from the rows and nodes it finds selected so that the rounds are full
-    // (one item per CU at the root); the grid holds the rounds of the largest case.
-    // Rows in place in groups of quads: the root, whose rows are the matrix in its own order,
-    // is read from the quad columns like a narrow matrix (one launch per group streams its
-    // columns once; the groups of the record kernel share only half of their reads there).
-    const bool records = indexed_ && (rec_one_launch_ || !root);
-    const unsigned cus = records ? hist_cus_ : cus_;
-    const unsigned grid = std::min(BalancedPlanItems(rows_max, (unsigned)L, kMaxHistRows, cus), max_hist_items_);
-    Mark(kPlan);
-    Plan(state, L, select_smaller ? 1 : 0, kMaxHistRows, d_hwork_, d_nwork_, level, nullptr, grid, cus);
+  // ---- plans of stand-alone histogram launches.
+  // A CU holds one work item at a time, so the launch runs in rounds of as many items as it has compute
+  // units to itself: the planner sizes the items from the rows and nodes it finds selected so that the
+  // rounds are full (one item per CU at the root); the grid holds the rounds of the largest case.
+  // Rows in place in groups of quads: the root, whose rows are the matrix in its own order,
+  // is read from the quad columns like a narrow matrix (one launch per group streams its
+  // columns once; the groups of the record kernel share only half of their reads there).
+  bool HistOnRecords(bool root) const { return indexed_ && (rec_one_launch_ || !root); }
+  unsigned HistCus(bool root) const {
+    if (wide_) return std::max(1u, cus_ / (unsigned)WideGroups());
+    return HistOnRecords(root) ? hist_cus_ : cus_;
+  }
+  int WideGroups() const { return (F_ + wide_group_ - 1) / wide_group_; }
+  unsigned HistGrid(int L, bool root) const {
+    const size_t rows_max = root || !trick_ ? n_ : n_ / 2;
+    return std::min(BalancedPlanItems(rows_max, (unsigned)L, kMaxHistRows, HistCus(root)), max_hist_items_);
+  }
+  // rows per work item of the root histogram (k_tree_end and k_first_root plan it)
+  unsigned RootRowsPerItem() const {
+    unsigned items = 0;
+    return BalancedRowsPerItem(n_, 1, kMaxHistRows, HistCus(true), &items);
+  }
+
+  // Histograms of contiguous node ranges in `cur` (level order); the work plan is in d_hwork_.
+  void HistOfNodes(const RowBuffers &cur, int L, bool root) {
+    const bool records = HistOnRecords(root);
+    const unsigned grid = HistGrid(L, root);
+    if (root) root_rows_scanned_ += n_;
     Mark(root ? kHistRoot : kHistDeep);
     if (wide_) {
-      for (int f0 = 0; f0 < F_; f0 += wide_group_) {
-        const int nf = std::min(wide_group_, F_ - f0);
-        const size_t lds = (size_t)nf * slots_ * 8 * (pair_ ? 2 : 1);
-        if (pair_) {
-          static std::once_flag configured;
-          AllowLdsOnce(configured, k_hist_wide<true>, kLdsBudget);
-          hipLaunchKernelGGL(k_hist_wide<true>, dim3(grid), dim3(kHistThreads), lds, stream_, cur.bins, stride_, f0, nf,
-                             slots_, cur.g, cur.h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_entries_);
-        } else {
-          static std::once_flag configured;
-          AllowLdsOnce(configured, k_hist_wide<false>, kLdsBudget);
-          hipLaunchKernelGGL(k_hist_wide<false>, dim3(grid), dim3(kHistThreads), lds, stream_, cur.bins, stride_, f0, nf,
-                             slots_, cur.g, cur.h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_entries_);
-        }
-        if (timing_) ++(root ? timings_.hist_root_launches : timings_.hist_deep_launches);
-      }
+      const size_t lds = (size_t)std::min(wide_group_, F_) * slots_ * 8 * (pair_ ? 2 : 1);
+#define ARB_HIST_WIDE(P)                                                                                              \
+  do {                                                                                                                \
+    static std::once_flag configured;                                                                                 \
+    AllowLdsOnce(configured, k_hist_wide<P>, kLdsBudget);                                                             \
+    hipLaunchKernelGGL(k_hist_wide<P>, dim3(grid, WideGroups()), dim3(kHistThreads), lds, stream_, cur.bins, stride_, \
+                       F_, wide_group_, slots_, cur.g, cur.h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_entries_); \
+  } while (0)
+      if (pair_) ARB_HIST_WIDE(true);
+      else ARB_HIST_WIDE(false);
+#undef ARB_HIST_WIDE
+      if (timing_) ++(root ? timings_.hist_root_launches : timings_.hist_deep_launches);
       if (timing_ && root) timings_.hist_root_rows += n_;
       return;
     }
@@ -1134,16 +1139,13 @@ class HipTreeBuilder : public TreeBuilder {
     if (timing_ && root) timings_.hist_root_rows += n_;
   }
 
-  // Gradient totals of the root: the sum over the slots of feature 0 of the root histogram, or, when
-  // ids of 256 are left out of the histograms, over the gradients themselves (tot[0].g / .h are
-  // zero: k_init_root).
-  void RootTotals(int hb, int state, const RowBuffers &orig) {
+  // Gradient totals of the root are the sum over the slots of feature 0 of the root histogram, made by
+  // its split scan (root_sum), or, when ids of 256 are left out of the histograms, the sum over the
+  // gradients themselves (tot[0].g / .h are zero then: k_first_root, k_tree_end, k_init_root).
+  void RootTotals(int state, const RowBuffers &orig) {
     if (hi_skip_)
       hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, orig.g,
                          pair_ ? orig.h : nullptr, 0, n_, d_shifts_, d_tot_[state]);
-    else
-      hipLaunchKernelGGL(k_root_from_hist, dim3(1), dim3(64), 0, stream_, d_hg_[hb], d_hh_[hb], d_tot_[state], slots_,
-                         hi_base_);
   }
 
   // k_hist over quads [q0, q0 + nq) of rows laid out with `stride` words between columns
@@ -1164,8 +1166,9 @@ class HipTreeBuilder : public TreeBuilder {
       LaunchHist<false>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_);
   }
 
-  // plan_state >= 0: one more block plans the fused pass over this level's nodes (d_tot_ / d_seg_
-  // [plan_state]) into the other set of (first item, items) per node, which is in use afterwards
+  // plan_state >= 0: one more block plans the row pass over this level's nodes (d_tot_ / d_seg_
+  // [plan_state]) that follows: the fused pass, whose slabs the next reduction finds by it, into the other
+  // set of (first item, items) per node, which is in use afterwards; or the partition of the other paths.
   void Reduce(int L, int hb, bool by_parent, int parent_state, bool trick, bool accumulate = false,
               int plan_state = -1) {
     Mark(kReduce);
@@ -1177,12 +1180,12 @@ class HipTreeBuilder : public TreeBuilder {
       plan.tot = d_tot_[plan_state];
       plan.seg_start = d_seg_[plan_state];
       plan.L = L;
-      plan.rows_per_item = FusedRowsPerItem(L);
+      plan.rows_per_item = fused_ ? FusedRowsPerItem(L) : part_rows_;
       plan.work = d_pwork_;
       plan.n_work = d_nwork_ + 1;
       plan.node_first = next_first;
       plan.node_items = next_items;
-      plan.max_items = FusedGrid(L);
+      plan.max_items = fused_ ? FusedGrid(L) : PartGrid(L);
       plan.overflow = d_overflow_;
       plan.cursor = d_cursor2_;
     }
@@ -1211,7 +1214,7 @@ class HipTreeBuilder : public TreeBuilder {
       else ARB_REDUCE(false, 16);
     }
 #undef ARB_REDUCE
-    if (plan_state >= 0) {
+    if (plan_state >= 0 && fused_) {
       d_node_first_ = next_first;
       d_node_items_ = next_items;
     }
@@ -1230,10 +1233,11 @@ class HipTreeBuilder : public TreeBuilder {
       return;
     }
 
-    // (the last pass of the previous tree has done this when it built the root histogram)
-    if (!root_hist_ready_)
-      hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0],
-                         (unsigned long long)n_);
+    // (the end of the previous tree has done this)
+    if (!root_planned_)
+      hipLaunchKernelGGL(k_first_root, dim3(1), dim3(256), 0, stream_, d_tot_[0], d_seg_[0], (unsigned)n_,
+                         RootRowsPerItem(), d_hwork_, d_nwork_, d_node_first_, d_node_items_);
+    root_planned_ = false;
     // The last pass of the tree can also build the root histogram of the next
     // one: logistic objective, gradients of the next round wanted, all quads in
     // one LDS histogram next to the node arrays.
@@ -1248,12 +1252,11 @@ class HipTreeBuilder : public TreeBuilder {
       const bool last = level + 2 >= D_;
       if (level == 0) {
         // the slabs of the root may have been written by the last pass of the previous tree
-        if (!root_hist_ready_) HistOfNodes(orig, state, 1, false, n_, true, 0);
+        if (!root_hist_ready_) HistOfNodes(orig, 1, true);
         root_hist_ready_ = false;
-        Reduce(1, hb, false, state, false, false, own_scan_ && !last ? state : -1);
-        // (the last pass of the previous tree has also summed the root's totals)
-        if (!root_totals_ready_) RootTotals(hb, state, orig);
-        root_totals_ready_ = false;
+        Reduce(1, hb, false, state, false, false, last ? -1 : state);
+        // (the last pass of the previous tree may have summed the root's totals)
+        if (!root_totals_ready_) RootTotals(state, orig);
       } else {
         // rows are in the order of level-1; the parents' state is state ^ 1
         const int ps = state ^ 1, PL = L >> 1;
@@ -1293,11 +1296,9 @@ class HipTreeBuilder : public TreeBuilder {
             if (timing_ && (last || !dominant_only_ || trees_grown_ % sample_every_ == 0))
             ++(last ? timings_.fused_last_launches : timings_.hist_deep_launches);
           }
-          Reduce(L, hb, true, ps, true, false, own_scan_ && !last ? state : -1);
+          Reduce(L, hb, true, ps, true, false, last ? -1 : state);
         } else {
-          const unsigned grid = (unsigned)std::min<size_t>(n_ / part_rows_ + 2 * PL + 1, max_part_items_);
-          Mark(kPlan);
-          Plan(ps, PL, 0, part_rows_, d_pwork_, d_nwork_ + 1, -1, nullptr, grid, 0, indexed_ ? d_cursor2_ : nullptr);
+          const unsigned grid = PartGrid(PL);  // (planned by the reduction of the level above)
           Mark(kPartition);
           if (indexed_) {
             // decisions, claims of the children's ranges and the move of (row id, g, h) in one launch
@@ -1314,61 +1315,62 @@ class HipTreeBuilder : public TreeBuilder {
                                d_pwork_, d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_);
             LaunchPartRows(grid, src, dst, ps);
           }
-          HistOfNodes(dst, state, L, trick_, trick_ ? n_ / 2 : n_, false, level);
-          Reduce(L, hb, false, ps, trick_);
+          HistOfNodes(dst, L, false);  // (planned with the splits of the level above)
+          Reduce(L, hb, false, ps, trick_, false, last ? -1 : state);
         }
       }
       if (inspect_) KeepHist(level, L, hb, state);
-      // (own_scan_: only the scan; the pass of the next level selects the splits of this level's nodes)
-      LaunchSplit(level, L, hb, state, gp, fused_ && !last, own_scan_ && !last);
-      if (last && !final_hist) LaunchLeafWeights(L, state, gp);
+      // own_scan_: the pass of the next level selects the splits of this level's nodes; those of the last
+      // level are selected at the end of the tree
+      LaunchScan(level, L, hb, state, gp, level == 0 && !root_totals_ready_ && !hi_skip_);
+      root_totals_ready_ = false;
+      if (!last && !own_scan_) LaunchSelect(level, L, state);
       state ^= 1;
     }
     // ---- leaf of every row, y_hat update, gradients of the next round
     Mark(kLeaf);
-    bool record_written = false;
-    {
-      if (final_hist) {
-        // leaf weights, tree record, state and plan of the next tree's root in
-        // one launch, then one pass: leaves, predictions, gradients and the
-        // root histogram of the next tree
-        const int last_L = 1 << (D_ - 2), last_state = state ^ 1;
-        const unsigned per_item = HistRowsPerItem(n_, 256);
-        const unsigned grid = (unsigned)std::min<size_t>(n_ / per_item + 2, max_hist_items_);
-        if ((n_ + per_item - 1) / per_item > grid) throw std::runtime_error("internal: root plan exceeds its grid");
-#define ARB_END(D)                                                                                                \
-  hipLaunchKernelGGL((k_tree_end<true, D>), dim3((last_L + 127) / 128 + 1), dim3(128), 0, stream_, d_split_,      \
-                     d_tot_[last_state], last_L, d_shifts_, gp, cfg_.tree.eta, d_weights_, d_tfid_, d_tbin_,      \
-                     d_tgain_, d_overflow_, d_records_ + pending_.size() * RecordWords(), d_tot_[0], d_seg_[0],   \
-                     (unsigned)n_, per_item, d_hwork_, d_nwork_, d_node_first_, d_node_items_, d_rows_scanned_)
-        if (f64_) ARB_END(true);
-        else ARB_END(false);
-#undef ARB_END
-        record_written = true;
-        LaunchFinalHist(grid, label, final_lds);
-        root_hist_ready_ = true;
-        root_totals_ready_ = true;
-        leaf_valid_ = false;  // not recorded by this pass; GetLeaves walks the tree when asked
-      } else {
-        LaunchFinal(dm_->bins, stride_, 0, n_, label, next_grad);
-        leaf_valid_ = true;
-      }
-      grad_ready_ = next_grad;
+    const int last_state = state ^ 1;
+    if (final_hist) {
+      // one pass: leaves, predictions, gradients and the root histogram of the next tree
+      const unsigned per_item = HistRowsPerItem(n_, 256);
+      const unsigned grid = (unsigned)std::min<size_t>(n_ / per_item + 2, max_hist_items_);
+      if ((n_ + per_item - 1) / per_item > grid) throw std::runtime_error("internal: root plan exceeds its grid");
+      LaunchTreeEnd(last_state, gp, per_item);
+      LaunchFinalHist(grid, label, final_lds);
+      root_rows_scanned_ += n_;
+      root_hist_ready_ = true;
+      root_totals_ready_ = true;
+      leaf_valid_ = false;  // not recorded by this pass; GetLeaves walks the tree when asked
+    } else {
+      LaunchTreeEnd(last_state, gp, RootRowsPerItem());
+      LaunchFinal(dm_->bins, stride_, 0, n_, label, next_grad);
+      leaf_valid_ = true;
     }
-    if (record_written) Mark(kNone);
-    else
-      EnqueueRecord();
+    root_planned_ = true;
+    grad_ready_ = next_grad;
+    Mark(kNone);
   }
 
-  // Tree record into the next slot of the device ring; FlushTrees reads it.
-  size_t RecordWords() const { return (size_t)3 * ((1 << (D_ - 1)) - 1) + (size_t)(1 << (D_ - 1)) + 1; }
-  void EnqueueRecord() {
-    Mark(kNone);
-    const int internal = (1 << (D_ - 1)) - 1, leaves = 1 << (D_ - 1);
-    hipLaunchKernelGGL(k_pack_record, dim3((leaves + 255) / 256), dim3(256), 0, stream_, d_tfid_, d_tbin_, d_tgain_,
-                       d_weights_, d_overflow_, internal, leaves, d_records_ + pending_.size() * RecordWords());
+  // Splits of the last level, leaf weights, record (into the next slot of the device ring; FlushTrees reads it)
+  // and, with rows_per_item, the state and plan of the next tree's root.
+  void LaunchTreeEnd(int last_state, const GainParams &gp, unsigned rows_per_item) {
+    const int L = 1 << (D_ - 2);
+    const unsigned char *active = sampling_ ? d_active_ + (size_t)(D_ - 2) * F_ : (const unsigned char *)nullptr;
+#define ARB_END(P, D)                                                                                              \
+  hipLaunchKernelGGL((k_tree_end<P, D>), dim3((L + 3) / 4 + 1), dim3(256), 0, stream_, d_cand_, F_, active,        \
+                     d_tot_[last_state], L, d_shifts_, gp, cfg_.tree.eta, d_weights_, d_tfid_, d_tbin_, d_tgain_,  \
+                     d_overflow_, d_records_ + pending_.size() * RecordWords(), d_tot_[0], d_seg_[0],              \
+                     (unsigned)n_, rows_per_item, rows_per_item ? d_hwork_ : (WorkItem *)nullptr, d_nwork_,        \
+                     d_node_first_, d_node_items_)
+    if (pair_ && f64_) ARB_END(true, true);
+    else if (pair_) ARB_END(true, false);
+    else if (f64_) ARB_END(false, true);
+    else ARB_END(false, false);
+#undef ARB_END
     HIP_OK(hipGetLastError());
   }
+
+  size_t RecordWords() const { return (size_t)3 * ((1 << (D_ - 1)) - 1) + (size_t)(1 << (D_ - 1)) + 1; }
 
   // ---- streamed matrices -------------------------------------------------
   // Block `b` of the matrix into one of the two device buffers, on the copy
@@ -1424,52 +1426,48 @@ class HipTreeBuilder : public TreeBuilder {
     return buf;
   }
 
-  // plan_next: also plan the fused pass of the next level over these nodes
-  // scan_only: candidates per (node, feature) only (k_split_scan); the next fused pass selects
-  void LaunchSplit(int level, int L, int hb, int state, const GainParams &gp, bool plan_next = false,
-                   bool scan_only = false) {
+  // Candidates per (node, feature) of a level.
+  void LaunchScan(int level, int L, int hb, int state, const GainParams &gp, bool root_sum) {
     Mark(kSplit);
     const int hs = std::min(data_->hist_size, slots_);  // data_->hist_size: the configuration's, or the distinct values (exact method)
-    const unsigned char *active = sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr;
-    const unsigned per_item = FusedRowsPerItem(L);
-    // From 32 nodes on, one launch: a workgroup per node scans its features and
-    // selects.  With fewer nodes that would leave the gain arithmetic (28
-    // features x 256 bins in double precision per node) on a few CUs, and the
-    // scan over (feature, node) waves followed by the selection is faster.
-    if (L >= 32 && !scan_only) {
-#define ARB_SCAN_SELECT(P, D)                                                                                     \
-  hipLaunchKernelGGL((k_scan_select<P, D>), dim3(L + (plan_next ? 1 : 0)), dim3(1024), 0, stream_, d_hg_[hb],     \
-                     d_hh_[hb], d_hc_[hb], nbin_total_, F_, slots_, L, d_tot_[state], d_shifts_, gp, hs,          \
-                     d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,   \
-                     L - 1, active, plan_next ? 1 : 0, per_item, d_pwork_, d_nwork_ + 1, d_node_first_,           \
-                     d_node_items_, ScanCounter(level + 1), FusedGrid(L), d_overflow_, d_cursor2_)
-      if (pair_ && f64_) ARB_SCAN_SELECT(true, true);
-      else if (pair_) ARB_SCAN_SELECT(true, false);
-      else if (f64_) ARB_SCAN_SELECT(false, true);
-      else ARB_SCAN_SELECT(false, false);
-#undef ARB_SCAN_SELECT
-      return;
-    }
-    dim3 grid(F_, L);
-#define ARB_SCAN(P, D) \
-  hipLaunchKernelGGL((k_split_scan<P, D>), grid, dim3(64), 0, stream_, d_hg_[hb], d_hh_[hb], d_hc_[hb], \
-                     nbin_total_, F_, slots_, d_tot_[state], d_shifts_, gp, hs, d_cand_)
-    if (pair_ && f64_) ARB_SCAN(true, true);
-    else if (pair_) ARB_SCAN(true, false);
-    else if (f64_) ARB_SCAN(false, true);
-    else ARB_SCAN(false, false);
+    const dim3 grid((F_ + 3) / 4, L);
+#define ARB_SCAN(P, D, B)                                                                                          \
+  hipLaunchKernelGGL((k_split_scan<P, D, B>), grid, dim3(256), 0, stream_, d_hg_[hb], d_hh_[hb], d_hc_[hb],       \
+                     nbin_total_, F_, slots_, d_tot_[state], d_shifts_, gp, hs, d_cand_, root_sum ? 1 : 0, hi_base_)
+#define ARB_SCAN_B(P, D)                       \
+  do {                                         \
+    if (hs <= 64) ARB_SCAN(P, D, 1);           \
+    else if (hs <= 128) ARB_SCAN(P, D, 2);     \
+    else ARB_SCAN(P, D, 4);                    \
+  } while (0)
+    if (pair_ && f64_) ARB_SCAN_B(true, true);
+    else if (pair_) ARB_SCAN_B(true, false);
+    else if (f64_) ARB_SCAN_B(false, true);
+    else ARB_SCAN_B(false, false);
+#undef ARB_SCAN_B
 #undef ARB_SCAN
-    if (scan_only) return;
-    if (plan_next) {
+  }
+
+  // Splits of a level's nodes from the candidates; on the paths with stand-alone histogram launches also the
+  // plan of the children's histograms: in the same launch while one workgroup selects for all nodes
+  // as fast as several would (up to 64 nodes).
+  void LaunchSelect(int level, int L, int state) {
+    const unsigned char *active = sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr;
+    const bool plan_hist = !fused_ && !streamed_;
+    if (plan_hist && L <= 64) {
       hipLaunchKernelGGL(k_select_plan, dim3(1), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
                          d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,
-                         L - 1, active, per_item, d_pwork_, d_nwork_ + 1, d_node_first_, d_node_items_,
-                         ScanCounter(level + 1), FusedGrid(L), d_overflow_, d_cursor2_);
-    } else {
-      hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L,
-                         d_tot_[state], d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_,
-                         d_tfid_, d_tbin_, d_tgain_, L - 1, active);
+                         L - 1, active, trick_ ? 1 : 0, kMaxHistRows, d_hwork_, d_nwork_, d_node_first_, d_node_items_,
+                         ScanCounter(level + 1), HistGrid(2 * L, false), d_overflow_, HistCus(false));
+      return;
     }
+    hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L,
+                       d_tot_[state], d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_,
+                       d_tfid_, d_tbin_, d_tgain_, L - 1, active,
+                       fused_ && !streamed_ ? ScanCounter(level + 1) : (unsigned long long *)nullptr);
+    if (plan_hist)
+      PlanOn(d_tot_[state ^ 1], d_seg_[state ^ 1], 2 * L, trick_ ? 1 : 0, kMaxHistRows, d_hwork_, d_nwork_, level + 1,
+             nullptr, HistGrid(2 * L, false), HistCus(false));
   }
 
   // Stand-alone partition: groups of up to eight words per launch; the first
@@ -1498,6 +1496,8 @@ class HipTreeBuilder : public TreeBuilder {
     }
   }
 
+  // launch bound of a stand-alone partition over PL parent nodes
+  unsigned PartGrid(int PL) const { return (unsigned)std::min<size_t>(n_ / part_rows_ + 2 * PL + 1, max_part_items_); }
   // launch bound of the fused pass over PL parent nodes
   unsigned FusedGrid(int PL) const {
     return (unsigned)std::min<size_t>(n_ / FusedRowsPerItem(PL) + 2 * PL + 1, max_hist_items_);  // (a slab each)
@@ -1513,19 +1513,6 @@ class HipTreeBuilder : public TreeBuilder {
   unsigned FusedRowsPerItem(int PL) const {
     const size_t target = PL <= 32 ? (size_t)(254 - PL) : (size_t)std::max(256, 508 - PL);
     return HistRowsPerItem(n_, target);
-  }
-
-  void LaunchLeafWeights(int L, int state, const GainParams &gp) {
-    Mark(kLeaf);
-    const int blocks = (L + 127) / 128;
-#define ARB_LEAF(P, D) \
-  hipLaunchKernelGGL((k_leaf_weights<P, D>), dim3(blocks), dim3(128), 0, stream_, d_split_, d_tot_[state], L, \
-                     d_shifts_, gp, cfg_.tree.eta, d_weights_)
-    if (pair_ && f64_) ARB_LEAF(true, true);
-    else if (pair_) ARB_LEAF(true, false);
-    else if (f64_) ARB_LEAF(false, true);
-    else ARB_LEAF(false, false);
-#undef ARB_LEAF
   }
 
   void LaunchFinal(const uint32_t *bins, size_t stride, size_t row0, size_t rows, int label, bool next_grad) {
@@ -1644,17 +1631,18 @@ class HipTreeBuilder : public TreeBuilder {
         if (in_place) DoneWithBlock(buf);
         Reduce(L, hb, false, state, false, b > 0);
       }
-      if (level == 0) RootTotals(hb, state, orig);
+      if (level == 0) RootTotals(state, orig);
       if (trick)
         hipLaunchKernelGGL(k_sibling, dim3((nbin_total_ + 255) / 256, L), dim3(256), 0, stream_, d_hg_[hb], d_hh_[hb],
                            d_hc_[hb], d_hg_[hb ^ 1], d_hh_[hb ^ 1], d_hc_[hb ^ 1], d_tot_[state], level, nbin_total_);
       if (inspect_) KeepHist(level, L, hb, state);
-      LaunchSplit(level, L, hb, state, gp);
-      if (level + 2 >= D_) LaunchLeafWeights(L, state, gp);
+      LaunchScan(level, L, hb, state, gp, level == 0 && !hi_skip_);
+      if (level + 2 < D_) LaunchSelect(level, L, state);
       state ^= 1;
     }
     // leaves, y_hat, next gradients: one more pass over the blocks
     Mark(kLeaf);
+    LaunchTreeEnd(state ^ 1, gp, 0);
     const bool next_grad = !inspect_ && K_ == 1;
     for (size_t b = 0; b < nblocks; ++b) {
       const size_t row0 = b * br;
@@ -1665,7 +1653,7 @@ class HipTreeBuilder : public TreeBuilder {
       DoneWithBlock(buf);
     }
     grad_ready_ = next_grad;
-    EnqueueRecord();
+    Mark(kNone);
   }
 
   // Column sampling of one tree (InitGrowingTree / InitTreeLevel,
@@ -1760,6 +1748,8 @@ class HipTreeBuilder : public TreeBuilder {
   int slots_ = kSlots;
   int wide_group_ = 2;    // features per histogram launch with 16-bit bins
   BinCode code_ = BinCode{2, 8};
+  bool root_planned_ = false;     // d_tot_[0][0], d_seg_[0][0] and d_hwork_ describe the root of the tree grown next
+  unsigned long long root_rows_scanned_ = 0;
   bool root_hist_ready_ = false;  // the slabs hold the root histogram of the tree grown next
   static constexpr int kScanLevels = 32;      // per-level counters of rows accumulated into histograms
   static constexpr size_t kRecordRing = 64;  // trees whose records may wait on the device

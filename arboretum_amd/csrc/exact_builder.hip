@@ -406,7 +406,8 @@ class ExactSortBuilder : public TreeBuilder {
                          F_, d_cand_);
       hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
                          d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,
-                         L - 1, sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr);
+                         L - 1, sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr,
+                         (unsigned long long *)nullptr);
       hipLaunchKernelGGL(k_ex_decide, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, sd_->ranks, stride_, d_split_,
                          d_node_of_, d_went_right_, n_);
       if (last) {

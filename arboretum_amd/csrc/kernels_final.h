@@ -3,6 +3,7 @@
 #define ARBORETUM_AMD_KERNELS_FINAL_H_
 #include "device_common.h"
 #include "kernels_hist.h"
+#include "kernels_split.h"
 #include "memory_pool.h"
 
 namespace arb {
@@ -34,53 +35,79 @@ __global__ void k_leaf_weights(const SplitRec *__restrict__ split, const NodeSum
   weights[2 * nd + 1] = LeafWeight<PAIR, F64>(GR, HR, t.c - s.left.c, gp) * eta;
 }
 
-// Leaf weights of a finished tree and, in the same launch, what would
-// otherwise be three more one-wave kernels in front of the last pass: the
-// tree's record into its slot of the record ring (layout of k_pack_record) and
-// the state and work plan of the next tree's root histogram over all n rows
-// (k_init_root + k_plan for one node starting at row 0).
-// grid ceil(L / 128) + 1, 128 threads: the last block writes the plan.
+// State and work plan of a tree's root histogram over all n rows: one node from row 0 on.  Called by
+// one workgroup.
+__device__ __forceinline__ void RootPlan(unsigned n, unsigned rows_per_item, WorkItem *__restrict__ work,
+                                         unsigned *__restrict__ n_work, unsigned *__restrict__ node_first,
+                                         unsigned *__restrict__ node_items) {
+  const unsigned items = (n + rows_per_item - 1) / rows_per_item;
+  for (unsigned w = threadIdx.x; w < items; w += blockDim.x) {
+    WorkItem it;
+    it.node = 0;
+    it.begin = w * rows_per_item;
+    it.end = min(n, it.begin + rows_per_item);
+    it.first = 0;
+    work[w] = it;
+  }
+  if (threadIdx.x == 0) {
+    node_first[0] = 0;
+    node_items[0] = items;
+    *n_work = items;
+  }
+}
+// The same for the first tree of a booster (k_tree_end does it for the others).
+__global__ void __launch_bounds__(256)
+k_first_root(NodeSum *__restrict__ root_tot, unsigned *__restrict__ root_seg, unsigned n, unsigned rows_per_item,
+             WorkItem *__restrict__ work, unsigned *__restrict__ n_work, unsigned *__restrict__ node_first,
+             unsigned *__restrict__ node_items) {
+  RootPlan(n, rows_per_item, work, n_work, node_first, node_items);
+  if (threadIdx.x == 0) {
+    root_tot[0] = NodeSum{0, 0, n};
+    root_seg[0] = 0;
+  }
+}
+
+// End of a tree in one launch, in front of the last pass: the splits of the last level from the
+// candidates of its scan (BestOfNode), the leaf weights (UpdateLeafWeight, garden.cu:487-503,
+// split.cu:25-35: left = Weight(left sum), right = Weight(parent - left) with the subtraction in the sum
+// type), the tree's record into its slot of the record ring (layout of k_pack_record), and, when the
+// rows are resident (work set), the state and work plan of the next tree's root histogram.  As kernels of their own these
+// took 2 to 5 us each, and the last level's scan and selection in one workgroup per node 15 to 90 us.
+// grid ceil(L / 4) + 1, 256 threads, a wave per node; the last block writes the plan.
 template <bool PAIR, bool F64>
-__global__ void __launch_bounds__(128)
-k_tree_end(const SplitRec *__restrict__ split, const NodeSum *__restrict__ tot, int L,
+__global__ void __launch_bounds__(256)
+k_tree_end(const Cand *__restrict__ cand, int F, const unsigned char *__restrict__ active, const NodeSum *tot, int L,
            const int *__restrict__ shifts, GainParams gp, float eta, float *__restrict__ weights,
-           const int *__restrict__ t_fid, const int *__restrict__ t_bin, const float *__restrict__ t_gain,
+           int *__restrict__ t_fid, int *__restrict__ t_bin, float *__restrict__ t_gain,
            const unsigned *__restrict__ overflow, uint32_t *__restrict__ record,
-           NodeSum *__restrict__ root_tot, unsigned *__restrict__ root_seg, unsigned n, unsigned rows_per_item,
+           NodeSum *root_tot, unsigned *__restrict__ root_seg, unsigned n, unsigned rows_per_item,
            WorkItem *__restrict__ work, unsigned *__restrict__ n_work, unsigned *__restrict__ node_first,
-           unsigned *__restrict__ node_items, unsigned long long *__restrict__ rows_scanned) {
+           unsigned *__restrict__ node_items) {
   const int internal = 2 * L - 1, leaves = 2 * L;
   const int node_blocks = (int)gridDim.x - 1;
   if ((int)blockIdx.x == node_blocks) {
-    const unsigned items = (n + rows_per_item - 1) / rows_per_item;
-    for (unsigned w = threadIdx.x; w < items; w += blockDim.x) {
-      WorkItem it;
-      it.node = 0;
-      it.begin = w * rows_per_item;
-      it.end = min(n, it.begin + rows_per_item);
-      it.first = 0;
-      work[w] = it;
-    }
-    if (threadIdx.x == 0) {
-      node_first[0] = 0;
-      node_items[0] = items;
-      *n_work = items;
-      *rows_scanned += n;
-      record[3 * internal + leaves] = *overflow;
-    }
+    if (work != nullptr) RootPlan(n, rows_per_item, work, n_work, node_first, node_items);
+    if (threadIdx.x == 0) record[3 * internal + leaves] = *overflow;
     return;
   }
-  const int nd = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int i = nd; i < internal; i += node_blocks * (int)blockDim.x) {
+  // the nodes above the last level
+  for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < L - 1; i += node_blocks * (int)blockDim.x) {
     record[i] = (uint32_t)t_fid[i];
     record[internal + i] = (uint32_t)t_bin[i];
     record[2 * internal + i] = __float_as_uint(t_gain[i]);
   }
+  const int nd = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (nd >= L) return;
-  const int sg = shifts[0], sh = shifts[1];
-  const SplitRec s = split[nd];
   const NodeSum t = tot[nd];
-  const double GL = FromFixed<F64>(s.left.g, sg), HL = PAIR ? FromFixed<F64>(s.left.h, sh) : 0.0;
+  Cand c;
+  c.gain = 0.0f;
+  c.bin = -1;
+  c.left = t;
+  const int fid = t.c == 0 ? -1 : BestOfNode(cand + (size_t)nd * F, F, active, lane, &c);
+  if (lane != 0) return;
+  if (fid < 0) c.left = t;  // not split: every row stays left
+  const int sg = shifts[0], sh = shifts[1];
+  const double GL = FromFixed<F64>(c.left.g, sg), HL = PAIR ? FromFixed<F64>(c.left.h, sh) : 0.0;
   const double GP = FromFixed<F64>(t.g, sg), HP = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
   double GR, HR;
   if (F64) {
@@ -90,17 +117,22 @@ k_tree_end(const SplitRec *__restrict__ split, const NodeSum *__restrict__ tot, 
     GR = (double)((float)GP - (float)GL);
     HR = (double)((float)HP - (float)HL);
   }
-  if (nd == 0) {
-    // root_tot may be the array `tot` of this level: entry 0 has been read above, by this thread
-    root_tot[0].g = 0;
-    root_tot[0].h = 0;
-    root_tot[0].c = n;
+  if (nd == 0 && work != nullptr) {
+    // root_tot may be the array `tot` of this level: entry 0 has been read above, by this wave
+    root_tot[0] = NodeSum{0, 0, n};
     root_seg[0] = 0;
   }
-  const float wl = LeafWeight<PAIR, F64>(GL, HL, s.left.c, gp) * eta;
-  const float wr = LeafWeight<PAIR, F64>(GR, HR, t.c - s.left.c, gp) * eta;
+  const float wl = LeafWeight<PAIR, F64>(GL, HL, c.left.c, gp) * eta;
+  const float wr = LeafWeight<PAIR, F64>(GR, HR, t.c - c.left.c, gp) * eta;
+  const int at = L - 1 + nd;
+  t_fid[at] = fid < 0 ? 0 : fid;  // garden.cu:471-481
+  t_bin[at] = fid < 0 ? -1 : c.bin;
+  t_gain[at] = fid < 0 ? 0.0f : c.gain;
   weights[2 * nd] = wl;
   weights[2 * nd + 1] = wr;
+  record[at] = (uint32_t)(fid < 0 ? 0 : fid);
+  record[internal + at] = (uint32_t)(fid < 0 ? -1 : c.bin);
+  record[2 * internal + at] = __float_as_uint(fid < 0 ? 0.0f : c.gain);
   record[3 * internal + 2 * nd] = __float_as_uint(wl);
   record[3 * internal + 2 * nd + 1] = __float_as_uint(wr);
 }

@@ -161,13 +161,14 @@ k_hist(const uint32_t *__restrict__ bins, size_t stride, int q0, int F,
   FlushSlab<PAIR, NQ, HI>(lds, slab, w, slab_entries, q0);
 }
 
-// Histogram of contiguous row ranges with 16-bit bins: features [f0, f0 + nf)
-// (f0 even), `slots` histogram slots per feature, LDS layout f * slots + bin,
+// Histogram of contiguous row ranges with 16-bit bins: a workgroup per work item and group of
+// group_nf features (an even number; grid.y groups, in one launch: one after the other each waited for
+// its own rows, 10 us a group at 500,000 rows), `slots` histogram slots per feature, LDS layout f * slots + bin,
 // word0 of every entry first, then (PAIR) word1.  The slab of a work item has
 // the same feature-major order: word0[slab_entries], word1[slab_entries].
 template <bool PAIR>
 __global__ void __launch_bounds__(kHistThreads)
-k_hist_wide(const uint32_t *__restrict__ bins, size_t stride, int f0, int nf, int slots,
+k_hist_wide(const uint32_t *__restrict__ bins, size_t stride, int F, int group_nf, int slots,
             const float *__restrict__ g, const float *__restrict__ h, const int *__restrict__ shifts,
             const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
             unsigned long long *__restrict__ slab, int slab_entries) {
@@ -175,6 +176,7 @@ k_hist_wide(const uint32_t *__restrict__ bins, size_t stride, int f0, int nf, in
   const unsigned w = blockIdx.x;
   if (w >= *n_work) return;
   const WorkItem it = work[w];
+  const int f0 = (int)blockIdx.y * group_nf, nf = min(group_nf, F - f0);
   const int entries = nf * slots;
   for (int i = threadIdx.x; i < entries * (PAIR ? 2 : 1); i += kHistThreads) lds[i] = 0ull;
   __syncthreads();

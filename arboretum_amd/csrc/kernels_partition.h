@@ -693,7 +693,7 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
 // (matrices with a ninth-bit word); one more block of the grid (the last one)
 // reduces it into cell hi_base + f of the node's histogram, behind the 256-bin
 // histograms of the features.
-// Work plan of the next fused pass, made by one more block of the slab reduction (the ranges of
+// Work plan of the row pass over this level's nodes that follows (fused pass or partition), made by one more block of the slab reduction (the ranges of
 // the nodes are known since their parents were split): work == null, none.  node_first /
 // node_items must be other arrays than the ones this reduction reads.
 struct NextPlan {
@@ -831,31 +831,6 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
       if (with_h) hh[so] = ph[po] - ah;
       hc[so] = pc[po] - cnt;
     }
-  }
-}
-
-// Root totals = sum over the slots of feature 0 of the root histogram (every
-// row, NaN included, sits in exactly one slot).  Replaces the reduction over
-// the gradient array of garden.cu:432-435.  One wave.
-// hi_cell > 0: the cell of feature 0's bin 256 (matrices with a ninth-bit word).
-// hh may be null (no hessians).
-__global__ void __launch_bounds__(64)
-k_root_from_hist(const long long *__restrict__ hg, const long long *__restrict__ hh,
-                 NodeSum *__restrict__ tot, int slots, int hi_cell = 0) {
-  long long a = 0, b = 0;
-  for (int i = threadIdx.x; i < slots; i += 64) {
-    a += hg[i];
-    if (hh != nullptr) b += hh[i];
-  }
-  if (hi_cell > 0 && threadIdx.x == 0) {
-    a += hg[hi_cell];
-    if (hh != nullptr) b += hh[hi_cell];
-  }
-  a = WaveSumLL(a);
-  b = WaveSumLL(b);
-  if (threadIdx.x == 0) {
-    tot[0].g = a;
-    tot[0].h = b;
   }
 }
 

@@ -40,7 +40,10 @@ namespace {
 // per bin < hist_size, arg-max with ties to the HIGHEST bin (builder.h:39-49),
 // only gains > 0 (hist_tree_grower.cu:31).  `first` is the index of the
 // feature's slot 0 in the histogram arrays.  The result is valid in lane 0.
-template <bool PAIR, bool F64>
+// BPL: neighbouring bins per lane, 64 BPL bins at a time.  The gains of a lane's
+// bins are double-precision arithmetic one after the other, so a feature of 64
+// bins is scanned with one bin per lane (with four, 16 lanes did the work of 64).
+template <bool PAIR, bool F64, int BPL>
 __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, const long long *__restrict__ hh,
                                             const unsigned long long *__restrict__ hc, size_t first, int slots,
                                             const NodeSum &t, const int *__restrict__ shifts,
@@ -54,36 +57,36 @@ __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, co
     const int sg = shifts[0], sh = shifts[1];
     const double GT = FromFixed<F64>(t.g, sg);
     const double HT = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
-    // sums of the slots below the current chunk of 256
+    // sums of the slots below the current chunk
     long long carry_g = 0, carry_h = 0;
     unsigned long long carry_c = 0;
-    for (int chunk = 0; chunk < slots && chunk < hist_size; chunk += 256) {
-      const size_t base = first + chunk + lane * 4;
-      long long g4[4], h4[4];
-      unsigned long long c4[4];
+    for (int chunk = 0; chunk < slots && chunk < hist_size; chunk += 64 * BPL) {
+      const size_t base = first + chunk + lane * BPL;
+      long long g4[BPL], h4[BPL];
+      unsigned long long c4[BPL];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) g4[j] = h4[j] = 0, c4[j] = 0;
-      // lanes whose four slots all lie at or past hist_size (missing values, unused slots) hold no
+      for (int j = 0; j < BPL; ++j) g4[j] = h4[j] = 0, c4[j] = 0;
+      // lanes whose slots all lie at or past hist_size (missing values, unused slots) hold no
       // candidate and are in no candidate's prefix: they read nothing
-      if (chunk + lane * 4 < hist_size) {
+      if (chunk + lane * BPL < hist_size) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < BPL; ++j) {
           g4[j] = hg[base + j];
           h4[j] = PAIR ? hh[base + j] : 0;
           c4[j] = hc[base + j];
         }
       }
 #pragma unroll
-      for (int j = 1; j < 4; ++j) {
+      for (int j = 1; j < BPL; ++j) {
         g4[j] += g4[j - 1];
         h4[j] += h4[j - 1];
         c4[j] += c4[j - 1];
       }
-      long long ig = g4[3], ih = h4[3];
-      unsigned long long ic = c4[3];
+      long long ig = g4[BPL - 1], ih = h4[BPL - 1];
+      unsigned long long ic = c4[BPL - 1];
       for (int off = 1; off < 64; off <<= 1) {
         const long long og = __shfl_up(ig, off);
-        const long long oh = __shfl_up(ih, off);
+        const long long oh = PAIR ? __shfl_up(ih, off) : 0;
         const unsigned long long oc = __shfl_up(ic, off);
         if (lane >= off) {
           ig += og;
@@ -91,11 +94,11 @@ __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, co
           ic += oc;
         }
       }
-      const long long eg = carry_g + ig - g4[3], eh = carry_h + ih - h4[3];
-      const unsigned long long ec = carry_c + ic - c4[3];
+      const long long eg = carry_g + ig - g4[BPL - 1], eh = carry_h + ih - h4[BPL - 1];
+      const unsigned long long ec = carry_c + ic - c4[BPL - 1];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int bin = chunk + lane * 4 + j;
+      for (int j = 0; j < BPL; ++j) {
+        const int bin = chunk + lane * BPL + j;
         if (bin < hist_size) {
           const long long lg = eg + g4[j], lh = eh + h4[j];
           const unsigned long long lc = ec + c4[j];
@@ -112,38 +115,63 @@ __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, co
         }
       }
       carry_g += __shfl(ig, 63);
-      carry_h += __shfl(ih, 63);
+      if (PAIR) carry_h += __shfl(ih, 63);
       carry_c += __shfl(ic, 63);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-      const float og = __shfl_down(best.gain, off);
-      const int ob = __shfl_down(best.bin, off);
-      const long long olg = __shfl_down(best.left.g, off);
-      const long long olh = __shfl_down(best.left.h, off);
-      const unsigned long long olc = __shfl_down(best.left.c, off);
-      if (ob >= 0 && (best.bin < 0 || og > best.gain || (og == best.gain && ob > best.bin))) {
-        best.gain = og;
-        best.bin = ob;
-        best.left.g = olg;
-        best.left.h = olh;
-        best.left.c = olc;
-      }
+    // highest gain, ties to the highest bin: one key, then the winner's sums
+    unsigned long long key = best.bin < 0 ? 0ull : ((unsigned long long)__float_as_uint(best.gain) << 32) | (unsigned)(best.bin + 1);
+    unsigned long long top = key;
+    for (int off = 32; off > 0; off >>= 1) top = max(top, (unsigned long long)__shfl_xor(top, off));
+    if (top != 0) {  // uniform
+      const int from = __ffsll((unsigned long long)__ballot(key == top)) - 1;  // (keys differ by their bins)
+      best.gain = __shfl(best.gain, from);
+      best.bin = __shfl(best.bin, from);
+      best.left.g = __shfl(best.left.g, from);
+      best.left.h = PAIR ? __shfl(best.left.h, from) : 0;
+      best.left.c = __shfl(best.left.c, from);
     }
   }
   return best;
 }
 
-// grid (F, L), 64 threads: one wave per (feature, node), candidates to `cand`.
-template <bool PAIR, bool F64>
-__global__ void __launch_bounds__(64)
+// grid (ceil(F / 4), L), 256 threads: one wave per (feature, node), candidates to `cand`.
+// root_sum (the root level): the gradient totals of the root are the sum over the slots of feature 0
+// of its histogram (every row, NaN included, sits in exactly one slot; replaces the reduction over the
+// gradient array of garden.cu:432-435).  Every wave makes that sum for itself, a kilobyte or two out of
+// the cache, and one writes it to tot[0]: no kernel of its own in between.  hi_cell > 0: the cell of
+// feature 0's bin 256 (matrices with a ninth-bit word).
+template <bool PAIR, bool F64, int BPL>
+__global__ void __launch_bounds__(256)
 k_split_scan(const long long *__restrict__ hg, const long long *__restrict__ hh,
              const unsigned long long *__restrict__ hc, int nbin_total, int F, int slots,
-             const NodeSum *__restrict__ tot, const int *__restrict__ shifts, GainParams gp,
-             int hist_size, Cand *__restrict__ cand) {
-  const int f = blockIdx.x, nd = blockIdx.y, lane = threadIdx.x;
-  const NodeSum t = tot[nd];
-  const Cand best = ScanFeature<PAIR, F64>(hg, hh, hc, (size_t)nd * nbin_total + (size_t)f * slots, slots, t, shifts,
-                                           gp, hist_size, lane);
+             NodeSum *__restrict__ tot, const int *__restrict__ shifts, GainParams gp,
+             int hist_size, Cand *__restrict__ cand, int root_sum, int hi_cell) {
+  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), nd = blockIdx.y, lane = threadIdx.x & 63;
+  if (f >= F) return;
+  NodeSum t = tot[nd];
+  if (root_sum) {
+    long long a = 0, b = 0;
+    for (int i = lane; i < slots; i += 64) {
+      a += hg[i];
+      if (PAIR) b += hh[i];
+    }
+    if (hi_cell > 0 && lane == 0) {
+      a += hg[hi_cell];
+      if (PAIR) b += hh[hi_cell];
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      a += __shfl_xor(a, off);
+      if (PAIR) b += __shfl_xor(b, off);
+    }
+    t.g = a;
+    t.h = b;
+    if (f == 0 && lane == 0) {
+      tot[0].g = a;
+      tot[0].h = b;
+    }
+  }
+  const Cand best = ScanFeature<PAIR, F64, BPL>(hg, hh, hc, (size_t)nd * nbin_total + (size_t)f * slots, slots, t, shifts,
+                                                gp, hist_size, lane);
   if (lane == 0) cand[(size_t)nd * F + f] = best;
 }
 
@@ -291,10 +319,10 @@ __device__ __forceinline__ void WriteEmptyNodes(const LevelScan &a, const NodeSu
 // row left.
 // One wave per node: lane l looks at features l, l + 64, ...; the wave keeps
 // the candidate with the highest gain, ties to the lowest feature id.
-__device__ __forceinline__ void SelectNode(int nd, int lane, const Cand *__restrict__ cand, int F,
+__device__ __forceinline__ SplitRec SelectNode(int nd, int lane, const Cand *__restrict__ cand, int F,
                                            const NodeSum *__restrict__ tot,
                                            const unsigned *__restrict__ seg_start,
-                                           NodeSum *__restrict__ tot_next, unsigned *__restrict__ seg_next,
+                                           NodeSum *tot_next, unsigned *seg_next,
                                            SplitRec *__restrict__ split, int *__restrict__ t_fid,
                                            int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
                                            const unsigned char *__restrict__ active) {
@@ -304,128 +332,50 @@ __device__ __forceinline__ void SelectNode(int nd, int lane, const Cand *__restr
   c.bin = -1;
   c.left = NodeSum{0, 0, 0};
   const int fid = t.c == 0 ? -1 : BestOfNode(cand + (size_t)nd * F, F, active, lane, &c);
-  if (lane != 0) return;
-  WriteNode(nd, t, c.gain, fid, c.bin, c.left.g, c.left.h, c.left.c, seg_start, tot_next, seg_next, split, t_fid, t_bin,
-            t_gain, heap_off);
+  SplitRec rec{};
+  if (lane == 0)
+    rec = WriteNode(nd, t, c.gain, fid, c.bin, c.left.g, c.left.h, c.left.c, seg_start, tot_next, seg_next, split, t_fid,
+                    t_bin, t_gain, heap_off);
+  return rec;  // valid in lane 0
 }
 
-// grid ceil(L / 16), 1024 threads: one wave per node
+// grid ceil(L / 16), 1024 threads: one wave per node.  rows_scanned (optional): advanced by the rows of
+// the smaller side of every split.
 __global__ void __launch_bounds__(1024)
 k_split_select(const Cand *__restrict__ cand, int F, int L, const NodeSum *__restrict__ tot,
                const unsigned *__restrict__ seg_start, NodeSum *__restrict__ tot_next,
                unsigned *__restrict__ seg_next, SplitRec *__restrict__ split, int *__restrict__ t_fid,
                int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
-               const unsigned char *__restrict__ active) {
+               const unsigned char *__restrict__ active, unsigned long long *__restrict__ rows_scanned) {
   const int nd = blockIdx.x * 16 + (threadIdx.x >> 6);
-  if (nd < L)
-    SelectNode(nd, threadIdx.x & 63, cand, F, tot, seg_start, tot_next, seg_next, split, t_fid, t_bin, t_gain,
-               heap_off, active);
+  if (nd >= L) return;
+  const SplitRec r = SelectNode(nd, threadIdx.x & 63, cand, F, tot, seg_start, tot_next, seg_next, split, t_fid, t_bin,
+                                t_gain, heap_off, active);
+  if (rows_scanned && (threadIdx.x & 63) == 0) {
+    const unsigned long long c = tot[nd].c;
+    if (c != 0) atomicAdd(rows_scanned, min(r.left.c, c - r.left.c));
+  }
 }
 
-// k_split_select followed, in the same workgroup, by the work plan of the
-// fused pass over these nodes' rows (the plan needs the splits only for the
-// row statistics).  One workgroup of 1024 threads.
+// k_split_select followed, in the same workgroup, by the work plan of the histograms of the
+// children (select: PlanBody's; the items are balanced over balance_cus compute units).  For levels
+// of few nodes: one workgroup selects for all of them.
 __global__ void __launch_bounds__(1024)
 k_select_plan(const Cand *__restrict__ cand, int F, int L, const NodeSum *__restrict__ tot,
-              const unsigned *__restrict__ seg_start, NodeSum *__restrict__ tot_next,
-              unsigned *__restrict__ seg_next, SplitRec *__restrict__ split, int *__restrict__ t_fid,
+              const unsigned *__restrict__ seg_start, NodeSum *tot_next, unsigned *seg_next,
+              SplitRec *__restrict__ split, int *__restrict__ t_fid,
               int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
-              const unsigned char *__restrict__ active, unsigned rows_per_item,
+              const unsigned char *__restrict__ active, int select, unsigned rows_per_item,
               WorkItem *__restrict__ work, unsigned *__restrict__ n_work,
               unsigned *__restrict__ node_first, unsigned *__restrict__ node_items,
               unsigned long long *__restrict__ rows_scanned, unsigned max_items,
-              unsigned *__restrict__ overflow, unsigned *__restrict__ cursor) {
+              unsigned *__restrict__ overflow, unsigned balance_cus) {
   for (int nd = threadIdx.x >> 6; nd < L; nd += 16)
     SelectNode(nd, threadIdx.x & 63, cand, F, tot, seg_start, tot_next, seg_next, split, t_fid, t_bin, t_gain,
                heap_off, active);
-  __syncthreads();  // the splits written above are read by the plan
-  PlanBody(tot, seg_start, L, 0, rows_per_item, work, n_work, node_first, node_items, rows_scanned, split,
-           max_items, overflow, cursor);
-}
-
-// Split scan and selection in one launch: workgroup `nd` < L scans the
-// features of node nd (wave w takes features w, w + 16, ...), keeps the
-// candidate with the highest gain, ties to the lowest feature id, and writes
-// the node's record; with `plan` set, workgroup L cuts the row ranges of these
-// nodes into the work items of the fused pass that follows, and every node adds
-// the rows of its smaller side to rows_scanned.  grid L (+ 1), 1024 threads.
-template <bool PAIR, bool F64>
-__global__ void __launch_bounds__(1024)
-k_scan_select(const long long *__restrict__ hg, const long long *__restrict__ hh,
-              const unsigned long long *__restrict__ hc, int nbin_total, int F, int slots, int L,
-              const NodeSum *__restrict__ tot, const int *__restrict__ shifts, GainParams gp, int hist_size,
-              const unsigned *__restrict__ seg_start, NodeSum *__restrict__ tot_next,
-              unsigned *__restrict__ seg_next, SplitRec *__restrict__ split, int *__restrict__ t_fid,
-              int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
-              const unsigned char *__restrict__ active, int plan, unsigned rows_per_item,
-              WorkItem *__restrict__ work, unsigned *__restrict__ n_work, unsigned *__restrict__ node_first,
-              unsigned *__restrict__ node_items, unsigned long long *__restrict__ rows_scanned,
-              unsigned max_items, unsigned *__restrict__ overflow, unsigned *__restrict__ cursor) {
-  if ((int)blockIdx.x >= L) {  // uniform per workgroup
-    PlanBody(tot, seg_start, L, 0, rows_per_item, work, n_work, node_first, node_items, nullptr, nullptr, max_items,
-             overflow, cursor);
-    return;
-  }
-  __shared__ Cand s_cand[16];
-  __shared__ int s_fid[16];
-  const int nd = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const NodeSum t = tot[nd];
-  Cand mine;
-  mine.gain = 0.0f;
-  mine.bin = -1;
-  mine.left.g = mine.left.h = 0;
-  mine.left.c = 0;
-  int mine_fid = -1;
-  for (int f = wave; f < F; f += 16) {
-    if (active && !active[f]) continue;  // feature not sampled at this level
-    const Cand c = ScanFeature<PAIR, F64>(hg, hh, hc, (size_t)nd * nbin_total + (size_t)f * slots, slots, t, shifts,
-                                          gp, hist_size, lane);
-    if (c.bin >= 0 && (mine_fid < 0 || mine.gain < c.gain)) {  // features ascend: ties keep the lower id
-      mine = c;
-      mine_fid = f;
-    }
-  }
-  if (lane == 0) {
-    s_cand[wave] = mine;
-    s_fid[wave] = mine_fid;
-  }
-  __syncthreads();
-  if (wave != 0) return;
-  float gain = 0.0f;
-  int fid = -1, bin = -1;
-  long long lg = 0, lh = 0;
-  unsigned long long lc = 0;
-  if (lane < 16 && s_fid[lane] >= 0) {
-    const Cand c = s_cand[lane];
-    gain = c.gain;
-    fid = s_fid[lane];
-    bin = c.bin;
-    lg = c.left.g;
-    lh = c.left.h;
-    lc = c.left.c;
-  }
-  for (int off = 8; off > 0; off >>= 1) {
-    const float og = __shfl_down(gain, off);
-    const int of = __shfl_down(fid, off);
-    const int ob = __shfl_down(bin, off);
-    const long long olg = __shfl_down(lg, off);
-    const long long olh = __shfl_down(lh, off);
-    const unsigned long long olc = __shfl_down(lc, off);
-    if (of >= 0 && (fid < 0 || og > gain || (og == gain && of < fid))) {
-      gain = og;
-      fid = of;
-      bin = ob;
-      lg = olg;
-      lh = olh;
-      lc = olc;
-    }
-  }
-  if (lane != 0) return;
-  WriteNode(nd, t, gain, fid, bin, lg, lh, lc, seg_start, tot_next, seg_next, split, t_fid, t_bin, t_gain, heap_off);
-  if (plan && rows_scanned && t.c != 0) {
-    const unsigned long long cl = fid < 0 ? t.c : lc;
-    atomicAdd(rows_scanned, min(cl, t.c - cl));
-  }
+  __syncthreads();  // the children's totals and ranges written above are read by the plan
+  PlanBody(tot_next, seg_next, 2 * L, select, rows_per_item, work, n_work, node_first, node_items, rows_scanned, nullptr,
+           max_items, overflow, nullptr, balance_cus);
 }
 
 }  // namespace
