@@ -8,7 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libarboretum.so")
-SOURCES = ["fused_pass_pair.hip", "fused_pass_single.hip", "device_builder.hip", "exact_builder.hip", "hist_sum.hip", "quantiser.hip", "predictor.hip", "memory_pool.hip", "staging.hip", "booster.cpp",
+SOURCES = ["fused_pass_pair.hip", "fused_pass_single.hip", "device_builder.hip", "exact_builder.hip", "hist_sum.hip", "quantiser.hip", "predictor.hip", "float_rows.hip", "memory_pool.hip", "staging.hip", "booster.cpp",
            "config.cpp", "parallel.cpp",
            "wrapper.cpp"]
 # -ffp-contract=off: the gain arithmetic must round exactly like the host

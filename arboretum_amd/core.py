@@ -42,6 +42,8 @@ def _load_lib():
         # extensions (include/arboretum_ext.h)
         "ADeviceCount": [P(c_int)],
         "ADeviceCopyProbe": [ctypes.c_ulonglong],
+        "APredictInto": [c_void_p, c_void_p, c_void_p, ctypes.c_ulonglong, c_int],
+        "AGetYInto": [c_void_p, c_void_p, c_void_p, ctypes.c_ulonglong],
         "ACreateFromQuantized": [c_void_p, ctypes.c_longlong, c_int, P(c_void_p)],
         "ACreateFromQuantizedBlocks": [c_void_p, c_int, ctypes.c_longlong, ctypes.c_longlong, c_int, P(c_void_p)],
         "AQuantize": [c_void_p, c_int],
@@ -278,23 +280,21 @@ class Garden(object):
         self._ensure()
         _check(_LIB.AAppendLastTree(self.handle, data.handle))
 
-    def _take(self, preds, length):
-        shape = (length,) if self.labels_count == 1 else (length, self.labels_count)
-        res = np.copy(np.ctypeslib.as_array(preds, shape=shape))
-        _check(_LIB.ADeleteArray(preds))
-        return res
+    def _results(self, data):
+        rows = int(data.rows)
+        return np.empty(rows if self.labels_count == 1 else (rows, self.labels_count), dtype=np.float32)
 
     def get_y(self, data):
         self._ensure()
-        preds = ctypes.POINTER(ctypes.c_float)()
-        _check(_LIB.AGetY(self.handle, data.handle, ctypes.byref(preds)))
-        return self._take(preds, int(data.rows))
+        out = self._results(data)
+        _check(_LIB.AGetYInto(self.handle, data.handle, out.ctypes.data, out.size))
+        return out
 
     def predict(self, data, n_rounds=-1):
         self._ensure()
-        preds = ctypes.POINTER(ctypes.c_float)()
-        _check(_LIB.APredict(self.handle, data.handle, ctypes.byref(preds), int(n_rounds)))
-        return self._take(preds, int(data.rows))
+        out = self._results(data)
+        _check(_LIB.APredictInto(self.handle, data.handle, out.ctypes.data, out.size, int(n_rounds)))
+        return out
 
     def dump(self):
         self._ensure()

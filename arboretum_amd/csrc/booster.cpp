@@ -24,6 +24,25 @@ DataMatrix::~DataMatrix() {
   if (exact_sort) FreeExactSortData(exact_sort);
 }
 
+std::vector<std::vector<float>> DataMatrix::Columns() const {
+  const float *x = values->OnHost();
+  std::vector<std::vector<float>> out(columns_dense);
+  // the columns are allocated (and their pages first touched) by several threads
+  ParallelTasks(columns_dense, [&](size_t f) { out[f].resize(rows); });
+  // in tiles of 256 rows, so that a tile's lines of every column stay in cache while its rows are
+  // read once
+  ParallelFor(rows, [&](size_t b, size_t e) {
+    for (size_t r0 = b; r0 < e; r0 += 256) {
+      const size_t r1 = std::min(e, r0 + 256);
+      for (size_t f = 0; f < columns_dense; ++f) {
+        float *dst = out[f].data();
+        for (size_t i = r0; i < r1; ++i) dst[i] = x[i * columns_dense + f];
+      }
+    }
+  });
+  return out;
+}
+
 void DataMatrix::SetY(const float *v) {
   y.resize(rows);
   std::mutex guard;
@@ -78,33 +97,33 @@ RegTree::RegTree(unsigned depth, unsigned label) : depth(depth), label(label) {
 void RegTree::PredictRows(const DataMatrix &data, size_t begin, size_t end, float *out) const {
   const size_t offset = ((size_t)1 << (depth - 1)) - 1;
   const size_t F = data.columns_dense;
-  if (!data.is_prebinned) {
-    // float columns: no per-value dispatch, no branch on the comparison
-    bool foreign = false;  // a feature id outside the matrix (foreign model) behaves like NaN: right
+  float *dst = out + (size_t)label * data.rows;
+  if (data.values) {
+    const float *x = data.values->OnHost() + begin * F;
+    const unsigned *fids = fid.data();
+    const float *thr = threshold.data();
+    // a feature id outside the matrix (foreign model) behaves like NaN: right
+    bool foreign = false;
     for (unsigned f : fid) foreign = foreign || f >= F;
-    if (!foreign) {
-      std::vector<const float *> cols(F);
-      for (size_t f = 0; f < F; ++f) cols[f] = data.data[f].data();
-      const unsigned *fids = fid.data();
-      const float *thr = threshold.data();
-      float *dst = out + (size_t)label * data.rows;
-      for (size_t i = begin; i < end; ++i) {
-        size_t id = 0;
-        for (unsigned j = 1; j < depth; ++j) id = 2 * id + 2 - (size_t)(cols[fids[id]][i] < thr[id]);
-        dst[i] += weights[id - offset];
+    for (size_t i = begin; i < end; ++i, x += F) {
+      size_t id = 0;
+      if (!foreign) {  // no branch on the comparison
+        for (unsigned j = 1; j < depth; ++j) id = 2 * id + 2 - (size_t)(x[fids[id]] < thr[id]);
+      } else {
+        for (unsigned j = 1; j < depth; ++j) id = 2 * id + 2 - (size_t)(fids[id] < F && x[fids[id]] < thr[id]);
       }
-      return;
+      dst[i] += weights[id - offset];
     }
+    return;
   }
   for (size_t i = begin; i < end; ++i) {
     size_t id = 0;
     for (unsigned j = 1; j < depth; ++j) {
       const unsigned f = fid[id];
-      // a feature id outside the matrix (foreign model) behaves like NaN: right
-      const bool left = f < F && data.value(f, i) < threshold[id];
+      const bool left = f < F && data.BinValue(f, i) < threshold[id];
       id = left ? 2 * id + 1 : 2 * id + 2;
     }
-    out[i + (size_t)label * data.rows] += weights[id - offset];
+    dst[i] += weights[id - offset];
   }
 }
 
@@ -135,11 +154,6 @@ Garden::~Garden() {}
 float Garden::IntoInternal(float v) const {
   if (cfg.objective == kLogisticRegression) return std::log(v / (1 - v));
   return v;
-}
-
-void Garden::FromInternal(const std::vector<float> &in, std::vector<float> *out) const {
-  out->resize(in.size());
-  FromInternal(in.data(), in.size(), out->data());
 }
 
 void Garden::FromInternal(const float *in, size_t count, float *out) const {
@@ -201,20 +215,25 @@ void Garden::GrowTree(DataMatrix *data, const float *grad) {
   builder_->GrowRound(&trees_);
 }
 
+bool Garden::WalksOnDevice(const DataMatrix *data) const {
+  return predict_on_device_ && data->rows > 0 && DeviceCount() > 0;
+}
+
 void Garden::Predict(const DataMatrix *data, float *out, int n_rounds) const {
   const size_t K = cfg.tree.labels_count;
   SyncTrees();
   const long long use = std::min<long long>(n_rounds, (long long)trees_.size());
   const float init = IntoInternal(cfg.tree.initial_y);
-  if (predict_on_device_ && use > 0 && data->rows > 0 && DeviceCount() > 0) {
+  if (use > 0 && WalksOnDevice(data)) {
+    std::lock_guard<std::mutex> lock(predictor_mutex_);
     if (!predictor_) predictor_.reset(CreateDevicePredictor());
-    const float *sums = PredictOnDevice(predictor_.get(), *data, trees_, (size_t)use, K, init);
+    const float *sums = PredictOnDevice(predictor_.get(), *data, trees_, 0, (size_t)use, K, init);
     FromInternal(sums, data->rows * K, out);
     return;
   }
   std::vector<float> tmp(data->rows * K, init);
   // Every tree over one block of rows before the next block: the block's
-  // feature values (column-major, 4096 rows of every column) stay in cache, so
+  // feature values (4096 rows) stay in cache, so
   // the matrix is read once, not once per tree.  Sums per row are added in tree
   // order either way.
   constexpr size_t kBlock = 4096;
@@ -232,11 +251,23 @@ void Garden::UpdateByLastTree(DataMatrix *data) {
   if (!data->HasYHat()) data->ResetYHat(data->rows * K, IntoInternal(cfg.tree.initial_y));
   if (trees_.size() < K) return;
   SyncTrees();
-  for (size_t t = trees_.size() - K; t < trees_.size(); ++t) trees_[t].Predict(*data, data->YHat().data());
+  std::vector<float> &y_hat = data->YHat();
+  if (WalksOnDevice(data)) {
+    // (a predictor of its own: the other one keeps the whole model laid out)
+    std::lock_guard<std::mutex> lock(predictor_mutex_);
+    if (!round_predictor_) round_predictor_.reset(CreateDevicePredictor());
+    const float *sums = PredictOnDevice(round_predictor_.get(), *data, trees_, trees_.size() - K, trees_.size(), K, 0.0f);
+    ParallelFor(y_hat.size(), [&](size_t b, size_t e) {
+      for (size_t i = b; i < e; ++i) y_hat[i] += sums[i];
+    });
+    return;
+  }
+  for (size_t t = trees_.size() - K; t < trees_.size(); ++t) trees_[t].Predict(*data, y_hat.data());
 }
 
-void Garden::GetY(DataMatrix *data, std::vector<float> *out) const {
-  FromInternal(data->YHat(), out);
+void Garden::GetY(DataMatrix *data, float *out) const {
+  const std::vector<float> &y_hat = data->YHat();
+  FromInternal(y_hat.data(), y_hat.size(), out);
 }
 
 // src/core/model_helper.cpp:16-23, json_conversion.h:13-40

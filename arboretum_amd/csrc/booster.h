@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "config.h"
+#include "float_rows.h"
 
 namespace arb {
 
@@ -31,10 +32,12 @@ class DataMatrix {
   // the same address (device-side caches are keyed by it).
   const uint64_t uid;
 
-  // Column-major host store, one contiguous vector per feature (io.h:22).
-  std::vector<std::vector<float>> data;
+  // The feature values (io.h:22), row-major; null for a pre-quantised matrix.
+  std::unique_ptr<FloatRows> values;
+  // One contiguous vector per feature: a copy, for the host sorts of the exact method.
+  std::vector<std::vector<float>> Columns() const;
   // Pre-quantised input: row-major [rows][columns_dense] bin ids instead of
-  // floats (extension; `data` is then empty).
+  // floats (extension; `values` is then null).
   std::vector<uint8_t> prebinned;
   bool is_prebinned = false;
   std::vector<std::vector<unsigned>> data_categories;
@@ -80,9 +83,8 @@ class DataMatrix {
   // The blocks belong to the caller (ACreateFromQuantizedBlocks): never copied, never freed.
   bool external_blocks = false;
 
-  // Feature value as seen by host prediction.
-  inline float value(size_t f, size_t i) const {
-    if (!is_prebinned) return data[f][i];
+  // Feature value of a pre-quantised matrix as seen by host prediction.
+  inline float BinValue(size_t f, size_t i) const {
     if (!prebinned.empty()) return (float)prebinned[i * columns_dense + f];
     const uint32_t q = stream_blocks[i / stream_block_rows][(f >> 2) * stream_block_rows + i % stream_block_rows];
     return (float)((q >> (8 * (f & 3))) & 255u);
@@ -155,12 +157,6 @@ class TreeBuilder {
   virtual void Synchronize() = 0;
 };
 
-// quantiser.hip: thresholds of one column by a device radix sort
-struct SortWorkspace;
-SortWorkspace *CreateSortWorkspace(size_t n, int hist_size);
-void FreeSortWorkspace(SortWorkspace *ws);
-void DeviceThresholds(SortWorkspace *ws, const float *d_col, std::vector<float> *thr, int *size, bool *has_nan);
-
 // device_builder.hip
 // streamed = false: bins resident in HBM; true: bins in pinned host blocks of
 // block_rows rows, copied to the GPU block by block at every tree level.
@@ -182,14 +178,15 @@ int DeviceCount();
 void CopyProbe(size_t bytes);
 
 // predictor.hip: tree walks of a matrix (floats or bin ids) on the GPU.  Returns [labels][rows]
-// sums of leaf weights of trees[0, use) on top of `init`, bit-identical to the
+// sums of leaf weights of trees[begin, end) on top of `init`, bit-identical to the
 // host walk (RegTree::Predict in tree order), in pinned host memory that the
-// predictor owns and overwrites on its next call.
+// predictor owns and overwrites on its next call.  One predictor serves one vector of trees,
+// which only grows.
 struct DevicePredictor;
 DevicePredictor *CreateDevicePredictor();
 void FreeDevicePredictor(DevicePredictor *p);
 const float *PredictOnDevice(DevicePredictor *p, const DataMatrix &data, const std::vector<RegTree> &trees,
-                             size_t use, size_t labels, float init);
+                             size_t begin, size_t end, size_t labels, float init);
 
 class Garden {
  public:
@@ -201,12 +198,11 @@ class Garden {
   // out: rows * labels_count floats
   void Predict(const DataMatrix *data, float *out, int n_rounds) const;  // :643-657
   void UpdateByLastTree(DataMatrix *data);                   // :627-635
-  void GetY(DataMatrix *data, std::vector<float> *out) const;  // :637-641
+  void GetY(DataMatrix *data, float *out) const;             // :637-641; out: rows * labels_count floats
   const char *GetModel();                                    // :659-665
   void Restore(const char *json_model);                      // :667-677
 
   float IntoInternal(float v) const;                         // objective.h:20,55-57
-  void FromInternal(const std::vector<float> &in, std::vector<float> *out) const;
   void FromInternal(const float *in, size_t count, float *out) const;  // count = rows * labels_count
 
   // Inspection / timing switches; they also apply to a builder created later.
@@ -233,6 +229,9 @@ class Garden {
   bool inspect_ = false;
   int timing_ = 0;
   bool predict_on_device_ = true;
+  bool WalksOnDevice(const DataMatrix *data) const;
+  mutable std::mutex predictor_mutex_;  // the predictors' results are read under it
+  mutable std::unique_ptr<DevicePredictor, void (*)(DevicePredictor *)> round_predictor_{nullptr, FreeDevicePredictor};
   mutable std::unique_ptr<DevicePredictor, void (*)(DevicePredictor *)> predictor_{nullptr, FreeDevicePredictor};
 };
 

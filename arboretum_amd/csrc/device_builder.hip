@@ -48,6 +48,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <limits>
 #include <random>
 #include <stdexcept>
@@ -71,6 +72,7 @@
 #include "kernels_stream.h"
 #include "memory_pool.h"
 #include "parallel.h"
+#include "quantiser.h"
 #include "staging.h"
 
 namespace arb {
@@ -176,9 +178,10 @@ static std::vector<uint16_t> ExactRanks(DataMatrix *data, size_t *most_distinct,
   std::vector<std::vector<float>> mapping(F);
   std::atomic<bool> has_nan{false};
   std::atomic<int> too_many{-1};
+  const std::vector<std::vector<float>> columns = data->Columns();
   ParallelTasks((size_t)F, [&](size_t f) {
     if (has_nan || too_many >= 0) return;
-    std::vector<float> m(data->data[f]);
+    std::vector<float> m(columns[f]);
     for (float v : m)
       if (v != v) has_nan = true;
     if (has_nan) return;
@@ -188,7 +191,7 @@ static std::vector<uint16_t> ExactRanks(DataMatrix *data, size_t *most_distinct,
       too_many = (int)f;
       return;
     }
-    const float *col = data->data[f].data();
+    const float *col = columns[f].data();
     for (size_t i = 0; i < n; ++i)
       ranks[i * F + f] = (uint16_t)(std::lower_bound(m.begin(), m.end(), col[i]) - m.begin());
     mapping[f].swap(m);
@@ -212,6 +215,141 @@ static std::vector<uint16_t> ExactRanks(DataMatrix *data, size_t *most_distinct,
     for (size_t k = 0; k + 1 < mapping[f].size(); ++k) data->thresholds[f][k] = mapping[f][k + 1];
   }
   return ranks;
+}
+
+// Thresholds and bin ids of a float matrix: fills data->thresholds / reduced_size and the bins of
+// `dm` (16-bit ones when a feature has more ids than 8 bits hold).  d_hi: columns of ninth-bit words,
+// or null.  Streamed: quad q of all rows goes to store_quad(q, device address).
+static void QuantiseFloats(DataMatrix *data, DeviceMatrix *dm, int hist_size, bool verbose, uint32_t *d_hi, int hi_words,
+                           const std::function<void(int, const uint32_t *)> &store_quad) {
+  const size_t n = dm->rows;
+  const int F = dm->F;
+  const bool streamed = dm->streamed;
+  // Columns per batch: their floats, the sort's two key buffers and, streamed, their quads.  Few
+  // columns of many rows are sorted one at a time.
+  constexpr size_t kBatchBytes = (size_t)6 << 30;
+  const int batch = (int)std::min<size_t>(std::min((size_t)(F + 3) / 4 * 4, (size_t)1 << 14), std::max<size_t>(4, kBatchBytes / (13 * n) / 4 * 4));
+  const size_t left = kBatchBytes > 5 * n * batch ? kBatchBytes - 5 * n * batch : 0;
+  const int sorted_at_once = (int)std::min<size_t>(batch, std::max<size_t>(1, left / (8 * n)));
+  struct Buffers {
+    hipStream_t st = StreamPoolTake();
+    SortWorkspace *ws = nullptr;
+    void *p[4] = {};
+    void *Words(int k, size_t count) { return p[k] = DevicePoolTake(count * sizeof(uint32_t)); }
+    ~Buffers() {
+      (void)hipStreamSynchronize(st);
+      FreeSortWorkspace(ws);
+      for (void *q : p) DevicePoolGive(q);
+      StreamPoolGive(st);
+    }
+  } buf;
+  buf.ws = CreateSortWorkspace(n, hist_size, sorted_at_once);
+  float *d_x = static_cast<float *>(buf.Words(0, (size_t)batch * n));
+  // thresholds, sizes and NaN flags of all features in one block: they come back in one copy
+  const size_t thr_words = (size_t)F * hist_size;
+  uint32_t *d_facts = static_cast<uint32_t *>(buf.Words(1, thr_words + 2 * (size_t)F));
+  float *d_thr = reinterpret_cast<float *>(d_facts);
+  int *d_size = reinterpret_cast<int *>(d_facts + thr_words);
+  unsigned *d_nan = d_facts + thr_words + F;
+  uint32_t *d_quads = streamed ? static_cast<uint32_t *>(buf.Words(2, (size_t)(batch / 4) * dm->stride)) : nullptr;
+  const float *rows = data->values->OnDevice();
+  if (!rows) buf.Words(3, kStageBytes / sizeof(float));
+  if (d_hi) HIP_OK(hipMemsetAsync(d_hi, 0, (size_t)hi_words * dm->stride * sizeof(uint32_t), buf.st));
+
+  auto load = [&](int f0, int nf) {
+    if (rows) {
+      RowsToColumns(rows, n, F, f0, nf, d_x, n, 0, buf.st);
+      return;
+    }
+    const float *host = data->values->OnHost();
+    const size_t piece = kStageBytes / sizeof(float) / nf;
+    if (piece == 0) throw std::runtime_error("too many features");
+    auto rows_of = [&](size_t k) { return std::min(piece, n - k * piece); };
+    float *d_piece = static_cast<float *>(buf.p[3]);
+    StageToDevice((n + piece - 1) / piece, [&](size_t k) { return rows_of(k) * nf * sizeof(float); },
+                  [&](size_t k, void *p) {
+                    float *dst = static_cast<float *>(p);
+                    const float *src = host + k * piece * F + f0;
+                    ParallelFor(rows_of(k), [&](size_t b, size_t e) {
+                      for (size_t r = b; r < e; ++r) std::memcpy(dst + r * nf, src + r * F, nf * sizeof(float));
+                    }, 1024);
+                  },
+                  [&](size_t) { return d_piece; },
+                  [&](size_t k) { RowsToColumns(d_piece, rows_of(k), nf, 0, nf, d_x, n, k * piece, buf.st); }, buf.st);
+  };
+  std::vector<uint32_t> facts(thr_words + 2 * (size_t)F);
+  int known = 0;  // features whose thresholds have been found
+  // One pass over the columns with `bits` bits per bin id; false when a feature needs more ids than
+  // 8 bits hold.
+  auto quantise = [&](int bits) -> bool {
+    for (int f0 = 0; f0 < F; f0 += batch) {
+      const int nf = std::min(batch, F - f0);
+      if (F > batch || known < F) load(f0, nf);
+      if (known <= f0) {
+        for (int c = 0; c < nf; c += sorted_at_once) {
+          const int nc = std::min(sorted_at_once, nf - c), f = f0 + c;
+          DeviceThresholds(buf.ws, d_x + (size_t)c * n, nc, d_thr + (size_t)f * hist_size, d_size + f, d_nan + f, buf.st);
+        }
+        if (nf == F) {
+          CopyToHost(facts.data(), d_facts, facts.size() * sizeof(uint32_t), buf.st);
+        } else {
+          CopyToHost(facts.data() + (size_t)f0 * hist_size, d_thr + (size_t)f0 * hist_size, (size_t)nf * hist_size * sizeof(float), buf.st);
+          CopyToHost(facts.data() + thr_words + f0, d_size + f0, nf * sizeof(int), buf.st);
+          CopyToHost(facts.data() + thr_words + F + f0, d_nan + f0, nf * sizeof(unsigned), buf.st);
+        }
+        for (int f = f0; f < f0 + nf; ++f) {
+          data->thresholds[f].resize(hist_size);
+          std::memcpy(data->thresholds[f].data(), facts.data() + (size_t)f * hist_size, hist_size * sizeof(float));
+          data->reduced_size[f] = (int)facts[thr_words + f];
+          if (verbose)
+            printf("feature %d has been reduced to %d bits \n", f, 32 - __builtin_clz((unsigned)data->reduced_size[f]));
+        }
+        known = f0 + nf;
+      }
+      for (int f = f0; bits == 8 && f < f0 + nf; ++f)
+        if (data->reduced_size[f] + (facts[thr_words + F + f] ? 1 : 0) > kSlots) {
+          // id 256: the ninth-bit words take it, where the matrix has them
+          if (d_hi == nullptr || data->reduced_size[f] + 1 > kSlots + 1) return false;
+          dm->hi = true;
+          dm->H = hi_words;
+        }
+      const int W = 32 / bits, q0 = f0 / W, quads = (nf + W - 1) / W;
+      uint32_t *out = streamed ? d_quads : dm->bins + (size_t)q0 * dm->stride;
+      // (a workgroup reads its thresholds before it starts: many rows each, once the chip is full)
+      const dim3 grid((unsigned)GridFor(n, 256, std::max(64, 4096 / quads)), (unsigned)quads);
+      if (bits == 8)
+        hipLaunchKernelGGL(k_bin_assign, grid, dim3(256), 0, buf.st, d_x, f0, nf, d_thr, hist_size, d_size, out,
+                           dm->stride, n, d_hi, dm->stride);
+      else
+        hipLaunchKernelGGL(k_bin_assign_wide, grid, dim3(256), 2 * (size_t)hist_size * sizeof(float), buf.st, d_x, f0, nf,
+                           d_thr, hist_size, d_size, out, dm->stride, n);
+      HIP_OK(hipGetLastError());
+      if (streamed) {
+        HIP_OK(hipStreamSynchronize(buf.st));
+        for (int q = 0; q < quads; ++q) store_quad(q0 + q, d_quads + (size_t)q * dm->stride);
+      }
+    }
+    HIP_OK(hipStreamSynchronize(buf.st));
+    for (int w = 0; streamed && w < dm->H; ++w) store_quad(dm->Q + w, d_hi + (size_t)w * dm->stride);
+    return true;
+  };
+  if (quantise(8)) return;
+  // Some feature has more than 256 bin ids: 16-bit bins, two features per
+  // word, hist_size + 1 slots per feature rounded up to a power of two.
+  if (streamed) throw std::runtime_error("a feature needs more than 256 bin ids: 16-bit bins are not built for streamed matrices");
+  int slots = kSlots;
+  while (slots < hist_size + 1) slots *= 2;
+  if (slots > kMaxWideSlots) throw std::runtime_error("hist_size above 4095 is not supported");
+  HIP_OK(hipStreamSynchronize(buf.st));
+  DevicePoolGive(dm->bins);
+  dm->bins = nullptr;
+  dm->bits = 16;
+  dm->slots = slots;
+  dm->hi = false;
+  dm->H = 0;
+  dm->Q = dm->cols = (F + 1) / 2;
+  dm->bins = DevAlloc<uint32_t>((size_t)dm->Q * dm->stride);
+  if (!quantise(16)) throw std::runtime_error("internal: 16-bit quantisation failed");
 }
 
 void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool streamed, size_t block_rows, bool exact,
@@ -267,7 +405,6 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
   const bool may_need_hi = !exact && !data->is_prebinned && hist_size >= kSlots;
   const int hi_words = (F + 31) / 32;
   dm->cols = dm->Q + (may_need_hi ? hi_words : 0);
-  uint32_t *d_col = nullptr;  // streamed: one quad column at a time on the device
   uint32_t *d_hi = nullptr;   // the column of ninth-bit words while the features are quantised
   size_t nblocks = 0;
   if (streamed) {
@@ -281,14 +418,12 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
     dm->host_blocks.assign(nblocks, nullptr);
     for (size_t b = 0; b < nblocks; ++b)
       HIP_OK(hipHostMalloc((void **)&dm->host_blocks[b], (size_t)dm->cols * block_rows * sizeof(uint32_t), hipHostMallocDefault));
-    d_col = DevAlloc<uint32_t>(dm->stride);
     if (may_need_hi) d_hi = DevAlloc<uint32_t>((size_t)hi_words * dm->stride);
   } else {
     dm->bins = DevAlloc<uint32_t>((size_t)dm->cols * dm->stride);
     if (may_need_hi) d_hi = dm->bins + (size_t)dm->Q * dm->stride;
   }
-  if (d_hi) HIP_OK(hipMemset(d_hi, 0, (size_t)hi_words * dm->stride * sizeof(uint32_t)));
-  // streamed: quad q of all rows (in d_col) -> its slice of every host block
+  // streamed: quad q of all rows (on the device) -> its slice of every host block
   auto store_quad = [&](int q, const uint32_t *col) {
     for (size_t b = 0; b < nblocks; ++b) {
       const size_t r0 = b * block_rows, rows = std::min(block_rows, n - r0);
@@ -363,92 +498,8 @@ void QuantiseOnDevice(DataMatrix *data, int hist_size, bool verbose, bool stream
       std::vector<uint8_t>().swap(data->prebinned);  // the pinned blocks are the only copy from here on
     }
   } else {
-    // per quad: upload four columns, thresholds by device sort, bin assignment
-    std::unique_ptr<SortWorkspace, void (*)(SortWorkspace *)> ws(CreateSortWorkspace(n, hist_size), FreeSortWorkspace);
-    float *d_x = DevAlloc<float>(4 * n);
-    float *d_thr = DevAlloc<float>(4 * (size_t)hist_size);
-    int *d_size = DevAlloc<int>(4);
-    // Columns go through two pinned staging buffers: the next column is copied
-    // there by host threads while the GPU sorts the current one, and the copy
-    // to the device runs at the full host-to-device rate.
-    float *stage[2] = {nullptr, nullptr};
-    for (int k = 0; k < 2; ++k) HIP_OK(hipHostMalloc((void **)&stage[k], n * sizeof(float), hipHostMallocDefault));
-    auto stage_column = [&](int f, int slot) {
-      const float *src = data->data[f].data();
-      float *dst = stage[slot];
-      ParallelFor(n, [&](size_t b, size_t e) { std::memcpy(dst + b, src + b, (e - b) * sizeof(float)); });
-    };
-    // One pass over the columns with `bits` bits per bin id; false when a
-    // feature needs more ids than 8 bits hold.
-    auto quantise_columns = [&](int bits) -> bool {
-      const int W = 32 / bits;  // features per word
-      stage_column(0, 0);
-      for (int q = 0; q < dm->Q; ++q) {
-        const int nc = std::min(W, F - q * W);
-        int sizes[4] = {0, 0, 0, 0};
-        for (int c = 0; c < nc; ++c) {
-          const int f = q * W + c;
-          std::thread next;
-          if (f + 1 < F) next = std::thread(stage_column, f + 1, (f + 1) & 1);
-          struct Joiner {
-            std::thread &t;
-            ~Joiner() { if (t.joinable()) t.join(); }
-          } joiner{next};
-          HIP_OK(hipMemcpy(d_x + (size_t)c * n, stage[f & 1], n * sizeof(float), hipMemcpyHostToDevice));
-          bool has_nan = false;
-          DeviceThresholds(ws.get(), d_x + (size_t)c * n, &data->thresholds[f], &data->reduced_size[f], &has_nan);
-          if (bits == 8 && data->reduced_size[f] + (has_nan ? 1 : 0) > kSlots) {
-            // id 256: the ninth-bit words take it, where the matrix has them
-            if (d_hi == nullptr || data->reduced_size[f] + 1 > kSlots + 1) return false;
-            dm->hi = true;
-            dm->H = hi_words;
-          }
-          if (verbose)
-            printf("feature %d has been reduced to %d bits \n", f,
-                   32 - __builtin_clz((unsigned)data->reduced_size[f]));
-          HIP_OK(hipMemcpy(d_thr + (size_t)c * hist_size, data->thresholds[f].data(),
-                           hist_size * sizeof(float), hipMemcpyHostToDevice));
-          sizes[c] = data->reduced_size[f];
-        }
-        HIP_OK(hipMemcpy(d_size, sizes, sizeof(sizes), hipMemcpyHostToDevice));
-        uint32_t *out = streamed ? d_col : dm->bins + (size_t)q * dm->stride;
-        if (bits == 8)
-          hipLaunchKernelGGL(k_bin_assign, dim3(GridFor(n, 256)), dim3(256), 0, 0, d_x, nc, d_thr, hist_size, d_size,
-                             out, n, d_hi ? d_hi + (size_t)((q * W) >> 5) * dm->stride : nullptr, (q * W) & 31);
-        else
-          hipLaunchKernelGGL(k_bin_assign_wide, dim3(GridFor(n, 256)), dim3(256),
-                             2 * (size_t)hist_size * sizeof(float), 0, d_x, nc, d_thr, hist_size, d_size, out, n);
-        HIP_OK(hipGetLastError());
-        HIP_OK(hipDeviceSynchronize());
-        if (streamed) store_quad(q, d_col);
-      }
-      for (int w = 0; streamed && w < dm->H; ++w) store_quad(dm->Q + w, d_hi + (size_t)w * dm->stride);
-      return true;
-    };
-    if (!quantise_columns(8)) {
-      // Some feature has more than 256 bin ids: 16-bit bins, two features per
-      // word, hist_size + 1 slots per feature rounded up to a power of two.
-      if (streamed) throw std::runtime_error("a feature needs more than 256 bin ids: 16-bit bins are not built for streamed matrices");
-      int slots = kSlots;
-      while (slots < hist_size + 1) slots *= 2;
-      if (slots > kMaxWideSlots) throw std::runtime_error("hist_size above 4095 is not supported");
-      DevicePoolGive(dm->bins);
-      dm->bins = nullptr;
-      dm->bits = 16;
-      dm->slots = slots;
-      dm->hi = false;
-      dm->H = 0;
-      d_hi = nullptr;  // (was a part of dm->bins: a resident matrix)
-      dm->Q = dm->cols = (F + 1) / 2;
-      dm->bins = DevAlloc<uint32_t>((size_t)dm->Q * dm->stride);
-      if (!quantise_columns(16)) throw std::runtime_error("internal: 16-bit quantisation failed");
-    }
-    DevicePoolGive(d_x);
-    DevicePoolGive(d_thr);
-    DevicePoolGive(d_size);
-    for (int k = 0; k < 2; ++k) HIP_OK(hipHostFree(stage[k]));
+    QuantiseFloats(data, dm.get(), hist_size, verbose, d_hi, hi_words, store_quad);
   }
-  if (d_col) DevicePoolGive(d_col);
   if (streamed && d_hi) DevicePoolGive(d_hi);
   if (dm->hi) dm->slots = kSlots + 1;
   if (streamed) {

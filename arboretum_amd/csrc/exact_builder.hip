@@ -64,13 +64,14 @@ void PrepareExactSort(DataMatrix *data) {
   std::vector<uint32_t> ranks((size_t)F * stride, 0u), lists((size_t)F * stride, 0u), list_ranks((size_t)F * stride, 0u);
   std::vector<std::vector<float>> mapping(F);
   std::atomic<bool> has_nan{false};
+  const std::vector<std::vector<float>> columns = data->Columns();
   // one column per thread at a time (the columns are few and long)
   ParallelTasks((size_t)F, [&](size_t f) {
     if (has_nan) return;
     // (value, row) packed into one integer that sorts like the pair: the float's bits with the
     // sign folded so that unsigned order is numeric order, above the row id
     std::vector<uint64_t> keyed(n);
-    const float *col = data->data[f].data();
+    const float *col = columns[f].data();
     for (size_t i = 0; i < n; ++i) {
       if (col[i] != col[i]) has_nan = true;
       uint32_t u;

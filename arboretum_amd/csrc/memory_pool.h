@@ -32,6 +32,10 @@ void PinnedPoolGive(void *p) noexcept;
 void *HostPoolTake(size_t bytes);
 void HostPoolGive(void *p) noexcept;
 
+// Whether this process has taken memory or a stream of a GPU from these pools (a child made by fork
+// has not).
+bool GpuInUse() noexcept;
+
 // Streams (non-blocking, default priority) that are kept and handed out again; nothing may be pending
 // on one that is given back.
 hipStream_t StreamPoolTake();

@@ -1,7 +1,9 @@
 #include "memory_pool.h"
 
 #include <hip/hip_runtime.h>
+#include <unistd.h>
 
+#include <atomic>
 #include <chrono>
 #include <cstdlib>
 #include <map>
@@ -175,10 +177,16 @@ int CurrentDevice() {
   return dev;
 }
 
+std::atomic<pid_t> g_gpu_user{0};
+void NoteGpuInUse() { g_gpu_user.store(getpid(), std::memory_order_relaxed); }
+
 }  // namespace
+
+bool GpuInUse() noexcept { return g_gpu_user.load(std::memory_order_relaxed) == getpid(); }
 
 void *DevicePoolTake(size_t bytes) {
   void *p = DevicePool().Take(CurrentDevice(), bytes);
+  if (p) NoteGpuInUse();
   if (!p) throw std::runtime_error("HIP error: out of memory allocating " + std::to_string(bytes) + " bytes of device memory");
   return p;
 }
@@ -203,12 +211,14 @@ hipStream_t StreamPoolTake() {
       if (idle[k].first == dev) {
         hipStream_t s = idle[k].second;
         idle.erase(idle.begin() + k);
+        NoteGpuInUse();
         return s;
       }
   }
   hipStream_t s = nullptr;
   const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
   if (e != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e) + " creating a stream");
+  NoteGpuInUse();
   return s;
 }
 

@@ -1,16 +1,16 @@
 // Batch prediction on the GPU: the tree walks of RegTree::Predict /
 // Garden::Predict (src/core/garden.h:70-90, src/core/garden.cu:643-657) for a
 // float matrix (or a pre-quantised one, whose bin ids are compared as floats
-// like the host walk does), every tree over a block of rows while the next
-// block is staged.  The arithmetic is the host walk's: `x < threshold` goes left (NaN
-// right), the leaf weights of one label are added in tree order in fp32, so
-// the sums are bit-identical to the host path.  The link function stays with
-// the caller.
+// like the host walk does).  The arithmetic is the host walk's: `x < threshold`
+// goes left (NaN right), the leaf weights of one label are added in tree order
+// in fp32, so the sums are bit-identical to the host path.  The link function
+// stays with the caller.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -18,6 +18,7 @@
 #include "booster.h"
 #include "memory_pool.h"
 #include "parallel.h"
+#include "staging.h"
 
 namespace arb {
 namespace {
@@ -29,176 +30,327 @@ namespace {
       throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_) + " in " #expr); \
   } while (0)
 
-constexpr int kPredictThreads = 1024;          // rows per workgroup, one row per thread
-constexpr size_t kTreeLdsBytes = 64 * 1024;    // trees staged in LDS at a time: two workgroups per CU
-constexpr size_t kStageBytes = 32u << 20;      // one pinned staging buffer
-constexpr size_t kCacheBytes = (size_t)8 << 30;  // largest float matrix kept on the device between calls
+constexpr unsigned kWalkThreads = 1024;
+constexpr size_t kWalkLds = 159 * 1024;           // of the 160 KB of a CU: one workgroup of 16 waves has it
+constexpr size_t kTreeLds = 40 * 1024;            // trees staged at a time when rows are many
+constexpr unsigned kAhead = 5;                    // words per thread fetched while the chunk before is walked
+constexpr unsigned kChains = 4;                   // trees a thread walks side by side
+constexpr size_t kBlockBytes = (size_t)32 << 20;  // device block of rows that are not kept on the device
 
+// A tree as 8-byte words: its 2^(depth-1) - 1 nodes (feature, threshold bits) in heap order, then its
+// 2^(depth-1) leaf weights, two to a word.
 struct TreeRef {
-  unsigned node_off;  // first internal node in the flattened node array
-  unsigned leaf_off;  // first leaf weight
-  unsigned depth;     // internal depth: depth - 1 comparisons
-  unsigned label;
-};
-
-// Consecutive trees [t0, t1) whose nodes and leaves fit the LDS budget
-// together, or a single tree that does not (in_lds = 0, read from global).
-struct Chunk {
-  unsigned t0, t1, in_lds, n_nodes, n_leaves;
+  unsigned off, depth, label, unused;
 };
 
 // Where a row's feature values come from.
 enum Source {
-  kFloatCols = 0,  // float columns [F][ld]
-  kByteRows = 1,   // pre-quantised rows [rows][ld = F] of uint8 bin ids
+  kFloatRows = 0,  // float rows [n][F]
+  kByteRows = 1,   // pre-quantised rows [n][F] of uint8 bin ids
   kQuadCols = 2    // pre-quantised quad columns [Q][ld]: four uint8 bin ids per word
 };
 
-template <int SRC>
-__device__ __forceinline__ float Fetch(const void *__restrict__ base, size_t ld, unsigned r, unsigned f) {
-  if (SRC == kFloatCols) return static_cast<const float *>(base)[(size_t)f * ld + r];
-  if (SRC == kByteRows) return (float)static_cast<const uint8_t *>(base)[(size_t)r * ld + f];
-  return (float)((static_cast<const uint32_t *>(base)[(size_t)(f >> 2) * ld + r] >> (8u * (f & 3u))) & 255u);
-}
+struct Walk {
+  const void *base;
+  size_t ld;               // kQuadCols
+  unsigned n, F;           // rows at `base`, features
+  unsigned rows_log;       // log2 of the rows of a workgroup, 6 ... 10
+  const uint2 *words;
+  const TreeRef *refs;     // n_trees of them in order of labels, and one more whose `off` is the end
+  unsigned n_trees, per_chunk, labels;
+  unsigned tree_words;     // != 0: every tree has so many words and the depth `depth`
+  unsigned depth;
+  unsigned words_at, leaf_at;  // bytes: where in the LDS the trees and the leaf weights found stand
+  float init;
+  float *out;              // [labels][out_ld], at the first of the n rows
+  size_t out_ld;
+};
 
-// Walks trees [t0, t1) for row r of `base`.  acc holds the running sum of
-// label *cur.
-template <int SRC>
-__device__ __forceinline__ void WalkTrees(const uint2 *nd, const float *lf, unsigned node_base, unsigned leaf_base,
-                                          const TreeRef *__restrict__ refs, unsigned t0, unsigned t1,
-                                          const void *__restrict__ base, size_t ld, unsigned r,
-                                          float *__restrict__ out, size_t out_ld, bool live, int *cur, float *acc) {
-  for (unsigned t = t0; t < t1; ++t) {
-    const TreeRef ref = refs[t];
-    if ((int)ref.label != *cur) {
-      if (*cur >= 0 && live) out[(size_t)*cur * out_ld] = *acc;
-      *cur = (int)ref.label;
-      *acc = out[(size_t)ref.label * out_ld];
-    }
-    const uint2 *tn = nd + (ref.node_off - node_base);
-    unsigned id = 0;
-    for (unsigned j = 1; j < ref.depth; ++j) {
-      const uint2 n = tn[id];
-      const float v = Fetch<SRC>(base, ld, r, n.x);
-      id = 2 * id + 2 - (unsigned)(v < __uint_as_float(n.y));
-    }
-    *acc += lf[ref.leaf_off - leaf_base + (id - ((1u << (ref.depth - 1)) - 1))];
-  }
-}
-
-// base: this block's rows as SRC says; out: [labels][out_ld], already offset
-// to the block's first row.  grid ceil(rows / 1024).
-template <int SRC>
-__global__ void __launch_bounds__(kPredictThreads)
-k_predict(const void *__restrict__ base, size_t ld, unsigned rows, const uint2 *__restrict__ nodes,
-          const float *__restrict__ leaves, const TreeRef *__restrict__ refs, const Chunk *__restrict__ chunks,
-          int n_chunks, float *__restrict__ out, size_t out_ld) {
-  extern __shared__ unsigned char smem[];
-  const unsigned i = blockIdx.x * kPredictThreads + threadIdx.x;
-  const bool live = i < rows;
-  const unsigned r = live ? i : rows - 1;
-  float *o = out + r;
-  int cur = -1;
-  float acc = 0.0f;
-  for (int c = 0; c < n_chunks; ++c) {
-    const Chunk ch = chunks[c];
-    const unsigned node_base = refs[ch.t0].node_off, leaf_base = refs[ch.t0].leaf_off;
-    if (ch.in_lds) {
-      uint2 *s_nd = (uint2 *)smem;
-      float *s_lf = (float *)(smem + (size_t)ch.n_nodes * sizeof(uint2));
-      __syncthreads();  // the previous chunk's trees are no longer read
-      for (unsigned k = threadIdx.x; k < ch.n_nodes; k += kPredictThreads) s_nd[k] = nodes[node_base + k];
-      for (unsigned k = threadIdx.x; k < ch.n_leaves; k += kPredictThreads) s_lf[k] = leaves[leaf_base + k];
-      __syncthreads();
-      WalkTrees<SRC>(s_nd, s_lf, node_base, leaf_base, refs, ch.t0, ch.t1, base, ld, r, o, out_ld, live, &cur, &acc);
-    } else {
-      WalkTrees<SRC>(nodes + node_base, leaves + leaf_base, node_base, leaf_base, refs, ch.t0, ch.t1, base, ld, r, o,
-                     out_ld, live, &cur, &acc);
-    }
-  }
-  if (cur >= 0 && live) o[(size_t)cur * out_ld] = acc;
-}
-
-__global__ void __launch_bounds__(256) k_predict_fill(float *__restrict__ p, size_t n, float v) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
+// The LDS by byte address: a 32-bit register is the whole address of a read.
 template <typename T>
-struct DevBuf {
-  T *p = nullptr;
-  size_t n = 0;
-  ~DevBuf() { DevicePoolGive(p); }
-  void Reserve(size_t want) {
-    if (want <= n) return;
-    if (p) DevicePoolGive(p);
-    p = nullptr;
-    n = 0;
-    p = static_cast<decltype(p)>(DevicePoolTake(want * sizeof(T)));
-    n = want;
-  }
-  // blocking: the vector may be gone when the call returns
-  void Upload(const std::vector<T> &v) {
-    Reserve(std::max<size_t>(v.size(), 1));
-    if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+__device__ __forceinline__ T LdsAt(unsigned at) {
+  return *(const __attribute__((address_space(3))) T *)at;
+}
+__device__ __forceinline__ unsigned LdsAddress(const unsigned char *p) {
+  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char *)p;
+}
+
+template <int SRC>
+struct Values {
+  typedef unsigned char T;
+};
+template <>
+struct Values<kFloatRows> {
+  typedef float T;
+};
+
+// Value of feature f of the thread's row: from the LDS tile [F][R], or from memory.
+template <int SRC, bool TILE>
+struct Fetch {
+  unsigned R, r;  // bytes of R elements, LDS address of the row's value of feature 0
+  const Walk &a;
+  size_t row;
+  __device__ __forceinline__ float operator()(unsigned f) const {
+    if (TILE) return (float)LdsAt<typename Values<SRC>::T>(__umul24(f, R) + r);
+    if (SRC == kQuadCols)
+      return (float)((static_cast<const uint32_t *>(a.base)[(size_t)(f >> 2) * a.ld + row] >> (8u * (f & 3u))) & 255u);
+    return (float)static_cast<const typename Values<SRC>::T *>(a.base)[row * a.F + f];
   }
 };
 
+// (no class type: it is read through a pointer of an address space)
+typedef unsigned Node __attribute__((ext_vector_type(2)));
+
+// N trees walked side by side: their chains of a node and a value read per level overlap.  w: where
+// the trees start, LDS addresses or bytes from `words`.  The children of the node at byte p of its tree are at
+// 2 p + 8 and 2 p + 16, so there at 2 at - w + 8 (16): four vector instructions a level
+// beside the two reads (counting in nodes takes nine, and the walk is as much bound by them as by the LDS).
+template <bool IN_LDS, int N, typename F>
+__device__ __forceinline__ void WalkTrees(const unsigned char *words, const unsigned (&w)[N], unsigned depth,
+                                          const F &fetch, float *leaf) {
+  unsigned at[N], left[N], right[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    at[k] = w[k];
+    left[k] = 8u - w[k];
+    right[k] = 16u - w[k];
+    asm("" : "+v"(left[k]), "+v"(right[k]));  // (registers, not 8 and 16 less w again on every level)
+  }
+  for (unsigned j = 1; j < depth; ++j) {
+    Node nd[N];
+    float v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) nd[k] = IN_LDS ? LdsAt<Node>(at[k]) : *reinterpret_cast<const Node *>(words + at[k]);
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = fetch(nd[k].x);
+#pragma unroll
+    for (int k = 0; k < N; ++k) at[k] = (at[k] << 1) + (v[k] < __uint_as_float(nd[k].y) ? left[k] : right[k]);
+  }
+  // node id = (at - w) / 8; its leaf id - nodes stands 4 (id - nodes) bytes behind the 8 nodes bytes of nodes
+  const unsigned nodes = (1u << (depth - 1)) - 1u;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const unsigned l = w[k] + 4u * nodes + ((at[k] - w[k]) >> 1);
+    leaf[k] = IN_LDS ? LdsAt<float>(l) : *reinterpret_cast<const float *>(words + l);
+  }
+}
+
+// What bounds it: reads of the LDS, a node (8 bytes) and a value (4) per level, tree and row.  A
+// workgroup owns R rows and holds all their values feature-major, so the 64 rows of a wave read 64
+// banks whatever features their nodes ask for; the trees pass through the rest of the LDS in chunks,
+// the next one fetched into registers while one is walked.  R is 1024 when there are rows enough to
+// fill the chip: each staged tree then serves 1024 rows.  With fewer rows or more features R is
+// smaller and the 1024 / R slices of the workgroup take different trees; the leaf weights they find
+// meet in the LDS and are added in tree order.
+// 1,000,003 rows x 28 features, 200 trees of depth 8: 575 us (2370 with the values read from memory and
+// a tree at a time), of which the LDS is busy 210 and the vector units 270; 64 rows by 100 trees of
+// depth 6: 13 us (86).
+template <int SRC, bool TILE, bool TREES_IN_LDS>
+__global__ void __launch_bounds__(kWalkThreads) k_predict(const Walk a) {
+  typedef typename Values<SRC>::T T;
+  extern __shared__ __align__(16) unsigned char smem[];
+  T *tile = reinterpret_cast<T *>(smem);
+  uint2 *s_words = reinterpret_cast<uint2 *>(smem + a.words_at);
+  float *s_leaf = reinterpret_cast<float *>(smem + a.leaf_at);
+  const unsigned R = 1u << a.rows_log, r = threadIdx.x & (R - 1);
+  const unsigned slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> a.rows_log), S = kWalkThreads >> a.rows_log;
+  const unsigned row0 = blockIdx.x * R;
+  const unsigned row = min(row0 + r, a.n - 1);
+  const bool live = row0 + r < a.n;
+
+  auto offset = [&](unsigned t) { return a.tree_words ? t * a.tree_words : a.refs[t].off; };
+  auto chunk_end = [&](unsigned t0) { return min(a.n_trees, t0 + a.per_chunk); };
+  uint2 ahead[kAhead];
+  auto fetch_ahead = [&](unsigned t0) {
+    const unsigned b = offset(t0), e = offset(chunk_end(t0));
+#pragma unroll
+    for (unsigned k = 0; k < kAhead; ++k) {
+      const unsigned i = b + k * kWalkThreads + threadIdx.x;
+      if (i < e) ahead[k] = a.words[i];
+    }
+  };
+  if (TREES_IN_LDS) fetch_ahead(0);
+
+  if (TILE) {
+    const unsigned lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (SRC == kQuadCols) {
+      const uint32_t *q = static_cast<const uint32_t *>(a.base);
+      for (unsigned f4 = 4 * slice; f4 < a.F; f4 += 4 * S) {
+        const uint32_t v = q[(size_t)(f4 >> 2) * a.ld + row];
+        for (unsigned c = 0; c < min(4u, a.F - f4); ++c) tile[(f4 + c) * R + r] = (unsigned char)(v >> (8 * c));
+      }
+    } else {
+      // a wave takes 16 rows by 4 features at a time: its reads are runs of 4 values of each row (the
+      // lines are used up within the workgroup), its writes meet 4 to a bank
+      const T *x = static_cast<const T *>(a.base);
+      const unsigned fours = (a.F + 3) / 4, all = (R / 16) * fours;
+      for (unsigned g = wave; g < all; g += 4 * (kWalkThreads / 64)) {
+        T v[4];
+        unsigned at[4];
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) {
+          const unsigned i = g + k * (kWalkThreads / 64);
+          const unsigned rr = i / fours * 16 + (lane >> 2), f = i % fours * 4 + (lane & 3u);
+          at[k] = f * R + rr;
+          if (i < all && f < a.F) v[k] = x[(size_t)min(row0 + rr, a.n - 1) * a.F + f];
+          else at[k] = ~0u;
+        }
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k)
+          if (at[k] != ~0u) tile[at[k]] = v[k];
+      }
+    }
+  }
+  if (TILE && !TREES_IN_LDS) __syncthreads();
+
+  const Fetch<SRC, TILE> value{R * (unsigned)sizeof(T), LdsAddress(smem) + r * (unsigned)sizeof(T), a, row};
+  unsigned cur = 0;
+  float acc = a.init;
+  auto add = [&](unsigned t, float w) {
+    if (a.labels > 1) {
+      const unsigned label = a.refs[t].label;
+      while (cur != label) {
+        if (live) a.out[(size_t)cur * a.out_ld + row] = acc;
+        acc = a.init;
+        ++cur;
+      }
+    }
+    acc += w;
+  };
+
+  for (unsigned t0 = 0; t0 < a.n_trees; t0 = chunk_end(t0)) {
+    const unsigned t1 = chunk_end(t0);
+    const unsigned b = TREES_IN_LDS ? offset(t0) : 0u;
+    if (TREES_IN_LDS) {
+      const unsigned e = offset(t1);
+      __syncthreads();  // the chunk before is no longer read
+#pragma unroll
+      for (unsigned k = 0; k < kAhead; ++k) {
+        const unsigned i = k * kWalkThreads + threadIdx.x;
+        if (b + i < e) s_words[i] = ahead[k];
+      }
+      for (unsigned i = kAhead * kWalkThreads + threadIdx.x; b + i < e; i += kWalkThreads) s_words[i] = a.words[b + i];
+      __syncthreads();
+      if (t1 < a.n_trees) fetch_ahead(t1);
+    } else if (S > 1) {
+      __syncthreads();  // the leaf weights of the chunk before have been added
+    }
+    const unsigned char *words = reinterpret_cast<const unsigned char *>(a.words);
+    auto tree = [&](unsigned t) {
+      return (unsigned)__builtin_amdgcn_readfirstlane((TREES_IN_LDS ? LdsAddress(smem) + a.words_at : 0u) + (offset(t) - b) * (unsigned)sizeof(uint2));
+    };
+    auto depth = [&](unsigned t) { return a.tree_words ? a.depth : a.refs[t].depth; };
+    for (unsigned t = t0 + slice; t < t1;) {
+      float leaf[kChains];
+      const unsigned d = depth(t);
+      bool four = t + (kChains - 1) * S < t1;
+      for (unsigned k = 1; four && k < kChains; ++k) four = depth(t + k * S) == d;
+      if (four) {
+        unsigned w[kChains];
+#pragma unroll
+        for (unsigned k = 0; k < kChains; ++k) w[k] = tree(t + k * S);
+        WalkTrees<TREES_IN_LDS>(words, w, d, value, leaf);
+      } else {
+        const unsigned w[1] = {tree(t)};
+        WalkTrees<TREES_IN_LDS>(words, w, d, value, leaf);
+      }
+#pragma unroll
+      for (unsigned k = 0; k < kChains; ++k) {
+        if (k > 0 && !four) break;
+        if (S == 1) add(t + k, leaf[k]);
+        else s_leaf[(t + k * S - t0) * R + r] = leaf[k];
+      }
+      t += four ? kChains * S : S;
+    }
+    if (S > 1) {
+      __syncthreads();
+      if (slice == 0) {
+        unsigned t = t0;
+        for (; t + 8 <= t1; t += 8) {
+          float w[8];
+#pragma unroll
+          for (unsigned k = 0; k < 8; ++k) w[k] = s_leaf[(t + k - t0) * R + r];
+#pragma unroll
+          for (unsigned k = 0; k < 8; ++k) add(t + k, w[k]);
+        }
+        for (; t < t1; ++t) add(t, s_leaf[(t - t0) * R + r]);
+      }
+    }
+  }
+  if (slice == 0 && live)
+    for (; cur < a.labels; ++cur, acc = a.init) a.out[(size_t)cur * a.out_ld + row] = acc;
+}
+
+template <int SRC, bool TILE, bool TREES_IN_LDS>
+void Launch(const Walk &a, size_t lds, hipStream_t stream) {
+  static std::once_flag configured;
+  std::call_once(configured, [] {
+    HIP_OK(hipFuncSetAttribute((const void *)k_predict<SRC, TILE, TREES_IN_LDS>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWalkLds));
+  });
+  const unsigned R = 1u << a.rows_log;
+  hipLaunchKernelGGL((k_predict<SRC, TILE, TREES_IN_LDS>), dim3((a.n + R - 1) / R), dim3(kWalkThreads), lds, stream, a);
+  HIP_OK(hipGetLastError());
+}
+
 }  // namespace
 
-// Buffers kept between calls: staging and device blocks are sized once, and
-// the columns of the last matrix (up to kCacheBytes) stay on the device, so
-// that predicting on it again (an evaluation set, once per boosting round)
-// copies nothing.
+// Keeps the model laid out on the device between calls, and the memory of the results.
 struct DevicePredictor {
   hipStream_t stream = nullptr;
-  hipEvent_t copied[2] = {nullptr, nullptr};
-  float *stage[2] = {nullptr, nullptr};
-  size_t stage_floats = 0;
-  DevBuf<float> block, out, leaves, cache;
+  unsigned *model = nullptr;  // refs, then words
+  size_t model_bytes = 0, words_at = 0;
+  // of which trees, for how many features and labels `model` is (the trees of a booster are only added to)
+  size_t begin = 0, end = 0, features = 0, labels_of = 0;
+  unsigned largest = 0, tree_words = 0, depth = 0;
   float *result = nullptr;  // pinned; the sums of the last call
   size_t result_floats = 0;
-  uint64_t cached_uid = 0;  // matrix whose columns `cache` holds as [F][cache_ld]
-  size_t cache_ld = 0;
-  DevBuf<uint2> nodes;
-  DevBuf<TreeRef> refs;
-  DevBuf<Chunk> chunks;
 
   ~DevicePredictor() {
-    for (int k = 0; k < 2; ++k) {
-      if (stage[k]) (void)hipHostFree(stage[k]);
-      if (copied[k]) (void)hipEventDestroy(copied[k]);
-    }
-    if (result) (void)hipHostFree(result);
-    if (stream) (void)hipStreamDestroy(stream);
+    if (stream) (void)hipStreamSynchronize(stream);
+    DevicePoolGive(model);
+    PinnedPoolGive(result);
+    StreamPoolGive(stream);
   }
 
-  const float *Run(const DataMatrix &data, const std::vector<RegTree> &trees, size_t use, size_t labels, float init) {
-    const size_t n = data.rows, F = data.columns_dense;
-    if (n == 0 || F == 0) throw std::runtime_error("empty data matrix");
-    // only the block-wise walk of a streamed matrix indexes rows with 64 bits
-    if (n >= (1ull << 31) && !(data.is_prebinned && data.prebinned.empty() && !data.stream_blocks.empty()))
-      throw std::runtime_error("too many rows");
-    if (!stream) {
-      HIP_OK(hipStreamCreate(&stream));
-      for (int k = 0; k < 2; ++k) HIP_OK(hipEventCreateWithFlags(&copied[k], hipEventDisableTiming));
+  void LayOut(const std::vector<RegTree> &trees, size_t b, size_t e, size_t F, size_t labels) {
+    if (begin == b && end == e && features == F && labels_of == labels) return;
+    end = begin = 0;
+    // in order of labels (stable): the sums of one label are complete before the next one's start
+    std::vector<unsigned> order;
+    for (size_t k = 0; k < labels; ++k)
+      for (size_t t = b; t < e; ++t)
+        if (trees[t].label == k) order.push_back((unsigned)t);
+    if (order.size() != e - b) throw std::runtime_error("tree label out of range");
+    std::vector<TreeRef> refs;
+    size_t words = 0;
+    largest = tree_words = 0;
+    depth = trees[b].depth;
+    bool same = true;
+    for (unsigned t : order) {
+      const size_t w = trees[t].fid.size() + trees[t].weights.size() / 2;
+      refs.push_back(TreeRef{(unsigned)words, trees[t].depth, trees[t].label, 0u});
+      words += w;
+      if (words * sizeof(uint2) >= (1ull << 31)) throw std::runtime_error("model too large for device prediction");
+      largest = std::max(largest, (unsigned)w);
+      same = same && trees[t].depth == depth;
     }
-    // ---- the model, flattened in tree order
-    std::vector<uint2> h_nodes;
-    std::vector<float> h_leaves;
-    std::vector<TreeRef> h_refs;
-    std::vector<Chunk> h_chunks;
-    for (size_t t = 0; t < use; ++t) {
+    refs.push_back(TreeRef{(unsigned)words, 0u, 0u, 0u});
+    if (same) tree_words = largest;
+    words_at = refs.size() * sizeof(TreeRef);
+    const size_t bytes = words_at + words * sizeof(uint2);
+    if (bytes > model_bytes) {
+      DevicePoolGive(model);
+      model = nullptr;
+      model_bytes = 0;
+      model = static_cast<unsigned *>(DevicePoolTake(bytes));
+      model_bytes = bytes;
+    }
+    std::vector<unsigned char> host(bytes);
+    std::memcpy(host.data(), refs.data(), words_at);
+    unsigned char *at = host.data() + words_at;
+    for (unsigned t : order) {
       const RegTree &tr = trees[t];
-      if (tr.label >= labels) throw std::runtime_error("tree label out of range");
-      if (h_nodes.size() + tr.fid.size() >= (1ull << 32) || h_leaves.size() + tr.weights.size() >= (1ull << 32))
-        throw std::runtime_error("model too large for device prediction");
-      TreeRef ref;
-      ref.node_off = (unsigned)h_nodes.size();
-      ref.leaf_off = (unsigned)h_leaves.size();
-      ref.depth = tr.depth;
-      ref.label = tr.label;
-      h_refs.push_back(ref);
       for (size_t k = 0; k < tr.fid.size(); ++k) {
         uint2 nd;
         float thr = tr.threshold[k];
@@ -208,143 +360,141 @@ struct DevicePredictor {
           thr = -std::numeric_limits<float>::infinity();
         }
         std::memcpy(&nd.y, &thr, sizeof(float));
-        h_nodes.push_back(nd);
+        std::memcpy(at, &nd, sizeof(nd));
+        at += sizeof(nd);
       }
-      h_leaves.insert(h_leaves.end(), tr.weights.begin(), tr.weights.end());
-      const size_t bytes = tr.fid.size() * sizeof(uint2) + tr.weights.size() * sizeof(float);
-      const bool fits = bytes <= kTreeLdsBytes;
-      bool joined = false;
-      if (fits && !h_chunks.empty() && h_chunks.back().in_lds) {
-        Chunk &c = h_chunks.back();
-        const size_t total = (c.n_nodes + tr.fid.size()) * sizeof(uint2) + (c.n_leaves + tr.weights.size()) * sizeof(float);
-        if (total <= kTreeLdsBytes) {
-          c.t1 = (unsigned)t + 1;
-          c.n_nodes += (unsigned)tr.fid.size();
-          c.n_leaves += (unsigned)tr.weights.size();
-          joined = true;
-        }
-      }
-      if (!joined) {
-        Chunk c;
-        c.t0 = (unsigned)t;
-        c.t1 = (unsigned)t + 1;
-        c.in_lds = fits ? 1u : 0u;
-        c.n_nodes = (unsigned)tr.fid.size();
-        c.n_leaves = (unsigned)tr.weights.size();
-        h_chunks.push_back(c);
-      }
+      std::memcpy(at, tr.weights.data(), tr.weights.size() * sizeof(float));
+      at += tr.weights.size() * sizeof(float);
     }
-    nodes.Upload(h_nodes);
-    leaves.Upload(h_leaves);
-    refs.Upload(h_refs);
-    chunks.Upload(h_chunks);
-    out.Reserve(labels * n);
-    hipLaunchKernelGGL(k_predict_fill, dim3((unsigned)((labels * n + 255) / 256)), dim3(256), 0, stream, out.p,
-                       labels * n, init);
-    HIP_OK(hipGetLastError());
-    auto walk = [&](int src, const void *base, size_t ld, size_t r0, size_t rows) {
-      if (use == 0) return;
-      const dim3 grid((unsigned)((rows + kPredictThreads - 1) / kPredictThreads)), block_dim(kPredictThreads);
-#define ARB_WALK(S)                                                                                         \
-  hipLaunchKernelGGL((k_predict<S>), grid, block_dim, kTreeLdsBytes, stream, base, ld, (unsigned)rows, nodes.p, \
-                     leaves.p, refs.p, chunks.p, (int)h_chunks.size(), out.p + r0, n)
-      if (src == kFloatCols) ARB_WALK(kFloatCols);
-      else if (src == kByteRows) ARB_WALK(kByteRows);
-      else ARB_WALK(kQuadCols);
+    CopyToDevice(model, host.data(), bytes, stream);
+    begin = b;
+    end = e;
+    features = F;
+    labels_of = labels;
+  }
+
+  // rows [0, n) at `base` into out[label * out_ld + row]
+  void Rows(int src, const void *base, size_t ld, size_t n, size_t F, size_t labels, float init, float *out,
+            size_t out_ld) {
+    Walk a;
+    a.base = base;
+    a.ld = ld;
+    a.n = (unsigned)n;
+    a.F = (unsigned)F;
+    a.refs = reinterpret_cast<const TreeRef *>(model);
+    a.words = reinterpret_cast<const uint2 *>(reinterpret_cast<const unsigned char *>(model) + words_at);
+    a.n_trees = (unsigned)(end - begin);
+    a.labels = (unsigned)labels;
+    a.tree_words = tree_words;
+    a.depth = depth;
+    a.init = init;
+    a.out = out;
+    a.out_ld = out_ld;
+    const size_t element = src == kFloatRows ? sizeof(float) : 1;
+    const size_t tree_bytes = (size_t)largest * sizeof(uint2);
+    auto tile_bytes = [&](unsigned log) { return ((F << log) * element + 15) / 16 * 16; };
+    // As many rows as give a workgroup to every CU, and room for a good chunk of trees beside them.
+    unsigned log = 10;
+    while (log > 6 && (n >> log) < 256) --log;
+    const size_t trees_want = tree_bytes > kWalkLds / 2 ? 0 : std::max(tree_bytes, kTreeLds);
+    // (leaf weights found, per tree: eight trees at least)
+    auto leaves = [](unsigned log) { return log < 10 ? (size_t)4 << log : (size_t)0; };
+    while (log > 6 && tile_bytes(log) + trees_want + 8 * leaves(log) > kWalkLds) --log;
+    const bool tile = tile_bytes(log) + trees_want + 8 * leaves(log) <= kWalkLds;
+    size_t free_lds = kWalkLds - (tile ? tile_bytes(log) : 0);
+    const size_t leaf_bytes = leaves(log);
+    const bool trees_in_lds = tree_bytes + 8 * leaf_bytes <= free_lds;
+    // (whole model at once where rows are few: every chunk ends with a sum that 15 waves wait for)
+    if (log == 10) free_lds = std::min(free_lds, std::max(kTreeLds, tree_bytes));
+    a.rows_log = log;
+    a.words_at = tile ? (unsigned)tile_bytes(log) : 0u;
+    size_t per = free_lds / ((trees_in_lds ? tree_bytes : 0) + std::max<size_t>(leaf_bytes, trees_in_lds ? 0 : 4));
+    per = std::min<size_t>(std::max<size_t>(per, 1), a.n_trees);
+    a.per_chunk = (unsigned)per;
+    a.leaf_at = a.words_at + (unsigned)(trees_in_lds ? per * tree_bytes : 0);
+    const size_t lds = a.leaf_at + per * leaf_bytes;
+#define ARB_WALK(S)                                                    \
+  do {                                                                 \
+    if (tile && trees_in_lds) Launch<S, true, true>(a, lds, stream);   \
+    else if (tile) Launch<S, true, false>(a, lds, stream);             \
+    else if (trees_in_lds) Launch<S, false, true>(a, lds, stream);     \
+    else Launch<S, false, false>(a, lds, stream);                      \
+  } while (0)
+    if (src == kFloatRows) ARB_WALK(kFloatRows);
+    else if (src == kByteRows) ARB_WALK(kByteRows);
+    else ARB_WALK(kQuadCols);
 #undef ARB_WALK
-      HIP_OK(hipGetLastError());
-    };
-    auto reserve_stage = [&](size_t floats) {
-      if (floats <= stage_floats) return;
-      for (int k = 0; k < 2; ++k) {
-        if (stage[k]) HIP_OK(hipHostFree(stage[k]));
-        stage[k] = nullptr;
-      }
-      stage_floats = 0;
-      for (int k = 0; k < 2; ++k) HIP_OK(hipHostMalloc((void **)&stage[k], floats * sizeof(float), hipHostMallocDefault));
-      stage_floats = floats;
-    };
-    if (data.is_prebinned) {
-      cached_uid = 0;
-      if (!data.prebinned.empty()) {
-        // row-major bytes on the host: blocks of whole rows through the staging buffers
-        const size_t block_rows =
-            std::min(std::max<size_t>(kStageBytes / F / kPredictThreads, 1) * kPredictThreads, (n + 63) / 64 * 64);
-        const size_t floats = (block_rows * F + 3) / 4;
-        reserve_stage(floats);
-        block.Reserve(floats);
-        const size_t nblocks = (n + block_rows - 1) / block_rows;
-        for (size_t b = 0; b < nblocks; ++b) {
-          const int buf = (int)(b & 1);
-          const size_t r0 = b * block_rows, rows = std::min(block_rows, n - r0);
-          if (b >= 2) HIP_OK(hipEventSynchronize(copied[buf]));
-          uint8_t *dst = reinterpret_cast<uint8_t *>(stage[buf]);
-          const uint8_t *src = data.prebinned.data() + r0 * F;
-          ParallelFor(rows * F, [&](size_t lo, size_t hi) { std::memcpy(dst + lo, src + lo, hi - lo); });
-          HIP_OK(hipMemcpyAsync(block.p, dst, rows * F, hipMemcpyHostToDevice, stream));
-          HIP_OK(hipEventRecord(copied[buf], stream));
-          walk(kByteRows, block.p, F, r0, rows);
-        }
-      } else if (!data.stream_blocks.empty()) {
-        // streamed matrix: its pinned blocks of quad columns go up as they are
-        const size_t br = data.stream_block_rows, Q = (F + 3) / 4;
-        block.Reserve(Q * br);
-        for (size_t b = 0; b < data.stream_blocks.size(); ++b) {
-          const size_t r0 = b * br;
-          if (r0 >= n) break;
-          const size_t rows = std::min(br, n - r0);
-          HIP_OK(hipMemcpyAsync(block.p, data.stream_blocks[b], Q * br * sizeof(uint32_t), hipMemcpyHostToDevice,
-                                stream));
-          walk(kQuadCols, block.p, br, r0, rows);
-        }
-      } else {
-        throw std::runtime_error("pre-quantised matrix without bins");
-      }
-    } else {
-      const size_t ld_all = (n + 63) / 64 * 64;
-      const bool cacheable = F * ld_all * sizeof(float) <= kCacheBytes;
-      if (cacheable && cached_uid == data.uid && cache_ld == ld_all) {
-        walk(kFloatCols, cache.p, cache_ld, 0, n);  // the columns are on the device already
-      } else {
-        // ---- row blocks: [F][block_rows] floats, about kStageBytes each
-        size_t block_rows = std::max<size_t>(kStageBytes / (F * sizeof(float)) / kPredictThreads, 1) * kPredictThreads;
-        block_rows = std::min(block_rows, ld_all);
-        const size_t floats = F * block_rows;
-        reserve_stage(floats);
-        block.Reserve(floats);
-        cached_uid = 0;
-        if (cacheable) cache.Reserve(F * ld_all);
-        const size_t nblocks = (n + block_rows - 1) / block_rows;
-        for (size_t b = 0; b < nblocks; ++b) {
-          const int buf = (int)(b & 1);
-          const size_t r0 = b * block_rows, rows = std::min(block_rows, n - r0);
-          if (b >= 2) HIP_OK(hipEventSynchronize(copied[buf]));  // the copy out of this staging buffer is done
-          float *dst = stage[buf];
-          ParallelFor(rows, [&](size_t lo, size_t hi) {
-            for (size_t f = 0; f < F; ++f)
-              std::memcpy(dst + f * block_rows + lo, data.data[f].data() + r0 + lo, (hi - lo) * sizeof(float));
-          });
-          HIP_OK(hipMemcpyAsync(block.p, dst, floats * sizeof(float), hipMemcpyHostToDevice, stream));
-          HIP_OK(hipEventRecord(copied[buf], stream));
-          walk(kFloatCols, block.p, block_rows, r0, rows);
-          if (cacheable)  // rows [r0, r0 + rows) of every column into their place in the whole matrix
-            HIP_OK(hipMemcpy2DAsync(cache.p + r0, ld_all * sizeof(float), block.p, block_rows * sizeof(float),
-                                    rows * sizeof(float), F, hipMemcpyDeviceToDevice, stream));
-        }
-        if (cacheable) {
-          cached_uid = data.uid;
-          cache_ld = ld_all;
-        }
-      }
-    }
+  }
+
+  const float *Run(const DataMatrix &data, const std::vector<RegTree> &trees, size_t first, size_t use, size_t labels,
+                   float init) {
+    const size_t n = data.rows, F = data.columns_dense;
+    if (n == 0 || F == 0) throw std::runtime_error("empty data matrix");
+    // only the block-wise walk of a streamed matrix indexes rows with 64 bits
+    const bool blocks = data.is_prebinned && data.prebinned.empty() && !data.stream_blocks.empty();
+    if (n >= (1ull << 31) && !blocks) throw std::runtime_error("too many rows");
+    if (data.is_prebinned && data.prebinned.empty() && !blocks) throw std::runtime_error("pre-quantised matrix without bins");
+    if (!stream) stream = StreamPoolTake();
+    LayOut(trees, first, use, F, labels);
+    // Kernels write the sums where the host reads them: stores of 256 bytes a wave, at the rate of a copy
+    // and beside the walk.
     if (labels * n > result_floats) {
-      if (result) HIP_OK(hipHostFree(result));
+      PinnedPoolGive(result);
       result = nullptr;
       result_floats = 0;
-      HIP_OK(hipHostMalloc((void **)&result, labels * n * sizeof(float), hipHostMallocDefault));
+      result = static_cast<float *>(PinnedPoolTake(labels * n * sizeof(float)));
       result_floats = labels * n;
     }
-    HIP_OK(hipMemcpyAsync(result, out.p, labels * n * sizeof(float), hipMemcpyDeviceToHost, stream));
+    // rows on the host: piece by piece through pinned memory into one device block (the stream keeps
+    // a piece's copy behind the walk of the one before)
+    auto through_block = [&](int src, const void *rows, size_t row_bytes) {
+      const size_t piece = kStageBytes / row_bytes;
+      if (piece == 0) throw std::runtime_error("too many features for device prediction");
+      struct Block {
+        void *p;
+        ~Block() { DevicePoolGive(p); }  // (the staging has waited for the stream's copies, Run waits for its walks)
+      };
+      const size_t pieces = (n + piece - 1) / piece, group = std::max<size_t>(kBlockBytes / kStageBytes, 1);
+      Block block{DevicePoolTake(group * piece * row_bytes)};
+      auto rows_of = [&](size_t k) { return std::min(piece, n - k * piece); };
+      StageToDevice(pieces, [&](size_t k) { return rows_of(k) * row_bytes; },
+                    [&](size_t k, void *p) {
+                      const char *from = static_cast<const char *>(rows) + k * piece * row_bytes;
+                      ParallelFor(rows_of(k) * row_bytes, [&](size_t b, size_t e) {
+                        std::memcpy(static_cast<char *>(p) + b, from + b, e - b);
+                      }, (size_t)256 << 10);
+                    },
+                    [&](size_t k) { return static_cast<char *>(block.p) + k % group * piece * row_bytes; },
+                    [&](size_t k) {
+                      if (k % group != group - 1 && k != pieces - 1) return;
+                      const size_t r0 = k / group * group * piece;
+                      Rows(src, block.p, 0, std::min(group * piece, n - r0), F, labels, init, result + r0, n);
+                    }, stream);
+      HIP_OK(hipStreamSynchronize(stream));
+    };
+    if (!data.is_prebinned) {
+      if (const float *rows = data.values->OnDevice()) Rows(kFloatRows, rows, 0, n, F, labels, init, result, n);
+      else through_block(kFloatRows, data.values->OnHost(), F * sizeof(float));
+    } else if (!blocks) {
+      through_block(kByteRows, data.prebinned.data(), F);
+    } else {
+      // streamed matrix: its pinned blocks of quad columns go up as they are
+      const size_t br = data.stream_block_rows, Q = (F + 3) / 4;
+      void *block = DevicePoolTake(Q * br * sizeof(uint32_t));
+      try {
+        for (size_t b = 0; b < data.stream_blocks.size() && b * br < n; ++b) {
+          const size_t r0 = b * br;
+          HIP_OK(hipMemcpyAsync(block, data.stream_blocks[b], Q * br * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+          Rows(kQuadCols, block, br, std::min(br, n - r0), F, labels, init, result + r0, n);
+        }
+        HIP_OK(hipStreamSynchronize(stream));
+      } catch (...) {
+        (void)hipStreamSynchronize(stream);
+        DevicePoolGive(block);
+        throw;
+      }
+      DevicePoolGive(block);
+    }
     HIP_OK(hipStreamSynchronize(stream));
     return result;
   }
@@ -353,8 +503,8 @@ struct DevicePredictor {
 DevicePredictor *CreateDevicePredictor() { return new DevicePredictor(); }
 void FreeDevicePredictor(DevicePredictor *p) { delete p; }
 const float *PredictOnDevice(DevicePredictor *p, const DataMatrix &data, const std::vector<RegTree> &trees,
-                             size_t use, size_t labels, float init) {
-  return p->Run(data, trees, use, labels, init);
+                             size_t begin, size_t end, size_t labels, float init) {
+  return p->Run(data, trees, begin, end, labels, init);
 }
 
 }  // namespace arb

@@ -1,6 +1,7 @@
 // extern "C" boundary: marshalling only.  Mirrors
 // python-wrapper/arboretum_wrapper.cu:16-205 (same names, argument meaning and
 // error convention) plus the extensions declared in arboretum_ext.h.
+#include <algorithm>
 #include <cstring>
 #include <limits>
 #include <new>
@@ -58,12 +59,19 @@ TreeBuilder *BuilderOf(VoidPointer p) {
   return b;
 }
 
-const char *CopyOut(const std::vector<float> &v, const float **out) {
-  float *p = new (std::nothrow) float[v.size() ? v.size() : 1];
-  if (!p) return Fail("unable to allocate array");
-  if (!v.empty()) std::memcpy(p, v.data(), v.size() * sizeof(float));
-  *out = p;
-  return nullptr;
+// `count` results of fn into the caller's array of `capacity` floats; a caller that expects another
+// number gets the first ones, and zeros behind them.
+template <typename Fn>
+void Into(float *out, size_t capacity, size_t count, Fn &&fn) {
+  if (count == capacity) {
+    fn(out);
+    return;
+  }
+  std::vector<float> all(count);
+  fn(all.data());
+  const size_t n = std::min(count, capacity);
+  std::copy(all.begin(), all.begin() + n, out);
+  std::fill(out + n, out + capacity, 0.0f);
 }
 
 }  // namespace
@@ -74,28 +82,15 @@ const char *ACreateFromDenseMatrix(const float *data, const unsigned int *catego
                                    int ncol, int ccol, float /*missing*/, VoidPointer *out) {
   return Guard([&] {
     if (!data || !out || nrow < 0 || ncol < 0 || ccol < 0) throw std::runtime_error("bad arguments");
-    DataMatrix *mat = new DataMatrix((size_t)nrow, (size_t)ncol, (size_t)ccol);
-    const size_t rows = (size_t)nrow, cols = (size_t)ncol;
-    // the columns are allocated (and their pages first touched) by several threads
-    mat->data.resize(cols);
-    ParallelTasks(cols, [&](size_t f) { mat->data[f].resize(rows); });
-    // row-major -> column-major in tiles of 256 rows, so that a tile's lines of every
-    // column stay in cache while its rows are read once
-    ParallelFor(rows, [&](size_t b, size_t e) {
-      for (size_t r0 = b; r0 < e; r0 += 256) {
-        const size_t r1 = std::min(e, r0 + 256);
-        for (size_t f = 0; f < cols; ++f) {
-          float *dst = mat->data[f].data();
-          for (size_t i = r0; i < r1; ++i) dst[i] = data[i * cols + f];
-        }
-      }
-    });
+    std::unique_ptr<DataMatrix> mat(new DataMatrix((size_t)nrow, (size_t)ncol, (size_t)ccol));
+    const size_t rows = (size_t)nrow;
+    mat->values.reset(new FloatRows(data, rows, (size_t)ncol));
     if (ccol > 0 && categories) {
       mat->data_categories.assign(ccol, std::vector<unsigned>(rows));
       for (size_t i = 0; i < rows; ++i)
         for (int c = 0; c < ccol; ++c) mat->data_categories[c][i] = categories[i * ccol + c];
     }
-    *out = mat;
+    *out = mat.release();
   });
 }
 
@@ -170,12 +165,21 @@ const char *ALoadModel(const char *model, VoidPointer garden) {
 }
 
 const char *AGetY(VoidPointer garden, VoidPointer data, const float **out) {
-  std::vector<float> result;
+  float *result = nullptr;
   const char *err = Guard([&] {
     if (!out) throw std::runtime_error("bad arguments");
-    AsGarden(garden)->garden.GetY(AsData(data), &result);
+    DataMatrix *d = AsData(data);
+    const size_t count = d->YHat().size();
+    result = new (std::nothrow) float[count ? count : 1];
+    if (!result) throw std::runtime_error("unable to allocate array");
+    AsGarden(garden)->garden.GetY(d, result);
   });
-  return err ? err : CopyOut(result, out);
+  if (err) {
+    delete[] result;
+    return err;
+  }
+  *out = result;
+  return nullptr;
 }
 
 const char *AAppendLastTree(VoidPointer garden, VoidPointer data) {
@@ -202,6 +206,25 @@ const char *ADeviceCopyProbe(unsigned long long bytes) {
   return Guard([&] {
     if (DeviceCount() <= 0) throw std::runtime_error("no HIP device available");
     CopyProbe((size_t)bytes);
+  });
+}
+
+const char *APredictInto(VoidPointer garden, VoidPointer data, float *out, unsigned long long capacity, int n_rounds) {
+  return Guard([&] {
+    if (!out) throw std::runtime_error("bad arguments");
+    const Garden &g = AsGarden(garden)->garden;
+    const DataMatrix *d = AsData(data);
+    Into(out, capacity, d->rows * g.cfg.tree.labels_count,
+         [&](float *p) { g.Predict(d, p, n_rounds == -1 ? std::numeric_limits<int>::max() : n_rounds); });
+  });
+}
+
+const char *AGetYInto(VoidPointer garden, VoidPointer data, float *out, unsigned long long capacity) {
+  return Guard([&] {
+    if (!out) throw std::runtime_error("bad arguments");
+    const Garden &g = AsGarden(garden)->garden;
+    DataMatrix *d = AsData(data);
+    Into(out, capacity, d->YHat().size(), [&](float *p) { g.GetY(d, p); });
   });
 }
 

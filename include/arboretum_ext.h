@@ -70,6 +70,12 @@ const char *AGetThresholds(VoidPointer data, int fid, float *thr, int *size);
 const char *AGetBinLayout(VoidPointer data, int *bits, int *slots);
 const char *AGetBins16(VoidPointer data, unsigned short *out);
 
+/* APredict and AGetY into an array of the caller's, `capacity` floats: rows * labels_count of the
+ * booster.  (With another capacity the array gets the first results, and zeros behind the last.) */
+const char *APredictInto(VoidPointer garden, VoidPointer data, float *out, unsigned long long capacity,
+                         int n_rounds);
+const char *AGetYInto(VoidPointer garden, VoidPointer data, float *out, unsigned long long capacity);
+
 /* Where APredict walks the trees (src/core/garden.cu:643-657 does it on the
  * host): on != 0 (default) uses the GPU when a device is present, 0 the host
  * walk.  Both give the same bits. */
