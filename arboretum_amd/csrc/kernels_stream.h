@@ -101,7 +101,7 @@ k_stream_segments(unsigned *__restrict__ blk_cnt, int L, NodeSum *__restrict__ b
 
 // Copies the rows of the built nodes into the staging buffer, node by node.
 // The order inside a node is whatever the atomics give; sums are integers.
-// A workgroup takes a tile of kGatherTile consecutive rows and sorts it by node
+// A workgroup takes a tile of TILE consecutive rows and sorts it by node
 // in LDS first (rank of every row among the tile's rows of its node, one LDS
 // atomic per distinct node of a wave; start of every node inside the tile by a
 // scan; one global cursor atomic per node present in the tile), so that the
@@ -110,12 +110,13 @@ k_stream_segments(unsigned *__restrict__ blk_cnt, int L, NodeSum *__restrict__ b
 // wave writing its own row to wherever its node's cursor stood, a store touched
 // 64 lines for 256 bytes (measured 1.8 ms per block of 4 M rows x 128
 // features, 0.3 TB/s).
-// grid ceil(rows / kGatherTile), 1024 threads; LDS: GatherLdsBytes(L).
-constexpr unsigned kGatherTile = 8192;
-constexpr int kGatherPerThread = kGatherTile / 1024;
-inline size_t GatherLdsBytes(int L) { return (size_t)2 * kGatherTile * 4 + (size_t)3 * L * 4 + 64; }
+// Tiles are smaller in smaller blocks: at 8192 rows a block of 524,288 rows is
+// 64 workgroups on 256 CUs (175 us for 100 MB; at 2048 rows 45).
+// grid ceil(rows / TILE), 1024 threads; LDS: GatherLdsBytes(L, TILE).
+constexpr unsigned kGatherTile = 8192;  // the largest
+inline size_t GatherLdsBytes(int L, unsigned tile) { return (size_t)2 * tile * 4 + (size_t)3 * L * 4 + 128; }
 
-template <bool PAIR>
+template <bool PAIR, unsigned TILE>
 __global__ void __launch_bounds__(1024)
 k_stream_gather(const uint32_t *__restrict__ bins, size_t bstride, int Q, unsigned rows,
                 const float *__restrict__ g, const float *__restrict__ h,
@@ -124,15 +125,16 @@ k_stream_gather(const uint32_t *__restrict__ bins, size_t bstride, int Q, unsign
                 uint32_t *__restrict__ st_bins, size_t sstride, float *__restrict__ st_g,
                 float *__restrict__ st_h) {
   extern __shared__ unsigned s_gather[];
+  constexpr int kGatherPerThread = TILE / 1024;
   const int L = 1 << level;
   unsigned *s_src = s_gather;                 // row of the block at every sorted place of the tile
-  unsigned *s_dst = s_src + kGatherTile;      // its place in the staging buffer
-  unsigned *s_cnt = s_dst + kGatherTile;      // rows of the tile per node
+  unsigned *s_dst = s_src + TILE;      // its place in the staging buffer
+  unsigned *s_cnt = s_dst + TILE;      // rows of the tile per node
   unsigned *s_start = s_cnt + L;              // first sorted place of every node
   unsigned *s_base = s_start + L;             // first staging place claimed for the tile's rows of every node
   unsigned *s_misc = s_base + L;              // [0..15] wave sums, [16] carry
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const unsigned tile0 = blockIdx.x * kGatherTile;
+  const unsigned tile0 = blockIdx.x * TILE;
   for (int i = tid; i < L; i += 1024) s_cnt[i] = 0;
   if (tid == 0) s_misc[16] = 0;
   __syncthreads();

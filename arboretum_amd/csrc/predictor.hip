@@ -69,7 +69,7 @@ struct Walk {
 // The LDS by byte address: a 32-bit register is the whole address of a read.
 template <typename T>
 __device__ __forceinline__ T LdsAt(unsigned at) {
-  return *(const __attribute__((address_space(3))) T *)at;
+  return *(const __attribute__((address_space(3))) T *)(uintptr_t)at;
 }
 __device__ __forceinline__ unsigned LdsAddress(const unsigned char *p) {
   return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char *)p;
