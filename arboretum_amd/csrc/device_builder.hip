@@ -50,13 +50,13 @@
 #include <cstring>
 #include <functional>
 #include <limits>
-#include <random>
 #include <stdexcept>
 #include <string>
 #include <thread>
 #include <vector>
 
 #include "booster.h"
+#include "column_sampler.h"
 #include "device_common.h"
 #include "gain.h"
 #include "fused_pass.h"
@@ -849,8 +849,7 @@ class HipTreeBuilder : public TreeBuilder {
     d_tbin_ = DevAlloc<int>(internal);
     d_tgain_ = DevAlloc<float>(internal);
     d_weights_ = DevAlloc<float>(max_nodes);
-    d_active_ = DevAlloc<unsigned char>((size_t)(D_ - 1) * F_);
-    rnd_.seed(cfg.internal.seed);  // garden.cu:87
+    sampler_.Init(cfg, data->columns_dense + data->columns_category, F_, D_ - 1);
     int shifts[2] = {30, 0};
     if (cfg.objective == kLogisticRegression) {
       shifts[1] = 32;  // 0 <= h <= 1/4
@@ -865,9 +864,10 @@ class HipTreeBuilder : public TreeBuilder {
 
   void Release() noexcept {
     if (stream_) (void)hipStreamSynchronize(stream_);
+    sampler_.Release();
     void *ptrs[] = {d_yhat_, d_g_, d_h_, d_leaf_, d_split_, d_cand_, d_node_first2_,
                     d_node_items2_, d_hwork_, d_pwork_, d_nwork_, d_wave_left_, d_item_left_, d_slab_,
-                    d_shifts_, d_gmax_, d_rows_scanned_, d_tfid_, d_tbin_, d_tgain_, d_weights_, d_active_, d_overflow_, d_records_, d_cursor2_};
+                    d_shifts_, d_gmax_, d_rows_scanned_, d_tfid_, d_tbin_, d_tgain_, d_weights_, d_overflow_, d_records_, d_cursor2_};
     for (void *p : ptrs)
       DevicePoolGive(p);
     for (int b = 0; b < 2; ++b) {
@@ -1278,7 +1278,7 @@ class HipTreeBuilder : public TreeBuilder {
     orig.g = d_g_ + (size_t)label * n_;
     orig.h = d_h_ ? d_h_ + (size_t)label * n_ : nullptr;
     if (inspect_) kept_hist_.assign(D_ - 1, {});
-    SampleColumns();
+    sampler_.NextTree(stream_);
     if (streamed_) {
       GrowOneStreamed(label, orig, gp);
       return;
@@ -1333,7 +1333,7 @@ class HipTreeBuilder : public TreeBuilder {
               scan.t_bin = d_tbin_;
               scan.t_gain = d_tgain_;
               scan.heap_off = PL - 1;
-              scan.active = sampling_ ? d_active_ + (size_t)(level - 1) * F_ : (const unsigned char *)nullptr;
+              scan.active = sampler_.Active(level - 1);
               scan.node_first = d_node_first_;
               scan.rows_scanned = ScanCounter(level);
             }
@@ -1406,7 +1406,7 @@ class HipTreeBuilder : public TreeBuilder {
   // and, with rows_per_item, the state and plan of the next tree's root.
   void LaunchTreeEnd(int last_state, const GainParams &gp, unsigned rows_per_item) {
     const int L = 1 << (D_ - 2);
-    const unsigned char *active = sampling_ ? d_active_ + (size_t)(D_ - 2) * F_ : (const unsigned char *)nullptr;
+    const unsigned char *active = sampler_.Active(D_ - 2);
 #define ARB_END(P, D)                                                                                              \
   hipLaunchKernelGGL((k_tree_end<P, D>), dim3((L + 3) / 4 + 1), dim3(256), 0, stream_, d_cand_, F_, active,        \
                      d_tot_[last_state], L, d_shifts_, gp, cfg_.tree.eta, d_weights_, d_tfid_, d_tbin_, d_tgain_,  \
@@ -1519,7 +1519,7 @@ class HipTreeBuilder : public TreeBuilder {
   // plan of the children's histograms: in the same launch while one workgroup selects for all nodes
   // as fast as several would (up to 64 nodes).
   void LaunchSelect(int level, int L, int state) {
-    const unsigned char *active = sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr;
+    const unsigned char *active = sampler_.Active(level);
     const bool plan_hist = !fused_ && !streamed_;
     if (plan_hist && L <= 64) {
       hipLaunchKernelGGL(k_select_plan, dim3(1), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
@@ -1747,30 +1747,6 @@ class HipTreeBuilder : public TreeBuilder {
     Mark(kNone);
   }
 
-  // Column sampling of one tree (InitGrowingTree / InitTreeLevel,
-  // garden.cu:126-165, and the `take` prefix of FindBestSplits, :249-253): the
-  // ids are shuffled per tree, the first floor(bytree * columns) of them again
-  // per level, and the first floor(bylevel * bytree * columns) are active.
-  void SampleColumns() {
-    const size_t columns = data_->columns_dense + data_->columns_category;
-    const int take_tree = (int)(cfg_.tree.colsample_bytree * columns);
-    const unsigned take_level = (unsigned)(cfg_.tree.colsample_bylevel * cfg_.tree.colsample_bytree * columns);
-    sampling_ = take_level < columns;
-    if (!sampling_) return;
-    std::vector<unsigned> ids(columns);
-    for (size_t i = 0; i < columns; ++i) ids[i] = (unsigned)i;
-    std::shuffle(ids.begin(), ids.end(), rnd_);
-    active_host_.assign((size_t)(D_ - 1) * F_, 0);
-    for (int level = 0; level + 1 < D_; ++level) {
-      std::shuffle(ids.begin(), ids.begin() + take_tree, rnd_);
-      for (unsigned j = 0; j < take_level; ++j)
-        if (ids[j] < (unsigned)F_) active_host_[(size_t)level * F_ + ids[j]] = 1;
-    }
-    // the previous tree's kernels may still read the mask
-    HIP_OK(hipStreamSynchronize(stream_));
-    HIP_OK(hipMemcpy(d_active_, active_host_.data(), active_host_.size(), hipMemcpyHostToDevice));
-  }
-
   void KeepHist(int level, int L, int hb, int state) {
     const size_t cells = (size_t)L * nbin_total_;
     std::vector<long long> g(cells), h(cells);
@@ -1862,10 +1838,7 @@ class HipTreeBuilder : public TreeBuilder {
   std::shared_ptr<const float> y_held_;  // the matrix' target (d_y_, d_labels_)
   std::shared_ptr<const unsigned char> labels_held_;
   unsigned *d_overflow_ = nullptr;     // set by the planner when a launch bound was too small
-  unsigned char *d_active_ = nullptr;  // [level][feature] 1 = sampled at that level
-  std::vector<unsigned char> active_host_;
-  std::default_random_engine rnd_;
-  bool sampling_ = false;
+  ColumnSampler sampler_;
   unsigned *d_node_first2_ = nullptr, *d_node_items2_ = nullptr;  // both sets; d_node_first_ / d_node_items_: the one in use
   bool own_scan_ = false;  // the fused passes find the splits of their parents themselves (LevelScan)
   unsigned *d_leaf_ = nullptr, *d_node_first_ = nullptr, *d_node_items_ = nullptr, *d_nwork_ = nullptr,

@@ -17,12 +17,12 @@
 #include <cstring>
 #include <limits>
 #include <memory>
-#include <random>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "booster.h"
+#include "column_sampler.h"
 #include "device_common.h"
 #include "gain.h"
 #include "kernels_exact.h"
@@ -214,8 +214,7 @@ class ExactSortBuilder : public TreeBuilder {
     d_tbin_ = DevAlloc<int>(internal);
     d_tgain_ = DevAlloc<float>(internal);
     d_weights_ = DevAlloc<float>(max_nodes);
-    d_active_ = DevAlloc<unsigned char>((size_t)(D_ - 1) * F_);
-    rnd_.seed(cfg.internal.seed);  // garden.cu:87
+    sampler_.Init(cfg, data->columns_dense + data->columns_category, F_, D_ - 1);
     int shifts[2] = {30, 0};
     if (cfg.objective == kLogisticRegression) {
       shifts[1] = 32;  // 0 <= h <= 1/4
@@ -229,11 +228,12 @@ class ExactSortBuilder : public TreeBuilder {
 
   void Release() noexcept {
     if (stream_) (void)hipStreamSynchronize(stream_);
+    sampler_.Release();
     void *all[] = {d_yhat_, d_g_, d_h_, d_leaf_, d_node_of_, d_went_right_, d_gh_, d_ids_[0], d_ids_[1], d_ranks_[0],
                    d_ranks_[1], d_lg_[0], d_lg_[1], d_lh_[0], d_lh_[1], d_tot_[0],
                    d_tot_[1], d_seg_[0], d_seg_[1], d_split_, d_cand_, d_work_, d_n_work_, d_node_first_,
                    d_node_items_, d_part_, d_off_, d_best_, d_lefts_, d_left_off_, d_left_bits_, d_shifts_, d_records_, d_gmax_,
-                   d_overflow_, d_tfid_, d_tbin_, d_tgain_, d_weights_, d_active_};
+                   d_overflow_, d_tfid_, d_tbin_, d_tgain_, d_weights_};
     for (void *p : all)
       DevicePoolGive(p);
     StreamPoolGive(stream_);
@@ -338,31 +338,11 @@ class ExactSortBuilder : public TreeBuilder {
   static constexpr size_t kRecordRing = 64;  // trees whose records may wait on the device
   size_t RecordWords() const { return (size_t)3 * ((1 << (D_ - 1)) - 1) + (size_t)(1 << (D_ - 1)) + 1; }
 
-  // The features a tree may split on at every level (garden.cu:142-146, 162-165, 252-253).
-  void SampleColumns() {
-    const size_t columns = data_->columns_dense + data_->columns_category;
-    const int take_tree = (int)(cfg_.tree.colsample_bytree * columns);
-    const unsigned take_level = (unsigned)(cfg_.tree.colsample_bylevel * cfg_.tree.colsample_bytree * columns);
-    sampling_ = take_level < columns;
-    if (!sampling_) return;
-    std::vector<unsigned> ids(columns);
-    for (size_t i = 0; i < columns; ++i) ids[i] = (unsigned)i;
-    std::shuffle(ids.begin(), ids.end(), rnd_);
-    std::vector<unsigned char> active((size_t)(D_ - 1) * F_, 0);
-    for (int level = 0; level + 1 < D_; ++level) {
-      std::shuffle(ids.begin(), ids.begin() + take_tree, rnd_);
-      for (unsigned j = 0; j < take_level; ++j)
-        if (ids[j] < (unsigned)F_) active[(size_t)level * F_ + ids[j]] = 1;
-    }
-    HIP_OK(hipStreamSynchronize(stream_));  // the previous tree's kernels may still read the mask
-    HIP_OK(hipMemcpy(d_active_, active.data(), active.size(), hipMemcpyHostToDevice));
-  }
-
   void GrowOne(int label) {
     const GainParams gp = cfg_.gain_params();
     const float *g = d_g_ + (size_t)label * n_;
     const float *h = d_h_ ? d_h_ + (size_t)label * n_ : nullptr;
-    SampleColumns();
+    sampler_.NextTree(stream_);
     hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0], (unsigned long long)n_);
     hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, g, h, pack_ ? 1 : 0, n_, d_shifts_,
                        d_tot_[0]);
@@ -407,7 +387,7 @@ class ExactSortBuilder : public TreeBuilder {
                          F_, d_cand_);
       hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
                          d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,
-                         L - 1, sampling_ ? d_active_ + (size_t)level * F_ : (const unsigned char *)nullptr,
+                         L - 1, sampler_.Active(level),
                          (unsigned long long *)nullptr);
       hipLaunchKernelGGL(k_ex_decide, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, sd_->ranks, stride_, d_split_,
                          d_node_of_, d_went_right_, n_);
@@ -453,12 +433,11 @@ class ExactSortBuilder : public TreeBuilder {
   const ExactSortData *sd_ = nullptr;
   size_t n_ = 0, stride_ = 0;
   int F_ = 0, K_ = 1, D_ = 2;
-  bool pair_ = false, f64_ = false, inspect_ = false, sampling_ = false;
+  bool pair_ = false, f64_ = false, inspect_ = false;
   bool pack_ = false;  // logistic gradients packed into one float per row
   bool harr_ = false;  // the gradients are two arrays (g, h)
   unsigned max_items_ = 0;
   hipStream_t stream_ = nullptr;
-  std::default_random_engine rnd_;
   std::vector<RegTree> *owner_ = nullptr;
   std::vector<size_t> pending_;
 
@@ -482,7 +461,7 @@ class ExactSortBuilder : public TreeBuilder {
   WorkItem *d_work_ = nullptr;
   ExSum *d_part_ = nullptr, *d_off_ = nullptr;
   int *d_shifts_ = nullptr, *d_tfid_ = nullptr, *d_tbin_ = nullptr;
-  unsigned char *d_active_ = nullptr;
+  ColumnSampler sampler_;
 };
 
 }  // namespace
