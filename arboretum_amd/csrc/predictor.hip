@@ -303,12 +303,15 @@ struct DevicePredictor {
   // of which trees, for how many features and labels `model` is (the trees of a booster are only added to)
   size_t begin = 0, end = 0, features = 0, labels_of = 0;
   unsigned largest = 0, tree_words = 0, depth = 0;
+  unsigned char *staged = nullptr;  // pinned
+  size_t staged_bytes = 0;
   float *result = nullptr;  // pinned; the sums of the last call
   size_t result_floats = 0;
 
   ~DevicePredictor() {
     if (stream) (void)hipStreamSynchronize(stream);
     DevicePoolGive(model);
+    PinnedPoolGive(staged);
     PinnedPoolGive(result);
     StreamPoolGive(stream);
   }
@@ -346,9 +349,20 @@ struct DevicePredictor {
       model = static_cast<unsigned *>(DevicePoolTake(bytes));
       model_bytes = bytes;
     }
-    std::vector<unsigned char> host(bytes);
-    std::memcpy(host.data(), refs.data(), words_at);
-    unsigned char *at = host.data() + words_at;
+    // A small model (a round's trees) is copied from pinned memory behind nothing and waited for by
+    // nobody: Run waits for the stream before it returns.
+    const bool small = bytes <= ((size_t)256 << 10);
+    if (small && bytes > staged_bytes) {
+      PinnedPoolGive(staged);
+      staged = nullptr;
+      staged_bytes = 0;
+      staged = static_cast<unsigned char *>(PinnedPoolTake(bytes));
+      staged_bytes = bytes;
+    }
+    std::vector<unsigned char> large(small ? 0 : bytes);
+    unsigned char *host = small ? staged : large.data();
+    std::memcpy(host, refs.data(), words_at);
+    unsigned char *at = host + words_at;
     for (unsigned t : order) {
       const RegTree &tr = trees[t];
       for (size_t k = 0; k < tr.fid.size(); ++k) {
@@ -366,7 +380,8 @@ struct DevicePredictor {
       std::memcpy(at, tr.weights.data(), tr.weights.size() * sizeof(float));
       at += tr.weights.size() * sizeof(float);
     }
-    CopyToDevice(model, host.data(), bytes, stream);
+    if (small) HIP_OK(hipMemcpyAsync(model, host, bytes, hipMemcpyHostToDevice, stream));
+    else CopyToDevice(model, host, bytes, stream);
     begin = b;
     end = e;
     features = F;

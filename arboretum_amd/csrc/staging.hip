@@ -53,10 +53,25 @@ struct Slots {
   hipEvent_t copied[kStageSlots] = {};
 };
 
+// Up to this many bytes go through one pinned block, with no events and no threads.
+constexpr size_t kSmallCopy = (size_t)128 << 10;
+struct PinnedBlock {
+  explicit PinnedBlock(size_t bytes) : p(PinnedPoolTake(bytes)) {}
+  ~PinnedBlock() { PinnedPoolGive(p); }
+  void *const p;
+};
+
 }  // namespace
 
 void CopyToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return;
+  if (bytes <= kSmallCopy) {
+    PinnedBlock block(bytes);
+    HIP_OK(hipMemcpyAsync(block.p, src, bytes, hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipStreamSynchronize(stream));
+    std::memcpy(dst, block.p, bytes);
+    return;
+  }
   const size_t pieces = (bytes + kStageBytes - 1) / kStageBytes;
   Slots s((int)std::min<size_t>(pieces, kStageSlots), std::min(bytes, kStageBytes), stream);
   auto start = [&](size_t k) {
@@ -92,6 +107,14 @@ void StageToDevice(size_t pieces, const std::function<size_t(size_t)> &bytes_of,
 }
 
 void CopyToDevice(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+  if (bytes == 0) return;
+  if (bytes <= kSmallCopy) {
+    PinnedBlock block(bytes);
+    std::memcpy(block.p, src, bytes);
+    HIP_OK(hipMemcpyAsync(dst, block.p, bytes, hipMemcpyHostToDevice, stream));
+    HIP_OK(hipStreamSynchronize(stream));
+    return;
+  }
   auto bytes_of = [&](size_t k) { return std::min(kStageBytes, bytes - k * kStageBytes); };
   StageToDevice((bytes + kStageBytes - 1) / kStageBytes, bytes_of,
                 [&](size_t k, void *p) { ParallelCopy(p, (const char *)src + k * kStageBytes, bytes_of(k)); },
