@@ -1349,22 +1349,24 @@ class HipTreeBuilder : public TreeBuilder {
           }
           Reduce(L, hb, true, ps, true, false, last ? -1 : state);
         } else {
-          const unsigned grid = PartGrid(PL);  // (planned by the reduction of the level above)
+          const unsigned items = PartGrid(PL);  // (planned by the reduction of the level above)
+          const SelectPlan plan = SelectInPartition(PL) ? PlanOfPartition(level - 1, PL, ps) : SelectPlan{};
+          const unsigned grid = items + (plan.cand ? 1u : 0u);
           Mark(kPartition);
           if (indexed_) {
             // decisions, claims of the children's ranges and the move of (row id, g, h) in one launch
             if (pair_)
               hipLaunchKernelGGL(k_ix_part<true>, dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8,
                                  src.ids, dst.ids, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_,
-                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb);
+                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb, plan);
             else
               hipLaunchKernelGGL(k_ix_part<false>, dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8,
                                  src.ids, dst.ids, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_,
-                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb);
+                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb, plan);
           } else {
             hipLaunchKernelGGL(k_part_count, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, stride_, d_split_,
-                               d_pwork_, d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_);
-            LaunchPartRows(grid, src, dst, ps);
+                               d_pwork_, d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_, plan);
+            LaunchPartRows(items, src, dst, ps);
           }
           HistOfNodes(dst, L, false);  // (planned with the splits of the level above)
           Reduce(L, hb, false, ps, trick_, false, last ? -1 : state);
@@ -1375,7 +1377,7 @@ class HipTreeBuilder : public TreeBuilder {
       // level are selected at the end of the tree
       LaunchScan(level, L, hb, state, gp, level == 0 && !root_totals_ready_ && !hi_skip_);
       root_totals_ready_ = false;
-      if (!last && !own_scan_) LaunchSelect(level, L, state);
+      if (!last && !own_scan_ && !SelectInPartition(L)) LaunchSelect(level, L, state);
       state ^= 1;
     }
     // ---- leaf of every row, y_hat update, gradients of the next round
@@ -1515,19 +1517,40 @@ class HipTreeBuilder : public TreeBuilder {
 #undef ARB_SCAN
   }
 
-  // Splits of a level's nodes from the candidates; on the paths with stand-alone histogram launches also the
-  // plan of the children's histograms: in the same launch while one workgroup selects for all nodes
-  // as fast as several would (up to 64 nodes).
+  // Levels whose splits are selected, and whose children's histograms are planned, by the partition.
+  bool SelectInPartition(int L) const { return !fused_ && !streamed_ && L <= kSelectPlanNodes; }
+  SelectPlan PlanOfPartition(int level, int L, int state) {
+    SelectPlan p;
+    p.cand = d_cand_;
+    p.F = F_;
+    p.L = L;
+    p.tot = d_tot_[state];
+    p.seg_start = d_seg_[state];
+    p.tot_next = d_tot_[state ^ 1];
+    p.seg_next = d_seg_[state ^ 1];
+    p.split = d_split_;
+    p.t_fid = d_tfid_;
+    p.t_bin = d_tbin_;
+    p.t_gain = d_tgain_;
+    p.active = sampler_.Active(level);
+    p.select = trick_ ? 1 : 0;
+    p.rows_per_item = kMaxHistRows;
+    p.work = d_hwork_;
+    p.n_work = d_nwork_;
+    p.node_first = d_node_first_;
+    p.node_items = d_node_items_;
+    p.rows_scanned = ScanCounter(level + 1);
+    p.max_items = HistGrid(2 * L, false);
+    p.overflow = d_overflow_;
+    p.balance_cus = HistCus(false);
+    return p;
+  }
+
+  // Splits of a level's nodes from the candidates, and on the paths with stand-alone histogram launches
+  // the plan of the children's histograms, as launches of their own (SelectInPartition: not needed).
   void LaunchSelect(int level, int L, int state) {
     const unsigned char *active = sampler_.Active(level);
     const bool plan_hist = !fused_ && !streamed_;
-    if (plan_hist && L <= 64) {
-      hipLaunchKernelGGL(k_select_plan, dim3(1), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
-                         d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,
-                         L - 1, active, trick_ ? 1 : 0, kMaxHistRows, d_hwork_, d_nwork_, d_node_first_, d_node_items_,
-                         ScanCounter(level + 1), HistGrid(2 * L, false), d_overflow_, HistCus(false));
-      return;
-    }
     hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L,
                        d_tot_[state], d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_,
                        d_tfid_, d_tbin_, d_tgain_, L - 1, active,

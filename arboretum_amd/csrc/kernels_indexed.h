@@ -142,12 +142,17 @@ k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__r
           const float *__restrict__ h, float *__restrict__ h_out, const SplitRec *__restrict__ split,
           const unsigned *__restrict__ seg_start, const WorkItem *__restrict__ work,
           const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor, unsigned *__restrict__ item_base,
-          const uint8_t *__restrict__ hibits, size_t strideb) {
+          const uint8_t *__restrict__ hibits, size_t strideb, const SelectPlan plan) {
   __shared__ unsigned s_tmp[kItemWaves + 2];
-  const unsigned w = blockIdx.x;
+  __shared__ SplitRec s_rec;
+  unsigned w = blockIdx.x;
+  if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
+    SelectAndPlan(plan);
+    return;
+  }
   if (w >= *n_work) return;
   const WorkItem it = work[w];
-  const SplitRec s = split[it.node];
+  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
   const bool by_bit = hibits != nullptr && s.bin >= 255;  // uniform: only an id of 256 goes right

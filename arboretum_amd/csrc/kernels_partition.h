@@ -33,11 +33,17 @@ __device__ __forceinline__ unsigned ChunkOrigin(const WorkItem &it) { return it.
 __global__ void __launch_bounds__(kHistThreads)
 k_part_count(const uint32_t *__restrict__ bins, size_t stride, const SplitRec *__restrict__ split,
              const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
-             unsigned *__restrict__ wave_left, unsigned *__restrict__ item_left, BinCode code, int hi_word) {
-  const unsigned w = blockIdx.x;
+             unsigned *__restrict__ wave_left, unsigned *__restrict__ item_left, BinCode code, int hi_word,
+             const SelectPlan plan) {
+  __shared__ SplitRec s_rec;
+  unsigned w = blockIdx.x;
+  if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
+    SelectAndPlan(plan);
+    return;
+  }
   if (w >= *n_work) return;
   const WorkItem it = work[w];
-  const SplitRec s = split[it.node];
+  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
   const SplitTest test = MakeSplitTest(s, code, hi_word);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned cnt = 0;

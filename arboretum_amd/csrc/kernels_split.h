@@ -357,25 +357,50 @@ k_split_select(const Cand *__restrict__ cand, int F, int L, const NodeSum *__res
   }
 }
 
-// k_split_select followed, in the same workgroup, by the work plan of the histograms of the
-// children (select: PlanBody's; the items are balanced over balance_cus compute units).  For levels
-// of few nodes: one workgroup selects for all of them.
-__global__ void __launch_bounds__(1024)
-k_select_plan(const Cand *__restrict__ cand, int F, int L, const NodeSum *__restrict__ tot,
-              const unsigned *__restrict__ seg_start, NodeSum *tot_next, unsigned *seg_next,
-              SplitRec *__restrict__ split, int *__restrict__ t_fid,
-              int *__restrict__ t_bin, float *__restrict__ t_gain, int heap_off,
-              const unsigned char *__restrict__ active, int select, unsigned rows_per_item,
-              WorkItem *__restrict__ work, unsigned *__restrict__ n_work,
-              unsigned *__restrict__ node_first, unsigned *__restrict__ node_items,
-              unsigned long long *__restrict__ rows_scanned, unsigned max_items,
-              unsigned *__restrict__ overflow, unsigned balance_cus) {
-  for (int nd = threadIdx.x >> 6; nd < L; nd += 16)
-    SelectNode(nd, threadIdx.x & 63, cand, F, tot, seg_start, tot_next, seg_next, split, t_fid, t_bin, t_gain,
-               heap_off, active);
+// Splits of a level's nodes and the work plan of the children's histograms, made by the partition that
+// follows the split scan on the paths with stand-alone histogram launches: every workgroup selects for
+// its own node (SplitOf), and one more block of the grid (the first one) selects for all of them, writes
+// their records and plans (SelectAndPlan; `select`, balance_cus: PlanBody's).  A launch of its own
+// stood between scan and partition for 6.5 us a level, and the partition takes 3 us longer for it.  One workgroup
+// does it beside the partition while the level has few nodes: cand == null, the splits have been selected by k_split_select.
+struct SelectPlan {
+  const Cand *cand = nullptr;
+  int F = 0, L = 0;
+  const NodeSum *tot = nullptr;
+  const unsigned *seg_start = nullptr;
+  NodeSum *tot_next = nullptr;
+  unsigned *seg_next = nullptr;
+  SplitRec *split = nullptr;
+  int *t_fid = nullptr, *t_bin = nullptr;
+  float *t_gain = nullptr;
+  const unsigned char *active = nullptr;
+  int select = 0;
+  unsigned rows_per_item = 0;
+  WorkItem *work = nullptr;
+  unsigned *n_work = nullptr, *node_first = nullptr, *node_items = nullptr;
+  unsigned long long *rows_scanned = nullptr;
+  unsigned max_items = 0;
+  unsigned *overflow = nullptr;
+  unsigned balance_cus = 0;
+};
+constexpr int kSelectPlanNodes = 64;  // most nodes of a level whose partition selects and plans
+
+__device__ __forceinline__ void SelectAndPlan(const SelectPlan &a) {
+  for (int nd = threadIdx.x >> 6; nd < a.L; nd += blockDim.x / 64)
+    SelectNode(nd, threadIdx.x & 63, a.cand, a.F, a.tot, a.seg_start, a.tot_next, a.seg_next, a.split, a.t_fid, a.t_bin,
+               a.t_gain, a.L - 1, a.active);
   __syncthreads();  // the children's totals and ranges written above are read by the plan
-  PlanBody(tot_next, seg_next, 2 * L, select, rows_per_item, work, n_work, node_first, node_items, rows_scanned, nullptr,
-           max_items, overflow, nullptr, balance_cus);
+  PlanBody(a.tot_next, a.seg_next, 2 * a.L, a.select, a.rows_per_item, a.work, a.n_work, a.node_first, a.node_items,
+           a.rows_scanned, nullptr, a.max_items, a.overflow, nullptr, a.balance_cus);
+}
+// Called by all threads of the workgroup; s_rec holds one record.
+__device__ __forceinline__ SplitRec SplitOf(const SelectPlan &a, int nd, const SplitRec *__restrict__ split, SplitRec *s_rec) {
+  if (a.cand == nullptr) return split[nd];  // uniform
+  LevelScan scan{};
+  scan.cand = a.cand;
+  scan.F = a.F;
+  scan.active = a.active;
+  return SelectInPass(scan, nd, a.tot[nd], a.seg_start, false, s_rec);
 }
 
 }  // namespace
