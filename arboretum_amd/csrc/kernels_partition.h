@@ -717,7 +717,7 @@ struct NextPlan {
 // 64-bit counts: a streamed matrix may hold 2^32 rows and more, all of which can
 // sit in one cell (a constant feature, the bin of the missing values).
 template <bool PAIR, int LANES, typename CNT = unsigned>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, 8)
 k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int nbin_total,
               const unsigned *__restrict__ node_first, const unsigned *__restrict__ node_items,
               int by_parent, const SplitRec *__restrict__ parent_split,
@@ -779,6 +779,17 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
                                              : (size_t)slab_entries / kSlots * (size_t)(lds_slots + (hi_base > 0 ? 1 : 0)) * (PAIR ? 2 : 1);
   long long ag = 0, ah = 0;
   unsigned ac = 0;
+  const size_t cell = hi_row ? (size_t)hi_base + f : plain ? (size_t)entry : (size_t)f * kSlots + bin;
+  const bool writes = lane == 0 && live && stored;
+  // the parent's cell is on its way while the slabs are added up
+  long long parent_g = 0, parent_h = 0;
+  CNT parent_c = 0;
+  if (writes && trick) {
+    const size_t po = (size_t)(nd >> 1) * nbin_total + cell;
+    parent_g = pg[po];
+    parent_c = pc[po];
+    if (PAIR || hh != nullptr) parent_h = ph[po];
+  }
   if (live) {
     // plain slabs: word0 of every entry, then word1 of every entry; others: the
     // launches of the level (groups of group_blocks blocks, the last one maybe
@@ -811,13 +822,12 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
   s_c[lane][e] = ac;
   __syncthreads();
   // cells of bins the slabs do not hold are zero in every node histogram, once and for all
-  if (lane == 0 && live && stored) {
+  if (writes) {
     for (int k = 1; k < LANES; ++k) {
       ag += s_g[k][e];
       ah += s_h[k][e];
       ac += s_c[k][e];
     }
-    const size_t cell = hi_row ? (size_t)hi_base + f : plain ? (size_t)entry : (size_t)f * kSlots + bin;
     const size_t o = (size_t)nd * nbin_total + cell;
     // without hessians (count as hessian) the caller may pass no hh / ph arrays
     const bool with_h = PAIR || hh != nullptr;
@@ -831,11 +841,10 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
     if (with_h) hh[o] = ah;
     hc[o] = cnt;
     if (trick) {
-      const size_t po = (size_t)(nd >> 1) * nbin_total + cell;
       const size_t so = (size_t)(nd ^ 1) * nbin_total + cell;
-      hg[so] = pg[po] - ag;
-      if (with_h) hh[so] = ph[po] - ah;
-      hc[so] = pc[po] - cnt;
+      hg[so] = parent_g - ag;
+      if (with_h) hh[so] = parent_h - ah;
+      hc[so] = parent_c - cnt;
     }
   }
 }
