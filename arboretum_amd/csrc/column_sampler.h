@@ -76,6 +76,7 @@ class ColumnSampler {
     HIP_OK(hipEventRecord(copied_, stream));
     at_ = 0;
   }
+  bool Samples() const { return device_ != nullptr; }
   // Mask of a level of the current tree, a byte per feature; null: every feature.
   const unsigned char *Active(int level) const {
     return device_ ? device_ + at_ * MaskBytes() + (size_t)level * F_ : nullptr;

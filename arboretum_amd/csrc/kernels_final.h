@@ -191,7 +191,7 @@ k_final(const uint32_t *__restrict__ bins, size_t stride, const int *__restrict_
       }
       node = node * 2 + right;
     }
-    __builtin_nontemporal_store(node, &leaf_of[i]);
+    if (leaf_of != nullptr) __builtin_nontemporal_store(node, &leaf_of[i]);  // uniform
     const float yh = yh0 + weights[node];
     yhat[i] = yh;
     if (NEXT_GRAD == 1) {

@@ -157,7 +157,7 @@ __device__ __forceinline__ void PlanBody(const NodeSum *__restrict__ tot, const 
     s_base[L] = total;
     *n_work = total <= max_items ? total : 0;  // never exceed the launch bound
     if (total > max_items) *overflow = 1;      // reported as an error at the end of the tree
-    if (rows_scanned) *rows_scanned += s_rows;
+    if (rows_scanned) atomicAdd(rows_scanned, s_rows);  // (trees may grow side by side)
   }
   __syncthreads();
   if (total > max_items) return;
