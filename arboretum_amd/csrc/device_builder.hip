@@ -39,7 +39,7 @@
 //   k_split_select    hist_apply_candidates        src/core/hist_tree_grower.cu:37-102
 //   k_part_*          apply_split, set_segment, CreatePartitioningIndexes,
 //                     scatter_kernel               src/core/builder.h:51-59,107-123,287-300
-//   k_leaf_*          UpdateLeafWeight, update_by_last_tree
+//   k_tree_end        UpdateLeafWeight, update_by_last_tree
 //                                                  src/core/garden.cu:45-76,487-503
 #include <hip/hip_runtime.h>
 

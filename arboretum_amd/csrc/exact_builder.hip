@@ -193,12 +193,18 @@ class ExactSortBuilder : public TreeBuilder {
       d_seg_[s] = DevAlloc<unsigned>(max_nodes);
     }
     d_split_ = DevAlloc<SplitRec>(last_nodes);
-    d_cand_ = DevAlloc<Cand>((size_t)last_nodes * F_);
-    d_work_ = DevAlloc<WorkItem>(max_items_);
-    d_n_work_ = DevAlloc<unsigned>(1);
-    d_node_first_ = DevAlloc<unsigned>(last_nodes);
-    d_node_items_ = DevAlloc<unsigned>(last_nodes);
-    d_part_ = DevAlloc<ExSum>((size_t)F_ * max_items_);
+    for (ExPlan &p : plans_) {
+      p.work = DevAlloc<WorkItem>(max_items_);
+      p.n_work = DevAlloc<unsigned>(1);
+      p.node_first = DevAlloc<unsigned>(last_nodes);
+      p.node_items = DevAlloc<unsigned>(last_nodes);
+      p.part = DevAlloc<ExSum>((size_t)F_ * max_items_);
+    }
+    // the root's plan is the same for every tree
+    d_root_tot_ = DevAlloc<NodeSum>(1);
+    d_root_seg_ = DevAlloc<unsigned>(1);
+    hipLaunchKernelGGL(k_first_root, dim3(1), dim3(256), 0, stream_, d_root_tot_, d_root_seg_, (unsigned)n_, kExItem,
+                       plans_[2].work, plans_[2].n_work, plans_[2].node_first, plans_[2].node_items);
     d_off_ = DevAlloc<ExSum>((size_t)F_ * max_items_);
     d_best_ = DevAlloc<Cand>((size_t)F_ * max_items_);
     d_lefts_ = DevAlloc<unsigned>((size_t)F_ * max_items_);
@@ -231,25 +237,32 @@ class ExactSortBuilder : public TreeBuilder {
     sampler_.Release();
     void *all[] = {d_yhat_, d_g_, d_h_, d_leaf_, d_node_of_, d_went_right_, d_gh_, d_ids_[0], d_ids_[1], d_ranks_[0],
                    d_ranks_[1], d_lg_[0], d_lg_[1], d_lh_[0], d_lh_[1], d_tot_[0],
-                   d_tot_[1], d_seg_[0], d_seg_[1], d_split_, d_cand_, d_work_, d_n_work_, d_node_first_,
-                   d_node_items_, d_part_, d_off_, d_best_, d_lefts_, d_left_off_, d_left_bits_, d_shifts_, d_records_, d_gmax_,
+                   d_tot_[1], d_seg_[0], d_seg_[1], d_split_, d_root_tot_, d_root_seg_, d_off_, d_best_, d_lefts_, d_left_off_, d_left_bits_, d_shifts_, d_records_, d_gmax_,
                    d_overflow_, d_tfid_, d_tbin_, d_tgain_, d_weights_};
     for (void *p : all)
       DevicePoolGive(p);
+    for (const ExPlan &p : plans_) {
+      void *q[] = {p.work, p.n_work, p.node_first, p.node_items, p.part};
+      for (void *x : q) DevicePoolGive(x);
+    }
     StreamPoolGive(stream_);
   }
 
  public:
   void GrowRound(std::vector<RegTree> *trees) override {
-    if (cfg_.objective == kLinearRegression) {
-      const unsigned parts = (unsigned)GridFor(n_, 256, kGmaxParts);
-      hipLaunchKernelGGL(k_grad_squared, dim3(parts), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
-      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(1024), 0, stream_, d_gmax_, parts, d_shifts_);
+    if (grad_ready_) {
+      // written by the end of the tree before
+    } else if (cfg_.objective == kLinearRegression) {
+      gmax_parts_ = (unsigned)GridFor(n_, 256, kGmaxParts);
+      hipLaunchKernelGGL(k_grad_squared, dim3(gmax_parts_), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, n_, d_gmax_);
     } else if (cfg_.objective == kLogisticRegression) {
       hipLaunchKernelGGL(k_grad_logistic, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_y_, d_yhat_, d_g_, d_h_, n_);  // (no d_h_: packed)
     } else {
       hipLaunchKernelGGL(k_grad_softmax, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_labels_, d_yhat_, d_g_, d_h_, n_, K_);
     }
+    if (cfg_.objective == kLinearRegression)
+      hipLaunchKernelGGL(k_set_shift, dim3(1), dim3(1024), 0, stream_, d_gmax_, gmax_parts_, d_shifts_);
+    grad_ready_ = false;
     owner_ = trees;
     for (int k = 0; k < K_; ++k) {
       trees->emplace_back((unsigned)D_, (unsigned)k);
@@ -343,39 +356,39 @@ class ExactSortBuilder : public TreeBuilder {
     const float *g = d_g_ + (size_t)label * n_;
     const float *h = d_h_ ? d_h_ + (size_t)label * n_ : nullptr;
     sampler_.NextTree(stream_);
-    hipLaunchKernelGGL(k_init_root, dim3(1), dim3(64), 0, stream_, d_tot_[0], d_seg_[0], (unsigned long long)n_);
-    hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, g, h, pack_ ? 1 : 0, n_, d_shifts_,
-                       d_tot_[0]);
-    HIP_OK(hipMemsetAsync(d_node_of_, 0, n_ * sizeof(unsigned), stream_));
-    int state = 0;
+    const ExPlan &root = plans_[2];
     // the root's lists: every row, sorted once; this tree's gradients in that order
     const dim3 whole((unsigned)((n_ + kExItem - 1) / kExItem), (unsigned)F_);
-    if (harr_) {
+    if (harr_)
       hipLaunchKernelGGL(k_ex_pair, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, g, h, d_gh_, n_);
-      hipLaunchKernelGGL((k_ex_gather<true>), whole, dim3(kExThreads), 0, stream_, sd_->lists, stride_, g, d_gh_,
-                         d_lg_[1], d_lh_[1], n_);
-    } else {
-      hipLaunchKernelGGL((k_ex_gather<false>), whole, dim3(kExThreads), 0, stream_, sd_->lists, stride_, g,
-                         (const float2 *)nullptr, d_lg_[1], d_lh_[1], n_);
+#define ARB_EX_GATHER(P, K)                                                                                        \
+  hipLaunchKernelGGL((k_ex_gather<P, K>), whole, dim3(kExThreads), 0, stream_, sd_->lists, stride_, g, d_gh_,     \
+                     d_lg_[1], d_lh_[1], n_, d_shifts_, root.part, max_items_)
+    if (pack_) ARB_EX_GATHER(true, true);
+    else if (pair_) ARB_EX_GATHER(true, false);
+    else ARB_EX_GATHER(false, false);
+#undef ARB_EX_GATHER
+    const bool fold = n_ / kExItem <= kExFoldItems;
+    if (!fold) {
+      HIP_OK(hipMemsetAsync(d_root_tot_, 0, 2 * sizeof(long long), stream_));
+      hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, g, h, pack_ ? 1 : 0, n_,
+                         d_shifts_, d_root_tot_);
     }
     ExLists lists{sd_->lists, sd_->list_ranks, d_lg_[1], d_lh_[1]};
     for (int level = 0; level + 1 < D_; ++level) {
       const int L = 1 << level;
       const bool last = level + 2 >= D_;
-      const unsigned grid_items = (unsigned)(n_ / kExItem) + 2u * (unsigned)L + 2u;
+      const ExPlan &plan = level == 0 ? root : plans_[level & 1], &next = plans_[(level + 1) & 1];
+      NodeSum *tot = level == 0 ? d_root_tot_ : d_tot_[level & 1], *tot_next = d_tot_[(level + 1) & 1];
+      unsigned *seg = level == 0 ? d_root_seg_ : d_seg_[level & 1], *seg_next = d_seg_[(level + 1) & 1];
+      const unsigned grid_items = ItemsOf(L);
       const dim3 per_item(grid_items, (unsigned)F_), per_node((unsigned)L, (unsigned)F_);
-      hipLaunchKernelGGL(k_plan, dim3(1), dim3(1024), 0, stream_, d_tot_[state], d_seg_[state], L, 0, kExItem, d_work_,
-                         d_n_work_, d_node_first_, d_node_items_, (unsigned long long *)nullptr,
-                         (const SplitRec *)nullptr, grid_items, d_overflow_, 0u);
+      if (!fold)
+        hipLaunchKernelGGL((k_ex_offsets<ExSum>), per_node, dim3(64), 0, stream_, plan.part, d_off_, plan.node_first,
+                           plan.node_items, max_items_);
 #define ARB_EX(P, D, K)                                                                                               \
-  do {                                                                                                                \
-    hipLaunchKernelGGL((k_ex_partial<P, K>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_,      \
-                       d_work_, d_n_work_, d_part_, max_items_);                                                      \
-    hipLaunchKernelGGL((k_ex_offsets<ExSum>), per_node, dim3(64), 0, stream_, d_part_, d_off_, d_node_first_,        \
-                       d_node_items_, max_items_);                                                                    \
-    hipLaunchKernelGGL((k_ex_scan<P, D, K>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_,      \
-                       d_work_, d_n_work_, d_off_, d_tot_[state], d_seg_[state], gp, d_best_, max_items_);            \
-  } while (0)
+  hipLaunchKernelGGL((k_ex_scan<P, D, K>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_, plan,  \
+                     fold ? (const ExSum *)nullptr : d_off_, level == 0 ? 1 : 0, tot, seg, gp, d_best_, max_items_)
       if (pack_ && f64_) ARB_EX(true, true, true);
       else if (pack_) ARB_EX(true, false, true);
       else if (pair_ && f64_) ARB_EX(true, true, false);
@@ -383,50 +396,54 @@ class ExactSortBuilder : public TreeBuilder {
       else if (f64_) ARB_EX(false, true, false);
       else ARB_EX(false, false, false);
 #undef ARB_EX
-      hipLaunchKernelGGL(k_ex_merge, per_node, dim3(64), 0, stream_, d_best_, d_node_first_, d_node_items_, max_items_,
-                         F_, d_cand_);
-      hipLaunchKernelGGL(k_split_select, dim3((L + 15) / 16), dim3(1024), 0, stream_, d_cand_, F_, L, d_tot_[state],
-                         d_seg_[state], d_tot_[state ^ 1], d_seg_[state ^ 1], d_split_, d_tfid_, d_tbin_, d_tgain_,
-                         L - 1, sampler_.Active(level),
-                         (unsigned long long *)nullptr);
-      hipLaunchKernelGGL(k_ex_decide, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, sd_->ranks, stride_, d_split_,
-                         d_node_of_, d_went_right_, n_);
+#define ARB_EX_SELECT(P, D)                                                                                          \
+  hipLaunchKernelGGL((k_ex_select<P, D>), dim3((unsigned)L), dim3(1024), 0, stream_, d_best_, plan.node_first,      \
+                     plan.node_items, max_items_, F_, sampler_.Active(level), tot, seg, tot_next, seg_next, d_split_, \
+                     d_tfid_, d_tbin_, d_tgain_, L, last ? 1 : 0, d_shifts_, gp, cfg_.tree.eta, d_weights_,          \
+                     d_overflow_, d_records_ + pending_.size() * RecordWords())
+      if (pair_ && f64_) ARB_EX_SELECT(true, true);
+      else if (pair_) ARB_EX_SELECT(true, false);
+      else if (f64_) ARB_EX_SELECT(false, true);
+      else ARB_EX_SELECT(false, false);
+#undef ARB_EX_SELECT
       if (last) {
-        const int blocks = (L + 127) / 128;
-#define ARB_LEAF(P, D)                                                                                          \
-  hipLaunchKernelGGL((k_leaf_weights<P, D>), dim3(blocks), dim3(128), 0, stream_, d_split_, d_tot_[state], L, \
-                     d_shifts_, gp, cfg_.tree.eta, d_weights_)
-        if (pair_ && f64_) ARB_LEAF(true, true);
-        else if (pair_) ARB_LEAF(true, false);
-        else if (f64_) ARB_LEAF(false, true);
-        else ARB_LEAF(false, false);
-#undef ARB_LEAF
-        hipLaunchKernelGGL(k_ex_final, dim3(GridFor(n_, 256)), dim3(256), 0, stream_, d_node_of_, d_weights_,
-                           d_yhat_ + (size_t)label * n_, d_leaf_, n_);
+        const bool next_grad = !inspect_ && K_ == 1;
+        gmax_parts_ = (unsigned)GridFor(n_, 256, kGmaxParts);
+#define ARB_EX_FINAL(G)                                                                                              \
+  hipLaunchKernelGGL(k_ex_final<G>, dim3(gmax_parts_), dim3(256), 0, stream_, sd_->ranks, stride_, d_split_,        \
+                     d_node_of_, level == 0 ? 1 : 0, d_weights_, d_yhat_ + (size_t)label * n_, d_leaf_, n_, d_y_, d_g_, \
+                     d_h_, d_gmax_)
+        if (next_grad && cfg_.objective == kLinearRegression) ARB_EX_FINAL(1);
+        else if (next_grad && cfg_.objective == kLogisticRegression) ARB_EX_FINAL(2);
+        else ARB_EX_FINAL(0);
+#undef ARB_EX_FINAL
+        grad_ready_ = next_grad;
       } else {
         const int b = level & 1;
-        hipLaunchKernelGGL(k_ex_count, per_item, dim3(kExThreads), 0, stream_, lists.ids, stride_, d_went_right_,
-                           d_work_, d_n_work_, d_lefts_, d_left_bits_, max_items_);
-        hipLaunchKernelGGL((k_ex_offsets<unsigned>), per_node, dim3(64), 0, stream_, d_lefts_, d_left_off_,
-                           d_node_first_, d_node_items_, max_items_);
-        if (harr_)
-          hipLaunchKernelGGL((k_ex_scatter<true>), per_item, dim3(kExThreads), 0, stream_, lists, d_ids_[b], d_ranks_[b],
-                             d_lg_[b], d_lh_[b], stride_, d_left_bits_, d_work_, d_n_work_, d_left_off_,
-                             d_seg_[state], d_seg_[state ^ 1], max_items_);
-        else
-          hipLaunchKernelGGL((k_ex_scatter<false>), per_item, dim3(kExThreads), 0, stream_, lists, d_ids_[b], d_ranks_[b],
-                             d_lg_[b], d_lh_[b], stride_, d_left_bits_, d_work_, d_n_work_, d_left_off_,
-                             d_seg_[state], d_seg_[state ^ 1], max_items_);
+        hipLaunchKernelGGL(k_ex_decide, dim3(1 + GridFor(n_, 1024, 1024)), dim3(1024), 0, stream_, sd_->ranks, stride_,
+                           d_split_, d_node_of_, d_went_right_, n_, level == 0 ? 1 : 0, tot_next, seg_next, L, next,
+                           ItemsOf(2 * L), max_items_, F_, d_overflow_);
+        hipLaunchKernelGGL(k_ex_count, per_item, dim3(kExThreads), 0, stream_, lists.ids, stride_, d_went_right_, plan,
+                           d_lefts_, d_left_bits_, max_items_);
+        if (!fold)
+          hipLaunchKernelGGL((k_ex_offsets<unsigned>), per_node, dim3(64), 0, stream_, d_lefts_, d_left_off_,
+                             plan.node_first, plan.node_items, max_items_);
+#define ARB_EX_SCATTER(P, K)                                                                                        \
+  hipLaunchKernelGGL((k_ex_scatter<P, K>), per_item, dim3(kExThreads), 0, stream_, lists, d_ids_[b], d_ranks_[b],  \
+                     d_lg_[b], d_lh_[b], stride_, d_left_bits_, plan, d_lefts_,                                     \
+                     fold ? (const unsigned *)nullptr : d_left_off_, seg, seg_next, d_shifts_, next, max_items_)
+        if (pack_) ARB_EX_SCATTER(true, true);
+        else if (pair_) ARB_EX_SCATTER(true, false);
+        else ARB_EX_SCATTER(false, false);
+#undef ARB_EX_SCATTER
         lists = ExLists{d_ids_[b], d_ranks_[b], d_lg_[b], d_lh_[b]};
-        state ^= 1;
       }
       HIP_OK(hipGetLastError());
     }
-    const int internal = (1 << (D_ - 1)) - 1, leaves = 1 << (D_ - 1);
-    hipLaunchKernelGGL(k_pack_record, dim3((leaves + 255) / 256), dim3(256), 0, stream_, d_tfid_, d_tbin_, d_tgain_,
-                       d_weights_, d_overflow_, internal, leaves, d_records_ + pending_.size() * RecordWords());
-    HIP_OK(hipGetLastError());
   }
+
+  // launch bound of the passes over the lists of L nodes
+  unsigned ItemsOf(int L) const { return (unsigned)(n_ / kExItem) + 2u * (unsigned)L + 2u; }
 
   const Configuration cfg_;
   DataMatrix *data_;
@@ -446,9 +463,8 @@ class ExactSortBuilder : public TreeBuilder {
   const uint8_t *d_labels_ = nullptr;
   std::shared_ptr<const float> y_held_;  // the matrix' target (d_y_, d_labels_)
   std::shared_ptr<const unsigned char> labels_held_;
-  unsigned *d_leaf_ = nullptr, *d_node_of_ = nullptr, *d_seg_[2] = {nullptr, nullptr}, *d_n_work_ = nullptr,
-           *d_node_first_ = nullptr, *d_node_items_ = nullptr, *d_lefts_ = nullptr, *d_left_off_ = nullptr,
-           *d_overflow_ = nullptr;
+  unsigned *d_leaf_ = nullptr, *d_node_of_ = nullptr, *d_seg_[2] = {nullptr, nullptr}, *d_root_seg_ = nullptr,
+           *d_lefts_ = nullptr, *d_left_off_ = nullptr, *d_overflow_ = nullptr;
   float *d_gmax_ = nullptr;  // partial maxima of |g|
   uint32_t *d_ids_[2] = {nullptr, nullptr}, *d_ranks_[2] = {nullptr, nullptr}, *d_records_ = nullptr;
   float *d_lg_[2] = {nullptr, nullptr}, *d_lh_[2] = {nullptr, nullptr};
@@ -457,9 +473,12 @@ class ExactSortBuilder : public TreeBuilder {
   float2 *d_gh_ = nullptr;  // (g, h) of the tree's label side by side: one gather per row
   NodeSum *d_tot_[2] = {nullptr, nullptr};
   SplitRec *d_split_ = nullptr;
-  Cand *d_cand_ = nullptr, *d_best_ = nullptr;
-  WorkItem *d_work_ = nullptr;
-  ExSum *d_part_ = nullptr, *d_off_ = nullptr;
+  Cand *d_best_ = nullptr;
+  ExPlan plans_[3] = {};  // of the levels in turn, and of the root
+  NodeSum *d_root_tot_ = nullptr;
+  ExSum *d_off_ = nullptr;
+  unsigned gmax_parts_ = 0;
+  bool grad_ready_ = false;  // the end of the tree before has written this round's gradients
   int *d_shifts_ = nullptr, *d_tfid_ = nullptr, *d_tbin_ = nullptr;
   ColumnSampler sampler_;
 };

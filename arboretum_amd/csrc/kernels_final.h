@@ -10,31 +10,6 @@ namespace arb {
 namespace {
 
 // --------------------------------------------------------------- leaves
-// UpdateLeafWeight (garden.cu:487-503, split.cu:25-35): left = Weight(left
-// sum), right = Weight(parent - left) with the subtraction in the sum type.
-template <bool PAIR, bool F64>
-__global__ void k_leaf_weights(const SplitRec *__restrict__ split, const NodeSum *__restrict__ tot,
-                               int L, const int *__restrict__ shifts, GainParams gp, float eta,
-                               float *__restrict__ weights) {
-  const int nd = blockIdx.x * blockDim.x + threadIdx.x;
-  if (nd >= L) return;
-  const int sg = shifts[0], sh = shifts[1];
-  const SplitRec s = split[nd];
-  const NodeSum t = tot[nd];
-  const double GL = FromFixed<F64>(s.left.g, sg), HL = PAIR ? FromFixed<F64>(s.left.h, sh) : 0.0;
-  const double GP = FromFixed<F64>(t.g, sg), HP = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
-  double GR, HR;
-  if (F64) {
-    GR = GP - GL;
-    HR = HP - HL;
-  } else {
-    GR = (double)((float)GP - (float)GL);
-    HR = (double)((float)HP - (float)HL);
-  }
-  weights[2 * nd] = LeafWeight<PAIR, F64>(GL, HL, s.left.c, gp) * eta;
-  weights[2 * nd + 1] = LeafWeight<PAIR, F64>(GR, HR, t.c - s.left.c, gp) * eta;
-}
-
 // State and work plan of a tree's root histogram over all n rows: one node from row 0 on.  Called by
 // one workgroup.
 __device__ __forceinline__ void RootPlan(unsigned n, unsigned rows_per_item, WorkItem *__restrict__ work,
@@ -70,7 +45,7 @@ k_first_root(NodeSum *__restrict__ root_tot, unsigned *__restrict__ root_seg, un
 // End of a tree in one launch, in front of the last pass: the splits of the last level from the
 // candidates of its scan (BestOfNode), the leaf weights (UpdateLeafWeight, garden.cu:487-503,
 // split.cu:25-35: left = Weight(left sum), right = Weight(parent - left) with the subtraction in the sum
-// type), the tree's record into its slot of the record ring (layout of k_pack_record), and, when the
+// type), the tree's record into its slot of the record ring (fid[internal], bin[internal], gain[internal], weights[leaves], overflow flag), and, when the
 // rows are resident (work set), the state and work plan of the next tree's root histogram.  As kernels of their own these
 // took 2 to 5 us each, and the last level's scan and selection in one workgroup per node 15 to 90 us.
 // grid ceil(L / 4) + 1, 256 threads, a wave per node; the last block writes the plan.
@@ -387,22 +362,6 @@ k_leaf_ids(const uint32_t *__restrict__ bins, size_t stride, const int *__restri
     }
     leaf_of[i] = node;
   }
-}
-
-// Tree record of the tree just grown into one slot of the record ring:
-// fid[internal], bin[internal], gain[internal], weights[leaves], overflow flag.
-__global__ void k_pack_record(const int *__restrict__ t_fid, const int *__restrict__ t_bin,
-                              const float *__restrict__ t_gain, const float *__restrict__ weights,
-                              const unsigned *__restrict__ overflow, int internal, int leaves,
-                              uint32_t *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < internal) {
-    out[i] = (uint32_t)t_fid[i];
-    out[internal + i] = (uint32_t)t_bin[i];
-    out[2 * internal + i] = __float_as_uint(t_gain[i]);
-  }
-  if (i < leaves) out[3 * internal + i] = __float_as_uint(weights[i]);
-  if (i == 0) out[3 * internal + leaves] = *overflow;
 }
 
 __global__ void k_fill_f32(float *p, float v, size_t n) {
