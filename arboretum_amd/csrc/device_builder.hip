@@ -1430,7 +1430,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
             FusedArgs a{src.bins, last ? nullptr : dst.bins, stride_, F_, src.g, q0 == 0 ? dst.g : nullptr, src.h,
                         q0 == 0 ? dst.h : nullptr, d_shifts_, d_split_, d_tot_[ps], d_seg_[ps], d_pwork_,
                         d_nwork_ + 1, q0 == 0 ? d_cursor2_ : nullptr, d_item_left_, d_slab_, slab_stride_, src.bins,
-                        q0, scan};
+                        q0, FusedRowsPerItem(PL), scan};
             const bool group = !single_group_ && !hi_rows_;
             if (pair_) LaunchFusedPair(!last, group, pack_, hi_rows_, nq, stream_, grid, a);
             else LaunchFusedSingle(!last, group, hi_rows_, nq, stream_, grid, a);

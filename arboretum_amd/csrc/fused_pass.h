@@ -30,7 +30,8 @@ struct FusedArgs {
   int slab_entries;
   const uint32_t *split_bins;  // start of the whole matrix
   int q0;                      // first quad of this launch
-  LevelScan scan;              // hg set: the pass finds the splits of its parents itself
+  unsigned rows_per_item;      // most rows of a work item
+  LevelScan scan;              // cand set: the pass finds the splits of its parents itself
 };
 
 // with hessians (pack: packed logistic gradients) / without.  write: the rows move to the children
