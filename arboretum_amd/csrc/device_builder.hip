@@ -1453,6 +1453,15 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
               hipLaunchKernelGGL(k_ix_part<false>, dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8,
                                  src.ids, dst.ids, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_,
                                  d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb, plan);
+          } else if (part_rows_ <= kChunkStep) {
+            if (pair_ && !pack_)
+              hipLaunchKernelGGL(k_part_small<true>, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, dst.bins, stride_,
+                                 W_, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1, d_cursor2_,
+                                 d_item_left_, code_, hi_word_, plan);
+            else
+              hipLaunchKernelGGL(k_part_small<false>, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, dst.bins, stride_,
+                                 W_, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1, d_cursor2_,
+                                 d_item_left_, code_, hi_word_, plan);
           } else {
             hipLaunchKernelGGL(k_part_count, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, stride_, d_split_,
                                d_pwork_, d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_, plan);
@@ -1593,9 +1602,13 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
 #define ARB_SCAN(P, D, B)                                                                                          \
   hipLaunchKernelGGL((k_split_scan<P, D, B>), grid, dim3(256), 0, stream_, d_hg_[hb], d_hh_[hb], d_hc_[hb],       \
                      nbin_total_, F_, slots_, d_tot_[state], d_shifts_, gp, hs, d_cand_, root_sum ? 1 : 0, hi_base_)
+    // (more bins than a wave scans at a time: a workgroup per feature and node)
 #define ARB_SCAN_B(P, D)                       \
   do {                                         \
-    if (hs <= 64) ARB_SCAN(P, D, 1);           \
+    if (hs > 256)                              \
+      hipLaunchKernelGGL((k_split_scan_wide<P, D>), dim3(F_, L), dim3(256), 0, stream_, d_hg_[hb], d_hh_[hb], d_hc_[hb], \
+                         nbin_total_, F_, slots_, d_tot_[state], d_shifts_, gp, hs, d_cand_, root_sum ? 1 : 0);          \
+    else if (hs <= 64) ARB_SCAN(P, D, 1);      \
     else if (hs <= 128) ARB_SCAN(P, D, 2);     \
     else ARB_SCAN(P, D, 4);                    \
   } while (0)
@@ -1650,30 +1663,23 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
              nullptr, HistGrid(2 * L, false), HistCus(false));
   }
 
-  // Stand-alone partition: groups of up to eight words per launch; the first
-  // launch also moves the gradients.
-  void LaunchPartRows(unsigned grid, const RowBuffers &src, const RowBuffers &dst, int ps) {
-    for (int q0 = 0; q0 < W_; q0 += 8) {  // (the ninth-bit word moves like a quad)
-      const int nq = std::min(8, W_ - q0);
-#define ARB_PART(P, N, G)                                                                                        \
-  hipLaunchKernelGGL((k_part_rows<P, N, G>), dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, dst.bins,    \
-                     stride_, q0, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1,      \
+  // Stand-alone partition of larger items: groups of up to eight words side by side.
+  void LaunchPartRows(unsigned items, const RowBuffers &src, const RowBuffers &dst, int ps) {
+    const int groups = (W_ + 7) / 8, nq = (W_ + groups - 1) / groups;  // (the ninth-bit word moves like a quad)
+#define ARB_PART(P, N)                                                                                             \
+  hipLaunchKernelGGL((k_part_rows<P, N>), dim3(items, groups), dim3(kHistThreads), 0, stream_, src.bins, dst.bins, \
+                     stride_, W_, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1,         \
                      d_wave_left_, d_item_left_, code_, hi_word_)
-#define ARB_PART_N(N)                                          \
-  case N:                                                      \
-    if (q0 == 0) {                                             \
-      if (pair_ && !pack_) ARB_PART(true, N, true);            \
-      else ARB_PART(false, N, true);                           \
-    } else {                                                   \
-      ARB_PART(false, N, false);                               \
-    }                                                          \
+#define ARB_PART_N(N)                     \
+  case N:                                 \
+    if (pair_ && !pack_) ARB_PART(true, N); \
+    else ARB_PART(false, N);              \
     break;
-      switch (nq) {
-        ARB_PART_N(1) ARB_PART_N(2) ARB_PART_N(3) ARB_PART_N(4) ARB_PART_N(5) ARB_PART_N(6) ARB_PART_N(7) ARB_PART_N(8)
-      }
+    switch (nq) {
+      ARB_PART_N(1) ARB_PART_N(2) ARB_PART_N(3) ARB_PART_N(4) ARB_PART_N(5) ARB_PART_N(6) ARB_PART_N(7) ARB_PART_N(8)
+    }
 #undef ARB_PART_N
 #undef ARB_PART
-    }
   }
 
   // launch bound of a stand-alone partition over PL parent nodes

@@ -702,19 +702,23 @@ k_part_hist_small(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins
 }
 
 // Stable partition alone (matrices too wide for the fused pass, 16-bit bins):
-// words [q0, q0 + NQ) of every row, and with GH the gradients, go to the
-// children order through the two register queues of the fused pass.  One launch
-// per group of words; every launch reads the word of the split feature again.
-template <bool PAIR, int NQ, bool GH>
+// the words of every row and the gradients go to the
+// children order through the two register queues of the fused pass.  A group of NQ words per
+// blockIdx.y (the last one begins earlier where the words do not divide: it writes some words a second time);
+// the first group also moves the gradients; every group reads the word of the split feature.
+template <bool PAIR, int NQ>
 __global__ void __launch_bounds__(kHistThreads)
-k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, size_t stride, int q0,
+k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, size_t stride, int words,
             const float *__restrict__ g, float *__restrict__ g_out, const float *__restrict__ h,
             float *__restrict__ h_out, const SplitRec *__restrict__ split,
             const unsigned *__restrict__ seg_start, const WorkItem *__restrict__ work,
             const unsigned *__restrict__ n_work, const unsigned *__restrict__ wave_left,
             const unsigned *__restrict__ item_left, BinCode code, int hi_word) {
   __shared__ unsigned s_tmp[kItemWaves + 1];
+  constexpr bool GH = true;
   const unsigned w = blockIdx.x;
+  const int q0 = min((int)blockIdx.y * NQ, words - NQ);
+  if (blockIdx.y != 0) g_out = nullptr;  // uniform
   if (w >= *n_work) return;
   const WorkItem it = work[w];
   const SplitRec s = split[it.node];
@@ -744,10 +748,13 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
     }
     R.s0 = split_col[a0];
     R.s1 = split_col[a1];
-    R.r.g0 = GH ? __builtin_nontemporal_load(&g[a0]) : 0.0f;
-    R.r.g1 = GH ? __builtin_nontemporal_load(&g[a1]) : 0.0f;
-    R.r.h0 = GH && PAIR ? __builtin_nontemporal_load(&h[a0]) : 0.0f;
-    R.r.h1 = GH && PAIR ? __builtin_nontemporal_load(&h[a1]) : 0.0f;
+    R.r.g0 = R.r.g1 = R.r.h0 = R.r.h1 = 0.0f;
+    if (g_out != nullptr) {
+      R.r.g0 = __builtin_nontemporal_load(&g[a0]);
+      R.r.g1 = __builtin_nontemporal_load(&g[a1]);
+      R.r.h0 = PAIR ? __builtin_nontemporal_load(&h[a0]) : 0.0f;
+      R.r.h1 = PAIR ? __builtin_nontemporal_load(&h[a1]) : 0.0f;
+    }
   };
   auto process = [&](const Rows &R, unsigned base) {
     const unsigned r0 = base + lane, r1 = r0 + 64;
@@ -773,6 +780,78 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
   }
   FlushQueue<PAIR, NQ, false, GH>(nullptr, QL, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
   FlushQueue<PAIR, NQ, false, GH>(nullptr, QR, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+}
+
+// The stand-alone partition in one launch, where a work item has one chunk of 128 rows per wave (kChunkStep rows at most): the
+// split of the node (SplitOf), the decisions, the claims of the children's ranges on the node's cursors (ClaimWithCount; zero at launch, the
+// planner clears them) and the move of every word of the rows and their gradients, straight from registers.  The first words of
+// the rows are requested before the split is known.  Within a child the items lie in the order of their claims; no result
+// depends on it.  The first block of the grid selects and plans when plan.cand is set.
+// 500,000 rows of ten words: 17.4 us; by k_part_count and k_part_rows, then a launch per group of words, 30.
+template <bool PAIR>
+__global__ void __launch_bounds__(kHistThreads)
+k_part_small(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, size_t stride, int words,
+             const float *__restrict__ g, float *__restrict__ g_out, const float *__restrict__ h,
+             float *__restrict__ h_out, const SplitRec *__restrict__ split, const unsigned *__restrict__ seg_start,
+             const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor,
+             unsigned *__restrict__ item_base, BinCode code, int hi_word, const SelectPlan plan) {
+  __shared__ unsigned s_tmp[kItemWaves + 2];
+  __shared__ SplitRec s_rec;
+  unsigned w = blockIdx.x;
+  if (plan.cand != nullptr && w-- == 0) {
+    SelectAndPlan(plan);
+    return;
+  }
+  if (w >= *n_work) return;
+  const WorkItem it = work[w];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
+  const unsigned r0 = wb + lane, r1 = r0 + 64;
+  const unsigned a0 = min(r0, we - 1), a1 = min(r1, we - 1);  // past the end: the last row
+  constexpr int kBatch = 8;
+  uint32_t b0[kBatch], b1[kBatch];
+  auto load = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      const size_t at = (size_t)min(q0 + q, words - 1) * stride;
+      b0[q] = bins[at + a0];
+      b1[q] = bins[at + a1];
+    }
+  };
+  load(0);
+  const float g0 = g[a0], g1 = g[a1];
+  const float h0 = PAIR ? h[a0] : 0.0f, h1 = PAIR ? h[a1] : 0.0f;
+  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  const SplitTest test = MakeSplitTest(s, code, hi_word);
+  const uint32_t *col = bins + (size_t)test.word * stride;
+  const bool right0 = test.Right(col[a0]), right1 = test.Right(col[a1]);
+  const bool v0 = r0 >= it.begin && r0 < we, v1 = r1 < we;
+  const unsigned long long lm0 = __ballot(v0 && !right0), rm0 = __ballot(v0 && right0);
+  const unsigned long long lm1 = __ballot(v1 && !right1), rm1 = __ballot(v1 && right1);
+  unsigned lo, ro;
+  ClaimWithCount(it, w, s, seg_start[it.node], (unsigned)(__popcll(lm0) + __popcll(lm1)), cursor, item_base, wave, lane,
+                 s_tmp, &lo, &ro);
+  if (wb >= we) return;
+  const unsigned d0 = right0 ? ro + RankBelow(rm0) : lo + RankBelow(lm0);
+  const unsigned d1 = right1 ? ro + (unsigned)__popcll(rm0) + RankBelow(rm1) : lo + (unsigned)__popcll(lm0) + RankBelow(lm1);
+  if (v0) g_out[d0] = g0;
+  if (v1) g_out[d1] = g1;
+  if (PAIR) {
+    if (v0) h_out[d0] = h0;
+    if (v1) h_out[d1] = h1;
+  }
+  for (int q0 = 0;; load(q0)) {
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      if (q0 + q < words) {  // uniform
+        uint32_t *to = bins_out + (size_t)(q0 + q) * stride;
+        if (v0) to[d0] = b0[q];
+        if (v1) to[d1] = b1[q];
+      }
+    }
+    q0 += kBatch;
+    if (q0 >= words) break;
+  }
 }
 
 // Adds the slabs of every directly built node of a level (on top of the stored

@@ -32,6 +32,17 @@ def test_either_side_of_the_line(oracle, n, F, objective, bins, nan_frac):
     _same(arb, oracle, X, y, cfg, 2)
 
 
+@pytest.mark.parametrize("n", [1, 66, 5000, 1_048_577, 1_060_003])
+@pytest.mark.parametrize("F,bins,objective,nan_frac", [(5, 700, 1, 0.1), (19, 3000, 0, 0.0), (51, 255, 1, 0.0), (49, 256, 0, 0.1)])
+def test_stand_alone_partitions(oracle, n, F, bins, objective, nan_frac):
+    # 16-bit ids (one and two groups of words) and rows in place, on either side of a chunk of rows per wave
+    import arboretum_amd as arb
+    X, y = make_data(n, F, objective, seed=n + F, nan_frac=nan_frac)
+    cfg = {"objective": objective, "method": 1, "internals": {"hist_size": bins, "double_precision": True},
+           "tree": {"max_depth": 4, "eta": 0.3, "lambda": 1.0, "min_child_weight": 1.0}}
+    _same(arb, oracle, X, y, cfg, 2)
+
+
 @pytest.mark.parametrize("n,objective,extra", [(1_100_001, 1, {}), (1_100_001, 0, {"lambda": 0.0, "min_child_weight": 30.0}),
                                                (20_000, 1, {"lambda": 0.0, "min_child_weight": 0.0}),
                                                (20_000, 1, {"alpha": 0.7}), (20_000, 0, {"max_leaf_weight": 0.05})])
