@@ -1445,14 +1445,18 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
           Mark(kPartition);
           if (indexed_) {
             // decisions, claims of the children's ranges and the move of (row id, g, h) in one launch
-            if (pair_)
-              hipLaunchKernelGGL(k_ix_part<true>, dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8,
-                                 src.ids, dst.ids, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_,
-                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb, plan);
-            else
-              hipLaunchKernelGGL(k_ix_part<false>, dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8,
-                                 src.ids, dst.ids, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_,
-                                 d_nwork_ + 1, d_cursor2_, d_item_left_, dm_->hibits, dm_->strideb, plan);
+#define ARB_IX(K)                                                                                                  \
+  hipLaunchKernelGGL((K), dim3(grid), dim3(kHistThreads), 0, stream_, dm_->bytes, dm_->stride8, src.ids, dst.ids, src.g, \
+                     dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1, d_cursor2_, d_item_left_,   \
+                     dm_->hibits, dm_->strideb, plan)
+            if (part_rows_ <= kChunkStep) {
+              if (pair_) ARB_IX(k_ix_part_small<true>);
+              else ARB_IX(k_ix_part_small<false>);
+            } else {
+              if (pair_) ARB_IX(k_ix_part<true>);
+              else ARB_IX(k_ix_part<false>);
+            }
+#undef ARB_IX
           } else if (part_rows_ <= kChunkStep) {
             if (pair_ && !pack_)
               hipLaunchKernelGGL(k_part_small<true>, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, dst.bins, stride_,

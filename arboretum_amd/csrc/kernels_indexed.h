@@ -233,6 +233,67 @@ k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__r
   FlushQueue<PAIR, 1, false, true>(nullptr, QR, false, ids_out, 0, g_out, h_out, lane, 0, 0, 0);
 }
 
+// The same where a work item has one chunk of 128 rows per wave (kChunkStep rows at most): ids and gradients are requested before
+// the split is known and go from registers straight to their places.  (200,000 rows: 7.6 us, 10.0 by k_ix_part.)
+template <bool PAIR>
+__global__ void __launch_bounds__(kHistThreads)
+k_ix_part_small(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__restrict__ ids,
+                unsigned *__restrict__ ids_out, const float *__restrict__ g, float *__restrict__ g_out,
+                const float *__restrict__ h, float *__restrict__ h_out, const SplitRec *__restrict__ split,
+                const unsigned *__restrict__ seg_start, const WorkItem *__restrict__ work,
+                const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor, unsigned *__restrict__ item_base,
+                const uint8_t *__restrict__ hibits, size_t strideb, const SelectPlan plan) {
+  __shared__ unsigned s_tmp[kItemWaves + 2];
+  __shared__ SplitRec s_rec;
+  unsigned w = blockIdx.x;
+  if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
+    SelectAndPlan(plan);
+    return;
+  }
+  if (w >= *n_work) return;
+  const WorkItem it = work[w];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
+  const unsigned r0 = wb + lane, r1 = r0 + 64;
+  const unsigned a0 = min(r0, we - 1), a1 = min(r1, we - 1);  // past the end: the last row
+  const unsigned id0 = ids ? ids[a0] : a0, id1 = ids ? ids[a1] : a1;
+  const float g0 = g[a0], g1 = g[a1];
+  const float h0 = PAIR ? h[a0] : 0.0f, h1 = PAIR ? h[a1] : 0.0f;
+  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  bool right0 = false, right1 = false;
+  if (s.fid >= 0) {  // uniform
+    if (hibits != nullptr && s.bin >= 255) {  // only an id of 256 goes right
+      const uint8_t *col = hibits + (size_t)s.fid * strideb;
+      const unsigned x0 = col[id0 >> 3], x1 = col[id1 >> 3];
+      right0 = (x0 >> (id0 & 7u)) & 1u;
+      right1 = (x1 >> (id1 & 7u)) & 1u;
+    } else {
+      const uint8_t *col = bytes + (size_t)s.fid * stride8;
+      const int x0 = col[id0], x1 = col[id1];
+      right0 = x0 > s.bin;  // builder.h:107-123
+      right1 = x1 > s.bin;
+    }
+  }
+  const bool v0 = r0 >= it.begin && r0 < we, v1 = r1 < we;
+  const unsigned long long lm0 = __ballot(v0 && !right0), rm0 = __ballot(v0 && right0);
+  const unsigned long long lm1 = __ballot(v1 && !right1), rm1 = __ballot(v1 && right1);
+  unsigned lo, ro;
+  ClaimWithCount(it, w, s, seg_start[it.node], (unsigned)(__popcll(lm0) + __popcll(lm1)), cursor, item_base, wave, lane,
+                 s_tmp, &lo, &ro);
+  if (v0) {
+    const unsigned d = right0 ? ro + RankBelow(rm0) : lo + RankBelow(lm0);
+    ids_out[d] = id0;
+    g_out[d] = g0;
+    if (PAIR) h_out[d] = h0;
+  }
+  if (v1) {
+    const unsigned d = right1 ? ro + (unsigned)__popcll(rm0) + RankBelow(rm1) : lo + (unsigned)__popcll(lm0) + RankBelow(lm1);
+    ids_out[d] = id1;
+    g_out[d] = g1;
+    if (PAIR) h_out[d] = h1;
+  }
+}
+
 // Histogram over records, every feature in one LDS histogram of `slots` bins
 // per feature (possible when features x slots is small enough: 200 features of
 // 65 bins with one word per cell take 108 KB): the record of a row is read
