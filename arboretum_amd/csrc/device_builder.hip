@@ -811,7 +811,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       hist_cus_ = indexed_ ? std::max(1u, cus_ / (unsigned)rec_groups_) : cus_;
       for (int level = 0; level + 1 < D_; ++level)
         max_hist_items_ = std::max(max_hist_items_, BalancedPlanItems(plan_rows, 1u << level, kMaxHistRows, hist_cus_));
-      max_hist_items_ = std::max(max_hist_items_, BalancedPlanItems(plan_rows, 1u, kMaxHistRows, cus_));
+      max_hist_items_ = std::max(max_hist_items_, BalancedPlanItems(plan_rows, 1u, kMaxHistRows, HistCus(true)));
     }
     // Rows per work item of a partition that builds no histogram: two workgroups per CU as long as
     // an item of kPartRows rows, the most a workgroup takes, would leave CUs without one.  (At 16384 rows
@@ -1196,7 +1196,8 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   bool HistOnRecords(bool root) const { return indexed_ && (rec_one_launch_ || !root); }
   unsigned HistCus(bool root) const {
     if (wide_) return std::max(1u, cus_ / (unsigned)WideGroups());
-    return HistOnRecords(root) ? hist_cus_ : cus_;
+    // (the groups of quads of a work item are workgroups side by side)
+    return HistOnRecords(root) ? hist_cus_ : std::max(1u, cus_ / (unsigned)HistGroups());
   }
   int WideGroups() const { return (F_ + wide_group_ - 1) / wide_group_; }
   unsigned HistGrid(int L, bool root) const {
@@ -1231,33 +1232,31 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       if (timing_ && root) timings_.hist_root_rows += n_;
       return;
     }
-    for (int q0 = 0; q0 < Q_; q0 += quads_per_group_) {
-      const int nq = std::min(quads_per_group_, Q_ - q0);
-      if (records) {
-        // one launch: every feature in one LDS histogram at rec_slots_ bins, or the groups of
-        // quads at 256 bins side by side (a workgroup per work item and group)
-        const int total = HistBlocks(Q_);
-        const int pieces = rec_one_launch_ ? total : HistBlocks(quads_per_group_);
-        const int ngroups = (total + pieces - 1) / pieces;
-        const int slots = rec_one_launch_ ? rec_slots_ : kSlots;
-        const int lay = rec_one_launch_ ? rec_lay_blocks_ : 0;   // blocks the LDS image is laid out for
-        const size_t lds = (size_t)(lay > 0 ? lay : pieces) * kBlockFeatures * slots * 8 * (pair_ ? 2 : 1);
-        const size_t item_words = rec_one_launch_ ? lds / 8 : (size_t)slab_entries_ * (pair_ ? 2 : 1);
-        if (lds > kLdsBudget || (size_t)total * 4 > (size_t)dm_->RS || ngroups != rec_groups_ ||
-            item_words > (size_t)slab_entries_ * (pair_ ? 2 : 1))
-          throw std::runtime_error("internal: record histogram launch does not fit");
-        const unsigned blocks = (grid + 7u) / 8u * 8u * (unsigned)ngroups;
-        // a power of two of blocks in every group (the last may hold fewer), or in the padded layout
-        const int last_pieces = total - (ngroups - 1) * pieces;
-        const bool pow2 = lay > 0 ? (lay & (lay - 1)) == 0
-                                  : (pieces & (pieces - 1)) == 0 && (last_pieces & (last_pieces - 1)) == 0;
+    if (records) {
+      // one launch: every feature in one LDS histogram at rec_slots_ bins, or the groups of
+      // quads at 256 bins side by side (a workgroup per work item and group)
+      const int total = HistBlocks(Q_);
+      const int pieces = rec_one_launch_ ? total : HistBlocks(quads_per_group_);
+      const int ngroups = (total + pieces - 1) / pieces;
+      const int slots = rec_one_launch_ ? rec_slots_ : kSlots;
+      const int lay = rec_one_launch_ ? rec_lay_blocks_ : 0;   // blocks the LDS image is laid out for
+      const size_t lds = (size_t)(lay > 0 ? lay : pieces) * kBlockFeatures * slots * 8 * (pair_ ? 2 : 1);
+      const size_t item_words = rec_one_launch_ ? lds / 8 : (size_t)slab_entries_ * (pair_ ? 2 : 1);
+      if (lds > kLdsBudget || (size_t)total * 4 > (size_t)dm_->RS || ngroups != rec_groups_ ||
+          item_words > (size_t)slab_entries_ * (pair_ ? 2 : 1))
+        throw std::runtime_error("internal: record histogram launch does not fit");
+      const unsigned blocks = (grid + 7u) / 8u * 8u * (unsigned)ngroups;
+      // a power of two of blocks in every group (the last may hold fewer), or in the padded layout
+      const int last_pieces = total - (ngroups - 1) * pieces;
+      const bool pow2 = lay > 0 ? (lay & (lay - 1)) == 0
+                                : (pieces & (pieces - 1)) == 0 && (last_pieces & (last_pieces - 1)) == 0;
 #define ARB_REC(P, POW2, H)                                                                                      \
   do {                                                                                                            \
     static std::once_flag configured;                                                                             \
     AllowLdsOnce(configured, (k_hist_rec<P, POW2, H>), kLdsBudget);                                               \
     hipLaunchKernelGGL((k_hist_rec<P, POW2, H>), dim3(blocks), dim3(kHistThreads), lds, stream_, dm_->rec,        \
-                       dm_->RS, cur.ids, Q_, slots, cur.g, cur.h, d_shifts_, d_hwork_, d_nwork_, d_slab_, pieces, \
-                       total, ngroups, item_words, lay);                                                          \
+                     dm_->RS, cur.ids, Q_, slots, cur.g, cur.h, d_shifts_, d_hwork_, d_nwork_, d_slab_, pieces, \
+                     total, ngroups, item_words, lay);                                                          \
   } while (0)
 #define ARB_REC_P(P)                                   \
   do {                                                 \
@@ -1266,17 +1265,14 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
     else if (pow2) ARB_REC(P, true, false);            \
     else ARB_REC(P, false, false);                     \
   } while (0)
-        if (pair_) ARB_REC_P(true);
-        else ARB_REC_P(false);
+      if (pair_) ARB_REC_P(true);
+      else ARB_REC_P(false);
 #undef ARB_REC_P
 #undef ARB_REC
-        if (timing_) ++(root ? timings_.hist_root_launches : timings_.hist_deep_launches);
-        break;
-      } else {
-        HistLaunch(nq, grid, cur.bins, stride_, q0, cur.g, cur.h);
-      }
-      if (timing_) ++(root ? timings_.hist_root_launches : timings_.hist_deep_launches);
+    } else {
+      HistLaunch(grid, cur.bins, stride_, cur.g, cur.h);
     }
+    if (timing_) ++(root ? timings_.hist_root_launches : timings_.hist_deep_launches);
     if (timing_ && root) timings_.hist_root_rows += n_;
   }
 
@@ -1289,22 +1285,27 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
                          pair_ ? orig.h : nullptr, 0, n_, d_shifts_, d_tot_[state]);
   }
 
-  // k_hist over quads [q0, q0 + nq) of rows laid out with `stride` words between columns
-  void HistLaunch(int nq, unsigned grid, const uint32_t *bins, size_t stride, int q0, const float *g, const float *h) {
-    // the ninth-bit words of the 32 features of a group of eight quads: column Q_ + q0 / 8
-    const uint32_t *hi_col = hi_ ? bins + (size_t)(Q_ + q0 / 8) * stride : nullptr;
-    if (hi_skip_ && pair_)
-      LaunchHist<true, 2>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_, hi_col);
-    else if (hi_skip_)
-      LaunchHist<false, 2>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_, hi_col);
-    else if (hi_rows_ && pair_)
-      LaunchHist<true, 1>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_, hi_col);
-    else if (hi_rows_)
-      LaunchHist<false, 1>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_, hi_col);
-    else if (pair_)
-      LaunchHist<true>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_);
-    else
-      LaunchHist<false>(nq, stream_, grid, bins, stride, q0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_, slab_stride_);
+  int HistGroups() const { return (Q_ + quads_per_group_ - 1) / quads_per_group_; }
+  // k_hist over all quads of rows laid out with `stride` words between columns
+  void HistLaunch(unsigned grid, const uint32_t *bins, size_t stride, const float *g, const float *h) {
+    // the ninth-bit words of the 32 features of a group of eight quads: column Q_ + group
+    const uint32_t *hi_col = hi_ ? bins + (size_t)Q_ * stride : nullptr;
+#define ARB_HIST(P, H)                                                                                               \
+  do {                                                                                                               \
+    if (HistGroups() == 1)                                                                                           \
+      LaunchHist<P, H>(Q_, stream_, grid, bins, stride, 0, F_, g, h, d_shifts_, d_hwork_, d_nwork_, d_slab_,         \
+                       slab_stride_, hi_col);                                                                        \
+    else                                                                                                             \
+      LaunchHistGroups<P, H == 2 ? 2 : 0>(Q_, stream_, grid, bins, stride, F_, g, h, d_shifts_, d_hwork_, d_nwork_,  \
+                                          d_slab_, slab_stride_, hi_col);                                            \
+  } while (0)
+    if (hi_skip_ && pair_) ARB_HIST(true, 2);
+    else if (hi_skip_) ARB_HIST(false, 2);
+    else if (hi_rows_ && pair_) ARB_HIST(true, 1);  // (one group)
+    else if (hi_rows_) ARB_HIST(false, 1);
+    else if (pair_) ARB_HIST(true, 0);
+    else ARB_HIST(false, 0);
+#undef ARB_HIST
   }
 
   // plan_state >= 0: one more block plans the row pass over this level's nodes (d_tot_ / d_seg_
@@ -1785,15 +1786,12 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       DoneWithBlock(buf);
     }
     // histograms of the gathered rows, added to the level's histograms
-    const unsigned per_item = HistRowsPerItem(rows);
+    const unsigned per_item = HistRowsPerItem(rows, std::max(64, 512 / HistGroups()));
     const unsigned grid = (unsigned)std::min<size_t>(rows / per_item + 2 * L + 1, max_hist_items_);
     Mark(kPlan);
     PlanOn(d_blk_tot_, d_blk_seg_, L, 0, per_item, d_hwork_, d_nwork_, level == 0 ? -1 : level, nullptr, grid);
     Mark(level == 0 ? kHistRoot : kHistDeep);
-    for (int q0 = 0; q0 < Q_; q0 += quads_per_group_) {
-      const int nq = std::min(quads_per_group_, Q_ - q0);
-      HistLaunch(nq, grid, hist_bins, br, q0, hist_g, hist_h);
-    }
+    HistLaunch(grid, hist_bins, br, hist_g, hist_h);
     if (in_place) DoneWithBlock(buf);
     Reduce(L, level & 1, false, state, false, !first);
   }

@@ -157,15 +157,17 @@ void Enqueue(const HistSumArgs &a, const Shape &sh, unsigned char *mem, unsigned
                      a.shift_h, s.tot, s.seg, a.use_trick ? 1 : 0, per_item, s.work, s.n_work, s.node_first,
                      s.node_items, max_items, s.overflow, s.shifts, status);
   const unsigned grid = (unsigned)std::min<size_t>((size_t)a.nrow / per_item + 2 * (size_t)a.nodes + 1, max_items);
-  for (int q0 = 0; q0 < sh.Q; q0 += sh.quads_per_group) {
-    const int nq = std::min(sh.quads_per_group, sh.Q - q0);
-    if (pair)
-      LaunchHist<true>(nq, st, grid, a.bins, (size_t)a.stride, q0, a.ncol, a.grad, a.hess, s.shifts, s.work, s.n_work,
-                       s.slab, sh.slab_entries);
-    else
-      LaunchHist<false>(nq, st, grid, a.bins, (size_t)a.stride, q0, a.ncol, a.grad, a.hess, s.shifts, s.work, s.n_work,
-                        s.slab, sh.slab_entries);
+#define ARB_HIST(LAUNCH, ...)                                                                                        \
+  LAUNCH(sh.Q, st, grid, a.bins, (size_t)a.stride, __VA_ARGS__ a.ncol, a.grad, a.hess, s.shifts, s.work, s.n_work, s.slab, \
+         sh.slab_entries)
+  if (sh.Q > sh.quads_per_group) {
+    if (pair) ARB_HIST(LaunchHistGroups<true>);
+    else ARB_HIST(LaunchHistGroups<false>);
+  } else {
+    if (pair) ARB_HIST(LaunchHist<true>, 0, );
+    else ARB_HIST(LaunchHist<false>, 0, );
   }
+#undef ARB_HIST
   dim3 rgrid((sh.slab_entries + 63) / 64, a.nodes);
   if (pair)
     hipLaunchKernelGGL((k_hist_reduce<true, 16>), rgrid, dim3(1024), 0, st, s.slab, sh.slab_entries, sh.nbin_total,

@@ -114,13 +114,13 @@ __device__ __forceinline__ void FlushSlab(const unsigned long long *__restrict__
 // PAIR with h == nullptr: g holds packed logistic gradients (PackGrad).
 // HI: hi_col is the column of the ninth-bit words of features 4 q0 .. 4 q0 + 31
 // (AccumulateRow: 1 = accumulated in a 257th row of entries, 2 = skipped).
-template <bool PAIR, int NQ, int HI = 0>
-__global__ void __launch_bounds__(kHistThreads)
-k_hist(const uint32_t *__restrict__ bins, size_t stride, int q0, int F,
-       const float *__restrict__ g, const float *__restrict__ h, const int *__restrict__ shifts,
-       const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
-       unsigned long long *__restrict__ slab, int slab_entries, const uint32_t *__restrict__ hi_col = nullptr) {
-  extern __shared__ unsigned long long lds[];
+template <bool PAIR, int NQ, int HI>
+__device__ __forceinline__ void HistItem(unsigned long long *__restrict__ lds, const uint32_t *__restrict__ bins,
+                                         size_t stride, int q0, int F,
+                                         const float *__restrict__ g, const float *__restrict__ h,
+                                         const int *__restrict__ shifts, const WorkItem *__restrict__ work,
+                                         const unsigned *__restrict__ n_work, unsigned long long *__restrict__ slab,
+                                         int slab_entries, const uint32_t *__restrict__ hi_col) {
   const unsigned w = blockIdx.x;
   if (w >= *n_work) return;
   const WorkItem it = work[w];
@@ -159,6 +159,36 @@ k_hist(const uint32_t *__restrict__ bins, size_t stride, int q0, int F,
     if (v1) AccumulateRow<PAIR, NQ, HI>(lds, b1, g1, h1, sg, sh, q0, F);
   }
   FlushSlab<PAIR, NQ, HI>(lds, slab, w, slab_entries, q0);
+}
+
+template <bool PAIR, int NQ, int HI = 0>
+__global__ void __launch_bounds__(kHistThreads)
+k_hist(const uint32_t *__restrict__ bins, size_t stride, int q0, int F,
+       const float *__restrict__ g, const float *__restrict__ h, const int *__restrict__ shifts,
+       const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
+       unsigned long long *__restrict__ slab, int slab_entries, const uint32_t *__restrict__ hi_col = nullptr) {
+  extern __shared__ unsigned long long lds[];
+  HistItem<PAIR, NQ, HI>(lds, bins, stride, q0, F, g, h, shifts, work, n_work, slab, slab_entries, hi_col);
+}
+
+// The groups of a matrix of more quads than one LDS histogram takes, side by side: kMaxGroupQuads quads per blockIdx.y, NQ_LAST in
+// the last one.  A launch per group had 256 work items to itself, each with the slabs of all groups to clear, write and add up;
+// here 64 items by four groups fill the chip (1 M rows x 100, 256 bins, ten soft-max classes: 80 us a
+// tree in four launches; 50 trees 18.4 -> 16.6 ms).
+// hi_col: the first of the columns of ninth-bit words, one per group.
+template <bool PAIR, int NQ_LAST, int HI = 0>
+__global__ void __launch_bounds__(kHistThreads)
+k_hist_groups(const uint32_t *__restrict__ bins, size_t stride, int F,
+              const float *__restrict__ g, const float *__restrict__ h, const int *__restrict__ shifts,
+              const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
+              unsigned long long *__restrict__ slab, int slab_entries, const uint32_t *__restrict__ hi_col) {
+  extern __shared__ unsigned long long lds[];
+  const int q0 = (int)blockIdx.y * kMaxGroupQuads;
+  const uint32_t *hi = HI != 0 ? hi_col + (size_t)blockIdx.y * stride : nullptr;
+  if (blockIdx.y + 1 < gridDim.y)
+    HistItem<PAIR, kMaxGroupQuads, HI>(lds, bins, stride, q0, F, g, h, shifts, work, n_work, slab, slab_entries, hi);
+  else
+    HistItem<PAIR, NQ_LAST, HI>(lds, bins, stride, q0, F, g, h, shifts, work, n_work, slab, slab_entries, hi);
 }
 
 // Histogram of contiguous row ranges with 16-bit bins: a workgroup per work item and group of

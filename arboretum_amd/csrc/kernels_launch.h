@@ -49,6 +49,28 @@ void LaunchHist(int nq, hipStream_t st, unsigned grid, const uint32_t *bins, siz
 #undef ARB_CASE
 }
 
+// nq: all quads of the matrix, more than kMaxGroupQuads; grid: work items
+template <bool PAIR, int HI = 0>
+void LaunchHistGroups(int nq, hipStream_t st, unsigned grid, const uint32_t *bins, size_t stride, int F, const float *g,
+                      const float *h, const int *shifts, const WorkItem *work, const unsigned *n_work,
+                      unsigned long long *slab, int slab_entries, const uint32_t *hi_col = nullptr) {
+  const int groups = (nq + kMaxGroupQuads - 1) / kMaxGroupQuads;
+  const size_t lds = HistLdsBytes(kMaxGroupQuads, PAIR);
+#define ARB_CASE(N)                                                                                                   \
+  case N: {                                                                                                           \
+    static std::once_flag configured;                                                                                 \
+    AllowLdsOnce(configured, k_hist_groups<PAIR, N, HI>, lds);                                                        \
+    hipLaunchKernelGGL((k_hist_groups<PAIR, N, HI>), dim3(grid, groups), dim3(kHistThreads), lds, st, bins, stride, F, \
+                       g, h, shifts, work, n_work, slab, slab_entries, hi_col);                                       \
+    break;                                                                                                            \
+  }
+  switch (nq - (groups - 1) * kMaxGroupQuads) {
+    ARB_CASE(1) ARB_CASE(2) ARB_CASE(3) ARB_CASE(4) ARB_CASE(5) ARB_CASE(6) ARB_CASE(7) ARB_CASE(8)
+    default: throw std::runtime_error("internal: bad quad count");
+  }
+#undef ARB_CASE
+}
+
 }  // namespace
 }  // namespace arb
 #endif  // ARBORETUM_AMD_KERNELS_LAUNCH_H_
