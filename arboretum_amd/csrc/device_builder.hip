@@ -1314,23 +1314,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   void Reduce(int L, int hb, bool by_parent, int parent_state, bool trick, bool accumulate = false,
               int plan_state = -1) {
     Mark(kReduce);
-    const size_t last_nodes = (size_t)1 << (D_ - 2);
-    unsigned *next_first = d_node_first_ == d_node_first2_ ? d_node_first2_ + last_nodes : d_node_first2_;
-    unsigned *next_items = d_node_items_ == d_node_items2_ ? d_node_items2_ + last_nodes : d_node_items2_;
-    NextPlan plan;
-    if (plan_state >= 0) {
-      plan.tot = d_tot_[plan_state];
-      plan.seg_start = d_seg_[plan_state];
-      plan.L = L;
-      plan.rows_per_item = fused_ ? FusedRowsPerItem(L) : part_rows_;
-      plan.work = d_pwork_;
-      plan.n_work = d_nwork_ + 1;
-      plan.node_first = next_first;
-      plan.node_items = next_items;
-      plan.max_items = fused_ ? FusedGrid(L) : PartGrid(L);
-      plan.overflow = d_overflow_;
-      plan.cursor = d_cursor2_;
-    }
+    const NextPlan plan = PlanOfNextPass(L, plan_state);
     // many nodes: few slabs per node and the output dominates -> longer output runs per block
     const bool wide_blocks = L >= 32;
     const int entries = wide_blocks ? 256 : 64;
@@ -1356,10 +1340,71 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       else ARB_REDUCE(false, 16);
     }
 #undef ARB_REDUCE
-    if (plan_state >= 0 && fused_) {
-      d_node_first_ = next_first;
-      d_node_items_ = next_items;
-    }
+    UsePlanOfNextPass(plan);
+  }
+
+  // The work plan of the row pass over this level's nodes (none: plan_state < 0), and, once the kernel that makes it has been
+  // launched, its set of (first item, items) per node.
+  NextPlan PlanOfNextPass(int L, int plan_state) {
+    const size_t last_nodes = (size_t)1 << (D_ - 2);
+    unsigned *next_first = d_node_first_ == d_node_first2_ ? d_node_first2_ + last_nodes : d_node_first2_;
+    unsigned *next_items = d_node_items_ == d_node_items2_ ? d_node_items2_ + last_nodes : d_node_items2_;
+    NextPlan plan;
+    if (plan_state < 0) return plan;
+    plan.tot = d_tot_[plan_state];
+    plan.seg_start = d_seg_[plan_state];
+    plan.L = L;
+    plan.rows_per_item = fused_ ? FusedRowsPerItem(L) : part_rows_;
+    plan.work = d_pwork_;
+    plan.n_work = d_nwork_ + 1;
+    plan.node_first = next_first;
+    plan.node_items = next_items;
+    plan.max_items = fused_ ? FusedGrid(L) : PartGrid(L);
+    plan.overflow = d_overflow_;
+    plan.cursor = d_cursor2_;
+    return plan;
+  }
+  void UsePlanOfNextPass(const NextPlan &plan) {
+    if (plan.work == nullptr || !fused_) return;
+    d_node_first_ = plan.node_first;
+    d_node_items_ = plan.node_items;
+  }
+
+  // Levels whose slabs are added up and scanned by one kernel: a workgroup goes through the slabs of its pair of nodes one after
+  // the other, so there are either few of them (four work items a pair) or workgroups for every CU.  (10.5 M x 28, eight items a pair, 64
+  // and 128 workgroups: 16.6 + 6.4 us as two kernels, 30 as one.)
+  bool ReducesAndScans(int L) const {
+    if (!trick_ || wide_ || streamed_ || L < 2) return false;
+    const unsigned groups = (unsigned)L * (slab_entries_ / kBlockEntries), pairs = L / 2;
+    const unsigned items = fused_ ? (unsigned)(n_ / FusedRowsPerItem(pairs)) + pairs : HistGrid(L, false);
+    return groups >= cus_ || (groups >= cus_ / 8 && items <= 4 * pairs);
+  }
+  void ReduceAndScan(int L, int hb, int parent_state, int state, const GainParams &gp, bool store, int plan_state) {
+    Mark(kReduce);
+    const NextPlan plan = PlanOfNextPass(L, plan_state);
+    const bool one = indexed_ && rec_one_launch_;
+    const int hs = std::min(data_->hist_size, slots_);
+    const dim3 grid(2 * (slab_entries_ / kBlockEntries) + (plan_state >= 0 ? 1 : 0), L / 2);
+#define ARB_RS(P, D, B)                                                                                              \
+  hipLaunchKernelGGL((k_reduce_scan<P, D, B>), grid, dim3(1024), 0, stream_, d_slab_, slab_entries_, nbin_total_,    \
+                     d_node_first_, d_node_items_, fused_ ? 1 : 0, d_split_, d_tot_[parent_state], d_hg_[hb],        \
+                     d_hh_[hb], d_hc_[hb], d_hg_[hb ^ 1], d_hh_[hb ^ 1], d_hc_[hb ^ 1],                              \
+                     one ? HistBlocks(Q_) : HistBlocks(quads_per_group_), one ? rec_slots_ : kSlots,                 \
+                     one ? rec_lay_blocks_ : 0, hi_base_, store ? 1 : 0, d_tot_[state], F_, d_shifts_, gp, hs,       \
+                     d_cand_, plan)
+#define ARB_RS_B(P, D)              \
+  do {                              \
+    if (hs <= 64) ARB_RS(P, D, 1);  \
+    else if (hs <= 128) ARB_RS(P, D, 2); \
+    else ARB_RS(P, D, 4);           \
+  } while (0)
+    if (pair_ && f64_) ARB_RS_B(true, true);
+    else if (pair_) ARB_RS_B(true, false);
+    else if (f64_) ARB_RS_B(false, true);
+    else ARB_RS_B(false, false);
+#undef ARB_RS_B
+#undef ARB_RS
+    UsePlanOfNextPass(plan);
   }
 
   void GrowOne(int label) {
@@ -1438,7 +1483,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
             if (timing_ && (last || !dominant_only_ || trees_grown_ % sample_every_ == 0))
             ++(last ? timings_.fused_last_launches : timings_.hist_deep_launches);
           }
-          Reduce(L, hb, true, ps, true, false, last ? -1 : state);
+          if (!ReducesAndScans(L)) Reduce(L, hb, true, ps, true, false, last ? -1 : state);
         } else {
           const unsigned items = PartGrid(PL);  // (planned by the reduction of the level above)
           const SelectPlan plan = SelectInPartition(PL) ? PlanOfPartition(level - 1, PL, ps) : SelectPlan{};
@@ -1473,13 +1518,15 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
             LaunchPartRows(items, src, dst, ps);
           }
           HistOfNodes(dst, L, false);  // (planned with the splits of the level above)
-          Reduce(L, hb, false, ps, trick_, false, last ? -1 : state);
+          if (!ReducesAndScans(L)) Reduce(L, hb, false, ps, trick_, false, last ? -1 : state);
         }
       }
+      const bool both = level > 0 && ReducesAndScans(L);
+      if (both) ReduceAndScan(L, hb, state ^ 1, state, gp, !last || inspect_, last ? -1 : state);
       if (inspect_) KeepHist(level, L, hb, state);
       // own_scan_: the pass of the next level selects the splits of this level's nodes; those of the last
       // level are selected at the end of the tree
-      LaunchScan(level, L, hb, state, gp, level == 0 && !root_totals_ready_ && !hi_skip_);
+      if (!both) LaunchScan(level, L, hb, state, gp, level == 0 && !root_totals_ready_ && !hi_skip_);
       root_totals_ready_ = false;
       if (!last && !own_scan_ && !SelectInPartition(L)) LaunchSelect(level, L, state);
       state ^= 1;

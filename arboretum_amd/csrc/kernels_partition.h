@@ -1018,6 +1018,165 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
   }
 }
 
+// Slab reduction and split scan of a level of many nodes in one kernel (8-bit bins, sibling subtraction): a workgroup owns
+// eight features of a pair of siblings.  It adds up the slabs of the built child's features, stores both children's
+// histograms for the level below, and scans them: a wave per feature and child, the built one from the LDS, its sibling as
+// parent - built.  Deep levels are bound by the bytes of their histograms, 16 or 24 a cell of which most rows-poor nodes fill few: here
+// they are written once and not read again, and not written at all at the last level (store = 0), where no child needs
+// them.  Taken when pairs and features give enough workgroups (HipTreeBuilder::ReducesAndScans); a level of few nodes
+// needs its slabs shared out finer, by bins.  1.5 M rows x 200, 65 bins, max_depth 10: reductions and scans take 355 us a
+// tree, 453 with two kernels on every level.
+// Arguments as those of k_hist_reduce and k_split_scan.  grid (2 * blocks of 16 features, pairs) and one more block in x
+// with a plan, 1024 threads.
+template <bool PAIR, bool F64, int BPL>
+__global__ void __launch_bounds__(1024)
+k_reduce_scan(const unsigned long long *__restrict__ slab, int slab_entries, int nbin_total,
+              const unsigned *__restrict__ node_first, const unsigned *__restrict__ node_items, int by_parent,
+              const SplitRec *__restrict__ parent_split, const NodeSum *__restrict__ parent_tot,
+              long long *__restrict__ hg, long long *__restrict__ hh, unsigned long long *__restrict__ hc,
+              const long long *__restrict__ pg, const long long *__restrict__ ph,
+              const unsigned long long *__restrict__ pc, int group_blocks, int lds_slots, int lay_blocks, int hi_base,
+              int store, const NodeSum *__restrict__ tot, int F, const int *__restrict__ shifts, GainParams gp,
+              int hist_size, Cand *__restrict__ cand, const NextPlan plan) {
+  if (plan.work != nullptr && blockIdx.x + 1 == gridDim.x) {
+    if (blockIdx.y == 0)
+      PlanBody(plan.tot, plan.seg_start, plan.L, 0, plan.rows_per_item, plan.work, plan.n_work, plan.node_first,
+               plan.node_items, nullptr, nullptr, plan.max_items, plan.overflow, plan.cursor);
+    return;
+  }
+  constexpr int kFeatures = 8, kPad = kSlots + 2;
+  constexpr unsigned per = PAIR ? 2u : 1u;
+  __shared__ long long s_g[kFeatures][kPad], s_h[PAIR ? kFeatures : 1][kPad];
+  __shared__ unsigned s_c[kFeatures][kPad];  // (the slabs of one call hold fewer than 2^32 rows)
+  const int pair = blockIdx.y, block = blockIdx.x >> 1, f16 = (blockIdx.x & 1) * kFeatures;
+  int nd;
+  unsigned items, first;
+  if (by_parent) {
+    const unsigned long long cl = parent_split[pair].left.c, cr = parent_tot[pair].c - cl;
+    nd = 2 * pair + (cl > cr ? 1 : 0);
+    items = node_items[pair];
+    first = node_first[pair];
+  } else {
+    nd = 2 * pair + (node_items[2 * pair] == 0xffffffffu ? 1 : 0);
+    items = node_items[nd];
+    first = node_first[nd];
+  }
+  const size_t slab_words = lay_blocks > 0 ? (size_t)lay_blocks * kBlockFeatures * (size_t)lds_slots * per
+                                           : (size_t)slab_entries / kSlots * (size_t)(lds_slots + (hi_base > 0 ? 1 : 0)) * per;
+  const unsigned long long *from = slab + (size_t)first * slab_words;
+  auto sums = [&](unsigned word, long long *g, long long *h, unsigned *c) {
+    long long ag = 0, ah = 0;
+    unsigned ac = 0;
+    const unsigned long long *p = from + word;
+#pragma unroll 4
+    for (unsigned s = 0; s < items; ++s, p += slab_words) {
+      const unsigned long long w0 = p[0];
+      const long long gq = ((long long)(w0 << (64 - kCountShift))) >> (64 - kCountShift);
+      ag += gq;
+      ac += (unsigned)((w0 - (unsigned long long)gq) >> kCountShift);
+      if (PAIR) ah += (long long)p[kWord1];
+    }
+    *g = ag;
+    *h = ah;
+    *c = ac;
+  };
+  {
+    const int group = block / group_blocks;
+    const int blocks_here = lay_blocks > 0 ? lay_blocks : min(group_blocks, slab_entries / kBlockEntries - group * group_blocks);
+    const unsigned base = (unsigned)(group * group_blocks * kBlockEntries) * per;
+    const int f = threadIdx.x & (kFeatures - 1);
+    const unsigned entry = (unsigned)((block - group * group_blocks) * kBlockEntries + f16 + f);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int bin = (int)(threadIdx.x / kFeatures) + k * (1024 / kFeatures);
+      long long g = 0, h = 0;
+      unsigned c = 0;
+      if (bin < lds_slots) sums(base + HistWord<PAIR>(entry + (unsigned)bin * kBlockFeatures, blocks_here), &g, &h, &c);
+      s_g[f][bin] = g;
+      if (PAIR) s_h[f][bin] = h;
+      s_c[f][bin] = c;
+    }
+  }
+  const int f0 = block * kBlockFeatures + f16;
+  const int hist_cells = hi_base > 0 ? hi_base : nbin_total;  // cells of the 256-bin histograms
+  const size_t o = (size_t)nd * nbin_total, so = (size_t)(nd ^ 1) * nbin_total, po = (size_t)pair * nbin_total;
+  if (store && hi_base > 0 && threadIdx.x < kFeatures) {
+    // bin 256 of the features: behind the image of the 256 bins, laid out like one more bin
+    const int f = f0 + (int)threadIdx.x;
+    if (f * kSlots < hist_cells) {
+      long long g, h;
+      unsigned c;
+      sums((unsigned)slab_entries * per + (unsigned)(f / kBlockFeatures) * per * kBlockFeatures + (unsigned)(f % kBlockFeatures),
+           &g, &h, &c);
+      const size_t cell = (size_t)hi_base + f;
+      hg[o + cell] = g;
+      hg[so + cell] = pg[po + cell] - g;
+      if (PAIR) hh[o + cell] = h;
+      if (PAIR) hh[so + cell] = ph[po + cell] - h;
+      hc[o + cell] = c;
+      hc[so + cell] = pc[po + cell] - c;
+    }
+  }
+  __syncthreads();
+  if (store) {
+    // (cells of bins the slabs do not hold are zero in every node histogram, once and for all)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int i = (int)threadIdx.x + k * 1024, f = i / kSlots, bin = i & (kSlots - 1);
+      if (bin < lds_slots && (f0 + f) * kSlots < hist_cells) {
+        const size_t cell = (size_t)(f0 + f) * kSlots + bin;
+        const long long g = s_g[f][bin];
+        const unsigned c = s_c[f][bin];
+        hg[o + cell] = g;
+        hg[so + cell] = pg[po + cell] - g;
+        hc[o + cell] = c;
+        hc[so + cell] = pc[po + cell] - c;
+        if (PAIR) {
+          const long long h = s_h[f][bin];
+          hh[o + cell] = h;
+          hh[so + cell] = ph[po + cell] - h;
+        }
+      }
+    }
+  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, f = wave & (kFeatures - 1);
+  if (f0 + f >= F) return;
+  const bool sibling = wave >= kFeatures;  // uniform
+  const int of = sibling ? nd ^ 1 : nd;
+  const NodeSum t = tot[of];
+  Cand best;
+  best.gain = 0.0f;
+  best.bin = -1;
+  best.left = NodeSum{0, 0, 0};
+  if (t.c != 0) {
+    long long g4[BPL], h4[BPL];
+    unsigned long long c4[BPL];
+#pragma unroll
+    for (int j = 0; j < BPL; ++j) {
+      const int bin = lane * BPL + j;
+      g4[j] = h4[j] = 0;
+      c4[j] = 0;
+      if (bin < lds_slots) {
+        g4[j] = s_g[f][bin];
+        if (PAIR) h4[j] = s_h[f][bin];
+        c4[j] = s_c[f][bin];
+        if (sibling) {
+          const size_t cell = po + (size_t)(f0 + f) * kSlots + bin;
+          g4[j] = pg[cell] - g4[j];
+          if (PAIR) h4[j] = ph[cell] - h4[j];
+          c4[j] = pc[cell] - c4[j];
+        }
+      }
+    }
+    const int sg = shifts[0], sh = shifts[1];
+    NodeSum carry{0, 0, 0};
+    ScanChunk<PAIR, F64, BPL>(g4, h4, c4, 0, lane, FromFixed<F64>(t.g, sg), PAIR ? FromFixed<F64>(t.h, sh) : 0.0, t, sg, sh,
+                              gp, hist_size, &carry, &best);
+    BestOfWave<PAIR>(&best);
+  }
+  if (lane == 0) cand[(size_t)of * F + f0 + f] = best;
+}
+
 }  // namespace
 }  // namespace arb
 #endif  // ARBORETUM_AMD_KERNELS_PARTITION_H_

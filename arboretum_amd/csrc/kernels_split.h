@@ -36,6 +36,71 @@ namespace {
 
 // --------------------------------------------------------------- split scan
 
+// The candidates among 64 BPL neighbouring bins of a feature from `chunk` on, BPL of them in every lane (sums per bin; overwritten).
+// carry: the sums below them, and then with them.
+template <bool PAIR, bool F64, int BPL>
+__device__ __forceinline__ void ScanChunk(long long (&g4)[BPL], long long (&h4)[BPL], unsigned long long (&c4)[BPL],
+                                          int chunk, int lane, double GT, double HT, const NodeSum &t, int sg, int sh,
+                                          const GainParams &gp, int hist_size, NodeSum *carry, Cand *best) {
+#pragma unroll
+  for (int j = 1; j < BPL; ++j) {
+    g4[j] += g4[j - 1];
+    h4[j] += h4[j - 1];
+    c4[j] += c4[j - 1];
+  }
+  long long ig = g4[BPL - 1], ih = h4[BPL - 1];
+  unsigned long long ic = c4[BPL - 1];
+  for (int off = 1; off < 64; off <<= 1) {
+    const long long og = __shfl_up(ig, off);
+    const long long oh = PAIR ? __shfl_up(ih, off) : 0;
+    const unsigned long long oc = __shfl_up(ic, off);
+    if (lane >= off) {
+      ig += og;
+      ih += oh;
+      ic += oc;
+    }
+  }
+  const long long eg = carry->g + ig - g4[BPL - 1], eh = carry->h + ih - h4[BPL - 1];
+  const unsigned long long ec = carry->c + ic - c4[BPL - 1];
+#pragma unroll
+  for (int j = 0; j < BPL; ++j) {
+    const int bin = chunk + lane * BPL + j;
+    if (bin < hist_size) {
+      const long long lg = eg + g4[j], lh = eh + h4[j];
+      const unsigned long long lc = ec + c4[j];
+      const double GL = FromFixed<F64>(lg, sg);
+      const double HL = PAIR ? FromFixed<F64>(lh, sh) : 0.0;
+      const float gn = SplitGain<PAIR, F64>(GL, HL, lc, GT, HT, t.c, gp);
+      if (gn > 0.0f && gn >= best->gain) {
+        best->gain = gn;
+        best->bin = bin;
+        best->left.g = lg;
+        best->left.h = lh;
+        best->left.c = lc;
+      }
+    }
+  }
+  carry->g += __shfl(ig, 63);
+  if (PAIR) carry->h += __shfl(ih, 63);
+  carry->c += __shfl(ic, 63);
+}
+// The best candidate of a wave in every lane: highest gain, ties to the highest bin (bins differ).
+template <bool PAIR>
+__device__ __forceinline__ void BestOfWave(Cand *best) {
+  // one key, then the winner's sums
+  unsigned long long key = best->bin < 0 ? 0ull : ((unsigned long long)__float_as_uint(best->gain) << 32) | (unsigned)(best->bin + 1);
+  unsigned long long top = key;
+  for (int off = 32; off > 0; off >>= 1) top = max(top, (unsigned long long)__shfl_xor(top, off));
+  if (top != 0) {  // uniform
+    const int from = __ffsll((unsigned long long)__ballot(key == top)) - 1;  // (keys differ by their bins)
+    best->gain = __shfl(best->gain, from);
+    best->bin = __shfl(best->bin, from);
+    best->left.g = __shfl(best->left.g, from);
+    best->left.h = PAIR ? __shfl(best->left.h, from) : 0;
+    best->left.c = __shfl(best->left.c, from);
+  }
+}
+
 // One wave scans one (feature, node): inclusive prefix over the slots, gain
 // per bin < hist_size, arg-max with ties to the HIGHEST bin (builder.h:39-49),
 // only gains > 0 (hist_tree_grower.cu:31).  `first` is the index of the
@@ -57,9 +122,7 @@ __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, co
     const int sg = shifts[0], sh = shifts[1];
     const double GT = FromFixed<F64>(t.g, sg);
     const double HT = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
-    // sums of the slots below the current chunk
-    long long carry_g = 0, carry_h = 0;
-    unsigned long long carry_c = 0;
+    NodeSum carry{0, 0, 0};  // sums of the slots below the current chunk
     for (int chunk = 0; chunk < slots && chunk < hist_size; chunk += 64 * BPL) {
       const size_t base = first + chunk + lane * BPL;
       long long g4[BPL], h4[BPL];
@@ -76,60 +139,9 @@ __device__ __forceinline__ Cand ScanFeature(const long long *__restrict__ hg, co
           c4[j] = hc[base + j];
         }
       }
-#pragma unroll
-      for (int j = 1; j < BPL; ++j) {
-        g4[j] += g4[j - 1];
-        h4[j] += h4[j - 1];
-        c4[j] += c4[j - 1];
-      }
-      long long ig = g4[BPL - 1], ih = h4[BPL - 1];
-      unsigned long long ic = c4[BPL - 1];
-      for (int off = 1; off < 64; off <<= 1) {
-        const long long og = __shfl_up(ig, off);
-        const long long oh = PAIR ? __shfl_up(ih, off) : 0;
-        const unsigned long long oc = __shfl_up(ic, off);
-        if (lane >= off) {
-          ig += og;
-          ih += oh;
-          ic += oc;
-        }
-      }
-      const long long eg = carry_g + ig - g4[BPL - 1], eh = carry_h + ih - h4[BPL - 1];
-      const unsigned long long ec = carry_c + ic - c4[BPL - 1];
-#pragma unroll
-      for (int j = 0; j < BPL; ++j) {
-        const int bin = chunk + lane * BPL + j;
-        if (bin < hist_size) {
-          const long long lg = eg + g4[j], lh = eh + h4[j];
-          const unsigned long long lc = ec + c4[j];
-          const double GL = FromFixed<F64>(lg, sg);
-          const double HL = PAIR ? FromFixed<F64>(lh, sh) : 0.0;
-          const float gn = SplitGain<PAIR, F64>(GL, HL, lc, GT, HT, t.c, gp);
-          if (gn > 0.0f && gn >= best.gain) {
-            best.gain = gn;
-            best.bin = bin;
-            best.left.g = lg;
-            best.left.h = lh;
-            best.left.c = lc;
-          }
-        }
-      }
-      carry_g += __shfl(ig, 63);
-      if (PAIR) carry_h += __shfl(ih, 63);
-      carry_c += __shfl(ic, 63);
+      ScanChunk<PAIR, F64, BPL>(g4, h4, c4, chunk, lane, GT, HT, t, sg, sh, gp, hist_size, &carry, &best);
     }
-    // highest gain, ties to the highest bin: one key, then the winner's sums
-    unsigned long long key = best.bin < 0 ? 0ull : ((unsigned long long)__float_as_uint(best.gain) << 32) | (unsigned)(best.bin + 1);
-    unsigned long long top = key;
-    for (int off = 32; off > 0; off >>= 1) top = max(top, (unsigned long long)__shfl_xor(top, off));
-    if (top != 0) {  // uniform
-      const int from = __ffsll((unsigned long long)__ballot(key == top)) - 1;  // (keys differ by their bins)
-      best.gain = __shfl(best.gain, from);
-      best.bin = __shfl(best.bin, from);
-      best.left.g = __shfl(best.left.g, from);
-      best.left.h = PAIR ? __shfl(best.left.h, from) : 0;
-      best.left.c = __shfl(best.left.c, from);
-    }
+    BestOfWave<PAIR>(&best);
   }
   return best;
 }
