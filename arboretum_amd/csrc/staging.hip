@@ -25,9 +25,17 @@ void ParallelCopy(void *dst, const void *src, size_t bytes) {
 }
 
 // Up to kStageSlots pinned blocks and the event of the last copy that touched each.
+// two: the copies go to `stream` and a second one in turn (behind what `stream` holds already): one copy's start does not wait
+// for the end of the one before (13 us a piece: 112 MB to the device 2.48 -> 2.12 ms, 2.05 at the rate of the link).
 struct Slots {
-  explicit Slots(int count, size_t bytes, hipStream_t stream) : count(count), stream(stream) {
+  Slots(int count, size_t bytes, hipStream_t stream, bool two) : count(count), stream(stream) {
     try {
+      if (two) {
+        other = StreamPoolTake();
+        HIP_OK(hipEventCreateWithFlags(&before, hipEventDisableTiming));
+        HIP_OK(hipEventRecord(before, stream));
+        HIP_OK(hipStreamWaitEvent(other, before, 0));
+      }
       for (int k = 0; k < count; ++k) {
         block[k] = PinnedPoolTake(bytes);
         HIP_OK(hipEventCreateWithFlags(&copied[k], hipEventDisableTiming));
@@ -41,14 +49,19 @@ struct Slots {
     (void)hipStreamSynchronize(stream);  // (a failed call may leave a copy pending; else this was waited for)
     Release();
   }
+  hipStream_t Of(size_t piece) const { return other && (piece & 1) ? other : stream; }
   void Release() {
+    if (other) (void)hipStreamSynchronize(other);
+    StreamPoolGive(other);
+    if (before) (void)hipEventDestroy(before);
     for (int k = 0; k < kStageSlots; ++k) {
       PinnedPoolGive(block[k]);
       if (copied[k]) (void)hipEventDestroy(copied[k]);
     }
   }
   const int count;
-  hipStream_t stream;
+  hipStream_t stream, other = nullptr;
+  hipEvent_t before = nullptr;
   void *block[kStageSlots] = {};
   hipEvent_t copied[kStageSlots] = {};
 };
@@ -73,11 +86,11 @@ void CopyToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
     return;
   }
   const size_t pieces = (bytes + kStageBytes - 1) / kStageBytes;
-  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::min(bytes, kStageBytes), stream);
+  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::min(bytes, kStageBytes), stream, pieces > 2);
   auto start = [&](size_t k) {
     const size_t at = k * kStageBytes, len = std::min(kStageBytes, bytes - at);
-    HIP_OK(hipMemcpyAsync(s.block[k % s.count], (const char *)src + at, len, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipEventRecord(s.copied[k % s.count], stream));
+    HIP_OK(hipMemcpyAsync(s.block[k % s.count], (const char *)src + at, len, hipMemcpyDeviceToHost, s.Of(k)));
+    HIP_OK(hipEventRecord(s.copied[k % s.count], s.Of(k)));
   };
   for (size_t k = 0; k < pieces && k < (size_t)s.count; ++k) start(k);
   for (size_t k = 0; k < pieces; ++k) {
@@ -95,13 +108,14 @@ void StageToDevice(size_t pieces, const std::function<size_t(size_t)> &bytes_of,
   size_t most = 0;
   for (size_t k = 0; k < pieces; ++k) most = std::max(most, bytes_of(k));
   if (most > kStageBytes) throw std::runtime_error("internal: staging piece too large");
-  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::max<size_t>(most, 1), stream);
+  // (work that follows a piece on the stream keeps all of them there)
+  Slots s((int)std::min<size_t>(pieces, kStageSlots), std::max<size_t>(most, 1), stream, !then && pieces > 2);
   for (size_t k = 0; k < pieces; ++k) {
     const int slot = (int)(k % s.count);
     if (k >= (size_t)s.count) HIP_OK(hipEventSynchronize(s.copied[slot]));
     fill(k, s.block[slot]);
-    HIP_OK(hipMemcpyAsync(dst_of(k), s.block[slot], bytes_of(k), hipMemcpyHostToDevice, stream));
-    HIP_OK(hipEventRecord(s.copied[slot], stream));
+    HIP_OK(hipMemcpyAsync(dst_of(k), s.block[slot], bytes_of(k), hipMemcpyHostToDevice, s.Of(k)));
+    HIP_OK(hipEventRecord(s.copied[slot], s.Of(k)));
     if (then) then(k);
   }
 }
