@@ -252,17 +252,21 @@ void Garden::UpdateByLastTree(DataMatrix *data) {
   if (trees_.size() < K) return;
   SyncTrees();
   std::vector<float> &y_hat = data->YHat();
+  // (a matrix may carry the predictions of a booster of more classes, or of fewer: the classes both
+  // have are advanced)
+  const size_t classes = data->rows ? std::min(K, y_hat.size() / data->rows) : 0;
   if (WalksOnDevice(data)) {
     // (a predictor of its own: the other one keeps the whole model laid out)
     std::lock_guard<std::mutex> lock(predictor_mutex_);
     if (!round_predictor_) round_predictor_.reset(CreateDevicePredictor());
     const float *sums = PredictOnDevice(round_predictor_.get(), *data, trees_, trees_.size() - K, trees_.size(), K, 0.0f);
-    ParallelFor(y_hat.size(), [&](size_t b, size_t e) {
+    ParallelFor(classes * data->rows, [&](size_t b, size_t e) {
       for (size_t i = b; i < e; ++i) y_hat[i] += sums[i];
     });
     return;
   }
-  for (size_t t = trees_.size() - K; t < trees_.size(); ++t) trees_[t].Predict(*data, y_hat.data());
+  for (size_t t = trees_.size() - K; t < trees_.size(); ++t)
+    if (trees_[t].label < classes) trees_[t].Predict(*data, y_hat.data());
 }
 
 void Garden::GetY(DataMatrix *data, float *out) const {
