@@ -36,8 +36,9 @@ void HostPoolGive(void *p) noexcept;
 // has not).
 bool GpuInUse() noexcept;
 
-// Streams (non-blocking, default priority) that are kept and handed out again; nothing may be pending
-// on one that is given back.
+// Streams (non-blocking, default priority) of the current device that are kept and handed out again;
+// nothing may be pending on one that is given back.  Blocks and streams return to the device they came
+// from, whichever one is current when they are given back.
 hipStream_t StreamPoolTake();
 void StreamPoolGive(hipStream_t s) noexcept;  // s may be null
 

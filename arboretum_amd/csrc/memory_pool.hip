@@ -196,8 +196,12 @@ void DevicePoolTrim() noexcept { DevicePool().Trim(CurrentDevice()); }
 namespace {
 constexpr size_t kIdleStreams = 16;
 std::mutex g_streams_mutex;
-std::vector<std::pair<int, hipStream_t>> &IdleStreams() {
-  static auto *v = new std::vector<std::pair<int, hipStream_t>>();
+struct Streams {
+  std::vector<std::pair<int, hipStream_t>> idle;
+  std::unordered_map<hipStream_t, int> made_on;  // the device of every stream, in use or idle
+};
+Streams &PooledStreams() {
+  static auto *v = new Streams();
   return *v;
 }
 }  // namespace
@@ -206,7 +210,7 @@ hipStream_t StreamPoolTake() {
   const int dev = CurrentDevice();
   {
     std::lock_guard<std::mutex> lock(g_streams_mutex);
-    auto &idle = IdleStreams();
+    auto &idle = PooledStreams().idle;
     for (size_t k = 0; k < idle.size(); ++k)
       if (idle[k].first == dev) {
         hipStream_t s = idle[k].second;
@@ -218,6 +222,13 @@ hipStream_t StreamPoolTake() {
   hipStream_t s = nullptr;
   const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
   if (e != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e) + " creating a stream");
+  try {
+    std::lock_guard<std::mutex> lock(g_streams_mutex);
+    PooledStreams().made_on[s] = dev;
+  } catch (...) {
+    (void)hipStreamDestroy(s);
+    throw;
+  }
   NoteGpuInUse();
   return s;
 }
@@ -226,13 +237,17 @@ void StreamPoolGive(hipStream_t s) noexcept {
   if (!s) return;
   {
     std::lock_guard<std::mutex> lock(g_streams_mutex);
-    if (IdleStreams().size() < kIdleStreams) {
+    // back to the device it was made on: the thread that gives it may use another one
+    auto &pool = PooledStreams();
+    const auto it = pool.made_on.find(s);
+    if (it != pool.made_on.end() && pool.idle.size() < kIdleStreams) {
       try {
-        IdleStreams().emplace_back(CurrentDevice(), s);
+        pool.idle.emplace_back(it->second, s);
         return;
       } catch (...) {
       }
     }
+    if (it != pool.made_on.end()) pool.made_on.erase(it);
   }
   (void)hipStreamDestroy(s);
 }
