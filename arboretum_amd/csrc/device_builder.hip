@@ -912,6 +912,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   void MakeOtherLanes() {
     if (K_ < 2 || streamed_ || n_ > kLaneRows || sampler_.Samples()) return;
     HIP_OK(hipEventCreateWithFlags(&round_start_, hipEventDisableTiming));
+    other_lanes_.reserve(kLanes);
     while (other_lanes_.size() + 1 < std::min(kLanes, (size_t)K_)) {
       Lane lane;
       std::swap(static_cast<Lane &>(*this), lane);
@@ -926,10 +927,25 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       }
       std::swap(static_cast<Lane &>(*this), lane);
       if (!made) break;
-      HIP_OK(hipStreamSynchronize(lane.stream_));
       other_lanes_.push_back(lane);
+      HIP_OK(hipStreamSynchronize(lane.stream_));
     }
   }
+  // Another lane in use while the object lives (0: the first, nothing to do), also when growing a tree fails.
+  class UseLane {
+   public:
+    UseLane(HipTreeBuilder *b, size_t lane) : b_(b), lane_(lane) { Swap(); }
+    ~UseLane() { Swap(); }
+    UseLane(const UseLane &) = delete;
+    UseLane &operator=(const UseLane &) = delete;
+
+   private:
+    void Swap() noexcept {
+      if (lane_ > 0) std::swap(static_cast<Lane &>(*b_), b_->other_lanes_[lane_ - 1]);
+    }
+    HipTreeBuilder *const b_;
+    const size_t lane_;
+  };
   // The first lane's stream behind the work of the others.
   void JoinLanes() {
     for (Lane &lane : other_lanes_) {
@@ -995,21 +1011,32 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
       for (Lane &lane : other_lanes_) HIP_OK(hipStreamWaitEvent(lane.stream_, round_start_, 0));
     }
     record_leaves_ = !several;  // (trees side by side would overwrite each other's: GetLeaves walks the last one)
-    for (int k = 0; k < K_; ++k) {
-      // the record stays on the device until somebody needs it: no host
-      // synchronisation between trees
-      trees->emplace_back((unsigned)D_, (unsigned)k);
-      // the last tree of the round on the first lane
-      const size_t lane = several ? (size_t)(K_ - 1 - k) % (other_lanes_.size() + 1) : 0;
-      if (lane > 0) std::swap(static_cast<Lane &>(*this), other_lanes_[lane - 1]);
-      GrowOne(k);
-      if (lane > 0) std::swap(static_cast<Lane &>(*this), other_lanes_[lane - 1]);
-      ++trees_grown_;
-      pending_.push_back(trees->size() - 1);
-      if (inspect_ || pending_.size() == kRecordRing) {
-        if (several) JoinLanes();
-        FlushTrees();
+    const size_t before = trees->size();
+    size_t grown = 0;
+    try {
+      for (int k = 0; k < K_; ++k) {
+        // the record stays on the device until somebody needs it: no host
+        // synchronisation between trees
+        trees->emplace_back((unsigned)D_, (unsigned)k);
+        {
+          // the last tree of the round on the first lane
+          const UseLane use(this, several ? (size_t)(K_ - 1 - k) % (other_lanes_.size() + 1) : 0);
+          GrowOne(k);
+        }
+        ++trees_grown_;
+        pending_.push_back(trees->size() - 1);
+        ++grown;
+        if (inspect_ || pending_.size() == kRecordRing) {
+          if (several) JoinLanes();
+          FlushTrees();
+        }
       }
+    } catch (...) {
+      // the tree that failed is no part of the model, and nothing that reads on the first lane's stream
+      // overtakes the others
+      for (Lane &lane : other_lanes_) (void)hipStreamSynchronize(lane.stream_);
+      trees->resize(before + grown);
+      throw;
     }
     if (several) JoinLanes();
     // phase times are read back lazily as well (GetTimings), or when many events are waiting

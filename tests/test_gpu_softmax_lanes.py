@@ -40,3 +40,33 @@ def test_trees_of_a_round(oracle, n, F, K, rounds, bins, depth):
                 assert np.array_equal(to[key], tg[key], equal_nan=True), (key, t)
         assert np.array_equal(ob.leaf(), g.leaves())
         assert np.array_equal(ob.yhat(), g.train_yhat())
+
+
+def test_a_round_that_fails_leaves_the_booster_usable(oracle):
+    # an error that another user of the runtime left in this thread is found by the check behind the first
+    # tree's kernels, which belong to another stream's state: that tree goes, and the next round grows the
+    # trees it would have grown
+    import hipmem
+    import arboretum_amd as arb
+    X, labels = _problem(4000, 9, 3, seed=11)
+    cfg = {"objective": 4, "method": 1, "internals": {"hist_size": 64, "double_precision": True},
+           "tree": {"max_depth": 5, "eta": 0.3, "lambda": 1.0, "labels_count": 3}}
+    ob = oracle.Booster(X, labels=labels, config=cfg)
+    data = arb.DMatrix(X, labels=labels)
+    g = arb.Garden(cfg, data)
+    g.labels_count = 3
+    g.grow_tree()
+    assert hipmem.hip().hipSetDevice(99) != 0
+    with pytest.raises(arb.ArboretumError):
+        g.grow_tree()
+    assert g.num_trees() == 3
+    for _ in range(2):
+        g.grow_tree()
+    ob.grow(3)
+    assert g.num_trees() == 9
+    for t in range(9):
+        to, tg = ob.tree(t), g.tree(t)
+        for key in ("fid", "quantized", "gain", "weights"):
+            assert np.array_equal(to[key], tg[key], equal_nan=True), (key, t)
+    assert np.array_equal(ob.leaf(), g.leaves())
+    assert np.array_equal(ob.yhat(), g.train_yhat())
