@@ -41,6 +41,7 @@ def _load_lib():
         "ADeleteArray": [P(c_float)],
         # extensions (include/arboretum_ext.h)
         "ADeviceCount": [P(c_int)],
+        "AReleaseMemory": [],
         "ADeviceCopyProbe": [ctypes.c_ulonglong],
         "APredictInto": [c_void_p, c_void_p, c_void_p, ctypes.c_ulonglong, c_int],
         "AGetYInto": [c_void_p, c_void_p, c_void_p, ctypes.c_ulonglong],
@@ -92,6 +93,12 @@ def device_count():
     n = ctypes.c_int(0)
     _check(_LIB.ADeviceCount(ctypes.byref(n)))
     return n.value
+
+
+def release_memory():
+    """Gives back the work memory and streams that finished boosters, matrices and predictions have left
+    behind for the next ones (at most 16 GB of device memory); what objects in use hold stays."""
+    _check(_LIB.AReleaseMemory())
 
 
 def copy_probe(nbytes):

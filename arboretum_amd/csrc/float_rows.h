@@ -16,6 +16,9 @@ namespace arb {
 //   - more, no memory there, or no GPU in use by this process yet: host memory, and on the device from
 //     the first OnDevice() on if they fit there (a process that only builds matrices never starts
 //     the GPU, and may fork).
+// Rows on the device are memory of their matrix: they stay until it is freed, and a streamed matrix keeps
+// that much less of its bins resident meanwhile (its own rows never matter: where they fit, its bins, a quarter
+// of their size, do).
 class FloatRows {
  public:
   FloatRows(const float *rows, size_t n, size_t columns);

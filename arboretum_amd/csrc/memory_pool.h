@@ -12,9 +12,11 @@ namespace arb {
 // gives them back when it goes; hipMalloc and hipFree of them cost up to milliseconds (a free waits
 // for the device and unmaps), so blocks given back are kept and handed out again.
 //   - Bounded: at most kDevicePoolBytes of idle blocks per device, the oldest go first.
-//   - Given back to the driver: when a hipMalloc fails (everything idle is freed, then it is tried
+//   - Given back to the driver: when a hipMalloc here fails (everything idle is freed, then it is tried
 //     again), when the bound is passed, when a block has been idle for kPoolIdleSeconds (looked at
-//     on every call), and by DevicePoolTrim().
+//     on every call of the pool, so not while nobody calls it), by DevicePoolTrim() and by TrimPools().
+//     An allocation that fails elsewhere in the process gets nothing back by itself: TrimPools() (AReleaseMemory)
+//     is for a program that needs the memory for something else.
 //   - Safe with several threads and streams: one lock; a block may only be given back when no work
 //     that uses it is pending on any stream.
 // The contents of a block are undefined.
@@ -41,6 +43,9 @@ bool GpuInUse() noexcept;
 // from, whichever one is current when they are given back.
 hipStream_t StreamPoolTake();
 void StreamPoolGive(hipStream_t s) noexcept;  // s may be null
+
+// Frees everything idle in the pools above, on every device.
+void TrimPools() noexcept;
 
 }  // namespace arb
 #endif  // ARBORETUM_AMD_MEMORY_POOL_H_

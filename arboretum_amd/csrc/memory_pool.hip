@@ -86,6 +86,10 @@ class Pool {
     std::lock_guard<std::mutex> lock(mutex_);
     DropAll(device);
   }
+  void TrimAll() noexcept {
+    std::lock_guard<std::mutex> lock(mutex_);
+    while (!idle_.empty()) Drop(idle_.begin());
+  }
 
  private:
   struct Key {
@@ -265,5 +269,19 @@ void *HostPoolTake(size_t bytes) {
   return p;
 }
 void HostPoolGive(void *p) noexcept { HostPool().Give(p); }
+
+void TrimPools() noexcept {
+  HostPool().TrimAll();
+  if (!GpuInUse()) return;  // (what a parent's pools held is not a child's to free)
+  DevicePool().TrimAll();
+  PinnedPool().TrimAll();
+  std::lock_guard<std::mutex> lock(g_streams_mutex);
+  auto &pool = PooledStreams();
+  for (const auto &s : pool.idle) {
+    pool.made_on.erase(s.second);
+    (void)hipStreamDestroy(s.second);
+  }
+  pool.idle.clear();
+}
 
 }  // namespace arb

@@ -13,6 +13,7 @@
 #include "../../include/arboretum_ext.h"
 #include "booster.h"
 #include "hist_sum.h"
+#include "memory_pool.h"
 #include "parallel.h"
 
 using namespace arb;
@@ -200,6 +201,10 @@ const char *ADeleteArray(float *in) {
 // ------------------------------------------------------------- extensions
 const char *ADeviceCount(int *out) {
   return Guard([&] { *out = DeviceCount(); });
+}
+
+const char *AReleaseMemory(void) {
+  return Guard([] { TrimPools(); });
 }
 
 const char *ADeviceCopyProbe(unsigned long long bytes) {

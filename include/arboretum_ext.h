@@ -18,6 +18,12 @@ extern "C" {
 /* Number of HIP devices visible (0 on a CPU-only host). */
 const char *ADeviceCount(int *out);
 
+/* Boosters, matrices and predictions leave work memory (at most 16 GB of device memory, 256 MB of pinned and
+ * 1 GB of ordinary host memory) and streams to the next ones instead of giving them back one by one.  This
+ * gives back all of it that is idle, on every device: for a program that needs the memory elsewhere.  What is
+ * idle for a minute is given back by itself, but only when this library is called again. */
+const char *AReleaseMemory(void);
+
 /* Runs one plain device-to-device copy kernel (k_copy_probe) of `bytes` bytes:
  * a dispatch of exactly known HBM traffic, against which the FETCH_SIZE /
  * WRITE_SIZE counters of a profile are scaled. */

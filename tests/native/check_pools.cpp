@@ -97,9 +97,36 @@ int Bounds() {
   return 0;
 }
 
+// TrimPools gives back everything idle, of every device, and nothing in use.
+int Release() {
+  void *kept[3];
+  hipStream_t stream[3];
+  for (int device = 0; device < 3; ++device) {
+    fake::current = device;
+    kept[device] = arb::DevicePoolTake(1 << 16);
+    stream[device] = arb::StreamPoolTake();
+    arb::DevicePoolGive(arb::DevicePoolTake(1 << 20));
+    arb::PinnedPoolGive(arb::PinnedPoolTake(1 << 20));
+    hipStream_t other = arb::StreamPoolTake();
+    arb::StreamPoolGive(other);
+  }
+  CHECK(fake::blocks.size() == 6 && fake::streams.size() == 6 && fake::pinned.size() == 1);
+  arb::TrimPools();
+  CHECK(fake::blocks.size() == 3 && fake::streams.size() == 3 && fake::pinned.empty());
+  for (int device = 0; device < 3; ++device) {
+    CHECK(fake::blocks.count(kept[device]) && fake::streams.count(stream[device]));
+    arb::DevicePoolGive(kept[device]);
+    arb::StreamPoolGive(stream[device]);
+  }
+  arb::TrimPools();
+  CHECK(fake::blocks.empty() && fake::streams.empty());
+  return 0;
+}
+
 int main(int, char **argv) {
   if (!std::strcmp(argv[1], "other_device")) return OtherDevice();
   if (!std::strcmp(argv[1], "threads")) return Threads();
   if (!std::strcmp(argv[1], "bounds")) return Bounds();
+  if (!std::strcmp(argv[1], "release")) return Release();
   return 2;
 }

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["other_device", "threads", "bounds"])
+@pytest.mark.parametrize("check", ["other_device", "threads", "bounds", "release"])
 def test_pool(program, check):
     r = subprocess.run([program, check], stdout=subprocess.PIPE, timeout=60)
     assert r.returncode == 0, r.stdout.decode()
