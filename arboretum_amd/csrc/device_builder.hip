@@ -840,24 +840,30 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
     if (streamed_) KeepBlocksResident(cfg.internal.stream_resident_bytes);
   }
 
+  template <typename T>
+  T *LaneAlloc(size_t n) {
+    lane_bytes_ += n * sizeof(T);
+    return DevAlloc<T>(n);
+  }
   // The memory of the lane in use; its stream is there.
   void AllocLane() {
+    lane_bytes_ = 0;
     const int max_nodes = 1 << (D_ - 1), last_nodes = 1 << (D_ - 2), internal = max_nodes - 1;
     // ping-pong row buffers in node order (not needed for a single split level)
     if (D_ > 2 && !streamed_) {
       for (int b = 0; b < 2; ++b) {
-        if (indexed_) buf_[b].ids = DevAlloc<unsigned>(n_);
-        else buf_[b].bins = DevAlloc<uint32_t>((size_t)W_ * stride_);
-        buf_[b].g = DevAlloc<float>(n_);
-        buf_[b].h = pack_ ? nullptr : DevAlloc<float>(n_);
+        if (indexed_) buf_[b].ids = LaneAlloc<unsigned>(n_);
+        else buf_[b].bins = LaneAlloc<uint32_t>((size_t)W_ * stride_);
+        buf_[b].g = LaneAlloc<float>(n_);
+        buf_[b].h = pack_ ? nullptr : LaneAlloc<float>(n_);
       }
     }
     for (int b = 0; b < 2; ++b) {
-      d_tot_[b] = DevAlloc<NodeSum>(max_nodes);
-      d_seg_[b] = DevAlloc<unsigned>(max_nodes);
-      d_hg_[b] = DevAlloc<long long>((size_t)last_nodes * nbin_total_);
-      if (pair_) d_hh_[b] = DevAlloc<long long>((size_t)last_nodes * nbin_total_);  // (null without hessians: the kernels leave it out)
-      d_hc_[b] = DevAlloc<unsigned long long>((size_t)last_nodes * nbin_total_);
+      d_tot_[b] = LaneAlloc<NodeSum>(max_nodes);
+      d_seg_[b] = LaneAlloc<unsigned>(max_nodes);
+      d_hg_[b] = LaneAlloc<long long>((size_t)last_nodes * nbin_total_);
+      if (pair_) d_hh_[b] = LaneAlloc<long long>((size_t)last_nodes * nbin_total_);  // (null without hessians: the kernels leave it out)
+      d_hc_[b] = LaneAlloc<unsigned long long>((size_t)last_nodes * nbin_total_);
       // cells of bins that no row can have are never written (rows in place with fewer than 256
       // bins in use) and must read as zero
       if (indexed_ && rec_one_launch_ && rec_slots_ < kSlots) {
@@ -866,25 +872,25 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
         HIP_OK(hipMemsetAsync(d_hc_[b], 0, (size_t)last_nodes * nbin_total_ * sizeof(unsigned long long), stream_));
       }
     }
-    d_split_ = DevAlloc<SplitRec>(last_nodes);
-    d_cand_ = DevAlloc<Cand>((size_t)last_nodes * F_);
+    d_split_ = LaneAlloc<SplitRec>(last_nodes);
+    d_cand_ = LaneAlloc<Cand>((size_t)last_nodes * F_);
     // two sets of (first item, items) per node: a slab reduction reads the plan of the pass before it
     // while it writes the plan of the pass after it
-    d_node_first2_ = DevAlloc<unsigned>((size_t)2 * last_nodes);
-    d_node_items2_ = DevAlloc<unsigned>((size_t)2 * last_nodes);
+    d_node_first2_ = LaneAlloc<unsigned>((size_t)2 * last_nodes);
+    d_node_items2_ = LaneAlloc<unsigned>((size_t)2 * last_nodes);
     d_node_first_ = d_node_first2_;
     d_node_items_ = d_node_items2_;
-    d_hwork_ = DevAlloc<WorkItem>(max_hist_items_);
-    d_pwork_ = DevAlloc<WorkItem>(max_part_items_);
-    d_nwork_ = DevAlloc<unsigned>(2);
-    d_wave_left_ = DevAlloc<unsigned>((size_t)max_part_items_ * kItemWaves);
-    d_item_left_ = DevAlloc<unsigned>((size_t)2 * max_part_items_);  // also the claimed bases of the fused pass
-    d_cursor2_ = DevAlloc<unsigned>((size_t)2 * last_nodes);
-    d_slab_ = DevAlloc<unsigned long long>((size_t)max_hist_items_ * slab_stride_ * (pair_ ? 2 : 1));
-    d_tfid_ = DevAlloc<int>(internal);
-    d_tbin_ = DevAlloc<int>(internal);
-    d_tgain_ = DevAlloc<float>(internal);
-    d_weights_ = DevAlloc<float>(max_nodes);
+    d_hwork_ = LaneAlloc<WorkItem>(max_hist_items_);
+    d_pwork_ = LaneAlloc<WorkItem>(max_part_items_);
+    d_nwork_ = LaneAlloc<unsigned>(2);
+    d_wave_left_ = LaneAlloc<unsigned>((size_t)max_part_items_ * kItemWaves);
+    d_item_left_ = LaneAlloc<unsigned>((size_t)2 * max_part_items_);  // also the claimed bases of the fused pass
+    d_cursor2_ = LaneAlloc<unsigned>((size_t)2 * last_nodes);
+    d_slab_ = LaneAlloc<unsigned long long>((size_t)max_hist_items_ * slab_stride_ * (pair_ ? 2 : 1));
+    d_tfid_ = LaneAlloc<int>(internal);
+    d_tbin_ = LaneAlloc<int>(internal);
+    d_tgain_ = LaneAlloc<float>(internal);
+    d_weights_ = LaneAlloc<float>(max_nodes);
   }
   void ReleaseLane() noexcept {
     if (stream_) (void)hipStreamSynchronize(stream_);
@@ -908,12 +914,19 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   // 23.9 ms on one stream, 19.4 on two, 19.2 on three, 20.2 on four; 20,000 x 20, three classes: 5.4, 5.2,
   // 3.6, 4.1; 6 M x 20, four classes: 18.9, 19.0, 17.0, 17.2.
   static constexpr size_t kLanes = 3;
-  static constexpr size_t kLaneRows = (size_t)8 << 20;  // (beyond, the kernels fill the chip, and the memory counts)
+  // One stream beyond kLaneRows rows (the kernels fill the chip) and with sampled columns: the sampler copies its
+  // masks on the stream of the trees, and the gain is not there at a colsample_bytree or colsample_bylevel below 1.
+  static constexpr size_t kLaneRows = (size_t)8 << 20;
+  // What the lanes beside the first may take together: deep trees over wide matrices need gigabytes of
+  // histograms and slabs a lane (200 features of 256 bins, max_depth 10: 3 GB).
+  static constexpr size_t kOtherLanesBytes = (size_t)8 << 30;
   void MakeOtherLanes() {
     if (K_ < 2 || streamed_ || n_ > kLaneRows || sampler_.Samples()) return;
     HIP_OK(hipEventCreateWithFlags(&round_start_, hipEventDisableTiming));
     other_lanes_.reserve(kLanes);
-    while (other_lanes_.size() + 1 < std::min(kLanes, (size_t)K_)) {
+    const size_t lane_bytes = lane_bytes_;
+    while (other_lanes_.size() + 1 < std::min(kLanes, (size_t)K_) &&
+           (other_lanes_.size() + 1) * lane_bytes <= kOtherLanesBytes) {
       Lane lane;
       std::swap(static_cast<Lane &>(*this), lane);
       bool made = true;
@@ -2056,6 +2069,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   unsigned part_rows_ = kPartRows;  // rows per work item of a stand-alone partition
   unsigned long long *d_rows_scanned_ = nullptr;
   int *d_shifts_ = nullptr;
+  size_t lane_bytes_ = 0;          // device memory of one lane
   std::vector<Lane> other_lanes_;  // (the members inherited from Lane are the lane in use)
   hipEvent_t round_start_ = nullptr;
   std::vector<std::vector<int64_t>> kept_hist_;

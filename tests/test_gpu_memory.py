@@ -45,3 +45,33 @@ def test_release_memory(arb):
     arb.release_memory()
     assert free_device_bytes() > before - 16 * MB
     assert np.array_equal(use(), first)
+
+
+def _softmax_bytes(arb, F, depth, column_share):
+    """Device memory of a soft-max booster of four classes over F features of 256 bins."""
+    n, K = 3000, 4
+    rng = np.random.default_rng(F)
+    X = rng.integers(0, 256, size=(n, F), dtype=np.uint8)
+    labels = ((X[:, 0] > 100).astype(np.uint8) + 2 * (X[:, F - 1] > 60)).astype(np.uint8)
+    cfg = _config(depth, bins=256, labels_count=K, colsample_bytree=column_share)
+    cfg["objective"] = 4
+    data = arb.DMatrix(X, labels=labels, quantized=True)
+    data.quantize(256)
+    arb.train(dict(cfg, tree=dict(cfg["tree"], max_depth=1)), data, 1).synchronize()   # (records of the rows)
+    gc.collect()
+    arb.release_memory()
+    before = free_device_bytes()
+    g = arb.Garden(cfg, data)
+    g.labels_count = K
+    g.grow_tree()
+    g.synchronize()
+    return before - free_device_bytes()
+
+
+# lanes beside the first take 8 GB at most together: two more of 3 GB, one more of 6 GB, none of 10 GB
+@pytest.mark.parametrize("F,others", [(200, 2), (400, 1), (640, 0)])
+def test_lanes_of_a_wide_deep_softmax_are_bounded(arb, F, others):
+    one = _softmax_bytes(arb, F, 10, 1.0 - 0.5 / F)   # sampled columns: one lane
+    used = _softmax_bytes(arb, F, 10, 1.0)
+    assert used - one < 8 * 1024 * MB
+    assert abs(used - (1 + others) * one) < 0.1 * one, (used, one)
