@@ -224,7 +224,7 @@ void Garden::Predict(const DataMatrix *data, float *out, int n_rounds) const {
   SyncTrees();
   const long long use = std::min<long long>(n_rounds, (long long)trees_.size());
   const float init = IntoInternal(cfg.tree.initial_y);
-  if (use > 0 && WalksOnDevice(data)) {
+  if (use > 0 && WalksOnDevice(data) && DeviceWalkFits(*data, trees_, 0, (size_t)use)) {
     std::lock_guard<std::mutex> lock(predictor_mutex_);
     if (!predictor_) predictor_.reset(CreateDevicePredictor());
     const float *sums = PredictOnDevice(predictor_.get(), *data, trees_, 0, (size_t)use, K, init);
@@ -246,6 +246,9 @@ void Garden::Predict(const DataMatrix *data, float *out, int n_rounds) const {
   FromInternal(tmp.data(), tmp.size(), out);
 }
 
+// Floats of pinned memory AppendLastTree takes for its sums (128 MB).
+constexpr size_t kSumsAtOnce = (size_t)32 << 20;
+
 void Garden::UpdateByLastTree(DataMatrix *data) {
   const size_t K = cfg.tree.labels_count;
   if (!data->HasYHat()) data->ResetYHat(data->rows * K, IntoInternal(cfg.tree.initial_y));
@@ -255,17 +258,28 @@ void Garden::UpdateByLastTree(DataMatrix *data) {
   // (a matrix may carry the predictions of a booster of more classes, or of fewer: the classes both
   // have are advanced)
   const size_t classes = data->rows ? std::min(K, y_hat.size() / data->rows) : 0;
-  if (WalksOnDevice(data)) {
+  const size_t n = data->rows, first = trees_.size() - K;
+  // (matrices without dense columns and of 2^31 rows are the host's, as before there was a walk on the GPU here)
+  const bool blocks = data->InBlocks();
+  if (WalksOnDevice(data) && data->columns_dense > 0 && (n < (1ull << 31) || blocks) &&
+      DeviceWalkFits(*data, trees_, first, trees_.size())) {
     // (a predictor of its own: the other one keeps the whole model laid out)
     std::lock_guard<std::mutex> lock(predictor_mutex_);
     if (!round_predictor_) round_predictor_.reset(CreateDevicePredictor());
-    const float *sums = PredictOnDevice(round_predictor_.get(), *data, trees_, trees_.size() - K, trees_.size(), K, 0.0f);
-    ParallelFor(classes * data->rows, [&](size_t b, size_t e) {
-      for (size_t i = b; i < e; ++i) y_hat[i] += sums[i];
-    });
+    // a range of rows at a time: the sums come back in pinned memory
+    size_t step = std::max<size_t>(kSumsAtOnce / K, 1);
+    if (blocks) step = std::max<size_t>(step / data->stream_block_rows, 1) * data->stream_block_rows;
+    for (size_t r0 = 0; r0 < n; r0 += step) {
+      const size_t m = std::min(step, n - r0);
+      const float *sums = PredictOnDevice(round_predictor_.get(), *data, trees_, first, trees_.size(), K, 0.0f, r0, r0 + m);
+      for (size_t k = 0; k < classes; ++k)
+        ParallelFor(m, [&](size_t b, size_t e) {
+          for (size_t i = b; i < e; ++i) y_hat[k * n + r0 + i] += sums[k * m + i];
+        });
+    }
     return;
   }
-  for (size_t t = trees_.size() - K; t < trees_.size(); ++t)
+  for (size_t t = first; t < trees_.size(); ++t)
     if (trees_[t].label < classes) trees_[t].Predict(*data, y_hat.data());
 }
 

@@ -82,6 +82,8 @@ class DataMatrix {
   size_t stream_block_rows = 0;
   // The blocks belong to the caller (ACreateFromQuantizedBlocks): never copied, never freed.
   bool external_blocks = false;
+  // The bin ids are in those blocks and nowhere else.
+  bool InBlocks() const { return is_prebinned && prebinned.empty() && !stream_blocks.empty(); }
 
   // Feature value of a pre-quantised matrix as seen by host prediction.
   inline float BinValue(size_t f, size_t i) const {
@@ -180,13 +182,18 @@ void CopyProbe(size_t bytes);
 // predictor.hip: tree walks of a matrix (floats or bin ids) on the GPU.  Returns [labels][rows]
 // sums of leaf weights of trees[begin, end) on top of `init`, bit-identical to the
 // host walk (RegTree::Predict in tree order), in pinned host memory that the
-// predictor owns and overwrites on its next call.  One predictor serves one vector of trees,
+// predictor owns and overwrites on its next call.  `rows`: those of [row_begin, row_end), all by default; of a
+// streamed matrix a range starts at a block.  One predictor serves one vector of trees,
 // which only grows.
 struct DevicePredictor;
 DevicePredictor *CreateDevicePredictor();
 void FreeDevicePredictor(DevicePredictor *p);
 const float *PredictOnDevice(DevicePredictor *p, const DataMatrix &data, const std::vector<RegTree> &trees,
-                             size_t begin, size_t end, size_t labels, float init);
+                             size_t begin, size_t end, size_t labels, float init, size_t row_begin = 0,
+                             size_t row_end = SIZE_MAX);
+// False for what only the host walks: 2 GB of trees and more, and rows on the host of which not even one fits a
+// staging block (a million features).
+bool DeviceWalkFits(const DataMatrix &data, const std::vector<RegTree> &trees, size_t begin, size_t end);
 
 class Garden {
  public:

@@ -36,12 +36,15 @@ constexpr size_t kTreeLds = 40 * 1024;            // trees staged at a time when
 constexpr unsigned kAhead = 5;                    // words per thread fetched while the chunk before is walked
 constexpr unsigned kChains = 4;                   // trees a thread walks side by side
 constexpr size_t kBlockBytes = (size_t)32 << 20;  // device block of rows that are not kept on the device
+constexpr size_t kMostModelBytes = (size_t)1 << 31;  // (trees are addressed by 32-bit byte offsets)
 
 // A tree as 8-byte words: its 2^(depth-1) - 1 nodes (feature, threshold bits) in heap order, then its
 // 2^(depth-1) leaf weights, two to a word.
 struct TreeRef {
   unsigned off, depth, label, unused;
 };
+
+size_t TreeWords(const RegTree &t) { return t.fid.size() + t.weights.size() / 2; }
 
 // Where a row's feature values come from.
 enum Source {
@@ -331,10 +334,10 @@ struct DevicePredictor {
     depth = trees[b].depth;
     bool same = true;
     for (unsigned t : order) {
-      const size_t w = trees[t].fid.size() + trees[t].weights.size() / 2;
+      const size_t w = TreeWords(trees[t]);
       refs.push_back(TreeRef{(unsigned)words, trees[t].depth, trees[t].label, 0u});
       words += w;
-      if (words * sizeof(uint2) >= (1ull << 31)) throw std::runtime_error("model too large for device prediction");
+      if (words * sizeof(uint2) >= kMostModelBytes) throw std::runtime_error("model too large for device prediction");
       largest = std::max(largest, (unsigned)w);
       same = same && trees[t].depth == depth;
     }
@@ -442,11 +445,11 @@ struct DevicePredictor {
   }
 
   const float *Run(const DataMatrix &data, const std::vector<RegTree> &trees, size_t first, size_t use, size_t labels,
-                   float init) {
-    const size_t n = data.rows, F = data.columns_dense;
+                   float init, size_t row_begin, size_t row_end) {
+    const size_t n = std::min(row_end, data.rows) - row_begin, F = data.columns_dense;
     if (n == 0 || F == 0) throw std::runtime_error("empty data matrix");
     // only the block-wise walk of a streamed matrix indexes rows with 64 bits
-    const bool blocks = data.is_prebinned && data.prebinned.empty() && !data.stream_blocks.empty();
+    const bool blocks = data.InBlocks();
     if (n >= (1ull << 31) && !blocks) throw std::runtime_error("too many rows");
     if (data.is_prebinned && data.prebinned.empty() && !blocks) throw std::runtime_error("pre-quantised matrix without bins");
     if (!stream) stream = StreamPoolTake();
@@ -488,18 +491,19 @@ struct DevicePredictor {
       HIP_OK(hipStreamSynchronize(stream));
     };
     if (!data.is_prebinned) {
-      if (const float *rows = data.values->OnDevice()) Rows(kFloatRows, rows, 0, n, F, labels, init, result, n);
-      else through_block(kFloatRows, data.values->OnHost(), F * sizeof(float));
+      if (const float *rows = data.values->OnDevice()) Rows(kFloatRows, rows + row_begin * F, 0, n, F, labels, init, result, n);
+      else through_block(kFloatRows, data.values->OnHost() + row_begin * F, F * sizeof(float));
     } else if (!blocks) {
-      through_block(kByteRows, data.prebinned.data(), F);
+      through_block(kByteRows, data.prebinned.data() + row_begin * F, F);
     } else {
       // streamed matrix: its pinned blocks of quad columns go up as they are
       const size_t br = data.stream_block_rows, Q = (F + 3) / 4;
+      if (row_begin % br != 0) throw std::runtime_error("internal: a range of rows starts inside a block");
       void *block = DevicePoolTake(Q * br * sizeof(uint32_t));
       try {
-        for (size_t b = 0; b < data.stream_blocks.size() && b * br < n; ++b) {
+        for (size_t b = 0; b * br < n; ++b) {
           const size_t r0 = b * br;
-          HIP_OK(hipMemcpyAsync(block, data.stream_blocks[b], Q * br * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+          HIP_OK(hipMemcpyAsync(block, data.stream_blocks[row_begin / br + b], Q * br * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
           Rows(kQuadCols, block, br, std::min(br, n - r0), F, labels, init, result + r0, n);
         }
         HIP_OK(hipStreamSynchronize(stream));
@@ -518,8 +522,17 @@ struct DevicePredictor {
 DevicePredictor *CreateDevicePredictor() { return new DevicePredictor(); }
 void FreeDevicePredictor(DevicePredictor *p) { delete p; }
 const float *PredictOnDevice(DevicePredictor *p, const DataMatrix &data, const std::vector<RegTree> &trees,
-                             size_t begin, size_t end, size_t labels, float init) {
-  return p->Run(data, trees, begin, end, labels, init);
+                             size_t begin, size_t end, size_t labels, float init, size_t row_begin, size_t row_end) {
+  return p->Run(data, trees, begin, end, labels, init, row_begin, row_end);
+}
+
+bool DeviceWalkFits(const DataMatrix &data, const std::vector<RegTree> &trees, size_t begin, size_t end) {
+  size_t bytes = 0;
+  for (size_t t = begin; t < end; ++t) bytes += TreeWords(trees[t]) * sizeof(uint2);
+  if (bytes >= kMostModelBytes) return false;
+  const size_t F = data.columns_dense;
+  if (!data.is_prebinned) return F * sizeof(float) <= kStageBytes || data.values->OnDevice() != nullptr;
+  return data.InBlocks() || F <= kStageBytes;
 }
 
 }  // namespace arb
