@@ -1538,9 +1538,12 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
             if (part_rows_ <= kChunkStep) {
               if (pair_) ARB_IX(k_ix_part_small<true>);
               else ARB_IX(k_ix_part_small<false>);
+            } else if (plan.cand) {
+              if (pair_) ARB_IX((k_ix_part<true, true>));
+              else ARB_IX((k_ix_part<false, true>));
             } else {
-              if (pair_) ARB_IX(k_ix_part<true>);
-              else ARB_IX(k_ix_part<false>);
+              if (pair_) ARB_IX((k_ix_part<true, false>));
+              else ARB_IX((k_ix_part<false, false>));
             }
 #undef ARB_IX
           } else if (part_rows_ <= kChunkStep) {
@@ -1553,8 +1556,12 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
                                  W_, src.g, dst.g, src.h, dst.h, d_split_, d_seg_[ps], d_pwork_, d_nwork_ + 1, d_cursor2_,
                                  d_item_left_, code_, hi_word_, plan);
           } else {
-            hipLaunchKernelGGL(k_part_count, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, stride_, d_split_,
-                               d_pwork_, d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_, plan);
+#define ARB_COUNT(S)                                                                                                  \
+  hipLaunchKernelGGL(k_part_count<S>, dim3(grid), dim3(kHistThreads), 0, stream_, src.bins, stride_, d_split_, d_pwork_, \
+                     d_nwork_ + 1, d_wave_left_, d_item_left_, code_, hi_word_, plan)
+            if (plan.cand) ARB_COUNT(true);
+            else ARB_COUNT(false);
+#undef ARB_COUNT
             LaunchPartRows(items, src, dst, ps);
           }
           HistOfNodes(dst, L, false);  // (planned with the splits of the level above)
@@ -1712,8 +1719,15 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
 #undef ARB_SCAN
   }
 
-  // Levels whose splits are selected, and whose children's histograms are planned, by the partition.
-  bool SelectInPartition(int L) const { return !fused_ && !streamed_ && L <= kSelectPlanNodes; }
+  // Levels whose splits are selected, and whose children's histograms are planned, by the partition: those of few
+  // nodes, while its work items fit two rounds of the chip (two workgroups per CU).  Every workgroup selects
+  // before it moves a row, so each further round pays again, and a launch of its own costs the same
+  // however many there are.  Per tree with / without: 2 M rows x 200 features, max_depth 10: 1.43 / 1.47 ms, 12 M x 48, 8:
+  // 2.92 / 3.01, 10.5 M x 200, 10: 4.40 / 4.46, 16 M x 200: 6.20 / 6.20, 24 M x 200: 8.96 / 8.90, 20 M x 100, 6: 4.70 / 4.67,
+  // 50 M x 200: 18.1 / 17.8 (the partition alone 4.26 / 3.76).
+  bool SelectInPartition(int L) const {
+    return !fused_ && !streamed_ && L <= kSelectPlanNodes && n_ / part_rows_ <= 4 * (size_t)cus_;
+  }
   SelectPlan PlanOfPartition(int level, int L, int state) {
     SelectPlan p;
     p.cand = d_cand_;

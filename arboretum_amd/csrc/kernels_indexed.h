@@ -135,7 +135,7 @@ k_sum_grad(const float *__restrict__ g, const float *__restrict__ h, int packed,
 // right exactly the rows whose id is 256.
 constexpr int kIxChunks = (int)(kPartRows / kChunkStep);  // chunks of a wave in one work item
 static_assert(kIxChunks * 2 <= 32, "a lane's decisions of one work item must fit one register");
-template <bool PAIR>
+template <bool PAIR, bool SELECT>
 __global__ void __launch_bounds__(kHistThreads)
 k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__restrict__ ids,
           unsigned *__restrict__ ids_out, const float *__restrict__ g, float *__restrict__ g_out,
@@ -144,15 +144,14 @@ k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__r
           const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor, unsigned *__restrict__ item_base,
           const uint8_t *__restrict__ hibits, size_t strideb, const SelectPlan plan) {
   __shared__ unsigned s_tmp[kItemWaves + 2];
-  __shared__ SplitRec s_rec;
   unsigned w = blockIdx.x;
-  if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
+  if (SELECT && plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
     SelectAndPlan(plan);
     return;
   }
   if (w >= *n_work) return;
   const WorkItem it = work[w];
-  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  const SplitRec s = SELECT ? SplitOf(plan, (int)it.node, split) : split[it.node];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned wb = ChunkOrigin(it) + wave * kChunkRows, we = it.end;
   const bool by_bit = hibits != nullptr && s.bin >= 255;  // uniform: only an id of 256 goes right
@@ -244,7 +243,6 @@ k_ix_part_small(const uint8_t *__restrict__ bytes, size_t stride8, const unsigne
                 const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor, unsigned *__restrict__ item_base,
                 const uint8_t *__restrict__ hibits, size_t strideb, const SelectPlan plan) {
   __shared__ unsigned s_tmp[kItemWaves + 2];
-  __shared__ SplitRec s_rec;
   unsigned w = blockIdx.x;
   if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
     SelectAndPlan(plan);
@@ -259,7 +257,7 @@ k_ix_part_small(const uint8_t *__restrict__ bytes, size_t stride8, const unsigne
   const unsigned id0 = ids ? ids[a0] : a0, id1 = ids ? ids[a1] : a1;
   const float g0 = g[a0], g1 = g[a1];
   const float h0 = PAIR ? h[a0] : 0.0f, h1 = PAIR ? h[a1] : 0.0f;
-  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  const SplitRec s = SplitOf(plan, (int)it.node, split);
   bool right0 = false, right1 = false;
   if (s.fid >= 0) {  // uniform
     if (hibits != nullptr && s.bin >= 255) {  // only an id of 256 goes right

@@ -30,20 +30,20 @@ __device__ __forceinline__ bool GoesRight(const uint32_t *__restrict__ bins, siz
 __device__ __forceinline__ unsigned ChunkOrigin(const WorkItem &it) { return it.begin & ~63u; }
 
 // Rows going left, per (work item, wave range).
+template <bool SELECT>
 __global__ void __launch_bounds__(kHistThreads)
 k_part_count(const uint32_t *__restrict__ bins, size_t stride, const SplitRec *__restrict__ split,
              const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work,
              unsigned *__restrict__ wave_left, unsigned *__restrict__ item_left, BinCode code, int hi_word,
              const SelectPlan plan) {
-  __shared__ SplitRec s_rec;
   unsigned w = blockIdx.x;
-  if (plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
+  if (SELECT && plan.cand != nullptr && w-- == 0) {  // (the first block: it takes longest)
     SelectAndPlan(plan);
     return;
   }
   if (w >= *n_work) return;
   const WorkItem it = work[w];
-  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  const SplitRec s = SELECT ? SplitOf(plan, (int)it.node, split) : split[it.node];
   const SplitTest test = MakeSplitTest(s, code, hi_word);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned cnt = 0;
@@ -796,7 +796,6 @@ k_part_small(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out,
              const WorkItem *__restrict__ work, const unsigned *__restrict__ n_work, unsigned *__restrict__ cursor,
              unsigned *__restrict__ item_base, BinCode code, int hi_word, const SelectPlan plan) {
   __shared__ unsigned s_tmp[kItemWaves + 2];
-  __shared__ SplitRec s_rec;
   unsigned w = blockIdx.x;
   if (plan.cand != nullptr && w-- == 0) {
     SelectAndPlan(plan);
@@ -821,7 +820,7 @@ k_part_small(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out,
   load(0);
   const float g0 = g[a0], g1 = g[a1];
   const float h0 = PAIR ? h[a0] : 0.0f, h1 = PAIR ? h[a1] : 0.0f;
-  const SplitRec s = SplitOf(plan, (int)it.node, split, &s_rec);
+  const SplitRec s = SplitOf(plan, (int)it.node, split);
   const SplitTest test = MakeSplitTest(s, code, hi_word);
   const uint32_t *col = bins + (size_t)test.word * stride;
   const bool right0 = test.Right(col[a0]), right1 = test.Right(col[a1]);

@@ -495,8 +495,11 @@ k_split_select(const Cand *__restrict__ cand, int F, int L, const NodeSum *__res
 // follows the split scan on the paths with stand-alone histogram launches: every workgroup selects for
 // its own node (SplitOf), and one more block of the grid (the first one) selects for all of them, writes
 // their records and plans (SelectAndPlan; `select`, balance_cus: PlanBody's).  A launch of its own
-// stood between scan and partition for 6.5 us a level, and the partition takes 3 us longer for it.  One workgroup
-// does it beside the partition while the level has few nodes: cand == null, the splits have been selected by k_split_select.
+// stood between scan and partition for 6.5 us a level, and the partition takes 3 us longer for it while its work items fit
+// two rounds of the chip.  One workgroup does it beside the partition while the level has few nodes.  cand == null: the splits
+// have been selected by k_split_select (HipTreeBuilder::SelectInPartition); the kernels of large items have an instance for
+// that (SELECT = false) without the planner's 16 KB of LDS and a third of the scalar registers: 50 M x 200, max_depth
+// 10: 3.76 ms a tree, 4.11 by the other one.
 struct SelectPlan {
   const Cand *cand = nullptr;
   int F = 0, L = 0;
@@ -527,14 +530,15 @@ __device__ __forceinline__ void SelectAndPlan(const SelectPlan &a) {
   PlanBody(a.tot_next, a.seg_next, 2 * a.L, a.select, a.rows_per_item, a.work, a.n_work, a.node_first, a.node_items,
            a.rows_scanned, nullptr, a.max_items, a.overflow, nullptr, a.balance_cus);
 }
-// Called by all threads of the workgroup; s_rec holds one record.
-__device__ __forceinline__ SplitRec SplitOf(const SelectPlan &a, int nd, const SplitRec *__restrict__ split, SplitRec *s_rec) {
+// Called by all threads of the workgroup.
+__device__ __forceinline__ SplitRec SplitOf(const SelectPlan &a, int nd, const SplitRec *__restrict__ split) {
   if (a.cand == nullptr) return split[nd];  // uniform
+  __shared__ SplitRec s_rec;
   LevelScan scan{};
   scan.cand = a.cand;
   scan.F = a.F;
   scan.active = a.active;
-  return SelectInPass(scan, nd, a.tot[nd], a.seg_start, false, s_rec);
+  return SelectInPass(scan, nd, a.tot[nd], a.seg_start, false, &s_rec);
 }
 
 }  // namespace
