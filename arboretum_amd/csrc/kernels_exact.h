@@ -15,6 +15,7 @@
 #ifndef ARBORETUM_AMD_KERNELS_EXACT_H_
 #define ARBORETUM_AMD_KERNELS_EXACT_H_
 #include "device_common.h"
+#include "exact_filter.h"
 #include "gain.h"
 #include "kernels_split.h"
 
@@ -166,64 +167,8 @@ k_ex_offsets(const T *__restrict__ part, T *__restrict__ off, const unsigned *__
   }
 }
 
-// SplitGain (gain.h) with the parent's term, which is the same at every place of a node, taken
-// from the caller: `parent` = SideGain of the node's totals at their leaf weight.  The same
-// operations in the same order, so the same bits.
-template <bool PAIR, bool F64>
-__device__ __forceinline__ float ExParentGain(double gt, double ht, unsigned long long ct, const GainParams &p) {
-  return SideGain<PAIR, F64>(gt, ht, ct, LeafWeight<PAIR, F64>(gt, ht, ct, p), p);
-}
-template <bool PAIR, bool F64>
-__device__ __forceinline__ float ExSplitGain(double gl, double hl, unsigned long long cl, double gt, double ht,
-                                             unsigned long long ct, const GainParams &p, float parent) {
-  const unsigned long long cr = ct - cl;
-  double gr, hr;
-  if (F64) {
-    gr = gt - gl;
-    hr = ht - hl;
-  } else {
-    gr = (double)((float)gt - (float)gl);
-    hr = (double)((float)ht - (float)hl);
-  }
-  if (cl < p.min_leaf_size || cr < p.min_leaf_size) return 0.0f;
-  if (PAIR) {
-    if (F64) {
-      if (!(fabs(hl) >= (double)p.min_child_weight && fabs(hr) >= (double)p.min_child_weight)) return 0.0f;
-    } else {
-      if (!(fabsf((float)hl) >= p.min_child_weight && fabsf((float)hr) >= p.min_child_weight)) return 0.0f;
-    }
-  }
-  const float l = SideGain<PAIR, F64>(gl, hl, cl, LeafWeight<PAIR, F64>(gl, hl, cl, p), p);
-  const float r = SideGain<PAIR, F64>(gr, hr, cr, LeafWeight<PAIR, F64>(gr, hr, cr, p), p);
-  const float diff = l + r - parent;
-  return (float)(diff > p.gamma_absolute && diff > p.gamma_relative * parent) * diff;
-}
-
 __device__ __forceinline__ bool ExBetter(float og, int ob, float gain, int bin) {
   return ob >= 0 && (bin < 0 || og > gain || (og == gain && ob > bin));
-}
-
-// The sum of the two sides' gains at a place, S_l^2 / D_l + S_r^2 / D_r with S the sum of a side and D its hessian (or
-// count) + lambda: what ExSplitGain computes, but for the parent's term, when there is no alpha and no bound on the weights, and
-// within 1e-6 of itself.  Here within 5e-7, on the same operands, in a sixth of the instructions: no double-precision division.
-// Not finite, or negative for a place that has no gain by the limits on leaves.
-template <bool PAIR, bool F64>
-__device__ __forceinline__ float ExSides(double gl, double hl, unsigned long long cl, double gt, double ht,
-                                         unsigned long long ct, const GainParams &p) {
-  const unsigned long long cr = ct - cl;
-  const double gr = F64 ? gt - gl : (double)((float)gt - (float)gl);
-  double hr = F64 ? ht - hl : (double)((float)ht - (float)hl);
-  bool none = cl < p.min_leaf_size || cr < p.min_leaf_size;
-  if (PAIR) none = none || !(fabs(hl) >= (double)p.min_child_weight && fabs(hr) >= (double)p.min_child_weight);
-  if (!PAIR) {
-    hl = (double)(float)cl;
-    hr = (double)(float)cr;
-  }
-  const double dl = hl + (double)p.lambda, dr = hr + (double)p.lambda;
-  const float v = (float)(gl * gl * dr + gr * gr * dl) * __builtin_amdgcn_rcpf((float)(dl * dr));
-  // (LeafWeight: such a side has the weight 0)
-  const bool zero = !(hl >= (double)p.min_child_weight && hr >= (double)p.min_child_weight) || !(dl > 0.0 && dr > 0.0);
-  return none ? -1.0f : zero ? INFINITY : v;
 }
 
 // grid (items, F): running sums along every work item's piece of every list (on top of `off`, the
@@ -232,7 +177,7 @@ __device__ __forceinline__ float ExSides(double gl, double hl, unsigned long lon
 // best: [F][max_items].
 // What bounds it: the gains in double precision (21 of 50 us a level at 400,000 rows x 20), then the latency of a
 // chain of loads, scan and barriers, hidden by the workgroups of a CU.  Only the best place of a wave counts, so the
-// gains are computed where ExSides comes within 4e-6 of the wave's largest: usually at one place or two of 512
+// gains are computed where ExSides comes near the wave's largest (ExLeastSides): usually at one place or two of 512
 // (43 us; with fewer registers, six waves per SIMD, they spill: 76).
 template <bool PAIR, bool F64, bool PACK>
 __global__ void __launch_bounds__(kExThreads)
@@ -294,7 +239,7 @@ k_ex_scan(const ExLists ls, size_t stride, const int *__restrict__ shifts,
   const double GT = FromFixed<F64>(t.g, sg);
   const double HT = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
   const float parent = ExParentGain<PAIR, F64>(GT, HT, t.c, gp);
-  const bool prune = gp.alpha == 0.0f && gp.max_leaf_weight == 0.0f && gp.lambda >= 0.0f;
+  const bool prune = ExPrunes<PAIR>(HT, t.c, gp);
   // the places worth a look: bit j
   unsigned look = 0;
   float sides[kExPer], most = 0.0f;
@@ -308,13 +253,12 @@ k_ex_scan(const ExLists ls, size_t stride, const int *__restrict__ shifts,
     if (p < it.end && p + 1 < node_end && rk[j] != rk[j + 1]) look |= 1u << j;
     if (prune)  // uniform
       sides[j] = ExSides<PAIR, F64>(FromFixed<F64>(g_at, sg), PAIR ? FromFixed<F64>(h_at, sh) : 0.0, p - node_start + 1, GT,
-                                    HT, t.c, gp);
-    if (((look >> j) & 1u) && sides[j] <= 3.0e38f) most = fmaxf(most, sides[j]);
+                                    HT, t.c, gp, [](float x) { return __builtin_amdgcn_rcpf(x); });
+    if (((look >> j) & 1u) && sides[j] <= kExMostSides) most = fmaxf(most, sides[j]);
   }
   if (prune) {
     for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
-    // (near the smallest floats nothing is within 4e-6)
-    const float least = most < 1e-30f ? 0.0f : most * (1.0f - 4e-6f);
+    const float least = ExLeastSides<PAIR>(most);
 #pragma unroll
     for (int j = 0; j < kExPer; ++j)
       if (sides[j] < least) look &= ~(1u << j);  // (not finite: looked at)
