@@ -1,6 +1,6 @@
 // GPU tree builder for gfx950 (MI355X): quantised bins resident in HBM, one
-// stream, O(1) kernel launches per tree level and no host synchronisation
-// inside a tree.
+// stream per tree (the trees of a soft-max round on up to three), O(1) kernel
+// launches per tree level and no host synchronisation inside a tree.
 //
 // Data layout.  Bins are uint8, four features packed in one uint32 ("quad"),
 // stored quad-column-major: quad q of row r is bins[q * stride + r].  Every
@@ -29,7 +29,8 @@
 //   k_bin_assign      build_histogram              src/io/io.cu:293-312
 //                     (thresholds: quantiser.hip)
 //   k_grad_*          update_grad                  src/core/objective.cu:15-56
-//   k_root_from_hist  cub::DeviceReduce::Sum       src/core/garden.cu:432-435
+//   root totals (k_final_hist, the root's k_split_scan, k_sum_grad)
+//                     cub::DeviceReduce::Sum       src/core/garden.cu:432-435
 //   k_hist            hist_sum_node / hist_sum_multi_node
 //                                                  src/core/hist_grad_sum.cu:109-215,262-406
 //   k_hist_reduce     update_multi_node + global atomics
@@ -1218,12 +1219,10 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   unsigned long long *ScanCounter(int level) { return d_rows_scanned_ + std::min(level, kScanLevels - 1); }
   // count_level >= 0: the planned rows are histogram work of that tree level
   void PlanOn(const NodeSum *tot, const unsigned *seg, int L, int select, unsigned rows_per_item, WorkItem *work,
-              unsigned *n_work, int count_level, const SplitRec *split, unsigned max_items,
-              unsigned balance_cus = 0, unsigned *cursor = nullptr) {
+              unsigned *n_work, int count_level, unsigned max_items, unsigned balance_cus = 0) {
     hipLaunchKernelGGL(k_plan, dim3(1), dim3(1024), 0, stream_, tot, seg, L, select,
                        rows_per_item, work, n_work, d_node_first_, d_node_items_,
-                       count_level >= 0 ? ScanCounter(count_level) : (unsigned long long *)nullptr, split, max_items,
-                       d_overflow_, balance_cus, cursor);
+                       count_level >= 0 ? ScanCounter(count_level) : (unsigned long long *)nullptr, max_items, d_overflow_, balance_cus);
   }
 
   // ---- plans of stand-alone histogram launches.
@@ -1766,7 +1765,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
                        fused_ && !streamed_ ? ScanCounter(level + 1) : (unsigned long long *)nullptr);
     if (plan_hist)
       PlanOn(d_tot_[state ^ 1], d_seg_[state ^ 1], 2 * L, trick_ ? 1 : 0, kMaxHistRows, d_hwork_, d_nwork_, level + 1,
-             nullptr, HistGrid(2 * L, false), HistCus(false));
+             HistGrid(2 * L, false), HistCus(false));
   }
 
   // Stand-alone partition of larger items: groups of up to eight words side by side.
@@ -1890,7 +1889,7 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
     const unsigned per_item = HistRowsPerItem(rows, std::max(64, 512 / HistGroups()));
     const unsigned grid = (unsigned)std::min<size_t>(rows / per_item + 2 * L + 1, max_hist_items_);
     Mark(kPlan);
-    PlanOn(d_blk_tot_, d_blk_seg_, L, 0, per_item, d_hwork_, d_nwork_, level == 0 ? -1 : level, nullptr, grid);
+    PlanOn(d_blk_tot_, d_blk_seg_, L, 0, per_item, d_hwork_, d_nwork_, level == 0 ? -1 : level, grid);
     Mark(level == 0 ? kHistRoot : kHistDeep);
     HistLaunch(grid, hist_bins, br, hist_g, hist_h);
     if (in_place) DoneWithBlock(buf);

@@ -101,8 +101,7 @@ k_hist_sum_plan(const unsigned *__restrict__ node_size, int nodes, unsigned nrow
     seg[nd] = ok ? b : 0;
   }
   __syncthreads();  // the plan reads what this workgroup has just written
-  PlanBody(tot, seg, nodes, select, rows_per_item, work, n_work, node_first, node_items, nullptr, nullptr, max_items,
-           overflow);
+  PlanBody(tot, seg, nodes, select, rows_per_item, work, n_work, node_first, node_items, nullptr, max_items, overflow);
   if (threadIdx.x == 0) *status = s_bad != 0 ? 1u : *overflow != 0 ? 2u : 0u;  // (thread 0 wrote *overflow)
 }
 

@@ -407,7 +407,7 @@ k_ex_decide(const unsigned *__restrict__ ranks, size_t stride, const SplitRec *_
             unsigned grid_items, unsigned max_items, int F, unsigned *__restrict__ overflow) {
   if (blockIdx.x == 0) {
     PlanBody(tot_next, seg_next, 2 * L, 0, kExItem, next.work, next.n_work, next.node_first, next.node_items, nullptr,
-             nullptr, grid_items, overflow);
+             grid_items, overflow);
     return;
   }
   const size_t at = (size_t)(blockIdx.x - 1) * 1024 + threadIdx.x, step = (size_t)(gridDim.x - 1) * 1024;

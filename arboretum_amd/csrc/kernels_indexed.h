@@ -212,10 +212,10 @@ k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__r
     const unsigned long long lm0 = __ballot(v0 && !right0), rm0 = __ballot(v0 && right0);
     const unsigned long long lm1 = __ballot(v1 && !right1), rm1 = __ballot(v1 && right1);
     uint32_t *out = ids_out;
-    MergeRows<PAIR, 1, false, true>(nullptr, QL, R.b0, R.g0, R.h0, lm0, false, out, 0, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, 1, false, true>(nullptr, QR, R.b0, R.g0, R.h0, rm0, false, out, 0, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, 1, false, true>(nullptr, QL, R.b1, R.g1, R.h1, lm1, false, out, 0, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, 1, false, true>(nullptr, QR, R.b1, R.g1, R.h1, rm1, false, out, 0, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, 1, false>(nullptr, QL, R.b0, R.g0, R.h0, lm0, false, out, 0, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, 1, false>(nullptr, QR, R.b0, R.g0, R.h0, rm0, false, out, 0, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, 1, false>(nullptr, QL, R.b1, R.g1, R.h1, lm1, false, out, 0, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, 1, false>(nullptr, QR, R.b1, R.g1, R.h1, rm1, false, out, 0, g_out, h_out, lane, 0, 0, 0);
   };
   RowSet<1> A, B;
   load(A, wb);
@@ -228,8 +228,8 @@ k_ix_part(const uint8_t *__restrict__ bytes, size_t stride8, const unsigned *__r
     process(B, base + kChunkStep, chunk + 1);
     if (base + 2 * kChunkStep >= we) break;
   }
-  FlushQueue<PAIR, 1, false, true>(nullptr, QL, false, ids_out, 0, g_out, h_out, lane, 0, 0, 0);
-  FlushQueue<PAIR, 1, false, true>(nullptr, QR, false, ids_out, 0, g_out, h_out, lane, 0, 0, 0);
+  FlushQueue<PAIR, 1, false>(nullptr, QL, false, ids_out, 0, g_out, h_out, lane, 0, 0, 0);
+  FlushQueue<PAIR, 1, false>(nullptr, QR, false, ids_out, 0, g_out, h_out, lane, 0, 0, 0);
 }
 
 // The same where a work item has one chunk of 128 rows per wave (kChunkStep rows at most): ids and gradients are requested before

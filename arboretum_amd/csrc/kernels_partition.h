@@ -289,10 +289,10 @@ constexpr bool HeadKept() { return (!PAIR || PACK) && HI == 0; }
 
 // Writes lanes [from, to) of Q to their destination and, for the child whose
 // histogram is built, adds them to the LDS histogram.
-// HIST: the kernel builds a histogram; GH: the gradients move with the rows;
+// HIST: the kernel builds a histogram;
 // PACK: Q.g holds packed logistic gradients (PackGrad), there is no h array.
 // NQ quads and, with HI, the ninth-bit word behind them (moved like a quad).
-template <bool PAIR, int NQ, bool HIST = true, bool GH = true, bool PACK = false, int HI = 0>
+template <bool PAIR, int NQ, bool HIST = true, bool PACK = false, int HI = 0>
 __device__ __forceinline__ void EmitRows(unsigned long long *__restrict__ lds, const RowQueue<NQ + HI> &Q,
                                          unsigned from, unsigned to, bool built,
                                          uint32_t *__restrict__ bins_out, size_t stride,
@@ -303,7 +303,7 @@ __device__ __forceinline__ void EmitRows(unsigned long long *__restrict__ lds, c
     const unsigned d = Q.base + (unsigned)lane;
 #pragma unroll
     for (int q = 0; q < NQ + HI; ++q) __builtin_nontemporal_store(Q.b[q], &bins_out[(size_t)q * stride + d]);
-    if (GH && g_out != nullptr) {  // a group pass after the first leaves the gradients alone
+    if (g_out != nullptr) {  // a group pass after the first leaves the gradients alone
       __builtin_nontemporal_store(Q.g, &g_out[d]);
       if (PAIR && !PACK) __builtin_nontemporal_store(Q.h, &h_out[d]);
     }
@@ -317,7 +317,7 @@ __device__ __forceinline__ void EmitRows(unsigned long long *__restrict__ lds, c
 
 // The kept first batch of a wave (plain stores: it is about to be completed by
 // a neighbour), then what is left in the queue.
-template <bool PAIR, int NQ, bool HIST = true, bool GH = true, bool PACK = false, int HI = 0>
+template <bool PAIR, int NQ, bool HIST = true, bool PACK = false, int HI = 0>
 __device__ __forceinline__ void FlushQueue(unsigned long long *__restrict__ lds, const RowQueue<NQ + HI> &Q, bool built,
                                            uint32_t *__restrict__ bins_out, size_t stride,
                                            float *__restrict__ g_out, float *__restrict__ h_out, int lane,
@@ -326,15 +326,15 @@ __device__ __forceinline__ void FlushQueue(unsigned long long *__restrict__ lds,
     const unsigned d = Q.hbase + (unsigned)lane;
 #pragma unroll
     for (int q = 0; q < NQ + HI; ++q) bins_out[(size_t)q * stride + d] = Q.hb[q];
-    if (GH && g_out != nullptr) g_out[d] = Q.hg;
+    if (g_out != nullptr) g_out[d] = Q.hg;
   }
-  EmitRows<PAIR, NQ, HIST, GH, PACK, HI>(lds, Q, Q.skip, Q.n, built, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+  EmitRows<PAIR, NQ, HIST, PACK, HI>(lds, Q, Q.skip, Q.n, built, bins_out, stride, g_out, h_out, lane, sg, sh, F);
 }
 
 // Appends the rows of X flagged in xm (wave-uniform mask, one row per lane) to
 // Q in row order with one lane permute (ds_permute_b32) per register; a full queue is emitted
 // and the rest of X starts the next batch.
-template <bool PAIR, int NQ, bool HIST = true, bool GH = true, bool PACK = false, int HI = 0>
+template <bool PAIR, int NQ, bool HIST = true, bool PACK = false, int HI = 0>
 __device__ __forceinline__ void MergeRows(unsigned long long *__restrict__ lds, RowQueue<NQ + HI> &Q,
                                           const uint32_t (&xb)[NQ + HI], float xg, float xh,
                                           unsigned long long xm, bool built,
@@ -351,8 +351,8 @@ __device__ __forceinline__ void MergeRows(unsigned long long *__restrict__ lds, 
   uint32_t vb[NW];
 #pragma unroll
   for (int q = 0; q < NW; ++q) vb[q] = SendTo(dst, xb[q]);
-  const float vg = GH ? __uint_as_float(SendTo(dst, __float_as_uint(xg))) : 0.0f;
-  const float vh = GH && PAIR && !PACK ? __uint_as_float(SendTo(dst, __float_as_uint(xh))) : 0.0f;
+  const float vg = __uint_as_float(SendTo(dst, __float_as_uint(xg)));
+  const float vh = PAIR && !PACK ? __uint_as_float(SendTo(dst, __float_as_uint(xh))) : 0.0f;
   if (Q.n + nx >= 64u) {  // wave-uniform: the batch is complete
     const bool fill = (unsigned)lane >= Q.n;
 #pragma unroll
@@ -371,7 +371,7 @@ __device__ __forceinline__ void MergeRows(unsigned long long *__restrict__ lds, 
         AccumulateRow<PAIR, NQ, HI>(lds, Q.b, gv, hv, sg, sh, 0, F);
       }
     } else {
-      EmitRows<PAIR, NQ, HIST, GH, PACK, HI>(lds, Q, Q.skip, 64u, built, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+      EmitRows<PAIR, NQ, HIST, PACK, HI>(lds, Q, Q.skip, 64u, built, bins_out, stride, g_out, h_out, lane, sg, sh, F);
     }
     Q.base += 64u;
     Q.skip = 0u;
@@ -510,10 +510,10 @@ k_part_hist(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
       const bool right1 = v1 && goes_right(s1);
       const unsigned long long b0 = __ballot(v0 && right0 == build_right), o0 = __ballot(v0 && right0 != build_right);
       const unsigned long long b1 = __ballot(v1 && right1 == build_right), o1 = __ballot(v1 && right1 != build_right);
-      MergeRows<PAIR, NQ, true, true, PACK, HI>(lds, QO, R.b0, R.g0, R.h0, o0, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
-      MergeRows<PAIR, NQ, true, true, PACK, HI>(lds, QB, R.b0, R.g0, R.h0, b0, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
-      MergeRows<PAIR, NQ, true, true, PACK, HI>(lds, QO, R.b1, R.g1, R.h1, o1, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
-      MergeRows<PAIR, NQ, true, true, PACK, HI>(lds, QB, R.b1, R.g1, R.h1, b1, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+      MergeRows<PAIR, NQ, true, PACK, HI>(lds, QO, R.b0, R.g0, R.h0, o0, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+      MergeRows<PAIR, NQ, true, PACK, HI>(lds, QB, R.b0, R.g0, R.h0, b0, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+      MergeRows<PAIR, NQ, true, PACK, HI>(lds, QO, R.b1, R.g1, R.h1, o1, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+      MergeRows<PAIR, NQ, true, PACK, HI>(lds, QB, R.b1, R.g1, R.h1, b1, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
     };
     if (wb < we) {
       RowSet<NW> A, B;
@@ -527,8 +527,8 @@ k_part_hist(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
         if (base + 2 * kChunkStep >= we) break;
       }
     }
-    FlushQueue<PAIR, NQ, true, true, PACK, HI>(lds, QO, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
-    FlushQueue<PAIR, NQ, true, true, PACK, HI>(lds, QB, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+    FlushQueue<PAIR, NQ, true, PACK, HI>(lds, QO, false, bins_out, stride, g_out, h_out, lane, sg, sh, F);
+    FlushQueue<PAIR, NQ, true, PACK, HI>(lds, QB, true, bins_out, stride, g_out, h_out, lane, sg, sh, F);
   } else {
     // Rows selected for the histogram are queued by row id (slot 64 * j + lane
     // of the queue is lane `lane` of q[j]; slots [0, np) are occupied) and read
@@ -715,7 +715,6 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
             const unsigned *__restrict__ n_work, const unsigned *__restrict__ wave_left,
             const unsigned *__restrict__ item_left, BinCode code, int hi_word) {
   __shared__ unsigned s_tmp[kItemWaves + 1];
-  constexpr bool GH = true;
   const unsigned w = blockIdx.x;
   const int q0 = min((int)blockIdx.y * NQ, words - NQ);
   if (blockIdx.y != 0) g_out = nullptr;  // uniform
@@ -763,10 +762,10 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
     const bool right1 = v1 && test.Right(R.s1);
     const unsigned long long lm0 = __ballot(v0 && !right0), rm0 = __ballot(right0);
     const unsigned long long lm1 = __ballot(v1 && !right1), rm1 = __ballot(right1);
-    MergeRows<PAIR, NQ, false, GH>(nullptr, QL, R.r.b0, R.r.g0, R.r.h0, lm0, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, NQ, false, GH>(nullptr, QR, R.r.b0, R.r.g0, R.r.h0, rm0, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, NQ, false, GH>(nullptr, QL, R.r.b1, R.r.g1, R.r.h1, lm1, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
-    MergeRows<PAIR, NQ, false, GH>(nullptr, QR, R.r.b1, R.r.g1, R.r.h1, rm1, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, NQ, false>(nullptr, QL, R.r.b0, R.r.g0, R.r.h0, lm0, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, NQ, false>(nullptr, QR, R.r.b0, R.r.g0, R.r.h0, rm0, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, NQ, false>(nullptr, QL, R.r.b1, R.r.g1, R.r.h1, lm1, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+    MergeRows<PAIR, NQ, false>(nullptr, QR, R.r.b1, R.r.g1, R.r.h1, rm1, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
   };
   Rows A, B;
   load(A, wb);
@@ -778,8 +777,8 @@ k_part_rows(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out, 
     process(B, base + kChunkStep);
     if (base + 2 * kChunkStep >= we) break;
   }
-  FlushQueue<PAIR, NQ, false, GH>(nullptr, QL, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
-  FlushQueue<PAIR, NQ, false, GH>(nullptr, QR, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+  FlushQueue<PAIR, NQ, false>(nullptr, QL, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
+  FlushQueue<PAIR, NQ, false>(nullptr, QR, false, group_out, stride, g_out, h_out, lane, 0, 0, 0);
 }
 
 // The stand-alone partition in one launch, where a work item has one chunk of 128 rows per wave (kChunkStep rows at most): the
@@ -853,20 +852,6 @@ k_part_small(const uint32_t *__restrict__ bins, uint32_t *__restrict__ bins_out,
   }
 }
 
-// Adds the slabs of every directly built node of a level (on top of the stored
-// histogram when `accumulate`) and, with `trick`, derives its sibling as
-// parent - node.  Slabs are in LDS order (HistLds; `entry` below counts
-// k * 4096 + bin * 16 + f16 over all blocks of the matrix); the histograms
-// written here are feature-major: hist[node][f * 256 + bin].
-// grid (slab_entries/64, L), 1024 threads = 64 entries x 16 slab lanes.
-//   by_parent = 0: slabs belong to work items of the node itself
-//               (node_items == 0xffffffff marks a derived node);
-//   by_parent = 1: slabs belong to work items of the parent (fused pass); the
-//               built child is the smaller one, ties -> left.
-// hi_base > 0: the slabs hold one more row of entries, bin 256 of every feature
-// (matrices with a ninth-bit word); one more block of the grid (the last one)
-// reduces it into cell hi_base + f of the node's histogram, behind the 256-bin
-// histograms of the features.
 // Work plan of the row pass over this level's nodes that follows (fused pass or partition), made by one more block of the slab reduction (the ranges of
 // the nodes are known since their parents were split): work == null, none.  node_first /
 // node_items must be other arrays than the ones this reduction reads.
@@ -881,6 +866,20 @@ struct NextPlan {
   unsigned *overflow = nullptr, *cursor = nullptr;
 };
 
+// Adds the slabs of every directly built node of a level (on top of the stored
+// histogram when `accumulate`) and, with `trick`, derives its sibling as
+// parent - node.  Slabs are in LDS order (HistLds; `entry` below counts
+// k * 4096 + bin * 16 + f16 over all blocks of the matrix); the histograms
+// written here are feature-major: hist[node][f * 256 + bin].
+// grid (slab_entries/64, L), 1024 threads = 64 entries x 16 slab lanes.
+//   by_parent = 0: slabs belong to work items of the node itself
+//               (node_items == 0xffffffff marks a derived node);
+//   by_parent = 1: slabs belong to work items of the parent (fused pass); the
+//               built child is the smaller one, ties -> left.
+// hi_base > 0: the slabs hold one more row of entries, bin 256 of every feature
+// (matrices with a ninth-bit word); one more block of the grid (the last one)
+// reduces it into cell hi_base + f of the node's histogram, behind the 256-bin
+// histograms of the features.
 // CNT: type of the row counts of the node histograms.  The tree builder keeps
 // 64-bit counts: a streamed matrix may hold 2^32 rows and more, all of which can
 // sit in one cell (a constant feature, the bin of the missing values).
@@ -899,7 +898,7 @@ k_hist_reduce(const unsigned long long *__restrict__ slab, int slab_entries, int
   if (plan.work != nullptr && blockIdx.x + 1 == gridDim.x) {
     if (blockIdx.y == 0)
       PlanBody(plan.tot, plan.seg_start, plan.L, 0, plan.rows_per_item, plan.work, plan.n_work, plan.node_first,
-               plan.node_items, nullptr, nullptr, plan.max_items, plan.overflow, plan.cursor);
+               plan.node_items, nullptr, plan.max_items, plan.overflow, plan.cursor);
     return;
   }
   // LANES threads share the slabs of one entry; a block covers 1024 / LANES
@@ -1040,7 +1039,7 @@ k_reduce_scan(const unsigned long long *__restrict__ slab, int slab_entries, int
   if (plan.work != nullptr && blockIdx.x + 1 == gridDim.x) {
     if (blockIdx.y == 0)
       PlanBody(plan.tot, plan.seg_start, plan.L, 0, plan.rows_per_item, plan.work, plan.n_work, plan.node_first,
-               plan.node_items, nullptr, nullptr, plan.max_items, plan.overflow, plan.cursor);
+               plan.node_items, nullptr, plan.max_items, plan.overflow, plan.cursor);
     return;
   }
   constexpr int kFeatures = 8, kPad = kSlots + 2;

@@ -52,9 +52,7 @@ inline unsigned BalancedPlanItems(unsigned long long rows, unsigned nodes, unsig
 // at most `rows_per_item` rows (a multiple of 64; at most len / rows_per_item
 // + 2 items per node).  select: 0 = every node, 1 = the smaller
 // child of each sibling pair, ties -> left (hist_grad_sum.cu:279-294).
-// rows_scanned (optional) is advanced by the rows that will be accumulated
-// into histograms: the selected rows, or, when `split` is given (fused
-// partition + histogram over parent nodes), the smaller side of every split.
+// rows_scanned (optional) is advanced by the selected rows: those that will be accumulated into histograms.
 // cursor (optional): two words per node, cleared here; the fused pass claims
 // the destination ranges of its work items on them.
 // balance_cus (optional): rows_per_item is then the most an item may hold, and
@@ -66,8 +64,7 @@ __device__ __forceinline__ void PlanBody(const NodeSum *__restrict__ tot, const 
                                          int L, int select, unsigned rows_per_item,
                                          WorkItem *__restrict__ work, unsigned *__restrict__ n_work,
                                          unsigned *__restrict__ node_first, unsigned *__restrict__ node_items,
-                                         unsigned long long *__restrict__ rows_scanned,
-                                         const SplitRec *__restrict__ split, unsigned max_items,
+                                         unsigned long long *__restrict__ rows_scanned, unsigned max_items,
                                          unsigned *__restrict__ overflow,
                                          unsigned *__restrict__ cursor = nullptr, unsigned balance_cus = 0) {
   __shared__ unsigned s_base[kMaxPlanNodes + 1];
@@ -120,12 +117,7 @@ __device__ __forceinline__ void PlanBody(const NodeSum *__restrict__ tot, const 
         // rounded down to one, so that every item but a node's first begins on
         // a 256-byte boundary of the row arrays
         cnt = (unsigned)(((seg_start[nd] & 63u) + len + rows_per_item - 1) / rows_per_item);
-        unsigned long long acc = len;
-        if (split) {
-          const unsigned long long cl = split[nd].left.c;
-          acc = min(cl, len - cl);
-        }
-        atomicAdd(&s_rows, acc);
+        atomicAdd(&s_rows, len);
       }
       node_items[nd] = sel ? cnt : 0xffffffffu;  // 0xffffffff marks "not selected"
       if (cursor) {  // destination cursors of the node's two children in the fused pass
@@ -187,13 +179,11 @@ __global__ void __launch_bounds__(1024)
 k_plan(const NodeSum *__restrict__ tot, const unsigned *__restrict__ seg_start, int L, int select,
        unsigned rows_per_item, WorkItem *__restrict__ work, unsigned *__restrict__ n_work,
        unsigned *__restrict__ node_first, unsigned *__restrict__ node_items,
-       unsigned long long *__restrict__ rows_scanned, const SplitRec *__restrict__ split,
-       unsigned max_items, unsigned *__restrict__ overflow, unsigned balance_cus,
-       unsigned *__restrict__ cursor = nullptr) {
-  PlanBody(tot, seg_start, L, select, rows_per_item, work, n_work, node_first, node_items, rows_scanned, split,
-           max_items, overflow, cursor, balance_cus);
+       unsigned long long *__restrict__ rows_scanned, unsigned max_items, unsigned *__restrict__ overflow,
+       unsigned balance_cus) {
+  PlanBody(tot, seg_start, L, select, rows_per_item, work, n_work, node_first, node_items, rows_scanned, max_items, overflow,
+           nullptr, balance_cus);
 }
-
 
 }  // namespace
 }  // namespace arb

@@ -528,7 +528,7 @@ __device__ __forceinline__ void SelectAndPlan(const SelectPlan &a) {
                a.t_gain, a.L - 1, a.active);
   __syncthreads();  // the children's totals and ranges written above are read by the plan
   PlanBody(a.tot_next, a.seg_next, 2 * a.L, a.select, a.rows_per_item, a.work, a.n_work, a.node_first, a.node_items,
-           a.rows_scanned, nullptr, a.max_items, a.overflow, nullptr, a.balance_cus);
+           a.rows_scanned, a.max_items, a.overflow, nullptr, a.balance_cus);
 }
 // Called by all threads of the workgroup.
 __device__ __forceinline__ SplitRec SplitOf(const SelectPlan &a, int nd, const SplitRec *__restrict__ split) {
