@@ -229,8 +229,13 @@ class Garden {
  private:
   std::unique_ptr<TreeBuilder> builder_;
   DataMatrix *bound_ = nullptr;
-  // Records of freshly grown trees are fetched from the GPU on first use.
-  void SyncTrees() const { if (builder_) builder_->FlushTrees(); }
+  // Records of freshly grown trees are fetched from the GPU on first use, which may be by several threads at once
+  // (predictions).
+  void SyncTrees() const {
+    std::lock_guard<std::mutex> lock(sync_mutex_);
+    if (builder_) builder_->FlushTrees();
+  }
+  mutable std::mutex sync_mutex_;
   mutable std::vector<RegTree> trees_;
   std::string model_;
   bool inspect_ = false;

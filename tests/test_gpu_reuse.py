@@ -94,3 +94,31 @@ def test_new_target_leaves_a_running_booster_alone(arb, oracle):
         for t in range(booster.num_trees()):
             assert np.array_equal(ob.tree(t)["fid"], booster.tree(t)["fid"])
             assert np.array_equal(ob.tree(t)["weights"], booster.tree(t)["weights"])
+
+
+def test_threads_predict_on_one_booster(arb):
+    # the first of them fetches the trees from the GPU, and each has its own sums
+    X, y, cfg = _problem(4)
+    rng = np.random.default_rng(9)
+    rows = [rng.standard_normal((200 * (k + 1) + k, X.shape[1]), dtype=np.float32) for k in range(6)]
+    train = arb.DMatrix(X, y=y)
+    want = None
+    for _ in range(6):
+        g = arb.train(cfg, train, 3)
+        got = [None] * len(rows)
+        start = threading.Barrier(len(rows))
+
+        def work(k):
+            data = arb.DMatrix(rows[k])
+            start.wait()
+            for _ in range(4):
+                got[k] = g.predict(data)
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(len(rows))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        if want is None:
+            g.predict_on_device(False)
+            want = [g.predict(arb.DMatrix(r)) for r in rows]
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
