@@ -33,6 +33,15 @@ def test_walks_at_tile_edges(arb, n, F, depths):
     both_ways(g, arb.DMatrix(X))
 
 
+# the most features of which 64 rows have their values in the LDS, and one more: read from memory row by row
+@pytest.mark.parametrize("F", [467, 468])
+@pytest.mark.parametrize("n", [64, 16449])
+def test_walks_at_the_widest_tile(arb, n, F):
+    rng = np.random.default_rng(n + F)
+    g = arb.load(_random_model(rng, [7] * 30 + [4, 9], F, fid_max=F))
+    both_ways(g, arb.DMatrix(rng.standard_normal((n, F), dtype=np.float32)))
+
+
 @pytest.mark.parametrize("n", [1000, 70000])
 def test_many_trees_of_several_labels(arb, n):
     # several chunks of trees, the labels changing inside and between them; the model is laid out again
