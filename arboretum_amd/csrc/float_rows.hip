@@ -25,6 +25,15 @@ int CurrentDevice() {
   return dev;
 }
 
+// Another device current while the object lives.
+struct OnDeviceOf {
+  explicit OnDeviceOf(int device) : before(CurrentDevice()) {
+    if (device != before && hipSetDevice(device) != hipSuccess) throw std::runtime_error("HIP error: no such device");
+  }
+  ~OnDeviceOf() { (void)hipSetDevice(before); }
+  const int before;
+};
+
 struct PooledStream {
   hipStream_t s = StreamPoolTake();
   ~PooledStream() { StreamPoolGive(s); }
@@ -81,6 +90,7 @@ const float *FloatRows::OnHost() {
   if (pinned_) return pinned_;
   if (!host_ && device_) {
     const size_t bytes = n_ * columns_ * sizeof(float);
+    const OnDeviceOf device(device_id_);  // (the caller may use another one)
     PooledStream stream;
     float *p = static_cast<float *>(HostPoolTake(bytes));
     try {

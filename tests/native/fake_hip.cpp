@@ -1,6 +1,7 @@
 #include "fake_hip.h"
 
 #include <cstdlib>
+#include <cstring>
 
 namespace fake {
 thread_local int current = 0;
@@ -29,7 +30,7 @@ hipError_t hipSetDevice(int device) {
 hipError_t hipMalloc(void **p, size_t bytes) {
   std::lock_guard<std::mutex> lock(fake::mutex);
   if (fake::BytesOn(fake::current) + bytes > fake::capacity) return hipErrorOutOfMemory;
-  *p = std::malloc(1);  // (an address of its own)
+  *p = std::malloc(bytes);
   fake::blocks[*p] = {fake::current, bytes};
   return hipSuccess;
 }
@@ -41,7 +42,7 @@ hipError_t hipFree(void *p) {
 }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
   std::lock_guard<std::mutex> lock(fake::mutex);
-  *p = std::malloc(1);
+  *p = std::malloc(bytes);
   fake::pinned[*p] = bytes;
   return hipSuccess;
 }
@@ -61,6 +62,27 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   std::lock_guard<std::mutex> lock(fake::mutex);
   if (!fake::streams.erase(s)) std::abort();
   std::free(s);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+// at once, in order; a copy that touches memory of another device than its stream's is refused
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t bytes, hipMemcpyKind, hipStream_t s) {
+  {
+    std::lock_guard<std::mutex> lock(fake::mutex);
+    for (const auto &b : fake::blocks)
+      for (const void *p : {(const void *)to, from})
+        if (p >= b.first && p < static_cast<char *>(b.first) + b.second.second && fake::streams.at(s) != b.second.first)
+          return hipErrorInvalidDevice;
+  }
+  std::memcpy(to, from, bytes);
   return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
