@@ -272,10 +272,13 @@ void Garden::UpdateByLastTree(DataMatrix *data) {
     for (size_t r0 = 0; r0 < n; r0 += step) {
       const size_t m = std::min(step, n - r0);
       const float *sums = PredictOnDevice(round_predictor_.get(), *data, trees_, first, trees_.size(), K, 0.0f, r0, r0 + m);
-      for (size_t k = 0; k < classes; ++k)
-        ParallelFor(m, [&](size_t b, size_t e) {
-          for (size_t i = b; i < e; ++i) y_hat[k * n + r0 + i] += sums[k * m + i];
+      for (size_t k = 0; k < classes; ++k) {
+        float *out = y_hat.data() + k * n + r0;
+        const float *in = sums + k * m;
+        ParallelFor(m, [out, in](size_t b, size_t e) {
+          for (size_t i = b; i < e; ++i) out[i] += in[i];
         });
+      }
     }
     return;
   }

@@ -916,7 +916,8 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
   // 3.6, 4.1; 6 M x 20, four classes: 18.9, 19.0, 17.0, 17.2.
   static constexpr size_t kLanes = 3;
   // One stream beyond kLaneRows rows (the kernels fill the chip) and with sampled columns: the sampler copies its
-  // masks on the stream of the trees, and the gain is not there at a colsample_bytree or colsample_bylevel below 1.
+  // masks on the stream of the trees.  (Five rounds of that 1 M x 100: 14.1 ms on three streams, 19.0 at a colsample_bytree
+  // of 0.8 and 18.9 at 0.999, on one.)
   static constexpr size_t kLaneRows = (size_t)8 << 20;
   // What the lanes beside the first may take together: deep trees over wide matrices need gigabytes of
   // histograms and slabs a lane (200 features of 256 bins, max_depth 10: 3 GB).
