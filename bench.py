@@ -18,7 +18,7 @@ matrix.  Prints ONE JSON line.
                `moved_*` keys give what this implementation moves instead (it
                re-orders the rows themselves), `traffic` the HBM bytes per
                launch from hardware counters of a committed profile
-  cpu_baseline the CPU checker (oracle/, OpenMP) on a bounded row sample of the
+  cpu_baseline the CPU oracle (oracle/, OpenMP) on a bounded row sample of the
                same workload, timed on this host
 """
 import argparse
@@ -55,11 +55,11 @@ def lds_floor_us(rows_accumulated, features, words=2):
     return instr_per_cu * LDS_CYCLES_PER_ATOMIC / CLOCK_HZ * 1e6
 
 
-# the same for the matrices whose rows stay in place
+# the same for the matrices whose rows stay in place (50 M x 200, 20 M x 100)
 WIDE_KERNEL_SOURCES = ["kernels_indexed.h", "kernels_hist.h", "device_common.h", "kernels_plan.h", "kernels_launch.h",
                        "device_builder.hip"]
-WIDE_TRAFFIC_PROFILES = {"config2": "hbm_traffic_configs2_50Mx200_missing_depth10.txt",
-                         "config3": "hbm_traffic_configs3_20Mx100_softmax10_depth6.txt"}
+WIDE_TRAFFIC_PROFILES = {"config2": "hbm_traffic_50Mx200_missing_depth10.txt",
+                         "config3": "hbm_traffic_20Mx100_softmax10_depth6.txt"}
 
 
 def kernel_source_digest(sources=None):
@@ -90,7 +90,7 @@ def profiled_traffic(profile=TRAFFIC_PROFILE, key="fused_pass_hbm_bytes_per_laun
 
 
 def make_workload(rows, features=28, seed=0):
-    """features 0-20 ~ N(0,1), 21-27 log-normal(0,1); label ~
+    """The headline's matrix: features 0-20 ~ N(0,1), 21-27 log-normal(0,1); label ~
     Bernoulli(sigmoid(sum of 8 random depth-3 stump products + 0.5 N(0,1) + bias)),
     bias chosen for about 53 % positives."""
     rng = np.random.default_rng(seed)
@@ -119,7 +119,7 @@ def config(max_depth=8, hist_size=256):
 
 
 def make_stream_workload(rows, features=128, seed=0):
-    """BASELINE config 5 shape: uint8 bins, per column either U{0..255} or a
+    """A matrix for streaming: uint8 bins, per column either U{0..255} or a
     Binomial(255, 0.3) look-alike (rounded normal), labels from a random depth-6
     tree on the bins with 10 % flips.  A base tile of at most 4M rows is generated
     and repeated (the content does not change what is measured: PCIe streaming)."""
@@ -169,9 +169,12 @@ def stream_mode(args, arb):
     model.synchronize()
     dt = time.perf_counter() - t0
     scanned = model.rows_scanned() - s0
-    passes = args.max_depth + 1    # one pass over every block per level + the leaf pass
+    # a pass over every block per level below the root and one for the leaves, which also builds the next
+    # tree's root; passes go forwards and backwards in turn, so each starts on the two blocks that the copy buffers hold
+    passes = args.max_depth
     resident, blocks = model.stream_residency()
-    streamed_bytes = host_bytes * (blocks - resident) / max(blocks, 1)   # copied per pass
+    block_bytes = min(args.stream_block_rows, args.stream_rows) * ((args.stream_features + 3) // 4 * 4)
+    streamed_bytes = max(blocks - resident - 2, 0) * block_bytes   # copied per pass
     print(json.dumps({
         "metric": "streamed (out-of-core) tree growing, bins in pinned host memory",
         "sec_per_tree": dt / args.steps, "steps": args.steps,
@@ -185,7 +188,7 @@ def stream_mode(args, arb):
 
 
 def make_config2_bins(rows, features=200, seed=2):
-    """BASELINE configs[2] as the kernels see it: 64 bins per feature plus the missing-value bin (id
+    """A wide matrix with gaps as the kernels see it: 64 bins per feature plus the missing-value bin (id
     64, 30 % of the values, uniformly placed); half the columns uniform over the 64 bins, half
     integer categories 0..49 under Zipf(1.1); regression target = 20 random piecewise-constant
     functions of the bins plus noise.  Generated in row chunks (the fp32 matrix would be 40 GB)."""
@@ -221,7 +224,7 @@ def make_config2_bins(rows, features=200, seed=2):
 
 
 def make_config3(rows, features=100, classes=10, seed=3):
-    """N(0,1) features, labels = argmax(X W + Gumbel noise)."""
+    """A matrix of several classes: N(0,1) features, labels = argmax(X W + Gumbel noise)."""
     rng = np.random.default_rng(seed)
     X = rng.standard_normal(size=(rows, features), dtype=np.float32)
     W = rng.standard_normal(size=(features, classes)).astype(np.float32)
@@ -234,7 +237,8 @@ def make_config3(rows, features=100, classes=10, seed=3):
 
 
 def other_config(arb, workload, rows_arg, steps):
-    """BASELINE configs[2] / configs[3] at full size: seconds per tree (not the headline metric)."""
+    """50 M x 200 with gaps ("config2") or 20 M x 100 of ten classes ("config3"): seconds per tree (not the
+    headline metric)."""
     t0 = time.perf_counter()
     if workload == "config2":
         rows = rows_arg if rows_arg != 10_500_000 else 50_000_000
@@ -244,7 +248,7 @@ def other_config(arb, workload, rows_arg, steps):
         del bins
         cfg = {"objective": 0, "method": 1, "internals": {"hist_size": 64, "double_precision": True},
                "tree": {"max_depth": 10, "eta": 0.3, "lambda": 1.0}}
-        trees_per_round, name = 1, "configs[2]: %d x 200, 64 bins + missing bin (30 %%), squared error, max_depth 10" % rows
+        trees_per_round, name = 1, "%d x 200, 64 bins + missing bin (30 %%), squared error, max_depth 10" % rows
     else:
         rows = rows_arg if rows_arg != 10_500_000 else 20_000_000
         F, K = 100, 10
@@ -253,7 +257,7 @@ def other_config(arb, workload, rows_arg, steps):
         del X
         cfg = {"objective": 4, "method": 1, "internals": {"hist_size": 256, "double_precision": True},
                "tree": {"max_depth": 6, "eta": 0.2, "lambda": 1.0, "labels_count": K}}
-        trees_per_round, name = K, "configs[3]: %d x 100, 10 classes soft-max, 256 bins, max_depth 6" % rows
+        trees_per_round, name = K, "%d x 100, 10 classes soft-max, 256 bins, max_depth 6" % rows
     t_gen = time.perf_counter() - t0
     model = arb.Garden(cfg, data)
     t0 = time.perf_counter()
@@ -269,7 +273,7 @@ def other_config(arb, workload, rows_arg, steps):
     scanned = model.rows_scanned() - s0
     trees = steps * trees_per_round
     # The histogram kernels of these matrices (rows in place: k_hist_rec over the records of the
-    # smaller children, the root of configs[3] from the quad columns by k_hist) against the HBM
+    # smaller children, the root of the soft-max matrix from the quad columns by k_hist) against the HBM
     # roofline, by the same accounting as the headline: rows accumulated x (F bin bytes + 4 row id
     # + the gradient pair) + cells written once; and against the LDS atomic floor of those rows.
     # Phase times come from one more round with every phase bracketed by events.
@@ -333,7 +337,7 @@ def exact_workload(arb, rows, features, steps):
 
 
 def cpu_baseline(X, y, cfg, sample_rows, trees):
-    """The CPU checker on the first `sample_rows` rows (same columns, same
+    """The CPU oracle on the first `sample_rows` rows (same columns, same
     configuration), all host cores."""
     from oracle import oracle as orc
     cores = os.cpu_count() or 1
@@ -365,14 +369,14 @@ def main():
     ap.add_argument("--cpu-trees", type=int, default=16)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-other-configs", action="store_true",
-                    help="skip the full-size runs of BASELINE configs[2] and configs[3] reported under other_configs")
+                    help="skip the full-size runs of the two wide workloads reported under other_configs")
     ap.add_argument("--nan-frac", type=float, default=0.0,
                     help="stress variant: this fraction of the feature values is replaced by NaN (all land in "
                          "one bin per feature; below 1/256 with --hist-size 256 every feature then has 257 bin "
                          "ids, the last one kept as a ninth bit)")
     ap.add_argument("--mode", choices=["resident", "stream"], default="resident")
     ap.add_argument("--workload", choices=["headline", "config2", "config3", "exact"], default="headline",
-                    help="config2 / config3: BASELINE configs[2] / configs[3] at full size, seconds per tree only; "
+                    help="config2: 50 M x 200 with gaps, config3: 20 M x 100 of ten classes, seconds per tree only; "
                          "exact: the exact method (method 0) on the headline matrix, seconds per tree only")
     ap.add_argument("--stream-rows", type=int, default=64_000_000)
     ap.add_argument("--stream-features", type=int, default=128)
@@ -519,7 +523,7 @@ def main():
         "vs_baseline": None,
         "dtype": "int64",
         "data": "synthetic",
-        "config": {"workload": "binary classification %d rows x %d dense fp32 features (BASELINE configs[1]), "
+        "config": {"workload": "binary classification %d rows x %d dense fp32 features, "
                                "%d bins, max_depth %d, logistic, eta 0.1, lambda 1, min_child_weight 1"
                                % (R, F, args.hist_size, D),
                    "rows": R, "features": F, "bins": args.hist_size, "max_depth": D},
@@ -541,7 +545,7 @@ def main():
                      "traffic_over_algorithmic": traffic / algo_bytes if traffic else None,
                      "traffic_source": "profiles/" + os.path.basename(TRAFFIC_PROFILE) if traffic else None},
         "other_kernels": other,
-        # north_star asks for the histogram build at >= 0.60 of the HBM peak: not met.  The kernels
+        # The target for the histogram build is 0.60 of the HBM peak: not met.  The kernels
         # that only build histograms are bound by the LDS atomic unit (frac_of_lds_floor above),
         # whose floor for one pass over all rows is lds_floor_us_all_rows; 0.60 of the HBM peak
         # would be 79 us for the same pass.
@@ -561,8 +565,8 @@ def main():
     if not args.no_other_configs and (R, F, args.hist_size, D) == (10500000, 28, 256, 8):
         # the wide configurations at their full sizes, a few trees each (seconds per tree only)
         del model, data, X, y
-        out["other_configs"] = {"configs[2]": other_config(arb, "config2", 10_500_000, 3),
-                                "configs[3]": other_config(arb, "config3", 10_500_000, 2)}
+        out["other_configs"] = {"50Mx200_missing_depth10": other_config(arb, "config2", 10_500_000, 3),
+                                "20Mx100_softmax10_depth6": other_config(arb, "config3", 10_500_000, 2)}
     print(json.dumps(out))
 
 
