@@ -369,6 +369,7 @@ class ExactSortBuilder : public TreeBuilder {
     else ARB_EX_GATHER(false, false);
 #undef ARB_EX_GATHER
     const bool fold = n_ / kExItem <= kExFoldItems;
+    const bool filter = (n_ / kExItem + 1) * (size_t)F_ <= kExFilterItems;
     if (!fold) {
       HIP_OK(hipMemsetAsync(d_root_tot_, 0, 2 * sizeof(long long), stream_));
       hipLaunchKernelGGL(k_sum_grad, dim3(SumGradGrid(n_)), dim3(kSumThreads), 0, stream_, g, h, pack_ ? 1 : 0, n_,
@@ -386,9 +387,14 @@ class ExactSortBuilder : public TreeBuilder {
       if (!fold)
         hipLaunchKernelGGL((k_ex_offsets<ExSum>), per_node, dim3(64), 0, stream_, plan.part, d_off_, plan.node_first,
                            plan.node_items, max_items_);
-#define ARB_EX(P, D, K)                                                                                               \
-  hipLaunchKernelGGL((k_ex_scan<P, D, K>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_, plan,  \
+#define ARB_EX_F(P, D, K, FI)                                                                                         \
+  hipLaunchKernelGGL((k_ex_scan<P, D, K, FI>), per_item, dim3(kExThreads), 0, stream_, lists, stride_, d_shifts_, plan,  \
                      fold ? (const ExSum *)nullptr : d_off_, level == 0 ? 1 : 0, tot, seg, gp, d_best_, max_items_)
+#define ARB_EX(P, D, K)                  \
+  do {                                   \
+    if (filter) ARB_EX_F(P, D, K, true); \
+    else ARB_EX_F(P, D, K, false);       \
+  } while (0)
       if (pack_ && f64_) ARB_EX(true, true, true);
       else if (pack_) ARB_EX(true, false, true);
       else if (pair_ && f64_) ARB_EX(true, true, false);
@@ -396,6 +402,7 @@ class ExactSortBuilder : public TreeBuilder {
       else if (f64_) ARB_EX(false, true, false);
       else ARB_EX(false, false, false);
 #undef ARB_EX
+#undef ARB_EX_F
 #define ARB_EX_SELECT(P, D)                                                                                          \
   hipLaunchKernelGGL((k_ex_select<P, D>), dim3((unsigned)L), dim3(1024), 0, stream_, d_best_, plan.node_first,      \
                      plan.node_items, max_items_, F_, sampler_.Active(level), tot, seg, tot_next, seg_next, d_split_, \

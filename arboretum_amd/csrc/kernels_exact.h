@@ -132,6 +132,11 @@ struct ExPlan {
 // of 4.6 us less, twice a level.)
 constexpr unsigned kExFoldItems = 512;
 
+// Up to this many pieces of lists (work items x features) the scan filters its places.  Levels 0, 1 and 7 with / without, us, 28
+// features: 400,000 rows (5500) 65, 67, 77 / 74, 66, 84; 1 M (14,000) 163, 170, 160 / 181, 163, 172; 3 M (41,000) 389, 479, 408 /
+// 392, 394, 406; 10.5 M (144,000) 1500, 1829, 1516 / 1432, 1435, 1376.
+constexpr size_t kExFilterItems = 16384;
+
 // grid (L, F), one wave: exclusive scan of `part` over the work items of every node, per feature.
 template <typename T>
 __global__ void __launch_bounds__(64)
@@ -176,10 +181,11 @@ __device__ __forceinline__ bool ExBetter(float og, int ob, float gain, int bin) 
 // node, and the best candidate of the piece, ties to the highest rank.
 // best: [F][max_items].
 // What bounds it: the gains in double precision (21 of 50 us a level at 400,000 rows x 20), then the latency of a
-// chain of loads, scan and barriers, hidden by the workgroups of a CU.  Only the best place of a wave counts, so the
-// gains are computed where ExSides comes near the wave's largest (ExLeastSides): usually at one place or two of 512
-// (43 us; with fewer registers, six waves per SIMD, they spill: 76).
-template <bool PAIR, bool F64, bool PACK>
+// chain of loads, scan and barriers, hidden by the workgroups of a CU.  Only the best place of a wave counts, so with
+// FILTER the gains are computed where ExSides comes near the wave's largest (ExLeastSides): usually at one place or
+// two of 512 (43 us; with fewer registers, six waves per SIMD, they spill: 76).  That shortens a workgroup, and costs
+// arithmetic and registers that a chip full of workgroups has better use for (kExFilterItems).
+template <bool PAIR, bool F64, bool PACK, bool FILTER>
 __global__ void __launch_bounds__(kExThreads)
 k_ex_scan(const ExLists ls, size_t stride, const int *__restrict__ shifts,
           const ExPlan plan, const ExSum *__restrict__ off, int root,
@@ -239,7 +245,7 @@ k_ex_scan(const ExLists ls, size_t stride, const int *__restrict__ shifts,
   const double GT = FromFixed<F64>(t.g, sg);
   const double HT = PAIR ? FromFixed<F64>(t.h, sh) : 0.0;
   const float parent = ExParentGain<PAIR, F64>(GT, HT, t.c, gp);
-  const bool prune = ExPrunes<PAIR>(HT, t.c, gp);
+  const bool prune = FILTER && ExPrunes<PAIR>(HT, t.c, gp);
   // the places worth a look: bit j
   unsigned look = 0;
   float sides[kExPer], most = 0.0f;

@@ -307,3 +307,21 @@ def test_exact_limits_are_errors(arb):
                    arb.DMatrix(bins, y=np.arange(100, dtype=np.float32), quantized=True))
     with pytest.raises(arb.ArboretumError, match="float features"):
         g.grow_tree()
+
+
+@pytest.mark.parametrize("objective,double_precision,F", [(1, True, 111), (0, True, 112), (0, False, 112), (1, True, 112),
+                                                          (1, False, 112)])
+def test_sorted_lists_with_and_without_the_filter(arb, oracle, objective, double_precision, F):
+    # 147 work items a list: 111 lists are the most whose scan filters its places, 112 are scanned without
+    n = 146 * 2048 + 77
+    rng = np.random.default_rng(F + objective)
+    X = rng.integers(0, 6000, size=(n, F)).astype(np.float32)     # more values than a rank histogram holds, and ties
+    s = np.sin(X[:, 0] / 900) + (X[:, 7] > 2500) + 0.0002 * X[:, F - 1]
+    y = (s + 0.3 * rng.normal(size=n)).astype(np.float32) if objective == 0 else (s > np.median(s)).astype(np.float32)
+    cfg = {"objective": objective, "method": 0, "internals": {"double_precision": double_precision, "hist_size": 16,
+                                                              "exact_sort": 1},
+           "tree": {"max_depth": 3, "eta": 0.3, "lambda": 1.0, "min_child_weight": 0.0, "min_leaf_size": 1}}
+    ob = oracle.Booster(X, y=y, config=cfg)
+    data = arb.DMatrix(X, y=y)
+    g = arb.Garden(cfg, data)
+    _same_trees(ob, g, 1)
