@@ -911,9 +911,9 @@ class HipTreeBuilder : public TreeBuilder, private Lane {
 
   // The trees of a round (soft-max: one per class) need nothing of each other, and most kernels of
   // a tree over a few million rows leave much of the chip idle part of the time: they are grown on several
-  // streams, each with level state of its own.  Measured (1 M rows x 100, ten classes, 50 trees):
-  // 23.9 ms on one stream, 19.4 on two, 19.2 on three, 20.2 on four; 20,000 x 20, three classes: 5.4, 5.2,
-  // 3.6, 4.1; 6 M x 20, four classes: 18.9, 19.0, 17.0, 17.2.
+  // streams, each with level state of its own.  Measured on one, two, three and four streams, ms: 1 M rows x 100, ten classes,
+  // 50 trees 19.1, 14.8, 14.3, 14.3; 20,000 x 20, three classes, 30 trees 4.6, 3.4, 3.1, 3.6 (at times 2.5); 6 M x 20, four
+  // classes, 20 trees 13.3, 11.5, 11.6, 11.8.
   static constexpr size_t kLanes = 3;
   // One stream beyond kLaneRows rows (the kernels fill the chip) and with sampled columns: the sampler copies its
   // masks on the stream of the trees.  (Five rounds of that 1 M x 100: 14.1 ms on three streams, 19.0 at a colsample_bytree

@@ -54,7 +54,8 @@ const char *AInitGarden(const char *configuration, VoidPointer *garden);
 const char *AGrowTree(VoidPointer garden, VoidPointer data, const float *grad);
 
 /* arboretum_wrapper.cu:181-193 -> Garden::UpdateByLastTree (garden.cu:627-635):
- * adds the last round's trees to data->y_hat on the host. */
+ * adds the trees of the last boosting round to the predictions `data` carries
+ * (walked on the GPU when one is present, with the bits of the host walk). */
 const char *AAppendLastTree(VoidPointer garden, VoidPointer data);
 
 /* arboretum_wrapper.cu:153-179 -> Garden::GetY (garden.cu:637-641): link
