@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 def arb():
     import arboretum_amd
     if arboretum_amd.device_count() < 1:
-        pytest.fail("no HIP device: the GPU tests must run on the GPU box")
+        pytest.fail("no HIP device: the GPU tests need an MI355X")
     return arboretum_amd
 
 
